@@ -1507,24 +1507,69 @@ __global__ void k_jump_levels(const uint64_t *__restrict__ w, int64_t n, int32_t
     }
 }
 
-// nedge per lane: sum of generated degrees over reached vertices
-__global__ __launch_bounds__(256) void k_ms_nedge(const uint64_t *__restrict__ visited, const uint32_t *__restrict__ gdeg,
-                                                  int64_t n, unsigned long long *__restrict__ out)
+// nedge per lane: sum of generated degrees over reached vertices.  A wave
+// reads 64 vertices' degrees and visited words in coalesced loads (lane =
+// vertex, kNedgeGroups groups in flight).  Nearly all vertices carry one and
+// the same word (a search reaches the giant component whole), so each lane
+// only adds up the degrees under the wave's common word, reduced once at the
+// end; the other words are taken one distinct word at a time, lane = root.
+// Streaming 4 to 12 B per vertex bounds it: 116 us at scale 26, 46 at 24, 4 at
+// 16 (4755, 1146 and 178 us with a vertex per wave step, whose two dependent
+// loads had 12 B in flight, and 8192 workgroups adding to 64 addresses).
+constexpr int kNedgeGroups = 4;
+constexpr int kNedgeGrid = 1024;  // every workgroup ends with one atomic per lane
+
+__global__ __launch_bounds__(kBlock) void k_ms_nedge(const uint64_t *__restrict__ visited,
+                                                     const uint32_t *__restrict__ gdeg, int64_t n,
+                                                     unsigned long long *__restrict__ out)
 {
-    // thread t of a wave handles lane t for a strip of vertices
     const int lane = __lane_id();
-    unsigned long long acc = 0;
-    const int64_t waves = (int64_t)gridDim.x * (blockDim.x / 64);
-    for (int64_t v = blockIdx.x * (int64_t)(blockDim.x / 64) + (threadIdx.x >> 6); v < n; v += waves) {
-        const uint32_t d = gdeg[v];
-        if (d && (visited[v] >> lane & 1)) acc += d;
+    const int64_t waves = (int64_t)gridDim.x * (kBlock / 64);
+    unsigned long long acc = 0;     // root `lane`
+    uint64_t common = 0;            // the wave's common word (wave-uniform)
+    unsigned long long under = 0;   // this lane's degrees under it
+    for (int64_t g0 = (blockIdx.x * (int64_t)(kBlock / 64) + (threadIdx.x >> 6)) * kNedgeGroups; g0 * 64 < n;
+         g0 += waves * kNedgeGroups) {
+        uint32_t d[kNedgeGroups];
+        uint64_t w[kNedgeGroups];
+#pragma unroll
+        for (int k = 0; k < kNedgeGroups; ++k) {
+            const int64_t v = (g0 + k) * 64 + lane;
+            d[k] = v < n ? gdeg[v] : 0u;
+        }
+#pragma unroll
+        for (int k = 0; k < kNedgeGroups; ++k) {
+            const int64_t v = (g0 + k) * 64 + lane;
+            w[k] = d[k] ? visited[v] : 0ull;
+        }
+#pragma unroll
+        for (int k = 0; k < kNedgeGroups; ++k) {
+            uint64_t todo = __ballot(w[k] != 0);
+            if (!common && todo) common = lane_read64(w[k], __ffsll((long long)todo) - 1);
+            if (common && w[k] == common) under += d[k];
+            todo &= __ballot(w[k] != common);
+            while (todo) {
+                const int src = __ffsll((long long)todo) - 1;
+                const uint64_t p = lane_read64(w[k], src);
+                const uint64_t same = __ballot(w[k] == p);
+                todo &= ~same;
+                // degrees are 32-bit, a group's sum of them is not
+                const int64_t sum = (same & (same - 1)) ? g5_wave_sum(w[k] == p ? (int64_t)d[k] : 0)
+                                                        : (int64_t)lane_read(d[k], src);
+                if (p >> lane & 1) acc += (unsigned long long)sum;
+            }
+        }
     }
+    const int64_t total = g5_wave_sum((int64_t)under);
+    if (common >> lane & 1) acc += (unsigned long long)total;
     // the workgroup's 4 waves fold in LDS, then one atomic per lane slot
-    __shared__ unsigned long long s_acc[4][64];
+    __shared__ unsigned long long s_acc[kBlock / 64][64];
     s_acc[threadIdx.x >> 6][lane] = acc;
     __syncthreads();
     if (threadIdx.x < 64) {
-        const unsigned long long t = s_acc[0][lane] + s_acc[1][lane] + s_acc[2][lane] + s_acc[3][lane];
+        unsigned long long t = 0;
+#pragma unroll
+        for (int k = 0; k < kBlock / 64; ++k) t += s_acc[k][lane];
         if (t) atomicAdd(&out[lane], t);
     }
 }
@@ -1538,39 +1583,48 @@ __global__ void k_lane_masks(uint64_t *__restrict__ visited, int64_t n, uint64_t
         visited[i] = (visited[i] | set) & ~clear;
 }
 
-// One thread: root jr[i] (original id) starts lane jr[64 + i] in the frontier
-// the next level reads.  A root without neighbours is only marked visited:
-// its search is complete (and vertices outside the degree bins are never
-// rewritten by the pull kernels, so no frontier bit may be left there).
-// added[0..1] = new frontier vertices and their edges.
-__global__ void k_join(const int64_t *__restrict__ jr, int n, const uint32_t *__restrict__ old2new,
-                       const int64_t *__restrict__ rowptr, uint64_t *__restrict__ visited,
-                       uint64_t *__restrict__ front, uint64_t *__restrict__ act, int32_t *__restrict__ parent,
-                       uint8_t *__restrict__ level, const int64_t *__restrict__ cnt, int64_t *__restrict__ added)
+// One wave, a thread per root: root jr[i] (original id) starts lane jr[64 + i]
+// in the frontier the next level reads (roots may share a vertex, hence the
+// atomics; the one that finds its frontier word empty counts the vertex).  A
+// root without neighbours is only marked visited: its search is complete (and
+// vertices outside the degree bins are never rewritten by the pull kernels, so
+// no frontier bit may be left there).  added[0..1] = new frontier vertices and
+// their edges, added[2 + i] = root i's degree.
+__global__ __launch_bounds__(64) void k_join(const int64_t *__restrict__ jr, int n,
+                                             const uint32_t *__restrict__ old2new,
+                                             const int64_t *__restrict__ rowptr, uint64_t *__restrict__ visited,
+                                             uint64_t *__restrict__ front, uint64_t *__restrict__ act,
+                                             int32_t *__restrict__ parent, uint8_t *__restrict__ level,
+                                             const int64_t *__restrict__ cnt, int64_t *__restrict__ added)
 {
     // the next level finds the root's neighbours with byte cnt[kDepth]
     const uint8_t root_byte = (uint8_t)(cnt[kDepth] - 1);
+    const int i = threadIdx.x;
     int64_t nv = 0, ne = 0;
-    for (int i = 0; i < n; ++i) {
+    if (i < n) {
         const int64_t root = jr[i];
         const int lane = (int)jr[64 + i];
         const int64_t v = old2new[root];
-        const uint64_t bit = 1ull << lane;
+        const unsigned long long bit = 1ull << lane;
         const int64_t deg = rowptr[v + 1] - rowptr[v];
-        visited[v] |= bit;
+        atomicOr((unsigned long long *)&visited[v], bit);
         parent[root * 64 + lane] = (int32_t)root;
         level[root * 64 + lane] = root_byte;
         added[2 + i] = deg;
-        if (deg == 0) continue;
-        if (front[v] == 0) {
-            ++nv;
-            ne += deg;
+        if (deg) {
+            if (atomicOr((unsigned long long *)&front[v], bit) == 0) {
+                nv = 1;
+                ne = deg;
+            }
+            atomicOr((unsigned long long *)&act[v >> 6], 1ull << (v & 63));
         }
-        front[v] |= bit;
-        act[v >> 6] |= 1ull << (v & 63);
     }
-    added[0] = nv;
-    added[1] = ne;
+    nv = g5_wave_sum(nv);
+    ne = g5_wave_sum(ne);
+    if (i == 0) {
+        added[0] = nv;
+        added[1] = ne;
+    }
 }
 
 // Lanes in `mask` leave: per lane the sum of generated degrees over its
@@ -1578,20 +1632,30 @@ __global__ void k_join(const int64_t *__restrict__ jr, int n, const uint32_t *__
 // mix64(orig(v) << 32 | (pred(v) + 1)) mod 2^64, in original ids; then the
 // lanes are freed (visited set everywhere).  A wave takes 64 consecutive
 // vertices (lane = vertex: visited words, ids and degrees in coalesced
-// loads), then reads the parent records of the reached ones (by original
-// id) 8 vertices at a time with lane = root, all 8 loads issued before any
-// is used.
+// loads), then reads the reached ones' parent records (by original id) with
+// the wave split into 64 / 2^kLog vertices of 2^kLog leaving roots each (2^kLog
+// = the leaving lanes, rounded up): a wave step covers one vertex when all 64
+// lanes leave and 64 vertices when one does.  Up to kLeaveGroup steps' loads
+// are issued before any is used.  The records' 64 B sectors bound it: at scale
+// 20 the 7 departures of 96 roots take 28 (one or two lanes) to 124 us (all
+// 64), 359 us together against 593 with a vertex per step whatever leaves.
 constexpr int kLeaveGroup = 8;
+constexpr int kLeaveGrid = 1024;  // every workgroup ends with two atomics per leaving lane
 
-__device__ __forceinline__ uint64_t bcast64(uint64_t x, int l)
+template <int kLog>
+__device__ __forceinline__ uint32_t leave_pick(uint32_t x, int at, int sub)
 {
-    return ((uint64_t)lane_read((uint32_t)(x >> 32), l) << 32) | lane_read((uint32_t)x, l);
+    return kLog == 6 ? lane_read(x, at) : (uint32_t)__shfl((int)x, at + sub, 64);
 }
 
-__global__ __launch_bounds__(256) void k_leave(uint64_t *__restrict__ visited, const int32_t *__restrict__ parent,
-                                               const uint32_t *__restrict__ new2old, const uint32_t *__restrict__ gdeg,
-                                               int64_t n, uint64_t mask, unsigned long long *__restrict__ out)
+template <int kLog>
+__global__ __launch_bounds__(kBlock) void k_leave(uint64_t *__restrict__ visited, const int32_t *__restrict__ parent,
+                                                  const uint32_t *__restrict__ new2old,
+                                                  const uint32_t *__restrict__ gdeg, int64_t n, uint64_t mask,
+                                                  unsigned long long *__restrict__ out)
 {
+    constexpr int K = 1 << kLog, V = 64 / K;              // roots and vertices of a step
+    constexpr int U = K < kLeaveGroup ? K : kLeaveGroup;  // steps in flight
     __shared__ unsigned long long s_ck[64], s_dg[64];
     if (threadIdx.x < 64) {
         s_ck[threadIdx.x] = 0;
@@ -1599,7 +1663,14 @@ __global__ __launch_bounds__(256) void k_leave(uint64_t *__restrict__ visited, c
     }
     __syncthreads();
     const int lane = __lane_id();
-    unsigned long long ck = 0, dg = 0;  // root `lane`'s sums
+    const int sub = lane >> kLog;  // the vertex of a step this lane works on
+    int r = -1;                    // the leaving root it works for, if there are that many
+    {
+        uint64_t m = mask;
+        for (int i = lane & (K - 1); m && i > 0; --i) m &= m - 1;
+        if (m) r = __ffsll((long long)m) - 1;
+    }
+    unsigned long long ck = 0, dg = 0;
     for (int64_t base = blockIdx.x * (int64_t)kBlock + (threadIdx.x & ~63); base < n;
          base += (int64_t)gridDim.x * kBlock) {
         const int64_t v = base + lane;
@@ -1615,30 +1686,34 @@ __global__ __launch_bounds__(256) void k_leave(uint64_t *__restrict__ visited, c
             if (~vis & mask) visited[v] = vis | mask;
         }
         const uint64_t todo = __ballot(reach != 0);
-        for (int j0 = 0; j0 < 64; j0 += kLeaveGroup) {
-            if (((todo >> j0) & ((1ull << kLeaveGroup) - 1)) == 0) continue;
-            uint64_t rj[kLeaveGroup];
-            uint32_t oj[kLeaveGroup];
-            int32_t pj[kLeaveGroup];
+        for (int j0 = 0; j0 < 64; j0 += U * V) {
+            // U * V vertices; U * V == 64 only for the smallest kLog
+            constexpr uint64_t kSpan = U * V == 64 ? ~0ull : (1ull << (U * V & 63)) - 1;
+            if (((todo >> j0) & kSpan) == 0) continue;
+            uint32_t oj[U], dj[U];
+            int32_t pj[U];
+            bool hit[U];
 #pragma unroll
-            for (int k = 0; k < kLeaveGroup; ++k) {
-                rj[k] = bcast64(reach, j0 + k);
-                oj[k] = lane_read(o, j0 + k);
-                pj[k] = (rj[k] >> lane & 1) ? parent[(int64_t)oj[k] * 64 + lane] : 0;
+            for (int k = 0; k < U; ++k) {
+                const int at = j0 + k * V;
+                const uint64_t rj = (uint64_t)leave_pick<kLog>((uint32_t)(reach >> 32), at, sub) << 32 |
+                                    leave_pick<kLog>((uint32_t)reach, at, sub);
+                oj[k] = leave_pick<kLog>(o, at, sub);
+                dj[k] = leave_pick<kLog>(d, at, sub);
+                hit[k] = r >= 0 && (rj >> (r & 63) & 1);
+                pj[k] = hit[k] ? parent[(int64_t)oj[k] * 64 + r] : 0;
             }
 #pragma unroll
-            for (int k = 0; k < kLeaveGroup; ++k) {
-                const uint32_t dj = lane_read(d, j0 + k);
-                if (rj[k] >> lane & 1) {
+            for (int k = 0; k < U; ++k)
+                if (hit[k]) {
                     ck += g5_mix64(((uint64_t)oj[k] << 32) | (uint32_t)(pj[k] + 1));
-                    dg += dj;
+                    dg += dj[k];
                 }
-            }
         }
     }
-    if (mask >> lane & 1) {
-        atomicAdd(&s_ck[lane], ck);
-        atomicAdd(&s_dg[lane], dg);
+    if (r >= 0) {
+        atomicAdd(&s_ck[r], ck);
+        atomicAdd(&s_dg[r], dg);
     }
     __syncthreads();
     if (threadIdx.x < 64 && (mask >> threadIdx.x & 1)) {
@@ -2359,7 +2434,7 @@ extern "C" int g5_msbfs_join(g5_msbfs *m, const int64_t *roots, const int *lanes
     uint64_t *act = m->d_act + (m->p == 0 ? 0 : m->n / 64);
     G5_HIP(hipMemcpyAsync(m->d_join, h, sizeof(h), hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL(k_lane_masks, g5::grid_for(m->n, 256, 16384), 256, 0, s, m->d_visited, m->n, 0ull, mask);
-    hipLaunchKernelGGL(k_join, 1, 1, 0, s, (const int64_t *)m->d_join, n, (const uint32_t *)m->rl.old2new,
+    hipLaunchKernelGGL(k_join, 1, 64, 0, s, (const int64_t *)m->d_join, n, (const uint32_t *)m->rl.old2new,
                        (const int64_t *)m->rl.rowptr, m->d_visited, front, act, m->d_parent, m->d_level,
                        (const int64_t *)m->d_cnt, m->d_join + 128);
     G5_HIP(hipGetLastError());
@@ -2416,7 +2491,16 @@ extern "C" int g5_msbfs_leave(g5_msbfs *m, uint64_t lanes, int64_t *nedge, uint6
     if (!lanes) return G5_OK;
     hipStream_t s = m->s;
     G5_HIP(g5::fill_u64((uint64_t *)m->d_sums, 128, 0, s));
-    hipLaunchKernelGGL(k_leave, g5::grid_for(m->n, kBlock, 4096), kBlock, 0, s, m->d_visited,
+    int lg = 0;  // 2^lg >= the leaving lanes
+    while ((1 << lg) < __builtin_popcountll(lanes)) ++lg;
+    auto leave = lg == 0   ? k_leave<0>
+                 : lg == 1 ? k_leave<1>
+                 : lg == 2 ? k_leave<2>
+                 : lg == 3 ? k_leave<3>
+                 : lg == 4 ? k_leave<4>
+                 : lg == 5 ? k_leave<5>
+                           : k_leave<6>;
+    hipLaunchKernelGGL(leave, g5::grid_for(m->n, kBlock, kLeaveGrid), kBlock, 0, s, m->d_visited,
                        (const int32_t *)m->d_parent, (const uint32_t *)m->rl.new2old, (const uint32_t *)m->rl.gdeg,
                        m->n, lanes, m->d_sums);
     G5_HIP(hipGetLastError());
@@ -2578,20 +2662,16 @@ extern "C" int g5_msbfs_times(g5_msbfs *m, float *search_ms, float *finalize_ms)
 extern "C" int g5_msbfs_nedge(g5_msbfs *m, int64_t *nedge)
 {
     G5_REQUIRE(m && nedge, G5_E_ARG, "g5_msbfs_nedge: null argument");
-    unsigned long long *d = nullptr;
-    G5_HIP(hipMalloc(&d, 64 * 8));
-    hipError_t e = hipMemsetAsync(d, 0, 64 * 8, m->s);
-    if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_ms_nedge, g5::grid_for(m->n / 4 + 1, 1, 8192), 256, 0, m->s,
-                           (const uint64_t *)m->d_visited, (const uint32_t *)m->rl.gdeg, m->n, d);
-        e = hipGetLastError();
-    }
-    unsigned long long h[64];
-    if (e == hipSuccess) e = hipMemcpyAsync(h, d, 64 * 8, hipMemcpyDeviceToHost, m->s);
-    if (e == hipSuccess) e = hipStreamSynchronize(m->s);
-    (void)hipFree(d);
-    G5_HIP(e);
-    for (int r = 0; r < m->nroots; ++r) nedge[r] = (int64_t)(h[internal_lane(m, r)] / 2);
+    G5_HIP(g5::fill_u64((uint64_t *)m->d_sums, 64, 0, m->s));  // free between calls
+    hipLaunchKernelGGL(k_ms_nedge, g5::grid_for(m->n, kBlock * kNedgeGroups, kNedgeGrid), kBlock, 0, m->s,
+                       (const uint64_t *)m->d_visited, (const uint32_t *)m->rl.gdeg, m->n, m->d_sums);
+    G5_HIP(hipGetLastError());
+    // h_cnt is read by a level right after its own copy, so it is free too
+    static_assert(kHostSlots >= 64, "the lanes' sums do not fit the pinned slots");
+    G5_HIP(hipMemcpyAsync(m->h_cnt, m->d_sums, 64 * 8, hipMemcpyDeviceToHost, m->s));
+    G5_HIP(hipStreamSynchronize(m->s));
+    const int64_t *h = m->h_cnt;
+    for (int r = 0; r < m->nroots; ++r) nedge[r] = (int64_t)((unsigned long long)h[internal_lane(m, r)] / 2);
     return G5_OK;
 }
 

@@ -1,0 +1,87 @@
+"""The passes that sum over a lane's reached vertices (g5_msbfs_nedge and
+g5_msbfs_leave) where neighbouring vertices carry different lane sets: many
+small components, so that a wave meets up to 64 distinct words, degrees whose
+sums pass 32 bits, and every way of splitting a wave over the leaving lanes."""
+import numpy as np
+import pytest
+
+import gpugraph500_amd as g5
+import oracle_lib as O
+from test_gpu_continuous import checksum
+
+pytestmark = pytest.mark.gpu
+
+
+def rings(n, sizes, seed):
+    """n vertices in rings of the given sizes (repeated until n is full, the
+    rest edgeless), ids shuffled; gdeg up to 2^32 - 1."""
+    rng = np.random.default_rng(seed)
+    ids = rng.permutation(n)
+    adj = [[] for _ in range(n)]
+    at, i = 0, 0
+    comps = []
+    while at + sizes[i % len(sizes)] <= n:
+        c = ids[at:at + sizes[i % len(sizes)]]
+        at += len(c)
+        i += 1
+        comps.append(c)
+        for a, b in zip(c, np.roll(c, 1)):
+            if a != b:
+                adj[a].append(b)
+                adj[b].append(a)
+    rows = [np.unique(np.array(a, np.int64)) for a in adj]
+    rowptr = np.concatenate([[0], np.cumsum([len(r) for r in rows])])
+    cols = np.concatenate(rows).astype(np.uint32)
+    gdeg = rng.integers(1, 1 << 32, n, dtype=np.int64)
+    gdeg[rng.random(n) < 0.1] = 0
+    return rowptr, cols, gdeg, comps
+
+
+@pytest.mark.parametrize("n,sizes,lanes", [(64, (2,), 32), (64, (3, 5), 1), (320, (7, 2, 11), 64),
+                                           (4096, (50, 64, 3), 33), (70016, (1000, 1500), 64), (70016, (70000,), 5)])
+def test_sums_over_small_components(n, sizes, lanes):
+    rowptr, cols, gdeg, comps = rings(n, sizes, n + lanes)
+    g = g5.Graph.upload(rowptr, cols, n, gdeg=gdeg)
+    m = g5.MSBFS(g)
+    rng = np.random.default_rng(1)
+    roots = [int(comps[i % len(comps)][rng.integers(len(comps[i % len(comps)]))]) for i in range(lanes)]
+    member = {int(v): i for i, c in enumerate(comps) for v in c}
+    want = [int(gdeg[comps[member[r]]].astype(object).sum()) // 2 for r in roots]
+    m.run(roots)
+    assert m.nedge().tolist() == want
+
+    # the same lanes in continuous mode, leaving in groups of 1, 2, 3, 5, ...
+    m.open()
+    m.join(roots, list(range(lanes)))
+    for _ in range(40000):
+        live, _ = m.step()
+        if not live:
+            break
+    preds = [m.result(lane)[0] for lane in range(lanes)] if n <= 4096 else None
+    left = list(rng.permutation(lanes))
+    for k in (1, 2, 3, 5, 17, 64):
+        group, left = left[:k], left[k:]
+        if not group:
+            break
+        ne, ck = m.leave(sum(1 << int(x) for x in group))
+        for x in group:
+            assert int(ne[x]) == want[x], f"lane {x}"
+            if preds is not None:
+                assert int(ck[x]) == checksum(preds[x]), f"lane {x}"
+
+
+def test_leaving_lanes_match_the_oracle():
+    ref = O.build_csr(O.kronecker_edges(11))
+    g = g5.Graph.upload(ref.rowptr, ref.cols, ref.n_rows, gdeg=ref.gdeg)
+    m = g5.MSBFS(g)
+    roots = [int(r) for r in O.select_roots(ref, 1 << 11)][:64]
+    for k in (1, 2, 4, 7, 9, 16, 31, 32, 64):
+        m.open()
+        lanes = [(5 * i + 3) % 64 for i in range(k)]  # spread over the word
+        m.join(roots[:k], lanes)
+        while m.step()[0]:
+            pass
+        ne, ck = m.leave(sum(1 << x for x in lanes))
+        for r, x in zip(roots, lanes):
+            pred, lev, _ = O.bfs_bin(ref, r)
+            assert int(ne[x]) == O.nedge(ref, lev) and int(ck[x]) == checksum(pred)
