@@ -13,19 +13,17 @@ struct S4Codec {
     int64_t cap = 0;               // values
     uint8_t *d_base = nullptr;     // the buffer holding every device array below
     bool owned = false;            // d_base and h_meta were allocated by reserve()
-    int64_t *d_words = nullptr;    // per-miniblock word counts -> prefix, nblk + 1
-    int64_t *d_scan = nullptr;     // int64 scan scratch
-    int64_t *d_off = nullptr;      // decode: per-miniblock data offset
-    uint32_t *d_carry = nullptr;   // decode: per-miniblock carry records (5 words)
-    uint32_t *d_carry_scan = nullptr;
+    uint8_t *d_width = nullptr;    // encode: per-miniblock widths
+    int64_t *d_total = nullptr;    // encode: per-workgroup word totals
+    uint8_t *d_rec = nullptr;      // decode: per-workgroup running-sum records
     int64_t *d_grp = nullptr;      // decode: group header positions
-    int32_t *d_nxt = nullptr;      // decode: next group start per candidate start (4 + 4i)
-    int32_t *d_jmp = nullptr, *d_jtmp = nullptr;  // decode: 32-step jumps (pointer doubling)
-    int32_t *d_anchor = nullptr;   // decode: every 32nd group start
-    int64_t ncand_cap = 0;
+    int32_t *d_anchor = nullptr;   // decode: every 8th group start
+    int32_t *d_hop[6] = {};        // decode: group starts 8, 64, ... groups after each candidate start (4 + 4i)
+    int hop_cap = 0;               // tables there are
+    int64_t ncand_cap = 0;         // candidate starts a table holds
     int64_t *d_meta = nullptr;     // small device record
-    int64_t *d_nw = nullptr;       // [0] the last encode's stream length, [1] decode's input length
-    int64_t *h_meta = nullptr;     // pinned mirror
+    int64_t *d_nw = nullptr;       // the last encode's stream length
+    int64_t *h_meta = nullptr;     // owned: pinned, the kernels write to it
     // accounting of encode() and decode() (g5_exchange_profile), when set
     ExchangeTimer *acct = nullptr;
 
@@ -55,11 +53,9 @@ struct S4Codec {
     int roundtrip_result(size_t *nwords, const char *who);
 
 private:
-    int encode_launch(const uint32_t *d_in, int64_t n, uint32_t *d_out, hipStream_t s);
-    int search_launch(const uint32_t *d_in, const int64_t *nwp, int64_t words_bound, int64_t cap_values,
-                      bool serial, hipStream_t s);
-    int unpack_launch(const uint32_t *d_in, const int64_t *nwp, int64_t L, int64_t cap_values, uint32_t *d_out,
-                      int64_t *d_flag, hipStream_t s);
+    int encode_launch(const uint32_t *d_in, int64_t n, uint32_t *d_out, int64_t *host, hipStream_t s);
+    int decode_launch(const uint32_t *d_in, const int64_t *nwp, int64_t nwv, int64_t words_bound, int64_t cap_values,
+                      uint32_t *d_out, int64_t n_expect, int64_t *d_flag, int64_t *host, hipStream_t s);
 };
 
 }  // namespace g5

@@ -387,9 +387,7 @@ int g5_vreduce_min_pred_list(const int64_t *const *d_preds, int k, int64_t n, in
  * kernels, their algorithmic bytes and the calls: OR (k+1)*8*n_words,
  * min-pred (k+1)*8*n, encode 4n + 4*csize, decode 4*csize + 4n.  A
  * combine's time is its kernel's, from start to end; the codec's runs from
- * its first kernel's launch to its last kernel's end (launch gaps included),
- * and a decode's excludes the host round trip between its header search and
- * its unpacking. */
+ * its first kernel's launch to its last kernel's end (launch gaps included). */
 enum { G5_UNIT_OR = 0, G5_UNIT_MIN_PRED = 1, G5_UNIT_ENCODE = 2, G5_UNIT_DECODE = 3, G5_UNIT_COUNT = 4 };
 int g5_exchange_profile(int enable);
 int g5_exchange_stats(int unit, double *ms, double *bytes, int64_t *calls);
