@@ -16,12 +16,14 @@
 // Queues are born sorted and unique, so the reference's thrust::sort and host
 // unique_copy (cuda_bfs.cu:380-475) have no counterpart.
 //
-// g5_bfs_run (1x1 block, resident) also runs dense levels bottom-up
-// (k_bottom_up): each unvisited vertex scans its sorted neighbour list and
-// stops at the first frontier vertex, which is again the minimum-id frontier
-// neighbour, so both directions give identical parents and levels.  It
-// reads only the counters from the host per level, and builds the sorted
-// queue of step 4 only for a top-down level or the codec.
+// g5_bfs_run (1x1 block, resident) also runs dense levels bottom-up: each
+// unvisited vertex scans its sorted neighbour list and stops at the first
+// frontier vertex, which is again the minimum-id frontier neighbour, so both
+// directions give identical parents and levels.  Its levels are one kernel
+// each and decided on the device (k_level); with the codec, with accounting or
+// with a forced direction the host drives them from the level's counters
+// (k_expand or k_bottom_up, k_commit, and the sorted queue of step 4 where a
+// top-down level or the codec needs it).
 #include <algorithm>
 
 #include "g5_codec.hpp"
@@ -51,11 +53,6 @@ enum Cnt {
 // alpha 20: 3.32 ms per root at scale 26 against 3.51 ms with 14 and 3.94
 // with 8 (scale 22: within 1 %); beta barely matters (12..96: within 0.5 %)
 constexpr int64_t kAlpha = 20, kBeta = 24;
-// frontier bits gathered ahead per lane in the bottom-up scan: 4 on graphs
-// below 2^25 vertices, 2 above, where each gather past the first hit more
-// likely misses the caches (measured at scales 22, 24 and 26; 1 and 8 were
-// slower everywhere)
-constexpr int64_t kBuLarge = (int64_t)1 << 25;
 
 }  // namespace
 
@@ -96,6 +93,14 @@ struct g5_bfs {
     // g5_bfs_expand_bottom_up
     uint64_t *d_inbits = nullptr;
     bool inbits_valid = false;
+    // g5_bfs_run's levels on the device (k_level): a third frontier bitmap,
+    // the two levels' queues and their
+    // prefixes (kGroups times gcap entries each) and the control record
+    uint64_t *d_third = nullptr;
+    uint32_t *d_gq[2] = {nullptr, nullptr};
+    int64_t *d_goff[2] = {nullptr, nullptr};
+    int64_t gcap = 0;
+    struct LevelCtl *d_ctl = nullptr;
 };
 
 namespace {
@@ -219,48 +224,130 @@ __global__ __launch_bounds__(256) void k_commit(uint64_t *__restrict__ out, uint
     }
 }
 
-// Bottom-up level of the 1x1 search: every unvisited vertex scans its
-// neighbours in ascending id order and stops at the first one whose frontier
-// bit is set -- its minimum-id frontier neighbour, the parent CPUBFS_bin's
-// ascending scan keeps (cpu_2d/cpubfs_bin.cpp:150-173).  One wavefront per
-// 64-vertex bitmap word (lane = vertex), so the next-frontier word is the
-// wave's ballot and needs no atomics.  kBuUnroll frontier bits are gathered
-// before any is tested, to keep several loads in flight per lane.
-template <int kBuUnroll>
+// Bottom-up scans: every unvisited vertex looks through its neighbours in
+// ascending id order for the first one whose frontier bit is set -- its
+// minimum-id frontier neighbour, the parent CPUBFS_bin's ascending scan keeps
+// (cpu_2d/cpubfs_bin.cpp:150-173).  One wavefront per 64-vertex bitmap word
+// (lane = vertex), so the next-frontier word is the wave's ballot and needs no
+// atomics.
+//
+// A lane looks at its own row's first kBuFirst neighbours, where a dense
+// level's scans end.  The rows still open then share the wave: r of them get
+// 64 / r lanes each (a power of two), which take that many consecutive
+// neighbours kBuSteps times over, until all rows have ended.  A lane alone on a
+// long row is a chain of dependent loads with the other lanes idle, and its
+// row's lines are gone from the caches before the next step reads on.
+// Measured over a search's three bottom-up levels, commit included: 143 us at
+// scale 22 (lane per row to its end: 455), 500 at 24, 3.2 ms at 26 (3.5).
+// The first level's random frontier bits bound it, about one address per
+// clock and CU, then the row starts' lines.  kBuFirst 2 and 4: 1.02 and 1.13
+// times that at scale 24; kBuSteps 2: 1.07.
+constexpr int kBuFirst = 1;
+constexpr int kBuSteps = 1;
+struct BuScan {  // one wave's
+    int64_t at[64], end[64];
+    uint32_t owner[64], par[64];
+};
+
+__device__ __forceinline__ void bu_wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The first frontier neighbour in [j, e) of each lane's row (none: kNoParent;
+// j == e for lanes without a row); j becomes the end of what was looked at.
+__device__ __forceinline__ uint32_t bu_scan(int64_t &j, int64_t e, const uint32_t *__restrict__ cols,
+                                            const uint64_t *__restrict__ front, BuScan &s, int lane)
+{
+    uint32_t par = kNoParent;
+    {
+        uint32_t u[kBuFirst];
+        uint64_t fw[kBuFirst];
+#pragma unroll
+        for (int k = 0; k < kBuFirst; ++k) u[k] = j + k < e ? cols[j + k] : 0u;
+#pragma unroll
+        for (int k = 0; k < kBuFirst; ++k) fw[k] = j + k < e ? front[u[k] >> 6] : 0ull;
+#pragma unroll
+        for (int k = kBuFirst - 1; k >= 0; --k)
+            if (fw[k] >> (u[k] & 63) & 1) par = u[k];
+        j = min(e, j + kBuFirst);
+    }
+    uint64_t open = __ballot(par == kNoParent && j < e);
+    while (open) {
+        const int r = __popcll(open);
+        const int lg = r > 1 ? 6 - (32 - __clz(r - 1)) : 6;  // log2 of the lanes per row
+        const bool mine = open >> lane & 1;
+        if (mine) {
+            const int rank = __popcll(open & ((1ull << lane) - 1));
+            s.at[rank] = j;
+            s.end[rank] = e;
+            s.owner[rank] = lane;
+            s.par[lane] = kNoParent;
+        }
+        bu_wave_sync();
+        const int row = lane >> lg;
+        int64_t at = 0, end = 0;
+        uint32_t owner = 0;
+        if (row < r) {
+            at = s.at[row] + (lane & ((1 << lg) - 1));
+            end = s.end[row];
+            owner = s.owner[row];
+        }
+        uint32_t u[kBuSteps];
+        uint64_t fw[kBuSteps];
+#pragma unroll
+        for (int k = 0; k < kBuSteps; ++k) u[k] = at + (k << lg) < end ? cols[at + (k << lg)] : 0u;
+#pragma unroll
+        for (int k = 0; k < kBuSteps; ++k) fw[k] = at + (k << lg) < end ? front[u[k] >> 6] : 0ull;
+        // the row's first hit: the lowest lane of the earliest step
+        const uint64_t below = ((1ull << lane) - 1) & ~((1ull << (row << lg)) - 1);
+        const uint64_t group = lg == 6 ? ~0ull : ((1ull << (1 << lg)) - 1) << ((row << lg) & 63);
+        bool over = false;  // an earlier step hit
+#pragma unroll
+        for (int k = 0; k < kBuSteps; ++k) {
+            const bool hit = fw[k] >> (u[k] & 63) & 1;
+            const uint64_t hits = __ballot(hit);
+            if (hit && !over && !(hits & below)) s.par[owner] = u[k];
+            over = over || (hits & group);
+        }
+        bu_wave_sync();
+        if (mine) {
+            par = s.par[lane];
+            j = min(e, j + (kBuSteps << lg));
+        }
+        open = __ballot(mine && par == kNoParent && j < e);
+    }
+    return par;
+}
+
 __global__ __launch_bounds__(256) void k_bottom_up(const int64_t *__restrict__ rowptr,
                                                    const uint32_t *__restrict__ cols,
                                                    const uint64_t *__restrict__ visited,
                                                    const uint64_t *__restrict__ front, uint64_t *__restrict__ next,
                                                    uint32_t *__restrict__ parent, int64_t wc, int64_t *__restrict__ cnt)
 {
+    __shared__ BuScan s_scan[4];
     const int lane = __lane_id();
     int64_t nedges = 0, nverts = 0, newdeg = 0;
     for (int64_t w = blockIdx.x * 4 + (threadIdx.x >> 6); w < wc; w += (int64_t)gridDim.x * 4) {
         const uint64_t vis = visited[w];
-        bool hit = false;
+        const int64_t v = w * 64 + lane;
+        int64_t b = 0, e = 0;
         if (!(vis >> lane & 1)) {
-            const int64_t v = w * 64 + lane;
-            const int64_t b = rowptr[v], e = rowptr[v + 1];
-            int64_t j = b;
-            while (j < e && !hit) {
-                uint32_t u[kBuUnroll];
-                uint64_t fw[kBuUnroll];
-#pragma unroll
-                for (int k = 0; k < kBuUnroll; ++k) u[k] = j + k < e ? cols[j + k] : 0u;
-#pragma unroll
-                for (int k = 0; k < kBuUnroll; ++k) fw[k] = j + k < e ? front[u[k] >> 6] : 0ull;
-#pragma unroll
-                for (int k = 0; k < kBuUnroll; ++k)
-                    if (!hit && (fw[k] >> (u[k] & 63) & 1)) {
-                        hit = true;
-                        parent[v] = u[k];
-                    }
-                j += kBuUnroll;
-            }
-            nedges += min(j, e) - b;
+            b = rowptr[v];
+            e = rowptr[v + 1];
             ++nverts;
-            if (hit) newdeg += e - b;
         }
+        int64_t j = b;
+        const uint32_t par = bu_scan(j, e, cols, front, s_scan[threadIdx.x >> 6], lane);
+        const bool hit = par != kNoParent;
+        if (hit) {
+            parent[v] = par;
+            newdeg += e - b;
+        }
+        nedges += j - b;
         const uint64_t bits = __ballot(hit);
         if (lane == 0) next[w] = bits;
     }
@@ -307,13 +394,24 @@ __global__ void k_result(const uint32_t *__restrict__ parent, int64_t n, int64_t
     }
 }
 
-__global__ void k_nedge(const uint32_t *__restrict__ gdeg, const int32_t *__restrict__ level, int64_t n,
-                        int64_t *__restrict__ dst)
+// grids that end in one atomic per workgroup: same-address atomics take their
+// turns (4096 of them were 40 of k_nedge's 54 us at scale 22)
+constexpr int kSumGrid = 1024;
+
+// n is a multiple of 64
+__global__ __launch_bounds__(256) void k_nedge(const uint32_t *__restrict__ gdeg, const int32_t *__restrict__ level,
+                                               int64_t n, int64_t *__restrict__ dst)
 {
+    const uint4 *g4 = (const uint4 *)gdeg;
+    const int4 *l4 = (const int4 *)level;
     int64_t c = 0;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x)
-        if (level[i] >= 0) c += gdeg[i];
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n / 4;
+         i += (int64_t)gridDim.x * blockDim.x) {
+        const int4 l = l4[i];
+        const uint4 g = g4[i];
+        c += (int64_t)(l.x >= 0 ? g.x : 0u) + (l.y >= 0 ? g.y : 0u) + (int64_t)(l.z >= 0 ? g.z : 0u) +
+             (l.w >= 0 ? g.w : 0u);
+    }
     c = g5_block_sum256(c);
     if (threadIdx.x == 0 && c) atomicAdd((unsigned long long *)dst, (unsigned long long)c);
 }
@@ -421,6 +519,17 @@ __global__ void k_isolated(const int64_t *__restrict__ rowptr, int64_t wc, uint6
     }
 }
 
+// d_isolated, at the first search of a resident graph
+int find_isolated(g5_bfs *b)
+{
+    if (b->d_isolated) return G5_OK;
+    G5_HIP(hipMalloc(&b->d_isolated, (size_t)(b->wc ? b->wc : 1) * 8));
+    hipLaunchKernelGGL(k_isolated, g5::grid_for(b->wc * 64, 256, 4096), 256, 0, b->s,
+                       (const int64_t *)b->g->d_rowptr, b->wc, b->d_isolated);
+    G5_HIP(hipGetLastError());
+    return G5_OK;
+}
+
 // isolated: start with the block's edgeless vertices visited (g5_bfs_run on a
 // diagonal block: they are never reached, so results do not change)
 int reset_search(g5_bfs *b, int64_t root, bool isolated = false)
@@ -431,12 +540,6 @@ int reset_search(g5_bfs *b, int64_t root, bool isolated = false)
     const int64_t root_row = (root >= 0 && rr >= 0 && rr < g->n_rows) ? rr : -1;
     const int64_t root_col = (root >= 0 && rc >= 0 && rc < g->n_cols) ? rc : -1;
     if (isolated) {
-        if (!b->d_isolated) {
-            G5_HIP(hipMalloc(&b->d_isolated, (size_t)(b->wc ? b->wc : 1) * 8));
-            hipLaunchKernelGGL(k_isolated, g5::grid_for(b->wc * 64, 256, 4096), 256, 0, s,
-                               (const int64_t *)g->d_rowptr, b->wc, b->d_isolated);
-            G5_HIP(hipGetLastError());
-        }
         G5_HIP(hipMemcpyAsync(b->d_visited, b->d_isolated, (size_t)b->wc * 8, hipMemcpyDeviceToDevice, s));
     } else {
         G5_HIP(g5::fill_u64(b->d_visited, b->wc, 0, s));
@@ -451,6 +554,478 @@ int reset_search(g5_bfs *b, int64_t root, bool isolated = false)
     b->root = root;
     b->depth = 0;
     b->qlen = root_row >= 0 ? 1 : 0;
+    b->inbits_valid = false;
+    return G5_OK;
+}
+
+// ---- the resident search, decided on the device ----
+//
+// g5_bfs_run's levels as one kernel each, with no word from the host between
+// them: every workgroup reads the level before's totals, takes the same
+// decision (done, top-down or bottom-up), and does its share.  A level costs
+// one launch (about 10 before, and a host round trip); the host looks only
+// after a batch of levels.  A whole search with its maps and count: 399 -> 133
+// us at scale 16, 3.9-4.3 -> 3.3-3.6 ms at 26.
+//
+// Three frontier bitmaps rotate: a level reads the frontier, writes the next
+// one and clears the third.  Visited lags one level behind: the frontier is
+// merged into it by the level that expands it, so "visited" below is always
+// visited | frontier.  Both directions collect the new vertices per workgroup
+// in LDS and append them, with their degree prefix, to one of the next level's
+// kGroups queues; one packed atomic (vertices, edges) reserves both and is the
+// queue's total.  (Returning atomics on one address take 12 ns each: 100 us of
+// a level whose 8192 workgroups all append to one queue.)  The queues
+// are in no order, which no result depends on.  They are only complete
+// if the next level may run top-down: a workgroup whose buffer overflows (a
+// dense bottom-up level), a full queue, or a top-down level that has already
+// found more edges than the switch allows leave it out, and the next level
+// runs bottom-up.  From then on the level's totals need not be exact (the next
+// level's direction is settled, and some vertex was found), so workgroups that
+// see it collect nothing any more.
+constexpr int kLvBlock = 256;
+constexpr int kLvGrid = 4096;   // two rounds of 8 workgroups per CU, which differ in what they take
+constexpr int kLvTile = 1024;   // edges of a top-down tile
+constexpr int kLvSrc = 512;     // sources of a tile that are staged in LDS
+constexpr int kLvBuf = 1024;    // new vertices a workgroup keeps
+constexpr int kLvMem = 4096;    // words of LDS: the buffer and staged sources, or the scans' rows
+constexpr int kEdgeBits = 34;   // of a packed total; the vertices take the rest
+constexpr uint64_t kEdgeMask = (1ull << kEdgeBits) - 1;
+constexpr int kGroups = 16;
+constexpr int kMinQueue = 4096;  // entries of a group's queue at least
+
+enum Mode { kTopDown = 0, kBottomUp = 1, kDone = 2 };
+
+}  // namespace
+
+struct LevelCtl {
+    // written by level d at [d % 2], read by level d + 1
+    struct {
+        int64_t mode, m_u;
+    } lv[2];
+    int64_t pad[12];
+    // level d at [d % 3], every word in a line of its own: the groups' packed
+    // new vertices and edges, and whether the queues are incomplete (a hint
+    // within the level, so it is read and written through the XCD's own L2)
+    struct {
+        unsigned long long x;
+        unsigned long long pad[15];
+    } tot[3][16], lost[3];
+};
+
+namespace {
+
+struct LevelArgs {
+    const int64_t *rowptr;
+    const uint32_t *cols;
+    uint64_t *visited;
+    uint32_t *parent;
+    int32_t *level;
+    // this level's frontier, the next one's, and the bitmap to clear; its
+    // queue and prefix, and the next one's.  The host picks them (an index
+    // into arrays here would make every access to them a flat one)
+    uint64_t *front, *next, *third;
+    uint32_t *q, *qn;
+    int64_t *qoff, *qoffn;
+    LevelCtl *ctl;
+    int64_t *host;
+    int64_t n, wc, nnz, alpha, beta;
+    int64_t gcap;  // entries of a group's queue
+};
+
+// what a level's workgroups know of the frontier's queues
+struct Groups {
+    int64_t n[kGroups], edges[kGroups], tile0[kGroups + 1];
+};
+
+// The search's state at its start: visited = the edgeless vertices, the root
+// the only frontier vertex; one kernel.
+__global__ __launch_bounds__(kLvBlock) void k_reset(LevelArgs a, const uint64_t *__restrict__ isolated, int64_t root)
+{
+    const int64_t t = blockIdx.x * (int64_t)kLvBlock + threadIdx.x, stride = (int64_t)gridDim.x * kLvBlock;
+    for (int64_t w = t; w < a.wc; w += stride) {
+        a.visited[w] = isolated[w];
+        a.front[w] = w == root >> 6 ? 1ull << (root & 63) : 0ull;
+        a.next[w] = 0;
+        a.third[w] = 0;
+    }
+    // n is a multiple of 64
+    uint4 *p4 = (uint4 *)a.parent, *l4 = (uint4 *)a.level;
+    for (int64_t i = t; i < a.n / 4; i += stride) {
+        uint4 p = {kNoParent, kNoParent, kNoParent, kNoParent}, l = {~0u, ~0u, ~0u, ~0u};
+        if (i == root >> 2) {
+            (&p.x)[root & 3] = kRootMark;
+            (&l.x)[root & 3] = 0;
+        }
+        p4[i] = p;
+        l4[i] = l;
+    }
+    if (blockIdx.x == 0) {
+        for (int i = threadIdx.x; i < (int)(sizeof(LevelCtl) / 8); i += kLvBlock) ((uint64_t *)a.ctl)[i] = 0;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            static_assert(kGroups <= 16, "totals");
+            a.q[0] = (uint32_t)root;
+            a.qoff[0] = 0;
+            a.ctl->lv[1].mode = kTopDown;
+            a.ctl->lv[1].m_u = a.nnz;
+            a.ctl->tot[2][0].x = 1ull << kEdgeBits | (unsigned long long)(a.rowptr[root + 1] - a.rowptr[root]);
+        }
+    }
+}
+
+// last s in [lo, hi] with qoff[s] <= e, by a whole wave, 64 probes a round
+__device__ __forceinline__ int64_t wave_src_of(const int64_t *__restrict__ qoff, int64_t lo, int64_t hi, int64_t e)
+{
+    ++hi;
+    while (hi - lo > 1) {
+        const int64_t step = (hi - lo + 63) / 64, at = lo + step * __lane_id();
+        const uint64_t le = __ballot(at < hi && qoff[at] <= e);  // lane 0's always is
+        lo += step * (63 - __clzll((long long)le));
+        hi = min(hi, lo + step);
+    }
+    return lo;
+}
+
+// whether the level's queue is known to be incomplete
+__device__ __forceinline__ bool lost_yet(const LevelArgs &a, int d)
+{
+    return __hip_atomic_load(&a.ctl->lost[d % 3].x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != 0;
+}
+__device__ __forceinline__ void set_lost(const LevelArgs &a, int d)
+{
+    __hip_atomic_store(&a.ctl->lost[d % 3].x, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// The workgroup's new vertices s_v[0 .. cnt) of degrees s_d go to the queue
+// (all threads call it, after a barrier; s_v is free again after the next one)
+__device__ __forceinline__ void level_flush(const LevelArgs &a, int d, int64_t limit, int cnt, const uint32_t *s_v,
+                                            const uint32_t *s_d)
+{
+    __shared__ int64_t s_wave[kLvBlock / 64];
+    __shared__ unsigned long long s_at;
+    const int per = (cnt + kLvBlock - 1) / kLvBlock, i0 = threadIdx.x * per, i1 = min(cnt, i0 + per);
+    int64_t sum = 0;
+    for (int i = i0; i < i1; ++i) sum += s_d[i];
+    const int64_t inc = g5_wave_incl_scan(sum);
+    if ((threadIdx.x & 63) == 63) s_wave[threadIdx.x >> 6] = inc;
+    __syncthreads();
+    int64_t before = inc - sum, all = 0;
+    for (int w = 0; w < kLvBlock / 64; ++w) {
+        before += w < (int)(threadIdx.x >> 6) ? s_wave[w] : 0;
+        all += s_wave[w];
+    }
+    if (threadIdx.x == 0)
+        s_at = atomicAdd(&a.ctl->tot[d % 3][blockIdx.x % kGroups].x,
+                         (unsigned long long)cnt << kEdgeBits | (unsigned long long)all);
+    __syncthreads();
+    const int64_t pos = (int64_t)(s_at >> kEdgeBits), off = (int64_t)(s_at & kEdgeMask);
+    if (pos + cnt <= a.gcap && off <= limit) {
+        const int64_t base = (int64_t)(blockIdx.x % kGroups) * a.gcap + pos;
+        int64_t run = off + before;
+        for (int i = i0; i < i1; ++i) {
+            a.qn[base + i] = s_v[i];
+            a.qoffn[base + i] = run;
+            run += s_d[i];
+        }
+    } else if (threadIdx.x == 0) {
+        set_lost(a, d);
+    }
+}
+
+// Top-down: the queue's edges in tiles, every tile's sources staged in LDS.
+// The thread that sets a target's bit in the next frontier collects it; the
+// parent is lowered to the smallest source with atomicMin.
+__device__ __forceinline__ void level_top_down(const LevelArgs &a, int d, const Groups &gr, int64_t limit,
+                                               uint32_t *s_mem)
+{
+    __shared__ int64_t s_range[2];
+    __shared__ int s_n;
+    __shared__ unsigned int s_lost;
+    int32_t *s_off = (int32_t *)s_mem;                        // kLvSrc
+    uint32_t *s_u = s_mem + kLvSrc;                           // kLvSrc
+    int64_t *s_rb = (int64_t *)(s_mem + 2 * kLvSrc);          // kLvSrc
+    uint32_t *s_v = s_mem + 4 * kLvSrc, *s_d = s_v + kLvBuf;  // kLvBuf each
+    static_assert(4 * kLvSrc + 2 * kLvBuf <= kLvMem && kLvBuf >= kLvTile, "LDS");
+    const uint64_t *__restrict__ front = a.front;
+    if (threadIdx.x == 0) {
+        s_n = 0;
+        s_lost = 0;
+    }
+    for (int64_t w = blockIdx.x * (int64_t)kLvBlock + threadIdx.x; w < a.wc; w += (int64_t)gridDim.x * kLvBlock) {
+        const uint64_t f = front[w];
+        if (f) a.visited[w] |= f;
+        a.third[w] = 0;
+    }
+    __syncthreads();
+    for (int64_t t = blockIdx.x; t < gr.tile0[kGroups]; t += gridDim.x) {
+        const int lane = threadIdx.x & 63;
+        const int g = __popcll(__ballot(lane < kGroups && gr.tile0[lane] <= t)) - 1;  // the last such has tiles
+        const uint32_t *__restrict__ q = a.q + g * a.gcap;
+        const int64_t *__restrict__ qoff = a.qoff + g * a.gcap;
+        const int64_t t0 = (t - gr.tile0[g]) * kLvTile, t1 = min(gr.edges[g], t0 + (int64_t)kLvTile);
+        const int64_t qn = gr.n[g];
+        if (threadIdx.x < 128) {
+            const int64_t r = wave_src_of(qoff, 0, qn - 1, threadIdx.x < 64 ? t0 : t1 - 1);
+            if ((threadIdx.x & 63) == 0) s_range[threadIdx.x >> 6] = r;
+        } else if (threadIdx.x == 128) {
+            s_lost = lost_yet(a, d);
+        }
+        __syncthreads();
+        const int64_t lo = s_range[0], hi = s_range[1];
+        const bool collect = s_lost == 0;
+        const bool staged = hi - lo < kLvSrc;  // sources of two edges and more on average
+        if (staged)
+            for (int j = threadIdx.x; j <= (int)(hi - lo); j += kLvBlock) {
+                const uint32_t u = q[lo + j];
+                const int64_t o = qoff[lo + j];
+                s_u[j] = u;
+                s_rb[j] = a.rowptr[u] - o;
+                s_off[j] = (int32_t)max(o - t0, (int64_t)-1);
+            }
+        __syncthreads();
+        // a thread's edges together, so that their loads are in flight at once
+        constexpr int U = kLvTile / kLvBlock;
+        uint32_t u[U], v[U];
+        uint64_t seen[U];
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+            const int64_t e = t0 + threadIdx.x + k * kLvBlock;
+            u[k] = v[k] = kNoParent;
+            if (e >= t1) continue;
+            int64_t at;
+            if (staged) {
+                const int32_t rel = (int32_t)(e - t0);
+                int x = 0, y = (int)(hi - lo);  // last source that starts at or before rel
+                while (x < y) {
+                    const int mid = (x + y + 1) >> 1;
+                    if (s_off[mid] <= rel) x = mid;
+                    else y = mid - 1;
+                }
+                u[k] = s_u[x];
+                at = s_rb[x] + e;
+            } else {
+                const int64_t x = src_of(qoff, lo, hi, e);
+                u[k] = q[x];
+                at = a.rowptr[u[k]] + (e - qoff[x]);
+            }
+            v[k] = a.cols[at];
+        }
+#pragma unroll
+        for (int k = 0; k < U; ++k) seen[k] = v[k] == kNoParent ? ~0ull : a.visited[v[k] >> 6];
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+            const int64_t w = v[k] >> 6;
+            const uint64_t bit = 1ull << (v[k] & 63);
+            if (seen[k] & bit) continue;
+            if (front[w] & bit) continue;
+            const bool early = !(a.next[w] & bit);
+            if (early) {
+                if (!collect) {
+                    // the next level, bottom-up, writes the levels
+                    atomicOr((unsigned long long *)&a.next[w], (unsigned long long)bit);
+                } else if (!(atomicOr((unsigned long long *)&a.next[w], (unsigned long long)bit) & bit)) {
+                    a.level[v[k]] = d + 1;
+                    const int i = atomicAdd(&s_n, 1);
+                    s_v[i] = v[k];
+                    s_d[i] = (uint32_t)(a.rowptr[v[k] + 1] - a.rowptr[v[k]]);
+                }
+            }
+            // an early source's parent slot holds nothing smaller yet
+            if (early || a.parent[v[k]] > u[k]) atomicMin(&a.parent[v[k]], u[k]);
+        }
+        __syncthreads();
+        const int cnt = s_n;
+        if (cnt > kLvBuf - kLvTile) {
+            level_flush(a, d, limit, cnt, s_v, s_d);
+            __syncthreads();
+            if (threadIdx.x == 0) s_n = 0;
+            __syncthreads();
+        }
+    }
+    const int cnt = s_n;
+    if (cnt) level_flush(a, d, limit, cnt, s_v, s_d);
+}
+
+// Bottom-up: as k_bottom_up, a wave per 64-vertex word, with the level's
+// commit (levels, visited, the next frontier) in the same pass.
+__device__ __forceinline__ void level_bottom_up(const LevelArgs &a, int d, const int64_t *__restrict__ rowptr,
+                                                const uint32_t *__restrict__ cols,
+                                                const uint64_t *__restrict__ front, uint64_t *__restrict__ visited,
+                                                uint64_t *__restrict__ next, uint64_t *__restrict__ third,
+                                                uint32_t *__restrict__ parent, int32_t *__restrict__ level,
+                                                bool late, uint32_t *s_mem)
+{
+    __shared__ int s_n;
+    __shared__ unsigned int s_lost;
+    constexpr int kCap = kLvBuf;
+    uint32_t *s_v = s_mem, *s_d = s_mem + kCap;
+    static_assert(2 * kCap * 4 + sizeof(BuScan) * (kLvBlock / 64) <= kLvMem * 4 && 2 * kCap * 4 % 16 == 0, "LDS");
+    BuScan &s_scan = ((BuScan *)(s_mem + 2 * kCap))[threadIdx.x >> 6];
+    const int lane = __lane_id();
+    if (threadIdx.x == 0) s_n = 0;
+    __syncthreads();
+    for (int64_t w = blockIdx.x * (int64_t)(kLvBlock / 64) + (threadIdx.x >> 6); w < a.wc;
+         w += (int64_t)gridDim.x * (kLvBlock / 64)) {
+        const uint64_t fr = front[w], vis = visited[w] | fr;
+        const int64_t v = w * 64 + lane;
+        if (late && (fr >> lane & 1)) level[v] = d;  // found by a top-down level that left them out
+        int64_t b = 0, e = 0;
+        if (!(vis >> lane & 1)) {
+            b = rowptr[v];
+            e = rowptr[v + 1];
+        }
+        const int64_t deg = e - b;
+        const uint32_t par = bu_scan(b, e, cols, front, s_scan, lane);
+        const bool hit = par != kNoParent;
+        if (hit) {
+            parent[v] = par;
+            level[v] = d + 1;
+        }
+        const uint64_t bits = __ballot(hit);
+        if (lane == 0) {
+            next[w] = bits;
+            visited[w] = vis | bits;
+            third[w] = 0;
+        }
+        // the workgroup's new vertices, as long as they fit
+        if (bits) {
+            const int c = __popcll(bits);
+            int i = 0;
+            if (lane == 0) i = s_n <= kCap ? atomicAdd(&s_n, c) : kCap;
+            i = __builtin_amdgcn_readfirstlane(i) + __popcll(bits & ((1ull << lane) - 1));
+            if (hit && i < kCap) {
+                s_v[i] = (uint32_t)v;
+                s_d[i] = (uint32_t)deg;
+            }
+        }
+    }
+    if (threadIdx.x == 0) s_lost = lost_yet(a, d);
+    __syncthreads();
+    const int cnt = s_n;
+    if (cnt == 0 || s_lost) return;
+    if (cnt <= kCap) {
+        level_flush(a, d, INT64_MAX, cnt, s_v, s_d);
+    } else if (threadIdx.x == 0) {
+        // some vertices (the next level only asks if there are any)
+        atomicAdd(&a.ctl->tot[d % 3][blockIdx.x % kGroups].x, (unsigned long long)cnt << kEdgeBits);
+        set_lost(a, d);
+    }
+}
+
+__global__ __launch_bounds__(kLvBlock) void k_level(LevelArgs a, int d, const int64_t *__restrict__ rowptr,
+                                                    const uint32_t *__restrict__ cols,
+                                                    const uint64_t *__restrict__ front,
+                                                    uint64_t *__restrict__ visited, uint64_t *__restrict__ next,
+                                                    uint64_t *__restrict__ third, uint32_t *__restrict__ parent,
+                                                    int32_t *__restrict__ level)
+{
+    __shared__ __align__(16) uint32_t s_mem[kLvMem];
+    __shared__ int64_t s_mode, s_limit;
+    __shared__ bool s_late;
+    __shared__ Groups s_gr;
+    if (a.ctl->lv[(d + 1) & 1].mode == kDone) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) a.ctl->lv[d & 1].mode = kDone;
+        return;
+    }
+    if (threadIdx.x < 64) {
+        const int g = threadIdx.x;
+        const unsigned long long tot = g < kGroups ? a.ctl->tot[(d + 2) % 3][g].x : 0ull;
+        const int64_t n = (int64_t)(tot >> kEdgeBits), m = (int64_t)(tot & kEdgeMask);
+        const int64_t tiles = (m + kLvTile - 1) / kLvTile, tinc = g5_wave_incl_scan(tiles);
+        if (g < kGroups) {
+            s_gr.n[g] = n;
+            s_gr.edges[g] = m;
+            s_gr.tile0[g] = tinc - tiles;
+            if (g == kGroups - 1) s_gr.tile0[kGroups] = tinc;
+        }
+        const int64_t n_f = g5_wave_sum(n), m_f = g5_wave_sum(m);
+        if (blockIdx.x == 0 && g < kGroups) a.ctl->tot[(d + 1) % 3][g].x = 0;
+        if (g == 0) {
+            const int64_t was = a.ctl->lv[(d + 1) & 1].mode;
+            int64_t mode = was, m_u = a.ctl->lv[(d + 1) & 1].m_u;
+            bool late = false;
+            if (n_f == 0) mode = kDone;
+            else if (d > 0) {  // the first level is top-down
+                if (mode == kTopDown && m_f > m_u / a.alpha) mode = kBottomUp;
+                else if (mode == kBottomUp && n_f < a.n / a.beta) mode = kTopDown;
+                if (a.ctl->lost[(d + 2) % 3].x) mode = kBottomUp;
+                late = mode == kBottomUp && was == kTopDown;
+                if (mode == kTopDown) m_u -= m_f;
+            }
+            if (blockIdx.x == 0) {
+                a.ctl->lv[d & 1].mode = mode;
+                a.ctl->lv[d & 1].m_u = m_u;
+                a.ctl->lost[(d + 1) % 3].x = 0;
+                // the first level that finds its frontier empty says so
+                if (mode == kDone) *a.host = d;
+            }
+            s_mode = mode;
+            s_limit = m_u / a.alpha;
+            s_late = late;
+        }
+    }
+    __syncthreads();
+    if (s_mode == kTopDown) level_top_down(a, d, s_gr, s_limit, s_mem);
+    else if (s_mode == kBottomUp)
+        level_bottom_up(a, d, rowptr, cols, front, visited, next, third, parent, level, s_late, s_mem);
+}
+
+// The whole search with k_level; levels are launched in batches.
+int run_levels(g5_bfs *b, int64_t root)
+{
+    g5_graph *g = b->g;
+    hipStream_t s = b->s;
+    LevelArgs a{};
+    a.rowptr = g->d_rowptr;
+    a.cols = g->d_cols;
+    a.visited = b->d_visited;
+    uint64_t *bm[3] = {b->d_out, b->d_next, b->d_third};
+    auto at = [&](int d) {
+        a.front = bm[d % 3];
+        a.next = bm[(d + 1) % 3];
+        a.third = bm[(d + 2) % 3];
+        a.q = b->d_gq[d & 1];
+        a.qn = b->d_gq[(d + 1) & 1];
+        a.qoff = b->d_goff[d & 1];
+        a.qoffn = b->d_goff[(d + 1) & 1];
+    };
+    at(0);
+    a.parent = b->d_parent;
+    a.level = b->d_level;
+    a.ctl = b->d_ctl;
+    a.host = b->h_cnt + kNCnt;
+    a.n = g->n_rows;
+    a.wc = b->wc;
+    a.nnz = g->nnz;
+    a.alpha = b->alpha;
+    a.beta = b->beta;
+    a.gcap = b->gcap;
+    *a.host = 0;
+    hipLaunchKernelGGL(k_reset, g5::grid_for(a.n / 4, kLvBlock, 4096), kLvBlock, 0, s, a,
+                       (const uint64_t *)b->d_isolated, root - g->row_start);
+    const int grid = std::max(256, g5::grid_for(a.wc, kLvBlock / 64, kLvGrid));
+    // a Kronecker search runs 6 to 9 levels; a level past the end costs about
+    // 2 us, a look from the host about 10
+    int d = 0;
+    for (int batch = 8;; batch = d < 16 ? 4 : std::min(64, batch * 2)) {
+        for (int i = 0; i < batch; ++i, ++d) {
+            at(d);
+            hipLaunchKernelGGL(k_level, grid, kLvBlock, 0, s, a, d,
+                               a.rowptr, a.cols, (const uint64_t *)a.front, a.visited, a.next, a.third, a.parent, a.level);
+        }
+        G5_HIP(hipGetLastError());
+        G5_HIP(hipEventRecord(b->ev1, s));
+        G5_HIP(hipStreamSynchronize(s));
+        if (*a.host) break;
+    }
+    const int nlevels = (int)*a.host;
+    // as a search level by level leaves it: the frontier empty, all merged
+    b->depth = nlevels - 1;
+    b->d_out = bm[nlevels % 3];
+    b->d_next = bm[(nlevels + 1) % 3];
+    b->d_third = bm[(nlevels + 2) % 3];
+    b->qlen = 0;
+    b->root = root;
     b->inbits_valid = false;
     return G5_OK;
 }
@@ -481,7 +1056,18 @@ extern "C" int g5_bfs_create(g5_graph *g, g5_bfs **out)
     if (e == hipSuccess) e = hipMalloc(&b->d_qoff, (size_t)(g->n_rows + 2) * 8);
     if (e == hipSuccess) e = hipMalloc(&b->d_scratch, scr * 8);
     if (e == hipSuccess) e = hipMalloc(&b->d_cnt, kNCnt * 8);
-    if (e == hipSuccess) e = hipHostMalloc(&b->h_cnt, kNCnt * 8, hipHostMallocDefault);
+    if (e == hipSuccess) e = hipHostMalloc(&b->h_cnt, (kNCnt + 1) * 8, hipHostMallocDefault);  // k_level's end last
+    if (g->n_rows == g->n_cols && g->row_start == g->col_start) {  // g5_bfs_run
+        // twice n / 8 vertices spread evenly: a level that finds more runs on
+        // bottom-up
+        b->gcap = std::max<int64_t>(kMinQueue, nmax / 4 / kGroups);
+        if (e == hipSuccess) e = hipMalloc(&b->d_third, (size_t)std::max<int64_t>(b->wc, 1) * 8);
+        for (int k = 0; k < 2; ++k) {
+            if (e == hipSuccess) e = hipMalloc(&b->d_gq[k], (size_t)(kGroups * b->gcap) * 4);
+            if (e == hipSuccess) e = hipMalloc(&b->d_goff[k], (size_t)(kGroups * b->gcap) * 8);
+        }
+        if (e == hipSuccess) e = hipMalloc(&b->d_ctl, sizeof(LevelCtl));
+    }
     if (e == hipSuccess) e = hipEventCreate(&b->ev0);
     if (e == hipSuccess) e = hipEventCreate(&b->ev1);
     if (e == hipSuccess) e = hipEventCreate(&b->ek0);
@@ -496,7 +1082,8 @@ extern "C" int g5_bfs_free(g5_bfs *b)
     if (!b) return G5_OK;
     if (b->s) (void)hipStreamSynchronize(b->s);
     void *dev[] = {b->d_visited, b->d_out,     b->d_next, b->d_parent, b->d_level, b->d_queue,
-                   b->d_outq,    b->d_qoff,    b->d_scratch, b->d_cnt, b->d_words, b->d_isolated, b->d_inbits};
+                   b->d_outq,    b->d_qoff,    b->d_scratch, b->d_cnt, b->d_words, b->d_isolated, b->d_inbits,
+                   b->d_third,   b->d_gq[0],   b->d_gq[1], b->d_goff[0], b->d_goff[1], b->d_ctl};
     for (void *p : dev)
         if (p) (void)hipFree(p);
     if (b->h_cnt) (void)hipHostFree(b->h_cnt);
@@ -681,7 +1268,7 @@ extern "C" int g5_bfs_expand_bottom_up(g5_bfs *b, const g5_graph *gt, int *any_n
     if (b->prof) G5_HIP(hipEventRecord(b->ek0, s));
     // rows of gt = this block's columns, its columns = this block's rows: the
     // kernel's frontier bits are the row frontier, its parents local row ids
-    hipLaunchKernelGGL(gt->n_rows < kBuLarge ? k_bottom_up<4> : k_bottom_up<2>, g5::grid_for(b->wc, 4, 4096), 256, 0,
+    hipLaunchKernelGGL(k_bottom_up, g5::grid_for(b->wc, 4, 4096), 256, 0,
                        s, (const int64_t *)gt->d_rowptr, (const uint32_t *)gt->d_cols,
                        (const uint64_t *)b->d_visited, (const uint64_t *)b->d_inbits, b->d_out, b->d_parent, b->wc,
                        b->d_cnt);
@@ -725,7 +1312,7 @@ extern "C" int g5_bfs_nedge(g5_bfs *b, int64_t *nedge)
     G5_REQUIRE(b && nedge, G5_E_ARG, "g5_bfs_nedge: null argument");
     G5_REQUIRE(b->g->n_rows == b->g->n_cols, G5_E_STATE, "g5_bfs_nedge: needs a 1x1 block");
     hipLaunchKernelGGL(k_set_cnt, 1, 1, 0, b->s, b->d_cnt, (int)kOutLen, (int64_t)0);
-    hipLaunchKernelGGL(k_nedge, g5::grid_for(b->g->n_rows, 256, 4096), 256, 0, b->s,
+    hipLaunchKernelGGL(k_nedge, g5::grid_for(b->g->n_rows / 4, 256, kSumGrid), 256, 0, b->s,
                        (const uint32_t *)b->g->d_gdeg, (const int32_t *)b->d_level, b->g->n_rows,
                        b->d_cnt + kOutLen);
     G5_HIP(hipGetLastError());
@@ -744,7 +1331,7 @@ extern "C" int g5_bfs_summary(g5_bfs *b, int64_t *nedge, uint64_t *checksum)
     static_assert(kNewEdges == kOutLen + 1, "the summary's two slots must be adjacent");
     hipLaunchKernelGGL(k_set_cnt, 1, 1, 0, b->s, b->d_cnt, (int)kOutLen, (int64_t)0);
     hipLaunchKernelGGL(k_set_cnt, 1, 1, 0, b->s, b->d_cnt, (int)kNewEdges, (int64_t)0);
-    hipLaunchKernelGGL(k_summary, g5::grid_for(b->g->n_rows, 256, 4096), 256, 0, b->s,
+    hipLaunchKernelGGL(k_summary, g5::grid_for(b->g->n_rows, 256, kSumGrid), 256, 0, b->s,
                        (const uint32_t *)b->g->d_gdeg, (const int32_t *)b->d_level, (const uint32_t *)b->d_parent,
                        b->g->n_rows, b->d_cnt + kOutLen);
     G5_HIP(hipGetLastError());
@@ -772,8 +1359,20 @@ extern "C" int g5_bfs_run(g5_bfs *b, int64_t root, int flags, int32_t *nlevels, 
     }
     hipStream_t s = b->s;
     G5_HIP(hipStreamSynchronize(s));
+    int rc = find_isolated(b);
+    if (rc) return rc;
     G5_HIP(hipEventRecord(b->ev0, s));
-    int rc = reset_search(b, root, true);
+    // k_level decides the levels on the device; the codec's launches, the
+    // accounting and a forced direction need the host's view of each level,
+    // and a packed total holds 2^30 vertices and 2^34 edges
+    if (!codec && !topdown_only && !b->prof && g->n_rows <= (int64_t)1 << 30 && g->nnz < (int64_t)1 << kEdgeBits) {
+        rc = run_levels(b, root);
+        if (rc) return rc;
+        if (ms) G5_HIP(hipEventElapsedTime(ms, b->ev0, b->ev1));
+        if (nlevels) *nlevels = b->depth + 1;
+        return G5_OK;
+    }
+    rc = reset_search(b, root, true);
     if (rc) return rc;
     const int64_t n = g->n_rows;
     int64_t m_u = g->nnz;  // edges not yet checked top-down
@@ -783,7 +1382,7 @@ extern "C" int g5_bfs_run(g5_bfs *b, int64_t root, int flags, int32_t *nlevels, 
         uint64_t *fresh = b->d_out;
         if (bu) {
             if (b->prof) G5_HIP(hipEventRecord(b->ek0, s));
-            hipLaunchKernelGGL(g->n_rows < kBuLarge ? k_bottom_up<4> : k_bottom_up<2>, g5::grid_for(b->wc, 4, 4096),
+            hipLaunchKernelGGL(k_bottom_up, g5::grid_for(b->wc, 4, 4096),
                                256, 0, s, (const int64_t *)g->d_rowptr,
                                (const uint32_t *)g->d_cols, (const uint64_t *)b->d_visited,
                                (const uint64_t *)b->d_out, b->d_next, b->d_parent, b->wc, b->d_cnt);
