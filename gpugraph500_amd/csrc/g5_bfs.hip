@@ -673,19 +673,6 @@ __global__ __launch_bounds__(kLvBlock) void k_reset(LevelArgs a, const uint64_t 
     }
 }
 
-// last s in [lo, hi] with qoff[s] <= e, by a whole wave, 64 probes a round
-__device__ __forceinline__ int64_t wave_src_of(const int64_t *__restrict__ qoff, int64_t lo, int64_t hi, int64_t e)
-{
-    ++hi;
-    while (hi - lo > 1) {
-        const int64_t step = (hi - lo + 63) / 64, at = lo + step * __lane_id();
-        const uint64_t le = __ballot(at < hi && qoff[at] <= e);  // lane 0's always is
-        lo += step * (63 - __clzll((long long)le));
-        hi = min(hi, lo + step);
-    }
-    return lo;
-}
-
 // whether the level's queue is known to be incomplete
 __device__ __forceinline__ bool lost_yet(const LevelArgs &a, int d)
 {
@@ -765,7 +752,7 @@ __device__ __forceinline__ void level_top_down(const LevelArgs &a, int d, const 
         const int64_t t0 = (t - gr.tile0[g]) * kLvTile, t1 = min(gr.edges[g], t0 + (int64_t)kLvTile);
         const int64_t qn = gr.n[g];
         if (threadIdx.x < 128) {
-            const int64_t r = wave_src_of(qoff, 0, qn - 1, threadIdx.x < 64 ? t0 : t1 - 1);
+            const int64_t r = g5_wave_src_of(qoff, 0, qn - 1, threadIdx.x < 64 ? t0 : t1 - 1);
             if ((threadIdx.x & 63) == 0) s_range[threadIdx.x >> 6] = r;
         } else if (threadIdx.x == 128) {
             s_lost = lost_yet(a, d);

@@ -183,3 +183,17 @@ __device__ __forceinline__ int64_t g5_block_sum256(int64_t v)
     __syncthreads();  // s_part is free again for the next call
     return t;
 }
+
+// last s in [lo, hi] with off[s] <= e (off ascends, off[lo] <= e), by a whole
+// wave, 64 probes a round: 4 dependent loads for 2^24 entries
+__device__ __forceinline__ int64_t g5_wave_src_of(const int64_t *__restrict__ off, int64_t lo, int64_t hi, int64_t e)
+{
+    ++hi;
+    while (hi - lo > 1) {
+        const int64_t step = (hi - lo + 63) / 64, at = lo + step * __lane_id();
+        const uint64_t le = __ballot(at < hi && off[at] <= e);  // lane 0's always is
+        lo += step * (63 - __clzll((long long)le));
+        hi = min(hi, lo + step);
+    }
+    return lo;
+}

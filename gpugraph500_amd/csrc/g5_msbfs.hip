@@ -112,8 +112,8 @@ struct Tune {
 // root) pairs, edges read, vertices worked on, frontier words gathered, and
 // the next frontier's vertices and edges; then the OR of the next frontier's
 // words (the lanes still searching).  Then set-once slots: the level number,
-// the newly reached queue length (push), the frontier queue length and its
-// edge total (push), the lanes the block and wave kernels work on, the lanes
+// the frontier queue's length and its edge total (push; the host's copy only),
+// the lanes the block and wave kernels work on, the lanes
 // in use, the first word of level flags the level before wrote, the lanes
 // the thread kernel works on and the wave kernel's first step (the last five
 // written before each pull level, k_set_pull_lanes).
@@ -122,24 +122,23 @@ enum MsCnt {
     kUnitSlots = 6,
     kLive = kUnits * kUnitSlots,
     kAccum = kLive + 1,
-    kDepth = kAccum, kNq = kAccum + 1, kFqLen = kAccum + 2, kFqEdges = kAccum + 3, kPullLanes = kAccum + 4,
+    kDepth = kAccum, kFqLen = kAccum + 2, kFqEdges = kAccum + 3, kPullLanes = kAccum + 4,
     kUsed = kAccum + 5, kFlagWord = kAccum + 6, kThreadLanes = kAccum + 7, kWaveStep = kAccum + 8,
     kCntStride = 40
 };
 // Many workgroups adding into one address serialise in one L2 channel, so
 // the accumulated slots are striped: workgroup b adds into stripe b %
-// kStripes (stripes 320 B apart) and k_level_end folds the stripes into
-// stripe 0, which also holds the set-once slots.
+// kStripes (stripes 320 B apart) and k_level_end folds the stripes for the
+// host; stripe 0 also holds the set-once slots.
 constexpr int kStripes = 32;
 static_assert(kWaveStep < kCntStride, "counter stripe too small");
 // Per-lane frontier edges (counted by push levels, from their new-vertex
 // queue): kLaneStripes stripes of 64 slots, summed on the host.
 constexpr int kLaneStripes = 8;
-constexpr int kHostSlots = kCntStride + 64;  // stripe 0, then the folded per-lane edges
+constexpr int kHostSlots = kCntStride + 64;  // the folded counters, then the per-lane edges
 // edgeless roots remembered between batch runs (beyond: every edgeless
 // vertex's record is cleared)
 constexpr int64_t kDirtyCap = 1 << 16;
-static_assert(kStripes * kCntStride >= kHostSlots, "per-lane edges do not fit the folded stripes");
 
 // The degree-ordered copy of the block.
 struct Relabeled {
@@ -163,6 +162,12 @@ struct Relabeled {
     int64_t split_first[kBins + 1] = {0};  // the same on split levels (min(split_max, thread_max))
 };
 
+// the total of a part of a push queue, in a line of its own
+struct QueueTotal {
+    unsigned long long x;  // entries << kQueueEdgeBits | edges
+    unsigned long long pad[15];
+};
+
 }  // namespace
 
 struct g5_msbfs {
@@ -171,8 +176,10 @@ struct g5_msbfs {
     int64_t n = 0;                       // vertices (rows == cols)
     uint64_t *d_visited = nullptr, *d_fa = nullptr, *d_fb = nullptr;
     uint64_t *d_act = nullptr;           // two n/64-word active bitmaps (parity a, b)
-    uint32_t *d_fq = nullptr, *d_nq = nullptr;  // push: frontier queue, newly reached queue
-    int64_t *d_qoff = nullptr;                  // push: frontier degree prefix
+    // push: two queues (a level's frontier, the vertices it reaches)
+    uint32_t *d_qv[2] = {nullptr, nullptr};
+    int64_t *d_qo[2] = {nullptr, nullptr};
+    QueueTotal *d_qt = nullptr;  // kGroups each
     // records [n][64] by original vertex id: slot r of v holds lane r's
     // parent of v (original id) and its level byte
     int32_t *d_parent = nullptr;
@@ -212,13 +219,14 @@ struct g5_msbfs {
     int64_t lane_edges[64] = {};
     hipEvent_t ek_push[2] = {};  // split levels (profiled): around the pushed lanes' kernels
     int64_t split_levels = 0;
-    // the last push level's frontier queue, which lists the only non-zero
-    // words of the buffer the next push level writes (listed_ok: the level
-    // just run was that push level, or both buffers are clear)
-    uint32_t *d_fq2 = nullptr;
-    uint32_t *listed = nullptr;
+    // the last push level's frontier queue (listed: 0 or 1), which lists the
+    // only non-zero words of the buffer the next push level writes (listed_ok:
+    // the level just run was that push level, or both buffers are clear), and
+    // whether the other queue holds the frontier the next level reads
+    int listed = 0;
     int64_t listed_len = 0;
     bool listed_ok = false;
+    bool queue_ok = false;
     int64_t flag_word = INT64_MAX;     // the first word of lvflag the last level wrote (INT64_MAX: none)
     uint64_t *d_lvflag = nullptr;      // bit v: v's level record holds the next level's prediction
     bool last_empty = false;  // the level just run found no new (vertex, root) pair
@@ -822,6 +830,69 @@ constexpr int kPushTile = 1024;  // 20 KB of LDS per block (2048: 40 KB, 4 waves
 constexpr int kPushGrid = 4096;
 constexpr int kPushVertGrid = 2048;
 
+// A push queue: the frontier's vertices and their degree prefix, in kGroups
+// independent parts.  Workgroups reserve their entries (vertices and edges
+// together) with one packed atomic on their part's total; returning atomics on
+// one address take 12 ns each, hence the parts.  The bitmap's words are dealt
+// to the parts in order, kUnitWords at a time, so a part's entries fit where
+// its words' vertices would: the buffers hold one entry per vertex and no part
+// overflows.
+constexpr int kGroups = 16;
+constexpr int kQueueEdgeBits = 36;
+constexpr int kUnitWords = kBlock / 64 * 8;  // of the bitmap: what a workgroup takes at a time
+struct PushQueue {
+    uint32_t *v;
+    int64_t *off;  // relative to the part's first edge
+    QueueTotal *tot;  // kGroups
+    int64_t units;  // of the bitmap it was built from
+};
+
+__host__ __device__ __forceinline__ int64_t queue_units(int64_t nwords) { return (nwords + kUnitWords - 1) / kUnitWords; }
+
+// first entry of part g
+__device__ __forceinline__ int64_t part_base(const PushQueue &q, int g)
+{
+    return (g * q.units + kGroups - 1) / kGroups * (kUnitWords * 64);
+}
+
+// A queue's parts as a workgroup works through them: entries, edges, and the
+// prefixes over the parts of `per` edges' tiles and of entries
+struct Parts {
+    int64_t n[kGroups], edges[kGroups], tile0[kGroups + 1], n0[kGroups + 1];
+    int64_t base[kGroups];
+};
+
+// one wave; the others wait at the caller's barrier
+__device__ __forceinline__ void load_parts(Parts &s, const PushQueue &q, int64_t per)
+{
+    const int g = __lane_id();
+    const unsigned long long t = g < kGroups ? q.tot[g].x : 0ull;
+    const int64_t n = (int64_t)(t >> kQueueEdgeBits), m = (int64_t)(t & ((1ull << kQueueEdgeBits) - 1));
+    const int64_t tiles = (m + per - 1) / per;
+    const int64_t tinc = g5_wave_incl_scan(tiles), ninc = g5_wave_incl_scan(n);
+    if (g < kGroups) {
+        s.n[g] = n;
+        s.edges[g] = m;
+        s.tile0[g] = tinc - tiles;
+        s.n0[g] = ninc - n;
+        s.base[g] = part_base(q, g);
+        if (g == kGroups - 1) {
+            s.tile0[kGroups] = tinc;
+            s.n0[kGroups] = ninc;
+        }
+    }
+}
+
+// the part that holds entry i of all
+__device__ __forceinline__ int part_of(const Parts &s, int64_t i)
+{
+    int g = 0;
+#pragma unroll
+    for (int d = kGroups / 2; d >= 1; d >>= 1)
+        if (s.n0[g + d] <= i) g += d;
+    return g;
+}
+
 __device__ __forceinline__ int64_t fq_src(const int64_t *__restrict__ qoff, int64_t lo, int64_t hi, int64_t e)
 {
     while (lo < hi) {
@@ -830,24 +901,6 @@ __device__ __forceinline__ int64_t fq_src(const int64_t *__restrict__ qoff, int6
         else hi = mid - 1;
     }
     return lo;
-}
-
-// qoff[i] = degree of queue entry i; entries [queue length, bound) := 0, so
-// that a scan over `bound` entries (a host-side upper bound of the queue's
-// length) ends with the queue's edge total
-__global__ void k_fq_degrees(const uint32_t *__restrict__ fq, const int64_t *__restrict__ cnt,
-                             const int64_t *__restrict__ rowptr, int64_t *__restrict__ qoff, int64_t bound)
-{
-    const int64_t n = cnt[kFqLen];
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < bound;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        if (i < n) {
-            const uint32_t u = fq[i];
-            qoff[i] = rowptr[u + 1] - rowptr[u];
-        } else {
-            qoff[i] = 0;
-        }
-    }
 }
 
 // one pushed edge: u (relabelled id, uo its original id) -> v (vo).  mark (first
@@ -862,7 +915,9 @@ __device__ __forceinline__ void push_edge(uint32_t u, uint32_t uo, uint32_t v, u
                                           int32_t *__restrict__ parent, uint8_t *__restrict__ level, uint8_t lv,
                                           uint64_t lm, uint64_t *__restrict__ mark)
 {
-    const uint64_t f = frontier[u] & lm & ~visited[v];
+    // the minimum pass works on the pairs the level found: next holds exactly
+    // those (it may run after visited has them too)
+    const uint64_t f = frontier[u] & lm & (kMin ? next[v] : ~visited[v]);
     if (!kMin) {
         // (a plain load of next[v] first, to skip atomics whose bits are set,
         // cost more than it saved: level 2 at scale 26 1.95 -> 1.7 ms without)
@@ -874,7 +929,7 @@ __device__ __forceinline__ void push_edge(uint32_t u, uint32_t uo, uint32_t v, u
         if (fresh) write_slots(parent, level, vo, fresh, uo, lv);
         if (mark && old == 0) atomicOr((unsigned long long *)&mark[v >> 6], 1ull << (v & 63));
     } else if (f) {
-        uint64_t bits = f;  // every bit of f is new at this level (visited excludes older ones)
+        uint64_t bits = f;
         int32_t *rec = &parent[(int64_t)vo * 64];
         while (bits) {
             const int r = __ffsll((long long)bits) - 1;
@@ -939,204 +994,323 @@ __global__ __launch_bounds__(kBlock) void k_cand_commit(const uint32_t *__restri
     block_add(cnt + kUnitSlots * kPushUnit, {nbits, (int64_t)0, nv});
 }
 
-// the push unit's next-frontier edges so far, summed over the stripes
-__device__ __forceinline__ int64_t push_next_edges(const int64_t *__restrict__ cnt)
-{
-    int64_t t = 0;
-    for (int st = 0; st < kStripes; ++st) t += cnt[st * kCntStride + kUnitSlots * kPushUnit + kNextEdges];
-    return t;
-}
-
 // A tile's sources (at most kPushTile: every queue vertex has an edge) are
 // staged in LDS first -- their first edge's offset within the tile, their
 // relabelled and original ids and their row start less their queue offset --
 // so that each edge finds its source by a binary search in LDS rather than
 // in the global prefix.
-template <bool kMin, bool kCand = false>
-__global__ __launch_bounds__(kBlock) void k_push_edges(
-    const uint32_t *__restrict__ fq, const int64_t *__restrict__ qoff, const int64_t *__restrict__ rowptr,
-    const uint32_t *__restrict__ cols, const uint32_t *__restrict__ cols_orig, const uint32_t *__restrict__ new2old,
-    const uint64_t *__restrict__ visited, const uint64_t *__restrict__ frontier, uint64_t *__restrict__ next,
-    int32_t *__restrict__ parent, uint8_t *__restrict__ level, int64_t *__restrict__ cnt, uint64_t lm,
-    uint64_t *__restrict__ mark, int64_t vend, uint32_t *__restrict__ cand = nullptr, int npm = 0,
-    bool rows_ok = false)
+struct PushTile {
+    int64_t lo_hi[2];
+    int64_t rb[kPushTile];
+    int32_t off[kPushTile];
+    uint32_t u[kPushTile], uo[kPushTile];
+};
+
+struct PushArgs {
+    const int64_t *rowptr;
+    const uint32_t *cols, *cols_orig, *new2old;
+    const uint64_t *visited, *frontier;
+    uint64_t *next;
+    int32_t *parent;
+    uint8_t *level;
+};
+
+template <bool kMin, bool kCand>
+__device__ __forceinline__ void push_tiles(const PushArgs &a, const PushQueue &q, const Parts &s, PushTile &t,
+                                           uint8_t lv, uint64_t lm, uint64_t *__restrict__ mark, int64_t vend,
+                                           uint32_t *__restrict__ cand, int npm)
 {
-    __shared__ int64_t s_lo, s_hi;
-    // the minimum pass of a pure push level whose new vertices have fewer
-    // edges than its frontier runs by rows (k_min_rows)
-    if (kMin && rows_ok && push_next_edges(cnt) < cnt[kFqEdges]) return;
-    __shared__ int32_t s_off[kPushTile];
-    __shared__ uint32_t s_u[kPushTile], s_uo[kPushTile];
-    __shared__ int64_t s_rb[kPushTile];
-    const int64_t qn = cnt[kFqLen], E = cnt[kFqEdges];
-    const uint8_t lv = level_byte(cnt);
-    for (int64_t t0 = blockIdx.x * (int64_t)kPushTile; t0 < E; t0 += (int64_t)gridDim.x * kPushTile) {
-        const int64_t t1 = min(E, t0 + (int64_t)kPushTile);
-        if (threadIdx.x == 0) {
-            s_lo = fq_src(qoff, 0, qn - 1, t0);
-            s_hi = fq_src(qoff, s_lo, qn - 1, t1 - 1);
+    const int lane = __lane_id();
+    for (int64_t tile = blockIdx.x; tile < s.tile0[kGroups]; tile += gridDim.x) {
+        const int g = __popcll(__ballot(lane < kGroups && s.tile0[lane] <= tile)) - 1;  // the last such has tiles
+        const uint32_t *__restrict__ fq = q.v + s.base[g];
+        const int64_t *__restrict__ qoff = q.off + s.base[g];
+        const int64_t t0 = (tile - s.tile0[g]) * kPushTile, t1 = min(s.edges[g], t0 + (int64_t)kPushTile);
+        if (threadIdx.x < 128) {
+            const int64_t r = g5_wave_src_of(qoff, 0, s.n[g] - 1, threadIdx.x < 64 ? t0 : t1 - 1);
+            if (lane == 0) t.lo_hi[threadIdx.x >> 6] = r;
         }
         __syncthreads();
-        const int64_t lo = s_lo, hi = s_hi;
+        const int64_t lo = t.lo_hi[0], hi = t.lo_hi[1];
         const int ns = (int)min(hi - lo + 1, (int64_t)kPushTile + 1);
         if (ns <= kPushTile) {
             for (int j = threadIdx.x; j < ns; j += kBlock) {
                 const uint32_t u = fq[lo + j];
-                const int64_t q = qoff[lo + j];
-                s_u[j] = u;
-                s_uo[j] = new2old[u];
-                s_rb[j] = rowptr[u] - q;
-                s_off[j] = (int32_t)max(q - t0, (int64_t)0);
+                const int64_t o = qoff[lo + j];
+                t.u[j] = u;
+                t.uo[j] = a.new2old[u];
+                t.rb[j] = a.rowptr[u] - o;
+                t.off[j] = (int32_t)max(o - t0, (int64_t)0);
             }
             __syncthreads();
             int j = 0;  // the sources of a thread's edges ascend
             for (int64_t e = t0 + threadIdx.x; e < t1; e += kBlock) {
                 const int32_t rel = (int32_t)(e - t0);
-                int a = j, b = ns - 1;  // last j with s_off[j] <= rel
-                while (a < b) {
-                    const int mid = (a + b + 1) >> 1;
-                    if (s_off[mid] <= rel) a = mid;
-                    else b = mid - 1;
+                int x = j, y = ns - 1;  // last j with off[j] <= rel
+                while (x < y) {
+                    const int mid = (x + y + 1) >> 1;
+                    if (t.off[mid] <= rel) x = mid;
+                    else y = mid - 1;
                 }
-                j = a;
-                const int64_t pos = s_rb[j] + e;
-                const uint32_t v = cols[pos];
+                j = x;
+                const int64_t pos = t.rb[j] + e;
+                const uint32_t v = a.cols[pos];
                 if (v >= vend) continue;
-                if (kCand) push_cand(s_u[j], s_uo[j], v, visited, frontier, cand, npm, lm);
+                if (kCand) push_cand(t.u[j], t.uo[j], v, a.visited, a.frontier, cand, npm, lm);
                 else
-                    push_edge<kMin>(s_u[j], s_uo[j], v, cols_orig[pos], visited, frontier, next, parent, level, lv,
-                                    lm, mark);
+                    push_edge<kMin>(t.u[j], t.uo[j], v, a.cols_orig[pos], a.visited, a.frontier, a.next, a.parent,
+                                    a.level, lv, lm, mark);
             }
         } else {
             for (int64_t e = t0 + threadIdx.x; e < t1; e += kBlock) {
                 const int64_t si = fq_src(qoff, lo, hi, e);
                 const uint32_t u = fq[si];
-                const int64_t pos = rowptr[u] + (e - qoff[si]);
-                const uint32_t v = cols[pos];
+                const int64_t pos = a.rowptr[u] + (e - qoff[si]);
+                const uint32_t v = a.cols[pos];
                 if (v >= vend) continue;
-                if (kCand) push_cand(u, new2old[u], v, visited, frontier, cand, npm, lm);
+                if (kCand) push_cand(u, a.new2old[u], v, a.visited, a.frontier, cand, npm, lm);
                 else
-                    push_edge<kMin>(u, new2old[u], v, cols_orig[pos], visited, frontier, next, parent, level, lv,
-                                    lm, mark);
+                    push_edge<kMin>(u, a.new2old[u], v, a.cols_orig[pos], a.visited, a.frontier, a.next, a.parent,
+                                    a.level, lv, lm, mark);
             }
         }
         __syncthreads();
     }
-    if (!kMin && blockIdx.x == 0 && threadIdx.x == 0)
-        atomicAdd((unsigned long long *)&cnt[kUnitSlots * kPushUnit + kEdgesRead], (unsigned long long)E);
 }
 
-// next[list[i]] := 0 for i < len (the entries a pure push level's frontier
-// queue listed: the only non-zero words of the buffer two levels on)
-__global__ void k_zero_listed(uint64_t *__restrict__ next, const uint32_t *__restrict__ list, int64_t len)
+// The first pass over the queue's edges (kCand: the candidate pass).  fresh:
+// the totals of the queue that the level builds next, cleared here.
+template <bool kCand>
+__global__ __launch_bounds__(kBlock) void k_push_edges(PushArgs a, PushQueue q, int64_t *__restrict__ cnt, uint64_t lm,
+                                                       uint64_t *__restrict__ mark, int64_t vend,
+                                                       uint32_t *__restrict__ cand, int npm,
+                                                       QueueTotal *__restrict__ fresh)
 {
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < len; i += (int64_t)gridDim.x * blockDim.x)
-        next[list[i]] = 0;
+    __shared__ Parts s;
+    __shared__ PushTile t;
+    if (threadIdx.x < 64) load_parts(s, q, kPushTile);
+    __syncthreads();
+    if (blockIdx.x == 0) {
+        if (fresh && threadIdx.x < kGroups) fresh[threadIdx.x].x = 0;
+        if (threadIdx.x == 0) {
+            int64_t E = 0;
+            for (int g = 0; g < kGroups; ++g) E += s.edges[g];
+            atomicAdd((unsigned long long *)&cnt[kUnitSlots * kPushUnit + kEdgesRead], (unsigned long long)E);
+        }
+    }
+    push_tiles<false, kCand>(a, q, s, t, level_byte(cnt), lm, mark, vend, cand, npm);
 }
 
-// The minimum pass of a pure push level by rows, when its newly reached
-// vertices have fewer edges than its frontier (levels past the peak: few new
-// vertices of low degree): each new vertex scans its row in ascending
-// original-id order, and the first frontier neighbour of each new lane is
-// its parent.  The same minimum as the edge pass (k_push_edges<true>), which
-// runs instead otherwise; each of the two exits at once when not chosen.
-__global__ __launch_bounds__(kBlock) void k_min_rows(const uint32_t *__restrict__ nq,
-                                                     const int64_t *__restrict__ rowptr,
-                                                     const uint32_t *__restrict__ cols,
-                                                     const uint32_t *__restrict__ cols_orig,
-                                                     const uint32_t *__restrict__ new2old,
-                                                     const uint64_t *__restrict__ frontier,
-                                                     const uint64_t *__restrict__ next,
-                                                     int32_t *__restrict__ parent, const int64_t *__restrict__ cnt)
+// What a push level starts with: the next frontier's active bitmap clear, and
+// next itself, whole or at the entries of the queue whose words it holds (the
+// frontier queue of the push level before); clear: the totals of a queue that
+// is built next.
+__global__ void k_push_begin(uint64_t *__restrict__ act_next, int64_t nw, uint64_t *__restrict__ next, int64_t n,
+                             bool whole, PushQueue listed, QueueTotal *__restrict__ clear)
 {
-    if (push_next_edges(cnt) >= cnt[kFqEdges]) return;
-    const int64_t n = cnt[kNq];
-    for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
-        const uint32_t v = nq[i];
-        const uint64_t w = next[v];
-        const int64_t b = rowptr[v], e = rowptr[v + 1];
-        int32_t *rec = &parent[(int64_t)new2old[v] * 64];
+    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+    if (clear && t < kGroups) clear[t].x = 0;
+    for (int64_t i = t; i < nw; i += stride) act_next[i] = 0;
+    if (whole) {
+        for (int64_t i = t; i < n; i += stride) next[i] = 0;
+        return;
+    }
+    if (!listed.v) return;
+    __shared__ Parts s;
+    if (threadIdx.x < 64) load_parts(s, listed, kPushTile);
+    __syncthreads();
+    for (int64_t i = t; i < s.n0[kGroups]; i += stride) {
+        const int g = part_of(s, i);
+        next[listed.v[s.base[g] + i - s.n0[g]]] = 0;
+    }
+}
+
+// The minimum pass of a push level.  When the newly reached vertices have
+// fewer edges than the frontier (levels past the peak: few new vertices of low
+// degree) it runs by rows: each new vertex scans its row in ascending
+// original-id order, and the first frontier neighbour of each new lane is its
+// parent.  Otherwise over the frontier's edges again, lowering the parents of
+// the pairs found at this level.  Both give the same minimum.
+// A push level (whole) also counts each lane's frontier edges of the next
+// level here, from the new vertices' queue (k_queue sees them word by word,
+// mostly a few lanes at a time).
+__global__ __launch_bounds__(kBlock) void k_push_min(PushArgs a, PushQueue q, PushQueue nq,
+                                                     const int64_t *__restrict__ cnt, uint64_t lm, int64_t vend,
+                                                     bool whole, int64_t *__restrict__ lane_edges)
+{
+    __shared__ Parts s, sn;
+    __shared__ PushTile t;
+    __shared__ unsigned long long s_lane[64];
+    if (threadIdx.x < 64) {
+        load_parts(s, q, kPushTile);
+        if (whole) load_parts(sn, nq, kPushTile);
+        s_lane[threadIdx.x] = 0;
+    }
+    __syncthreads();
+    bool rows = false;
+    if (whole) {
+        for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < sn.n0[kGroups];
+             i += (int64_t)gridDim.x * kBlock) {
+            const int g = part_of(sn, i);
+            const uint32_t v = nq.v[sn.base[g] + i - sn.n0[g]];
+            const unsigned long long d = (unsigned long long)(a.rowptr[v + 1] - a.rowptr[v]);
+            for (uint64_t b = a.next[v]; b; b &= b - 1) atomicAdd(&s_lane[__ffsll((long long)b) - 1], d);
+        }
+        __syncthreads();
+        if (threadIdx.x < 64 && s_lane[threadIdx.x])
+            atomicAdd((unsigned long long *)&lane_edges[(blockIdx.x % kLaneStripes) * 64 + threadIdx.x],
+                      s_lane[threadIdx.x]);
+        int64_t E = 0, En = 0;
+        for (int g = 0; g < kGroups; ++g) {
+            E += s.edges[g];
+            En += sn.edges[g];
+        }
+        rows = En < E;
+    }
+    if (!rows) {
+        push_tiles<true, false>(a, q, s, t, level_byte(cnt), lm, nullptr, vend, nullptr, 0);
+        return;
+    }
+    for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < sn.n0[kGroups];
+         i += (int64_t)gridDim.x * kBlock) {
+        const int g = part_of(sn, i);
+        const uint32_t v = nq.v[sn.base[g] + i - sn.n0[g]];
+        const uint64_t w = a.next[v];
+        const int64_t b = a.rowptr[v], e = a.rowptr[v + 1];
+        int32_t *rec = &a.parent[(int64_t)a.new2old[v] * 64];
         uint64_t found = 0;
         for (int64_t j = b; j < e && found != w; j += 4) {
             uint64_t fr[4];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) fr[k] = j + k < e ? frontier[cols[j + k]] : 0ull;
+            for (int k = 0; k < 4; ++k) fr[k] = j + k < e ? a.frontier[a.cols[j + k]] : 0ull;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 uint64_t f = fr[k] & w & ~found;
                 if (!f) continue;
                 found |= f;
-                const int32_t uo = (int32_t)cols_orig[j + k];
+                const int32_t uo = (int32_t)a.cols_orig[j + k];
                 for (; f; f &= f - 1) rec[__ffsll((long long)f) - 1] = uo;
             }
         }
     }
 }
 
-// A pure push level's next frontier from its queue nq (cnt[kNq] entries)
-// instead of a pass over all n words: the push unit's next-frontier vertices
-// and edges, the live lanes and each lane's frontier edges (exact).
-__global__ __launch_bounds__(kBlock) void k_nq_counts(const uint32_t *__restrict__ nq,
-                                                      const uint64_t *__restrict__ next,
-                                                      const int64_t *__restrict__ rowptr, int64_t *__restrict__ cnt,
-                                                      int64_t *__restrict__ lane_edges)
+// The vertices of a bitmap, a workgroup per unit of its words (a wave per 8
+// words, lane = vertex, 8 words' loads in flight):
+//   kKind 0   their queue
+//   kKind 1   the same for a push level's newly reached vertices (next's
+//             bitmap), with the level's commit (visited |= next) and counts:
+//             pairs, the next frontier's vertices and edges, the live lanes
+//   kKind 2   a split level's vertices reached by the pushed lanes lm: commit
+//             and counts of pairs and vertices, no queue
+// A lane's vertices (one per word) lie next to each other in the queue, so one
+// scan over the lanes gives every entry its place and edge offset.
+template <int kKind>
+__global__ __launch_bounds__(kBlock) void k_queue(const uint64_t *__restrict__ bits, int64_t nwords,
+                                                  const int64_t *__restrict__ rowptr, PushQueue q,
+                                                  const uint64_t *__restrict__ next, uint64_t *__restrict__ visited,
+                                                  uint64_t lm, int64_t *__restrict__ cnt)
 {
-    __shared__ unsigned long long s_lane[64];
+    constexpr int W = kUnitWords / (kBlock / 64);
+    __shared__ unsigned long long s_wave[kBlock / 64], s_at;
     __shared__ uint64_t s_live[kBlock / 64];
-    const int64_t n = cnt[kNq];
-    if (threadIdx.x < 64) s_lane[threadIdx.x] = 0;
-    __syncthreads();
-    int64_t nv = 0, ne = 0;
+    const int lane = __lane_id(), wv = threadIdx.x >> 6;
+    int64_t nbits = 0, nv = 0, ne = 0;
     uint64_t live = 0;
-    for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
-        const uint32_t v = nq[i];
-        const uint64_t w = next[v];
-        const int64_t d = rowptr[v + 1] - rowptr[v];
-        ++nv;
-        ne += d;
-        live |= w;
-        for (uint64_t b = w; b; b &= b - 1) atomicAdd(&s_lane[__ffsll((long long)b) - 1], (unsigned long long)d);
-    }
-    live = g5_wave_or(live);
-    if (__lane_id() == 0) s_live[threadIdx.x >> 6] = live;
-    block_add(cnt + kUnitSlots * kPushUnit + kNextVerts, {nv, ne});  // its barriers order s_lane, s_live
-    if (threadIdx.x == 0) {
-        uint64_t t = 0;
+    const int64_t units = queue_units(nwords);
+    for (int64_t unit = blockIdx.x; unit < units; unit += gridDim.x) {
+        const int64_t w0 = unit * kUnitWords + wv * W;
+        uint64_t word = 0;  // lane k < W: word w0 + k
+        if (lane < W && w0 + lane < nwords) word = bits[w0 + lane];
+        const bool any = __ballot(word != 0) != 0;
+        uint32_t deg[W];
+        unsigned long long sum = 0;
+        if (any) {
+            int64_t lo[W], hi[W];
+            uint64_t x[W];
 #pragma unroll
-        for (int w = 0; w < kBlock / 64; ++w) t |= s_live[w];
-        if (t) atomicOr((unsigned long long *)&cnt[(blockIdx.x % kStripes) * kCntStride + kLive], (unsigned long long)t);
+            for (int k = 0; k < W; ++k) {
+                const int64_t v = (w0 + k) * 64 + lane;
+                const bool mine = lane_read64(word, k) >> lane & 1;
+                if (kKind != 2) {
+                    lo[k] = mine ? rowptr[v] : 0;
+                    hi[k] = mine ? rowptr[v + 1] : 0;
+                }
+                if (kKind != 0) x[k] = mine ? next[v] & lm : 0ull;
+            }
+#pragma unroll
+            for (int k = 0; k < W; ++k) {
+                const int64_t v = (w0 + k) * 64 + lane;
+                const bool mine = lane_read64(word, k) >> lane & 1;
+                if (kKind != 2) {
+                    deg[k] = (uint32_t)(hi[k] - lo[k]);
+                    sum += mine ? 1ull << kQueueEdgeBits | deg[k] : 0ull;
+                }
+                if (kKind != 0 && mine) {
+                    visited[v] |= x[k];
+                    nbits += __popcll(x[k]);
+                    ++nv;
+                    if (kKind == 1) {
+                        ne += deg[k];
+                        live |= x[k];
+                    }
+                }
+            }
+        }
+        if (kKind == 2) continue;
+        const unsigned long long inc = (unsigned long long)g5_wave_incl_scan((int64_t)sum);
+        if (lane == 63) s_wave[wv] = inc;
+        __syncthreads();
+        unsigned long long before = inc - sum, all = 0;
+#pragma unroll
+        for (int k = 0; k < kBlock / 64; ++k) {
+            before += k < wv ? s_wave[k] : 0ull;
+            all += s_wave[k];
+        }
+        const int g = (int)(unit * kGroups / units);
+        if (all) {
+            if (threadIdx.x == 0) s_at = atomicAdd(&q.tot[g].x, all);
+            __syncthreads();
+            before += s_at;
+            int64_t pos = part_base(q, g) + (int64_t)(before >> kQueueEdgeBits);
+            int64_t off = (int64_t)(before & ((1ull << kQueueEdgeBits) - 1));
+            if (any) {
+#pragma unroll
+                for (int k = 0; k < W; ++k)
+                    if (lane_read64(word, k) >> lane & 1) {
+                        q.v[pos] = (uint32_t)((w0 + k) * 64 + lane);
+                        q.off[pos] = off;
+                        ++pos;
+                        off += deg[k];
+                    }
+            }
+        }
+        __syncthreads();  // s_wave is rewritten by the next unit
     }
-    if (threadIdx.x < 64 && s_lane[threadIdx.x])
-        atomicAdd((unsigned long long *)&lane_edges[(blockIdx.x % kLaneStripes) * 64 + threadIdx.x],
-                  s_lane[threadIdx.x]);
+    if (kKind == 2) block_add(cnt + kUnitSlots * kPushUnit, {nbits, (int64_t)0, nv});
+    if (kKind == 1) {
+        live = g5_wave_or(live);
+        if (lane == 0) s_live[wv] = live;
+        // its barrier orders s_live
+        block_add(cnt + kUnitSlots * kPushUnit, {nbits, (int64_t)0, nv, (int64_t)0, nv, ne});
+        if (threadIdx.x == 0) {
+            uint64_t t = 0;
+#pragma unroll
+            for (int k = 0; k < kBlock / 64; ++k) t |= s_live[k];
+            if (t)
+                atomicOr((unsigned long long *)&cnt[(blockIdx.x % kStripes) * kCntStride + kLive],
+                         (unsigned long long)t);
+        }
+    }
 }
 
-// visited |= next over the newly reached queue, and the push unit's counts
-// (lanes lm only)
-__global__ __launch_bounds__(kBlock) void k_push_commit(const uint32_t *__restrict__ nq,
-                                                        const uint64_t *__restrict__ next,
-                                                        uint64_t *__restrict__ visited, int64_t *__restrict__ cnt,
-                                                        uint64_t lm)
-{
-    const int64_t n = cnt[kNq];
-    int64_t nbits = 0, nv = 0;
-    for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
-        const uint32_t v = nq[i];
-        const uint64_t w = next[v] & lm;
-        visited[v] |= w;
-        nbits += __popcll(w);
-        ++nv;
-    }
-    block_add(cnt + kUnitSlots * kPushUnit, {nbits, (int64_t)0, nv});
-}
-
-// one workgroup of kBlock threads: clear every stripe's accumulated slots
+// one workgroup of kBlock threads: clear every stripe's accumulated slots (the
+// first level's; every level's end leaves them clear for the next)
 __global__ void k_level_begin(int64_t *cnt, int64_t *lane_edges)
 {
     for (int i = threadIdx.x; i < kStripes * kCntStride; i += blockDim.x)
         if (i % kCntStride < kAccum) cnt[i] = 0;
     for (int i = threadIdx.x; i < kLaneStripes * 64; i += blockDim.x) lane_edges[i] = 0;
-    if (threadIdx.x == 0) cnt[kNq] = 0;
 }
 
 // active[w] bit i = ((next[64w + i] & lm) != 0).  A wave takes four
@@ -1203,27 +1377,54 @@ __global__ void k_set_pull_lanes(int64_t *cnt, uint64_t lanes, uint64_t thread_l
     cnt[kFlagWord] = flag_word;
 }
 
-// one workgroup: fold the stripes into stripe 0, then advance the level
-// ... and the per-lane frontier edges, summed over their stripes, into
-// slots [kCntStride, kCntStride + 64) (stripes 1 and 2, free once folded),
-// so that one copy of kHostSlots slots brings the level's counters home
-__global__ void k_level_end(int64_t *cnt, const int64_t *lane_edges)
+// one workgroup: the stripes' and the per-lane edges' sums, the pushed queue's
+// totals (when there was one) and the set-once slots go to the host's counters,
+// in pinned memory; the stripes are clear again, the level advances
+__global__ __launch_bounds__(kBlock) void k_level_end(int64_t *cnt, int64_t *lane_edges,
+                                                      const QueueTotal *__restrict__ pushed, int64_t *__restrict__ host)
 {
-    for (int i = threadIdx.x; i < kAccum; i += blockDim.x) {
-        int64_t t = 0;
-        if (i == kLive)
-            for (int st = 0; st < kStripes; ++st) t |= cnt[st * kCntStride + i];
-        else
-            for (int st = 0; st < kStripes; ++st) t += cnt[st * kCntStride + i];
-        cnt[i] = t;
-    }
-    if (threadIdx.x == 0) cnt[kDepth] += 1;
+    static_assert(kAccum <= kBlock / 2 && kStripes % 8 == 0 && kLaneStripes == 8, "fold");
+    // a thread per slot and 8 stripes, all loads in flight at once
+    __shared__ unsigned long long s_acc[kCntStride];
+    if (threadIdx.x < kCntStride) s_acc[threadIdx.x] = 0;
     __syncthreads();
-    for (int r = threadIdx.x; r < 64; r += blockDim.x) {
-        int64_t t = 0;
-        for (int st = 0; st < kLaneStripes; ++st) t += lane_edges[st * 64 + r];
-        cnt[kCntStride + r] = t;
+    for (int i = threadIdx.x; i < kAccum * (kStripes / 8); i += kBlock) {
+        const int slot = i % kAccum, st = i / kAccum * 8;
+        int64_t x[8], t = 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) x[k] = cnt[(st + k) * kCntStride + slot];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) t = slot == kLive ? t | x[k] : t + x[k];
+        if (slot == kLive) atomicOr(&s_acc[slot], (unsigned long long)t);
+        else if (t) atomicAdd(&s_acc[slot], (unsigned long long)t);
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (x[k]) cnt[(st + k) * kCntStride + slot] = 0;
     }
+    if (threadIdx.x < 64) {
+        int64_t x[8], t = 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) x[k] = lane_edges[k * 64 + threadIdx.x];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            t += x[k];
+            if (x[k]) lane_edges[k * 64 + threadIdx.x] = 0;
+        }
+        host[kCntStride + threadIdx.x] = t;
+    }
+    if (threadIdx.x >= 64 && threadIdx.x < 128) {  // the second wave
+        const int g = threadIdx.x - 64;
+        const unsigned long long x = pushed && g < kGroups ? pushed[g].x : 0ull;
+        const int64_t n = g5_wave_sum((int64_t)(x >> kQueueEdgeBits));
+        const int64_t m = g5_wave_sum((int64_t)(x & ((1ull << kQueueEdgeBits) - 1)));
+        if (g == 0) {
+            host[kFqLen] = n;
+            host[kFqEdges] = m;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < kAccum) host[threadIdx.x] = (int64_t)s_acc[threadIdx.x];
+    if (threadIdx.x == 0) cnt[kDepth] += 1;
 }
 
 // visited := unused lanes, both active bitmaps := 0 and, unless the caller
@@ -1761,7 +1962,6 @@ int level_launches(g5_msbfs *m, hipStream_t s, int p, bool act_check, bool prof 
     uint64_t *next = p == 0 ? m->d_fb : m->d_fa;
     const int64_t nw = m->n / 64;
     uint64_t *act_next = m->d_act + (p == 0 ? nw : 0);
-    hipLaunchKernelGGL(k_level_begin, 1, kBlock, 0, s, m->d_cnt, m->d_lane);
     pull_bins(m, s, p, act_check, prof, m->rl.bin_first);
     // the thread kernel wrote its words of the active bitmap; the block and
     // wave bins' words (and the live lanes among them) come from next
@@ -1769,147 +1969,122 @@ int level_launches(g5_msbfs *m, hipStream_t s, int p, bool act_check, bool prof 
     if (nw01)
         hipLaunchKernelGGL((k_build_active<false, true>), g5::grid_for(nw01, 16, 4096), kBlock, 0, s,
                            (const uint64_t *)next, nw01, (const int64_t *)m->rl.rowptr, act_next, m->d_cnt, ~0ull);
-    hipLaunchKernelGGL(k_level_end, 1, kBlock, 0, s, m->d_cnt, (const int64_t *)m->d_lane);
+    hipLaunchKernelGGL(k_level_end, 1, kBlock, 0, s, m->d_cnt, m->d_lane, (const QueueTotal *)nullptr, m->h_cnt);
     return hipGetLastError() == hipSuccess ? G5_OK : G5_E_HIP;
 }
 
-// The push kernels for the frontier lanes lm of parity p, after next has been
-// cleared (push level) or written by the pull kernels for the other lanes
-// (split level).  `act_front` holds the frontier's active bitmap restricted
-// to lm, fq_bound bounds its vertex count and fq receives its queue.  Ends
-// with next's active bitmap, the next frontier's counts and each lane's
-// frontier edges.  A push level (lm = every lane) finds its newly reached
-// vertices as it goes -- the edge that makes next[v] non-zero sets v's
-// active bit, in act_next cleared beforehand -- and counts them from their
-// queue, so it makes no pass over all n words; a split level builds the
-// bitmaps from next, and its newly reached vertices are those of the block
-// and wave bins.  When those bins' vertices times the pushed lanes fit in n
-// words, a split level takes the candidate path instead of the two passes:
-// one pass lowers per-pair candidates (push_cand) and k_cand_commit writes
-// the pairs out.
-int push_lanes(g5_msbfs *m, hipStream_t s, int p, const uint64_t *act_front, int64_t fq_bound, uint64_t lm,
-               uint32_t *fq)
+// queue i of the engine
+PushQueue push_queue(const g5_msbfs *m, int i)
+{
+    return PushQueue{m->d_qv[i], m->d_qo[i], m->d_qt + i * kGroups, queue_units(m->n / 64)};
+}
+
+PushArgs push_args(const g5_msbfs *m, int p)
 {
     const Relabeled &R = m->rl;
-    const uint64_t *front = p == 0 ? m->d_fa : m->d_fb;
-    uint64_t *next = p == 0 ? m->d_fb : m->d_fa;
-    const int64_t nw = m->n / 64;
-    uint64_t *act_next = m->d_act + (p == 0 ? nw : 0);
-    const bool whole = lm == ~0ull;
-    // a split level pushes only into the block and wave bins: the thread
-    // kernel pulls every lane of its vertices
-    const int64_t vend = whole ? m->n : R.split_first[2];
-    const int64_t nw_push = whole ? nw : (vend + 63) / 64;
-    G5_HIP(g5::bitmap_to_queue(act_front, nw, fq, m->d_cnt + kFqLen, m->d_scratch, s));
-    hipLaunchKernelGGL(k_fq_degrees, g5::grid_for(fq_bound, 256, 8192), 256, 0, s, (const uint32_t *)fq,
-                       (const int64_t *)m->d_cnt, (const int64_t *)R.rowptr, m->d_qoff, fq_bound);
-    G5_HIP(g5::exclusive_scan_i64(m->d_qoff, fq_bound, m->d_cnt + kFqEdges, m->d_scratch, s));
-    if (whole) G5_HIP(g5::fill_u64(act_next, nw, 0, s));
-    // a split level with few pushed lanes: one candidate pass into the newly
-    // reached queue's buffer (n words; idle on split levels) and a commit
-    const int npm = __builtin_popcountll(lm);
-    if (!whole && vend * npm <= m->n) {
-        uint32_t *cand = m->d_nq;
-        if (vend) {
-            G5_HIP(g5::fill_u32(cand, vend * npm, ~0u, s));
-            hipLaunchKernelGGL((k_push_edges<false, true>), kPushGrid, kBlock, 0, s, (const uint32_t *)fq,
-                               (const int64_t *)m->d_qoff, (const int64_t *)R.rowptr, (const uint32_t *)R.cols,
-                               (const uint32_t *)R.cols_orig, (const uint32_t *)R.new2old,
-                               (const uint64_t *)m->d_visited, front, next, m->d_parent, m->d_level, m->d_cnt, lm,
-                               (uint64_t *)nullptr, vend, cand, npm);
-            hipLaunchKernelGGL(k_cand_commit, g5::grid_for(vend, kBlock, 4096), kBlock, 0, s, (const uint32_t *)cand,
-                               npm, lm, vend, (const uint32_t *)R.new2old, next, m->d_visited, m->d_parent,
-                               m->d_level, m->d_cnt);
-        }
-        if (nw_push)
-            hipLaunchKernelGGL((k_build_active<true, true>), g5::grid_for(nw_push, 16, 4096), kBlock, 0, s,
-                               (const uint64_t *)next, nw_push, (const int64_t *)R.rowptr, act_next, m->d_cnt, ~0ull);
-        return hipGetLastError() == hipSuccess ? G5_OK : G5_E_HIP;
-    }
-    hipLaunchKernelGGL(k_push_edges<false>, kPushGrid, kBlock, 0, s, (const uint32_t *)fq,
-                       (const int64_t *)m->d_qoff, (const int64_t *)R.rowptr, (const uint32_t *)R.cols,
-                       (const uint32_t *)R.cols_orig, (const uint32_t *)R.new2old, (const uint64_t *)m->d_visited,
-                       front, next, m->d_parent,
-                       m->d_level, m->d_cnt, lm, whole ? act_next : (uint64_t *)nullptr, vend);
-    // the newly reached vertices of the lanes lm
-    if (!whole && nw_push)
-        hipLaunchKernelGGL((k_build_active<false, false>), g5::grid_for(nw_push, 16, 4096), kBlock, 0, s,
-                           (const uint64_t *)next, nw_push, (const int64_t *)R.rowptr, act_next, m->d_cnt, lm);
-    G5_HIP(g5::bitmap_to_queue(act_next, nw_push, m->d_nq, m->d_cnt + kNq, m->d_scratch, s));
-    if (whole)
-        hipLaunchKernelGGL(k_nq_counts, g5::grid_for(m->n, kBlock, 2048), kBlock, 0, s, (const uint32_t *)m->d_nq,
-                           (const uint64_t *)next, (const int64_t *)R.rowptr, m->d_cnt, m->d_lane);
-    hipLaunchKernelGGL(k_push_edges<true>, kPushGrid, kBlock, 0, s, (const uint32_t *)fq,
-                       (const int64_t *)m->d_qoff, (const int64_t *)R.rowptr, (const uint32_t *)R.cols,
-                       (const uint32_t *)R.cols_orig, (const uint32_t *)R.new2old, (const uint64_t *)m->d_visited,
-                       front, next, m->d_parent,
-                       m->d_level, m->d_cnt, lm, (uint64_t *)nullptr, vend, (uint32_t *)nullptr, 0, whole);
-    if (whole)
-        hipLaunchKernelGGL(k_min_rows, kPushVertGrid, kBlock, 0, s, (const uint32_t *)m->d_nq,
-                           (const int64_t *)R.rowptr, (const uint32_t *)R.cols, (const uint32_t *)R.cols_orig,
-                           (const uint32_t *)R.new2old, front, (const uint64_t *)next, m->d_parent,
-                           (const int64_t *)m->d_cnt);
-    hipLaunchKernelGGL(k_push_commit, kPushVertGrid, kBlock, 0, s, (const uint32_t *)m->d_nq,
-                       (const uint64_t *)next, m->d_visited, m->d_cnt, lm);
-    // the block and wave bins' part of the next frontier: active bitmap,
-    // counts, live lanes (the thread kernel has done its own bin's)
-    if (!whole && nw_push)
-        hipLaunchKernelGGL((k_build_active<true, true>), g5::grid_for(nw_push, 16, 4096), kBlock, 0, s,
-                           (const uint64_t *)next, nw_push, (const int64_t *)R.rowptr, act_next, m->d_cnt, ~0ull);
-    return hipGetLastError() == hipSuccess ? G5_OK : G5_E_HIP;
+    return PushArgs{R.rowptr, R.cols, R.cols_orig, R.new2old, m->d_visited, p == 0 ? m->d_fa : m->d_fb,
+                    p == 0 ? m->d_fb : m->d_fa, m->d_parent, m->d_level};
 }
 
-// One push level on parity p: direct launches (the frontier queue's length
-// sizes the degree scan on the host).  fqn = active vertices of the frontier.
-// next is cleared entry by entry when the level before was a push level too
-// (its frontier queue lists the only non-zero words of this level's next:
-// listed_in) and the list is short; otherwise by a fill of all n words.  The two push
-// queue buffers alternate, so that list survives into this level.
-int push_level(g5_msbfs *m, hipStream_t s, int p, int64_t fqn, bool listed_in, bool prof)
+unsigned queue_grid(int64_t nwords) { return (unsigned)g5::grid_for(queue_units(nwords), 1, kPushVertGrid); }
+
+// One push level on parity p.  fqn = active vertices of the frontier.
+// It starts with next's active bitmap and next itself clear -- entry by entry
+// when the level before was a push level too (its frontier queue lists the
+// only non-zero words of this level's next: listed_in) and the list is short,
+// otherwise whole -- and with the frontier's queue, which the level before
+// left if it pushed.  The edge that makes next[v] non-zero sets v's active
+// bit; k_queue then commits and counts the vertices of that bitmap and leaves
+// their queue, the next level's frontier's, so a push level makes no pass over
+// all n words.  Six launches or five (19 with separate queue, degree, prefix,
+// count and commit passes: a batch's four push levels at scale 16 took 260 us,
+// now 160).
+int push_level(g5_msbfs *m, hipStream_t s, int p, bool listed_in, bool queue_in, bool prof)
 {
-    uint64_t *next = p == 0 ? m->d_fb : m->d_fa;
+    const Relabeled &R = m->rl;
     const int64_t nw = m->n / 64;
     const uint64_t *act = m->d_act + (p == 0 ? 0 : nw);
-    hipLaunchKernelGGL(k_level_begin, 1, kBlock, 0, s, m->d_cnt, m->d_lane);
-    if (listed_in && m->listed_len * kListedFrac < m->n) {
-        if (m->listed_len)
-            hipLaunchKernelGGL(k_zero_listed, g5::grid_for(m->listed_len, 256, 4096), 256, 0, s, next,
-                               (const uint32_t *)m->listed, m->listed_len);
-    } else {
-        G5_HIP(g5::fill_u64(next, m->n, 0, s));
-    }
+    uint64_t *act_next = m->d_act + (p == 0 ? nw : 0);
+    const PushArgs a = push_args(m, p);
+    const PushQueue q = push_queue(m, 1 - m->listed), nq = push_queue(m, m->listed);
+    const bool whole = !(listed_in && m->listed_len * kListedFrac < m->n);
+    hipLaunchKernelGGL(k_push_begin, g5::grid_for(whole ? m->n : std::max(nw, m->listed_len), 256, 4096), 256, 0, s,
+                       act_next, nw, a.next, m->n, whole, m->listed_len ? nq : PushQueue{},
+                       queue_in ? (QueueTotal *)nullptr : q.tot);
     if (prof) G5_HIP(hipEventRecord(m->ek[0], s));
-    uint32_t *fq = m->listed == m->d_fq ? m->d_fq2 : m->d_fq;
-    int rc = push_lanes(m, s, p, act, fqn, ~0ull, fq);
-    if (rc) return rc;
-    m->listed = fq;
+    if (!queue_in)
+        hipLaunchKernelGGL(k_queue<0>, queue_grid(nw), kBlock, 0, s, act, nw, (const int64_t *)R.rowptr, q,
+                           (const uint64_t *)nullptr, (uint64_t *)nullptr, ~0ull, m->d_cnt);
+    hipLaunchKernelGGL(k_push_edges<false>, kPushGrid, kBlock, 0, s, a, q, m->d_cnt, ~0ull, act_next, m->n,
+                       (uint32_t *)nullptr, 0, nq.tot);
+    hipLaunchKernelGGL(k_queue<1>, queue_grid(nw), kBlock, 0, s, (const uint64_t *)act_next, nw,
+                       (const int64_t *)R.rowptr, nq, (const uint64_t *)a.next, m->d_visited, ~0ull, m->d_cnt);
+    hipLaunchKernelGGL(k_push_min, kPushGrid, kBlock, 0, s, a, q, nq, (const int64_t *)m->d_cnt, ~0ull, m->n, true,
+                       m->d_lane);
     if (prof) G5_HIP(hipEventRecord(m->ek[1], s));
-    hipLaunchKernelGGL(k_level_end, 1, kBlock, 0, s, m->d_cnt, (const int64_t *)m->d_lane);
+    hipLaunchKernelGGL(k_level_end, 1, kBlock, 0, s, m->d_cnt, m->d_lane, (const QueueTotal *)q.tot, m->h_cnt);
     G5_HIP(hipGetLastError());
+    m->listed = 1 - m->listed;  // q lists the buffer that the next push level writes
     return G5_OK;
 }
 
 // One split level on parity p: the block and wave kernels on the lanes in
-// cnt[kPullLanes] and the thread kernel on every frontier lane, then the
-// push kernels on the lanes pm (disjoint from cnt[kPullLanes]) into the
-// block and wave bins only.  fqn = active vertices of the whole frontier.
-int split_level(g5_msbfs *m, hipStream_t s, int p, uint64_t pm, bool act_check, int64_t fqn, bool prof)
+// cnt[kPullLanes] and the thread kernel on every frontier lane, then the push
+// kernels on the lanes pm (disjoint from cnt[kPullLanes]) into the block and
+// wave bins only (the thread kernel pulls every lane of its vertices), which
+// the pull kernels have written for the other lanes.  When those bins'
+// vertices times the pushed lanes fit in n words, one pass lowers per-pair
+// candidates (push_cand) and k_cand_commit writes the pairs out; otherwise the
+// passes of a push level run.  Ends with the bins' part of next's active
+// bitmap, counts and live lanes.
+int split_level(g5_msbfs *m, hipStream_t s, int p, uint64_t pm, bool act_check, bool prof)
 {
-    const uint64_t *front = p == 0 ? m->d_fa : m->d_fb;
+    const Relabeled &R = m->rl;
     const int64_t nw = m->n / 64;
     uint64_t *act_cur = m->d_act + (p == 0 ? 0 : nw);
-    hipLaunchKernelGGL(k_level_begin, 1, kBlock, 0, s, m->d_cnt, m->d_lane);
-    pull_bins(m, s, p, act_check, prof, m->rl.split_first);
+    uint64_t *act_next = m->d_act + (p == 0 ? nw : 0);
+    const PushArgs a = push_args(m, p);
+    const PushQueue q = push_queue(m, 1 - m->listed);
+    uint32_t *cand = m->d_qv[m->listed];  // the other queue, of one entry per vertex, holds the candidates
+    pull_bins(m, s, p, act_check, prof, R.split_first);
     if (prof) G5_HIP(hipEventRecord(m->ek_push[0], s));
     // the frontier vertices with a pushed lane, in the frontier's own active
     // bitmap (the pull kernels are done with it; the thread kernel has
     // written its words of act_next)
-    hipLaunchKernelGGL((k_build_active<false, false>), g5::grid_for(nw, 16, 4096), kBlock, 0, s, front, nw,
-                       (const int64_t *)m->rl.rowptr, act_cur, m->d_cnt, pm);
-    int rc = push_lanes(m, s, p, act_cur, fqn, pm, m->listed == m->d_fq ? m->d_fq2 : m->d_fq);
-    if (rc) return rc;
+    hipLaunchKernelGGL((k_build_active<false, false>), g5::grid_for(nw, 16, 4096), kBlock, 0, s, a.frontier, nw,
+                       (const int64_t *)R.rowptr, act_cur, m->d_cnt, pm);
+    hipLaunchKernelGGL(k_push_begin, 1, 256, 0, s, (uint64_t *)nullptr, (int64_t)0, (uint64_t *)nullptr, (int64_t)0,
+                       true, PushQueue{}, q.tot);
+    hipLaunchKernelGGL(k_queue<0>, queue_grid(nw), kBlock, 0, s, (const uint64_t *)act_cur, nw,
+                       (const int64_t *)R.rowptr, q, (const uint64_t *)nullptr, (uint64_t *)nullptr, ~0ull, m->d_cnt);
+    const int64_t vend = R.split_first[2], nw_push = (vend + 63) / 64;
+    const int npm = __builtin_popcountll(pm);
+    if (vend * npm <= m->n) {
+        if (vend) {
+            G5_HIP(g5::fill_u32(cand, vend * npm, ~0u, s));
+            hipLaunchKernelGGL(k_push_edges<true>, kPushGrid, kBlock, 0, s, a, q, m->d_cnt, pm, (uint64_t *)nullptr,
+                               vend, cand, npm, (QueueTotal *)nullptr);
+            hipLaunchKernelGGL(k_cand_commit, g5::grid_for(vend, kBlock, 4096), kBlock, 0, s, (const uint32_t *)cand,
+                               npm, pm, vend, (const uint32_t *)R.new2old, a.next, m->d_visited, m->d_parent,
+                               m->d_level, m->d_cnt);
+        }
+    } else {
+        hipLaunchKernelGGL(k_push_edges<false>, kPushGrid, kBlock, 0, s, a, q, m->d_cnt, pm, (uint64_t *)nullptr, vend,
+                           (uint32_t *)nullptr, 0, (QueueTotal *)nullptr);
+        // the newly reached vertices of the lanes pm
+        hipLaunchKernelGGL((k_build_active<false, false>), g5::grid_for(nw_push, 16, 4096), kBlock, 0, s,
+                           (const uint64_t *)a.next, nw_push, (const int64_t *)R.rowptr, act_next, m->d_cnt, pm);
+        hipLaunchKernelGGL(k_queue<2>, queue_grid(nw_push), kBlock, 0, s, (const uint64_t *)act_next, nw_push,
+                           (const int64_t *)R.rowptr, PushQueue{}, (const uint64_t *)a.next, m->d_visited, pm,
+                           m->d_cnt);
+        hipLaunchKernelGGL(k_push_min, kPushGrid, kBlock, 0, s, a, q, PushQueue{}, (const int64_t *)m->d_cnt, pm, vend,
+                           false, m->d_lane);
+    }
+    if (nw_push)
+        hipLaunchKernelGGL((k_build_active<true, true>), g5::grid_for(nw_push, 16, 4096), kBlock, 0, s,
+                           (const uint64_t *)a.next, nw_push, (const int64_t *)R.rowptr, act_next, m->d_cnt, ~0ull);
     if (prof) G5_HIP(hipEventRecord(m->ek_push[1], s));
-    hipLaunchKernelGGL(k_level_end, 1, kBlock, 0, s, m->d_cnt, (const int64_t *)m->d_lane);
+    hipLaunchKernelGGL(k_level_end, 1, kBlock, 0, s, m->d_cnt, m->d_lane, (const QueueTotal *)q.tot, m->h_cnt);
     G5_HIP(hipGetLastError());
     return G5_OK;
 }
@@ -2077,8 +2252,8 @@ int run_level(g5_msbfs *m, int64_t *new_bits_out, uint64_t *live_out)
     hipStream_t s = m->s;
     const int p = m->p;
     // until this level completes, the buffers' state is not known
-    const bool listed_in = m->listed_ok;
-    m->listed_ok = false;
+    const bool listed_in = m->listed_ok, queue_in = m->queue_ok;
+    m->listed_ok = m->queue_ok = false;
     m->last_empty = false;
     const int64_t act_verts = m->act_verts, act_edges = m->act_edges;
     const int64_t nnz = m->g->nnz;
@@ -2086,13 +2261,13 @@ int run_level(g5_msbfs *m, int64_t *new_bits_out, uint64_t *live_out)
     const bool act_check = act_edges < 0 || act_edges * m->tune.active_ratio < nnz;
     const uint64_t pm = push ? 0 : split_lanes(m);
     if (push) {
-        int rc = push_level(m, s, p, act_verts, listed_in, m->prof);
+        int rc = push_level(m, s, p, listed_in, queue_in, m->prof);
         if (rc) return rc;
     } else {
         hipLaunchKernelGGL(k_set_pull_lanes, 1, 1, 0, s, m->d_cnt, m->front_lanes & ~pm, m->front_lanes, used_lanes(m),
                            m->flag_word, pm ? (int64_t)64 : (int64_t)kWaveFirst);
         if (pm) {
-            int rc = split_level(m, s, p, pm, act_check, act_verts, m->prof);
+            int rc = split_level(m, s, p, pm, act_check, m->prof);
             if (rc) return rc;
         } else if (m->prof) {
             int rc = level_launches(m, s, p, act_check, true);
@@ -2101,8 +2276,7 @@ int run_level(g5_msbfs *m, int64_t *new_bits_out, uint64_t *live_out)
             G5_HIP(hipGraphLaunch(m->graph[p][act_check ? 1 : 0], s));
         }
     }
-    G5_HIP(hipMemcpyAsync(m->h_cnt, m->d_cnt, kHostSlots * 8, hipMemcpyDeviceToHost, s));
-    G5_HIP(hipStreamSynchronize(s));
+    G5_HIP(hipStreamSynchronize(s));  // k_level_end has written h_cnt
     int64_t new_bits = 0;
     const int64_t *h = m->h_cnt;
     int64_t next_verts = 0, next_edges = 0;
@@ -2117,7 +2291,7 @@ int run_level(g5_msbfs *m, int64_t *new_bits_out, uint64_t *live_out)
     m->lane_known = push ? ~0ull : 0ull;
     if (push)
         for (int r = 0; r < 64; ++r) m->lane_edges[r] = h[kCntStride + r];
-    m->listed_ok = push;
+    m->listed_ok = m->queue_ok = push;
     m->listed_len = push ? h[kFqLen] : 0;
     m->last_empty = new_bits == 0;
     m->split_ok = push;
@@ -2207,10 +2381,12 @@ extern "C" int g5_msbfs_create(g5_graph *g, g5_msbfs **out)
     if (e == hipSuccess) e = hipMalloc(&m->d_fb, (size_t)n * 8);
     if (e == hipSuccess) e = hipMalloc(&m->d_act, (size_t)(n / 64) * 2 * 8);
     if (e == hipSuccess) e = hipMalloc(&m->d_lvflag, (size_t)std::max<int64_t>(n / 64, 1) * 8);
-    if (e == hipSuccess) e = hipMalloc(&m->d_fq, (size_t)n * 4);
-    if (e == hipSuccess) e = hipMalloc(&m->d_fq2, (size_t)n * 4);
-    if (e == hipSuccess) e = hipMalloc(&m->d_nq, (size_t)n * 4);
-    if (e == hipSuccess) e = hipMalloc(&m->d_qoff, (size_t)(n + 1) * 8);
+    const int64_t nq = queue_units(n / 64) * (kUnitWords * 64);  // a queue's entries
+    for (int k = 0; k < 2; ++k) {
+        if (e == hipSuccess) e = hipMalloc(&m->d_qv[k], (size_t)nq * 4);
+        if (e == hipSuccess) e = hipMalloc(&m->d_qo[k], (size_t)nq * 8);
+    }
+    if (e == hipSuccess) e = hipMalloc(&m->d_qt, 2 * kGroups * sizeof(QueueTotal));
     if (e == hipSuccess) e = hipMalloc(&m->d_parent, (size_t)n * 64 * 4);
     if (e == hipSuccess) e = hipMalloc(&m->d_level, (size_t)n * 64);
     if (e == hipSuccess) e = hipMalloc(&m->d_dirty, (size_t)kDirtyCap * 8);
@@ -2251,7 +2427,7 @@ extern "C" int g5_msbfs_footprint(const g5_graph *g, int64_t *graph_bytes, int64
     const int64_t per_lane = 5 * n + (3 * n + 7) / 8;
     const int64_t all = 3 * 8 * n                      // visited, frontier buffers
                         + 3 * (n / 64) * 8             // active bitmaps, level flags
-                        + 3 * 4 * n + 8 * (n + 1)      // push queues, degree prefix
+                        + 2 * 12 * queue_units(n / 64) * (kUnitWords * 64) + 2 * kGroups * (int64_t)sizeof(QueueTotal)  // push queues
                         + 64 * 5 * n                   // parent and level records
                         + kDirtyCap * 8 + kStripes * kCntStride * 8 + kLaneStripes * 64 * 8 +
                         ((int64_t)g5::scan_scratch_words(n + 1) + 16) * 8 + 64 * 12 + 194 * 8 + 128 * 8 +
@@ -2270,10 +2446,10 @@ extern "C" int g5_msbfs_free(g5_msbfs *m)
     for (auto &gp : m->graph)
         for (hipGraphExec_t ge : gp)
             if (ge) (void)hipGraphExecDestroy(ge);
-    void *dev[] = {m->d_fq,      m->d_nq,      m->d_qoff,     m->d_act,   m->d_visited, m->d_fa,
+    void *dev[] = {m->d_qv[0],   m->d_qv[1],   m->d_qo[0],    m->d_qo[1],   m->d_qt,    m->d_act,   m->d_visited, m->d_fa,
                    m->d_fb,      m->d_parent,  m->d_cnt,      m->d_scratch, m->d_roots, m->d_join,
                    m->d_sums,    m->rl.new2old, m->rl.old2new, m->rl.rowptr, m->rl.cols, m->rl.gdeg,
-                   m->d_lane,    m->d_fq2,     m->rl.head,    m->d_level,   m->d_dirty,  m->rl.head_orig,
+                   m->d_lane,    m->rl.head,    m->d_level,   m->d_dirty,  m->rl.head_orig,
                    m->rl.cols_orig, m->d_lvflag};
     for (void *p : dev)
         if (p) (void)hipFree(p);
@@ -2328,10 +2504,11 @@ extern "C" int g5_msbfs_run(g5_msbfs *m, const int64_t *roots, int nroots, int32
     const bool listed = m->listed_ok && m->last_empty && m->listed_len * kListedFrac < m->n;
     hipLaunchKernelGGL(k_ms_init, g5::grid_for(m->n, 256, 16384), 256, 0, s, m->d_visited, m->d_fa, m->d_fb,
                        m->d_act, m->n, unused, !listed);
+    hipLaunchKernelGGL(k_level_begin, 1, kBlock, 0, s, m->d_cnt, m->d_lane);
     if (listed && m->listed_len) {
         uint64_t *last_front = m->p == 0 ? m->d_fb : m->d_fa;  // parity p ^ 1 read it
-        hipLaunchKernelGGL(k_zero_listed, g5::grid_for(m->listed_len, 256, 4096), 256, 0, s, last_front,
-                           (const uint32_t *)m->listed, m->listed_len);
+        hipLaunchKernelGGL(k_push_begin, g5::grid_for(m->listed_len, 256, 4096), 256, 0, s, (uint64_t *)nullptr,
+                           (int64_t)0, last_front, m->n, false, push_queue(m, m->listed), (QueueTotal *)nullptr);
     }
     hipLaunchKernelGGL(k_root_reach, nroots, 256, 0, s, (const int64_t *)d_roots, (const uint32_t *)m->rl.old2new,
                        (const int64_t *)m->rl.rowptr, (const uint32_t *)m->rl.cols, m->d_join);
@@ -2351,6 +2528,7 @@ extern "C" int g5_msbfs_run(g5_msbfs *m, const int64_t *roots, int nroots, int32
     m->split_levels = 0;
     m->listed_ok = true;  // k_ms_init cleared both frontier buffers
     m->listed_len = 0;
+    m->queue_ok = false;
     {
         int64_t tmp[64];
         std::copy(roots, roots + nroots, tmp);
@@ -2394,6 +2572,7 @@ extern "C" int g5_msbfs_open(g5_msbfs *m)
     // keep a vertex from the fully-visited early exit
     hipLaunchKernelGGL(k_ms_init, g5::grid_for(m->n, 256, 16384), 256, 0, s, m->d_visited, m->d_fa, m->d_fb,
                        m->d_act, m->n, ~0ull, true);
+    hipLaunchKernelGGL(k_level_begin, 1, kBlock, 0, s, m->d_cnt, m->d_lane);
     G5_HIP(hipGetLastError());
     G5_HIP(hipStreamSynchronize(s));
     m->cont = true;
@@ -2406,6 +2585,7 @@ extern "C" int g5_msbfs_open(g5_msbfs *m)
     m->front_lanes = 0;
     m->listed_ok = true;  // k_ms_init cleared both frontier buffers
     m->listed_len = 0;
+    m->queue_ok = false;
     m->lane_known = 0;  // no lane has a frontier; joins add theirs
     std::fill(m->lane_edges, m->lane_edges + 64, 0);
     m->split_levels = 0;
@@ -2458,6 +2638,7 @@ extern "C" int g5_msbfs_join(g5_msbfs *m, const int64_t *roots, const int *lanes
         if (added[2 + i]) m->front_lanes |= 1ull << lanes[i];
     }
     m->split_ok = true;
+    m->queue_ok = false;  // the roots are not in it
     m->flag_word = INT64_MAX;
     return G5_OK;
 }
