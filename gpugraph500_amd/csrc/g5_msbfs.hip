@@ -54,8 +54,8 @@
 // are; other bounds move some vertices into a neighbouring bin, which gives
 // the same results): one thread per vertex up to thread_max neighbours, one wavefront
 // (64 neighbours per step, first hits from an exclusive prefix-OR across
-// lanes) up to wave_max, one 256-thread workgroup beyond (Tune; 32 and 2048
-// by default).  Each pull level's launch
+// lanes) up to wave_max, one 256-thread workgroup beyond (Tune; 256 and 2048
+// by default, 32 and 2048 on graphs of fewer than 2^22 stored neighbours).  Each pull level's launch
 // sequence is captured once into a hipGraph per frontier parity and
 // replayed; the level number lives in device memory.
 //
@@ -94,14 +94,27 @@ constexpr int kUnits = kBins + 1;
 constexpr int kBlock = 256;
 constexpr int kLevelRec = 12;  // per level: ms[4], edges[4], new pairs, pushed, frontier vertices, edges
 // Shape parameters (g5_msbfs_tune / g5_msbfs_autotune).  Any values give the
-// same results; they only move work between kernels.
+// same results; they only move work between kernels.  The bounds a search
+// starts with were measured on Kronecker graphs, 64 (and 17) roots each.
+// From 2^22 stored neighbours on, thread_max 256 with split_max 32 is 1.02
+// (scale 17, edgefactor 16), 1.09 (18), 1.14 (20), 1.06 (22), 1.17 (24) times
+// as fast as 32 with 16 (64: 1.01-1.05, 128: 1.04-1.07).  Below it a thread's
+// longer list is a launch's longest chain and too few wavefronts run to hide
+// it: 256 takes 1.08 (scale 16), 1.06 (14) and 1.04 (12) times as long as 32;
+// around the line (scales 15 to 19, edgefactors 64 to 4) the two are within
+// 3 % either way.  lane_ratio 128 is 0.99-1.01 (scale 20 and below), 1.04
+// (22) and 1.07 (24) times as fast as 64; push_ratio 4 to 64 are within 7 %.
+constexpr int64_t kLargeNnz = (int64_t)1 << 22;
+constexpr int64_t kLeastWaveMax = 32;  // of a search whose thread_max was not set
 struct Tune {
     int64_t thread_max = 32;   // degree bound of the thread-per-vertex bin
+    int64_t thread_auto = 32;  // its starting value while the caller has not set
+                               // it (it follows a smaller wave_max), else 0
     int64_t wave_max = 2048;   // degree bound of the wavefront-per-vertex bin
     int64_t push_ratio = 16;   // push when the frontier's edges < nnz / push_ratio
     int64_t active_ratio = 2;  // pull levels consult the active bitmap when the
                                // frontier's edges < nnz / active_ratio
-    int64_t lane_ratio = 64;   // a pull level pushes the lanes whose frontier
+    int64_t lane_ratio = 128;  // a pull level pushes the lanes whose frontier
                                // edges < nnz / lane_ratio (0: never)
     int64_t split_max = 16;    // split levels bound the thread bin at
                                // min(split_max, thread_max)
@@ -2370,6 +2383,10 @@ extern "C" int g5_msbfs_create(g5_graph *g, g5_msbfs **out)
     g5_msbfs *m = new g5_msbfs();
     m->g = g;
     m->n = g->n_rows;
+    if (g->nnz >= kLargeNnz) {
+        m->tune.thread_max = m->tune.thread_auto = 256;
+        m->tune.split_max = 32;
+    }
     const int64_t n = std::max<int64_t>(m->n, 64);
     auto fail = [&](int rc) {
         g5_msbfs_free(m);
@@ -2939,8 +2956,14 @@ extern "C" int g5_msbfs_tune(g5_msbfs *m, int key, int64_t value)
     G5_REQUIRE(slot, G5_E_ARG, "g5_msbfs_tune: unknown key %d", key);
     Tune t = m->tune;
     switch (key) {
-    case G5_TUNE_THREAD_MAX: t.thread_max = value; break;
-    case G5_TUNE_WAVE_MAX: t.wave_max = value; break;
+    case G5_TUNE_THREAD_MAX:
+        t.thread_max = value;
+        t.thread_auto = 0;
+        break;
+    case G5_TUNE_WAVE_MAX:
+        t.wave_max = value;
+        if (t.thread_auto) t.thread_max = std::max(kLeastWaveMax, std::min(t.thread_auto, value));
+        break;
     case G5_TUNE_PUSH_RATIO: t.push_ratio = value; break;
     case G5_TUNE_ACTIVE_RATIO: t.active_ratio = value; break;
     case G5_TUNE_LANE_RATIO: t.lane_ratio = value; break;
@@ -3017,6 +3040,7 @@ extern "C" int g5_msbfs_autotune(g5_msbfs *m, const int64_t *roots, int nroots, 
                                         : &t.split_max;
                 if (*f == v) continue;
                 *f = v;
+                if (key == 0) t.thread_auto = 0;
                 if (t.wave_max < t.thread_max) continue;
                 double ms = 0;
                 rc = measure(t, &ms);

@@ -263,7 +263,7 @@ int g5_msbfs_nedge(g5_msbfs *m, int64_t *nedge);
 int g5_msbfs_set_mode(g5_msbfs *m, int mode);
 /* Per-kernel accounting.  Units 0..2 are the pull kernels of the degree bins
  * (0: workgroup per vertex, degree > 2048; 1: wavefront per vertex,
- * 33..2048; 2: thread per vertex, 1..32), unit 3 the push levels and the
+ * 257..2048; 2: thread per vertex, 1..256), unit 3 the push levels and the
  * pushed lanes of split levels.  Enabling runs pull levels as direct launches timed with
  * events (otherwise each pull level replays a captured hipGraph); bytes are
  * the algorithmic bytes of the unit's launches. */
@@ -294,15 +294,18 @@ int g5_msbfs_info(g5_msbfs *m, int64_t *bins, int cap);
  *                   g5_msbfs_result may be called for a lane before it leaves. */
 /* Shape parameters of the batched search (results never depend on them):
  * G5_TUNE_THREAD_MAX / G5_TUNE_WAVE_MAX bound the degree bins of the
- * thread-per-vertex and wavefront-per-vertex pull kernels (default 32, 2048;
- * higher degrees take a workgroup per vertex); G5_TUNE_PUSH_RATIO pushes a
+ * thread-per-vertex and wavefront-per-vertex pull kernels (default 256, 2048,
+ * or 32, 2048 on graphs of fewer than 2^22 stored neighbours; higher degrees
+ * take a workgroup per vertex; while THREAD_MAX has not been
+ * set it follows a smaller WAVE_MAX, down to 32); G5_TUNE_PUSH_RATIO pushes a
  * level whose frontier edges are below nnz / ratio (16); G5_TUNE_ACTIVE_RATIO
  * makes pull levels consult the active bitmap below nnz / ratio edges (2);
  * G5_TUNE_LANE_RATIO: a pull level that follows a push level pushes the
- * lanes whose frontier edges are below nnz / ratio (64; 0 = never), which
+ * lanes whose frontier edges are below nnz / ratio (128; 0 = never), which
  * stops one lagging root from making every vertex scan its whole list;
  * G5_TUNE_SPLIT_MAX: such split levels bound the thread-per-vertex bin at
- * min(split_max, thread_max) (16), as every row is scanned to its end there.
+ * min(split_max, thread_max) (32, or 16 on graphs of fewer than 2^22
+ * stored neighbours), as every row is scanned to its end there.
  * g5_msbfs_autotune searches these by coordinate descent over candidate
  * values (passes rounds, two timed batch searches of roots per candidate),
  * keeps the fastest and reports its time and the number of candidates run. */

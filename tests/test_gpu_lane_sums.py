@@ -85,3 +85,33 @@ def test_leaving_lanes_match_the_oracle():
         for r, x in zip(roots, lanes):
             pred, lev, _ = O.bfs_bin(ref, r)
             assert int(ne[x]) == O.nedge(ref, lev) and int(ck[x]) == checksum(pred)
+
+
+@pytest.mark.parametrize("scale, edgefactor, thread, split", [(11, 16, 32, 16), (18, 16, 256, 32)])
+def test_thread_bound_follows_a_smaller_wave_bound_until_it_is_set(scale, edgefactor, thread, split):
+    g = g5.Graph.kronecker(scale, edgefactor)
+    m = g5.MSBFS(g)
+    d = m.get_tune()
+    assert (d["thread_max"], d["wave_max"], d["split_max"]) == (thread, 2048, split)
+    roots = [int(r) for r in g.select_roots(g.nglobal, 20)]
+    m.run(roots)
+    want = [m.result(lane) for lane in range(20)]
+
+    def check():
+        m.run(roots)
+        for lane in range(20):
+            pred, lev = m.result(lane)
+            assert np.array_equal(pred, want[lane][0]) and np.array_equal(lev, want[lane][1])
+
+    for wave in (64, 32, 300, 100):
+        m.tune(wave_max=wave)
+        assert m.get_tune()["thread_max"] == min(thread, wave) and m.get_tune()["wave_max"] == wave
+        check()
+    with pytest.raises(g5.G5Error):
+        m.tune(wave_max=31)
+    m.tune(thread_max=8)
+    m.tune(wave_max=16)
+    assert m.get_tune()["thread_max"] == 8
+    check()
+    with pytest.raises(g5.G5Error):
+        m.tune(wave_max=7)
