@@ -34,8 +34,10 @@ namespace {
 constexpr uint32_t kNoParent = 0xFFFFFFFFu;
 constexpr uint32_t kRootMark = 0xFFFFFFFEu;  // parent slot of the root column
 constexpr int kExpandBlock = 256;
-constexpr int kExpandTile = 2048;            // edges per block tile
+constexpr int kExpandTile = 1024;            // edges per block tile
 constexpr int kExpandGrid = 4096;            // persistent grid, grid-stride over tiles
+constexpr int kTileSrc = 512;                // sources of a tile that are staged in LDS
+constexpr int kParts = 4096;                 // workgroups that leave a sum each, at most
 
 // kNewEdges: degree sum of the newly reached vertices (1x1 only); kBuEdges,
 // kBuVerts: neighbours checked and vertices scanned by a bottom-up level;
@@ -70,6 +72,11 @@ struct g5_bfs {
     int64_t *d_scratch = nullptr;
     int64_t *d_cnt = nullptr;
     int64_t *h_cnt = nullptr;     // pinned mirror of d_cnt
+    int64_t *d_part = nullptr;    // the workgroups' sums, 4 x kParts
+    // the frontier's queue is in d_queue with its length in cnt[kQLen]; its
+    // degree prefix in d_qoff with the total in cnt[kEdges].  Without a queue
+    // the frontier is in d_inbits
+    bool queue_ok = false, qoff_ok = false;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     g5::S4Codec codec;
     uint32_t *d_words = nullptr;  // codec stream for G5_RUN_CODEC
@@ -117,91 +124,173 @@ __device__ __forceinline__ int64_t src_of(const int64_t *__restrict__ qoff, int6
     return lo;
 }
 
-__global__ void k_queue_degrees(const uint32_t *__restrict__ q, const int64_t *__restrict__ d_qlen,
-                                const int64_t *__restrict__ rowptr, int64_t *__restrict__ qoff)
+// A queue given by the host: its degrees (for the prefix), its length, and the
+// out-bitmap cleared for the expansion.
+__global__ __launch_bounds__(256) void k_queue_degrees(const uint32_t *__restrict__ q, int64_t n,
+                                                       const int64_t *__restrict__ rowptr,
+                                                       int64_t *__restrict__ qoff, int64_t *__restrict__ cnt,
+                                                       uint64_t *__restrict__ out, int64_t wc)
 {
-    const int64_t n = *d_qlen;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = t; i < n; i += stride) {
         const uint32_t u = q[i];
         qoff[i] = rowptr[u + 1] - rowptr[u];
     }
+    for (int64_t w = t; w < wc; w += stride) out[w] = 0;
+    if (t == 0) cnt[kQLen] = n;
 }
 
+// The sources of the edges [t0, t1) of a queue with its degree prefix: the
+// first and the last by two waves' searches, all of them staged in LDS if they
+// are few (two edges and more each on average).  All 256 threads call it.
+struct TileSrc {
+    int64_t lo, hi;
+    bool staged;
+};
+__device__ __forceinline__ TileSrc stage_sources(const uint32_t *__restrict__ q, const int64_t *__restrict__ qoff,
+                                                 int64_t qn, const int64_t *__restrict__ rowptr, int64_t t0,
+                                                 int64_t t1, int64_t *s_range, int32_t *s_off, uint32_t *s_u,
+                                                 int64_t *s_rb)
+{
+    if (threadIdx.x < 128) {
+        const int64_t r = g5_wave_src_of(qoff, 0, qn - 1, threadIdx.x < 64 ? t0 : t1 - 1);
+        if ((threadIdx.x & 63) == 0) s_range[threadIdx.x >> 6] = r;
+    }
+    __syncthreads();
+    TileSrc t;
+    t.lo = s_range[0];
+    t.hi = s_range[1];
+    t.staged = t.hi - t.lo < kTileSrc;
+    if (t.staged)
+        for (int j = threadIdx.x; j <= (int)(t.hi - t.lo); j += 256) {
+            const uint32_t u = q[t.lo + j];
+            const int64_t o = qoff[t.lo + j];
+            s_u[j] = u;
+            s_rb[j] = rowptr[u] - o;
+            s_off[j] = (int32_t)max(o - t0, (int64_t)-1);
+        }
+    __syncthreads();
+    return t;
+}
+// the source of edge e, and the edge's place in the columns
+__device__ __forceinline__ uint32_t edge_source(const TileSrc &t, const uint32_t *__restrict__ q,
+                                                const int64_t *__restrict__ qoff,
+                                                const int64_t *__restrict__ rowptr, int64_t t0, int64_t e,
+                                                const int32_t *s_off, const uint32_t *s_u, const int64_t *s_rb,
+                                                int64_t &at)
+{
+    if (t.staged) {
+        const int32_t rel = (int32_t)(e - t0);
+        int x = 0, y = (int)(t.hi - t.lo);  // last source that starts at or before rel
+        while (x < y) {
+            const int mid = (x + y + 1) >> 1;
+            if (s_off[mid] <= rel) x = mid;
+            else y = mid - 1;
+        }
+        at = s_rb[x] + e;
+        return s_u[x];
+    }
+    const int64_t x = src_of(qoff, t.lo, t.hi, e);
+    const uint32_t u = q[x];
+    at = rowptr[u] + (e - qoff[x]);
+    return u;
+}
+
+// Top-down: the frontier's edges in tiles.  kCount: part[workgroup] = the out
+// bits it was the first to set.  One level of 2^20 edges at scale 22: MEASURE.
+template <bool kCount>
 __global__ __launch_bounds__(kExpandBlock) void k_expand(
     const uint32_t *__restrict__ q, const int64_t *__restrict__ qoff, const int64_t *__restrict__ cnt,
     const int64_t *__restrict__ rowptr, const uint32_t *__restrict__ cols,
-    const uint64_t *__restrict__ visited, uint64_t *__restrict__ out, uint32_t *__restrict__ parent)
+    const uint64_t *__restrict__ visited, uint64_t *out, uint32_t *parent, int64_t *__restrict__ part)
 {
-    __shared__ int64_t s_lo, s_hi;
+    __shared__ int64_t s_range[2], s_rb[kTileSrc];
+    __shared__ int32_t s_off[kTileSrc];
+    __shared__ uint32_t s_u[kTileSrc];
     const int64_t qn = cnt[kQLen];
     const int64_t E = cnt[kEdges];
+    int64_t found = 0;
     for (int64_t t0 = blockIdx.x * (int64_t)kExpandTile; t0 < E; t0 += (int64_t)gridDim.x * kExpandTile) {
         const int64_t t1 = min(E, t0 + (int64_t)kExpandTile);
-        if (threadIdx.x == 0) {
-            s_lo = src_of(qoff, 0, qn - 1, t0);
-            s_hi = src_of(qoff, s_lo, qn - 1, t1 - 1);
+        const TileSrc src = stage_sources(q, qoff, qn, rowptr, t0, t1, s_range, s_off, s_u, s_rb);
+        // a thread's edges together, so that their loads are in flight at once
+        constexpr int U = kExpandTile / kExpandBlock;
+        uint32_t u[U], v[U];
+        uint64_t seen[U];
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+            const int64_t e = t0 + threadIdx.x + k * kExpandBlock;
+            u[k] = v[k] = kNoParent;
+            if (e >= t1) continue;
+            int64_t at;
+            u[k] = edge_source(src, q, qoff, rowptr, t0, e, s_off, s_u, s_rb, at);
+            v[k] = cols[at];
         }
-        __syncthreads();
-        const int64_t lo = s_lo, hi = s_hi;
-        for (int64_t e = t0 + threadIdx.x; e < t1; e += kExpandBlock) {
-            const int64_t si = src_of(qoff, lo, hi, e);
-            const uint32_t u = q[si];
-            const uint32_t v = cols[rowptr[u] + (e - qoff[si])];
-            const uint64_t bit = 1ull << (v & 63);
-            if (visited[v >> 6] & bit) continue;
-            if (!(out[v >> 6] & bit)) atomicOr((unsigned long long *)&out[v >> 6], (unsigned long long)bit);
-            if (parent[v] > u) atomicMin(&parent[v], u);
+#pragma unroll
+        for (int k = 0; k < U; ++k) seen[k] = v[k] == kNoParent ? ~0ull : visited[v[k] >> 6];
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+            const int64_t w = v[k] >> 6;
+            const uint64_t bit = 1ull << (v[k] & 63);
+            if (seen[k] & bit) continue;
+            if (!(out[w] & bit)) {
+                if (kCount)
+                    found += !(atomicOr((unsigned long long *)&out[w], (unsigned long long)bit) & bit);
+                else
+                    atomicOr((unsigned long long *)&out[w], (unsigned long long)bit);
+            }
+            if (parent[v[k]] > u[k]) atomicMin(&parent[v[k]], u[k]);
         }
         __syncthreads();
     }
+    if (kCount) {
+        found = g5_block_sum256(found);
+        if (threadIdx.x == 0) part[blockIdx.x] = found;
+    }
 }
 
-// visited |= out (minus already visited), level := depth for new bits, count;
-// with rowptr (1x1 block) also the degree sum of the new vertices.  One
-// wavefront per 64 consecutive words: lane j commits word w0 + j; then the
-// wave walks the words with new bits 8 at a time, lane i taking vertex
-// 64 w + i, so a word's level stores and offset reads are coalesced, and the
-// 8 words' offset loads are all issued before any is used (a vertex's degree
-// is the next lane's offset minus its own; lane 63 loads the next word's
-// first offset).
+// visited |= in, out := the bits of in that are new, level := depth for them;
+// part (if not null): a bitmap tile's new vertices, and with rowptr (1x1
+// block) their degrees kTiles further.  in may be out.  A workgroup takes 64
+// words at a time, 16 to a wave (lane j commits word w0 + j); then the wave
+// walks the words with new bits 8 at a time, lane i taking vertex 64 w + i, so
+// a word's level stores and offset reads are coalesced, and the 8 words'
+// offset loads are all issued before any is used (a vertex's degree is the
+// next lane's offset minus its own; lane 63 loads the next word's first
+// offset).  The sums are stored per tile: added up with atomics on one
+// address they took their turns (scale 22, MEASURE).
 constexpr int kCommitGroup = 8;
+constexpr int kCommitWords = 16;
 
-__device__ __forceinline__ uint64_t bcast64(uint64_t x, int l)
-{
-    return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(x >> 32), l) << 32) |
-           (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, l);
-}
-
-__global__ __launch_bounds__(256) void k_commit(uint64_t *__restrict__ out, uint64_t *__restrict__ visited,
-                                                int32_t *__restrict__ level, int64_t wc, int32_t depth,
-                                                int64_t *__restrict__ cnt, const int64_t *__restrict__ rowptr)
+__global__ __launch_bounds__(256) void k_commit(const uint64_t *in, uint64_t *out, uint64_t *__restrict__ visited,
+                                                int32_t *__restrict__ level, int64_t wc, int64_t tile, int32_t depth,
+                                                const int64_t *__restrict__ rowptr, int64_t *__restrict__ part)
 {
     const int lane = __lane_id();
-    const int64_t nwaves = (int64_t)gridDim.x * (blockDim.x >> 6);
+    const int64_t end = min(wc, (blockIdx.x + 1) * tile);
     int64_t c = 0, ce = 0;
-    for (int64_t w0 = (blockIdx.x * (int64_t)(blockDim.x >> 6) + (threadIdx.x >> 6)) * 64; w0 < wc;
-         w0 += nwaves * 64) {
+    for (int64_t w0 = blockIdx.x * tile + (threadIdx.x >> 6) * kCommitWords; w0 < end; w0 += 64) {
         const int64_t w = w0 + lane;
         uint64_t nw = 0;
-        if (w < wc) {
-            const uint64_t o = out[w];
+        if (lane < kCommitWords && w < end) {
+            const uint64_t o = in[w];
             if (o) {
                 const uint64_t vis = visited[w];
                 nw = o & ~vis;
-                if (nw != o) out[w] = nw;
                 if (nw) visited[w] = vis | nw;
                 c += __popcll(nw);
             }
+            if (nw != o || in != out) out[w] = nw;
         }
         const uint64_t todo = __ballot(nw != 0);
-        for (int j0 = 0; j0 < 64; j0 += kCommitGroup) {
+#pragma unroll
+        for (int j0 = 0; j0 < kCommitWords; j0 += kCommitGroup) {
             if (((todo >> j0) & ((1ull << kCommitGroup) - 1)) == 0) continue;
             uint64_t bits[kCommitGroup];
             int64_t lo[kCommitGroup], hi[kCommitGroup];
 #pragma unroll
             for (int k = 0; k < kCommitGroup; ++k) {
-                bits[k] = bcast64(nw, j0 + k);  // zero for words past wc
+                bits[k] = g5_bcast64(nw, j0 + k);  // zero for words past the tile
                 const int64_t v = (w0 + j0 + k) * 64 + lane;
                 const bool any = bits[k] != 0;  // wave-uniform
                 lo[k] = (rowptr && any) ? rowptr[v] : 0;
@@ -216,11 +305,12 @@ __global__ __launch_bounds__(256) void k_commit(uint64_t *__restrict__ out, uint
             }
         }
     }
+    if (!part) return;
     c = g5_block_sum256(c);
     ce = g5_block_sum256(ce);
-    if (threadIdx.x == 0 && c) {
-        atomicAdd((unsigned long long *)&cnt[kNew], (unsigned long long)c);
-        if (ce) atomicAdd((unsigned long long *)&cnt[kNewEdges], (unsigned long long)ce);
+    if (threadIdx.x == 0) {
+        part[blockIdx.x] = c;
+        part[g5::kTiles + blockIdx.x] = ce;
     }
 }
 
@@ -322,15 +412,24 @@ __device__ __forceinline__ uint32_t bu_scan(int64_t &j, int64_t e, const uint32_
     return par;
 }
 
+// kCommit: with the level's commit (visited, levels) in the same pass.
+// part[j * kParts + workgroup]: new vertices, their degrees (with the row
+// offsets of their own rows), neighbours checked, vertices scanned.  Three
+// atomics per workgroup on one line were most of its time before: at scale 22,
+// commit included, 149 us a level (of three) -> MEASURE.
+enum BuPart { kPNew = 0, kPNewEdges = 1, kPBuEdges = 2, kPBuVerts = 3 };
+
+template <bool kCommit>
 __global__ __launch_bounds__(256) void k_bottom_up(const int64_t *__restrict__ rowptr,
                                                    const uint32_t *__restrict__ cols,
-                                                   const uint64_t *__restrict__ visited,
+                                                   uint64_t *__restrict__ visited,
                                                    const uint64_t *__restrict__ front, uint64_t *__restrict__ next,
-                                                   uint32_t *__restrict__ parent, int64_t wc, int64_t *__restrict__ cnt)
+                                                   uint32_t *__restrict__ parent, int32_t *__restrict__ level,
+                                                   int32_t depth, int64_t wc, int64_t *__restrict__ part)
 {
     __shared__ BuScan s_scan[4];
     const int lane = __lane_id();
-    int64_t nedges = 0, nverts = 0, newdeg = 0;
+    int64_t nedges = 0, nverts = 0, newdeg = 0, nnew = 0;
     for (int64_t w = blockIdx.x * 4 + (threadIdx.x >> 6); w < wc; w += (int64_t)gridDim.x * 4) {
         const uint64_t vis = visited[w];
         const int64_t v = w * 64 + lane;
@@ -345,43 +444,71 @@ __global__ __launch_bounds__(256) void k_bottom_up(const int64_t *__restrict__ r
         const bool hit = par != kNoParent;
         if (hit) {
             parent[v] = par;
+            if (kCommit) level[v] = depth;
             newdeg += e - b;
+            ++nnew;
         }
         nedges += j - b;
         const uint64_t bits = __ballot(hit);
-        if (lane == 0) next[w] = bits;
+        if (lane == 0) {
+            next[w] = bits;
+            if (kCommit && bits) visited[w] = vis | bits;
+        }
     }
+    nnew = g5_block_sum256(nnew);
+    newdeg = g5_block_sum256(newdeg);
     nedges = g5_block_sum256(nedges);
     nverts = g5_block_sum256(nverts);
-    newdeg = g5_block_sum256(newdeg);
     if (threadIdx.x == 0) {
-        if (nedges) atomicAdd((unsigned long long *)&cnt[kBuEdges], (unsigned long long)nedges);
-        if (nverts) atomicAdd((unsigned long long *)&cnt[kBuVerts], (unsigned long long)nverts);
-        if (newdeg) atomicAdd((unsigned long long *)&cnt[kNewEdges], (unsigned long long)newdeg);
+        part[kPNew * kParts + blockIdx.x] = nnew;
+        part[kPNewEdges * kParts + blockIdx.x] = newdeg;
+        part[kPBuEdges * kParts + blockIdx.x] = nedges;
+        part[kPBuVerts * kParts + blockIdx.x] = nverts;
     }
 }
 
-__global__ void k_count_bits(const uint64_t *__restrict__ bits, int64_t n, int64_t *__restrict__ dst)
+// A search's state at its start, in one launch (a fill each took seven): the
+// root's column visited at level 0 (isolated: with the edgeless vertices), its
+// bit in out (the frontier of a bottom-up first level), its row the queue.
+// n_cols is a multiple of 64.
+__global__ __launch_bounds__(256) void k_start(int64_t root_row, int64_t root_col, int64_t wc, int64_t n_cols,
+                                               const uint64_t *__restrict__ isolated,
+                                               const int64_t *__restrict__ rowptr, uint64_t *__restrict__ visited,
+                                               uint64_t *__restrict__ out, uint64_t *__restrict__ next,
+                                               uint32_t *__restrict__ parent, int32_t *__restrict__ level,
+                                               uint32_t *__restrict__ queue, int64_t *__restrict__ qoff,
+                                               int64_t *__restrict__ cnt)
 {
-    int64_t c = 0;
-    for (int64_t w = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; w < n;
-         w += (int64_t)gridDim.x * blockDim.x)
-        c += __popcll(bits[w]);
-    c = g5_block_sum256(c);
-    if (threadIdx.x == 0 && c) atomicAdd((unsigned long long *)dst, (unsigned long long)c);
+    const int64_t t = blockIdx.x * 256ll + threadIdx.x, stride = gridDim.x * 256ll;
+    for (int64_t w = t; w < wc; w += stride) {
+        const uint64_t bit = root_col >= 0 && w == root_col >> 6 ? 1ull << (root_col & 63) : 0ull;
+        visited[w] = (isolated ? isolated[w] : 0ull) | bit;
+        out[w] = bit;
+        next[w] = 0;
+    }
+    uint4 *p4 = (uint4 *)parent, *l4 = (uint4 *)level;
+    for (int64_t i = t; i < n_cols / 4; i += stride) {
+        const int at = i == root_col >> 2 ? (int)(root_col & 3) : 4;  // root_col -1: never
+        p4[i] = make_uint4(at == 0 ? kRootMark : kNoParent, at == 1 ? kRootMark : kNoParent,
+                           at == 2 ? kRootMark : kNoParent, at == 3 ? kRootMark : kNoParent);
+        l4[i] = make_uint4(at == 0 ? 0u : ~0u, at == 1 ? 0u : ~0u, at == 2 ? 0u : ~0u, at == 3 ? 0u : ~0u);
+    }
+    if (t < kNCnt) {
+        int64_t c = 0;
+        if (root_row >= 0 && t == kQLen) {
+            c = 1;
+            queue[0] = (uint32_t)root_row;
+            qoff[0] = 0;
+        }
+        if (root_row >= 0 && t == kEdges) c = rowptr[root_row + 1] - rowptr[root_row];
+        cnt[t] = c;
+    }
 }
 
-__global__ void k_start(int64_t root_row, int64_t root_col, uint32_t *queue, uint64_t *visited, uint64_t *out,
-                        int32_t *level, uint32_t *parent, int64_t *cnt)
+__global__ __launch_bounds__(256) void k_copy_words(const uint64_t *__restrict__ from, uint64_t *__restrict__ to,
+                                                    int64_t n)
 {
-    cnt[kQLen] = root_row >= 0 ? 1 : 0;
-    if (root_row >= 0) queue[0] = (uint32_t)root_row;
-    if (root_col >= 0) {
-        visited[root_col >> 6] |= 1ull << (root_col & 63);
-        out[root_col >> 6] = 1ull << (root_col & 63);  // the frontier of a bottom-up first level
-        level[root_col] = 0;
-        parent[root_col] = kRootMark;
-    }
+    for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < n; i += gridDim.x * 256ll) to[i] = from[i];
 }
 
 __global__ void k_result(const uint32_t *__restrict__ parent, int64_t n, int64_t row_start,
@@ -394,13 +521,12 @@ __global__ void k_result(const uint32_t *__restrict__ parent, int64_t n, int64_t
     }
 }
 
-// grids that end in one atomic per workgroup: same-address atomics take their
-// turns (4096 of them were 40 of k_nedge's 54 us at scale 22)
-constexpr int kSumGrid = 1024;
+constexpr int kSumGrid = 2048;
 
-// n is a multiple of 64
+// part[workgroup] = its share of the sum (one atomic each on one address, 1024
+// of them, were 4 us); n is a multiple of 64
 __global__ __launch_bounds__(256) void k_nedge(const uint32_t *__restrict__ gdeg, const int32_t *__restrict__ level,
-                                               int64_t n, int64_t *__restrict__ dst)
+                                               int64_t n, int64_t *__restrict__ part)
 {
     const uint4 *g4 = (const uint4 *)gdeg;
     const int4 *l4 = (const int4 *)level;
@@ -413,13 +539,13 @@ __global__ __launch_bounds__(256) void k_nedge(const uint32_t *__restrict__ gdeg
              (l.w >= 0 ? g.w : 0u);
     }
     c = g5_block_sum256(c);
-    if (threadIdx.x == 0 && c) atomicAdd((unsigned long long *)dst, (unsigned long long)c);
+    if (threadIdx.x == 0) part[blockIdx.x] = c;
 }
 
 // nedge's generated-degree sum and the predecessor-map checksum of a 1x1
 // search in one pass: sum over reached v of mix64(v << 32 | (pred(v) + 1))
 __global__ void k_summary(const uint32_t *__restrict__ gdeg, const int32_t *__restrict__ level,
-                          const uint32_t *__restrict__ parent, int64_t n, int64_t *__restrict__ dst)
+                          const uint32_t *__restrict__ parent, int64_t n, int64_t *__restrict__ part)
 {
     int64_t c = 0;
     uint64_t h = 0;
@@ -434,35 +560,76 @@ __global__ void k_summary(const uint32_t *__restrict__ gdeg, const int32_t *__re
     c = g5_block_sum256(c);
     h = g5_block_sum256_u64(h);
     if (threadIdx.x == 0) {
-        if (c) atomicAdd((unsigned long long *)dst, (unsigned long long)c);
-        if (h) atomicAdd((unsigned long long *)(dst + 1), (unsigned long long)h);
+        part[blockIdx.x] = c;
+        part[kParts + blockIdx.x] = (int64_t)h;
     }
 }
 
-__global__ void k_set_cnt(int64_t *cnt, int idx, int64_t v) { cnt[idx] = v; }
-
-// One level's expansion from the current in-queue (d_queue, cnt[kQLen]).
-int expand_level(g5_bfs *b)
+// The frontier of d_inbits or of a host's queue as a queue with its degree
+// prefix, and out cleared: one to three launches before an expansion, none of
+// them where the level before left both.
+int prepare_queue(g5_bfs *b, uint64_t *out)
 {
     g5_graph *g = b->g;
     hipStream_t s = b->s;
-    G5_HIP(g5::fill_u64(b->d_out, b->wc, 0, s));
-    hipLaunchKernelGGL(k_queue_degrees, g5::grid_for(g->n_rows, 256, 4096), 256, 0, s,
-                       (const uint32_t *)b->d_queue, (const int64_t *)b->d_cnt + kQLen,
-                       (const int64_t *)g->d_rowptr, b->d_qoff);
-    G5_HIP(hipGetLastError());
-    // the scan length must be known on the host: it is the in-queue length
-    G5_HIP(g5::exclusive_scan_i64(b->d_qoff, b->qlen, b->d_cnt + kEdges, b->d_scratch, s));
-    if (b->qlen > 0) {
-        // qoff[qlen] = total, so src_of never reads past the prefix
-        if (b->prof) G5_HIP(hipEventRecord(b->ek0, s));
-        hipLaunchKernelGGL(k_expand, kExpandGrid, kExpandBlock, 0, s, (const uint32_t *)b->d_queue,
-                           (const int64_t *)b->d_qoff, (const int64_t *)b->d_cnt,
-                           (const int64_t *)g->d_rowptr, (const uint32_t *)g->d_cols,
-                           (const uint64_t *)b->d_visited, b->d_out, b->d_parent);
+    if (b->queue_ok && b->qoff_ok) {
+        G5_HIP(g5::fill_u64(out, b->wc, 0, s));
+    } else if (b->queue_ok) {
+        hipLaunchKernelGGL(k_queue_degrees, g5::grid_for(std::max(b->qlen, b->wc), 256, 4096), 256, 0, s,
+                           (const uint32_t *)b->d_queue, b->qlen, (const int64_t *)g->d_rowptr, b->d_qoff, b->d_cnt,
+                           out, b->wc);
         G5_HIP(hipGetLastError());
-        if (b->prof) G5_HIP(hipEventRecord(b->ek1, s));
+        G5_HIP(g5::exclusive_scan_i64(b->d_qoff, b->qlen, b->d_cnt + kEdges, b->d_scratch, s));
+    } else {
+        g5::QueueOut o{};
+        o.q = b->d_queue;
+        o.qoff = b->d_qoff;
+        o.d_n = b->d_cnt + kQLen;
+        o.d_e = b->d_cnt + kEdges;
+        o.clear = out;
+        o.n_clear = b->wc;
+        G5_HIP(g5::bitmap_to_queue(b->d_inbits, b->wr, (const int64_t *)g->d_rowptr, o, b->d_part, false, s));
     }
+    b->queue_ok = b->qoff_ok = true;
+    return G5_OK;
+}
+
+// One level's expansion from the queue (d_queue, d_qoff, cnt[kQLen] and
+// cnt[kEdges]) into out; count: part[0 .. kExpandGrid) sum to its new bits.
+// E: its edges if the host knows them, else -1.
+int expand_level(g5_bfs *b, uint64_t *out, bool count, int64_t E)
+{
+    g5_graph *g = b->g;
+    hipStream_t s = b->s;
+    if (b->prof) G5_HIP(hipEventRecord(b->ek0, s));
+    static_assert(kExpandGrid <= kParts, "a sum per workgroup");
+    hipLaunchKernelGGL(count ? k_expand<true> : k_expand<false>,
+                       count || E < 0 ? kExpandGrid : g5::grid_for(E, kExpandTile, kExpandGrid), kExpandBlock, 0, s,
+                       (const uint32_t *)b->d_queue, (const int64_t *)b->d_qoff, (const int64_t *)b->d_cnt,
+                       (const int64_t *)g->d_rowptr, (const uint32_t *)g->d_cols, (const uint64_t *)b->d_visited, out,
+                       b->d_parent, b->d_part);
+    G5_HIP(hipGetLastError());
+    if (b->prof) G5_HIP(hipEventRecord(b->ek1, s));
+    return G5_OK;
+}
+
+// The workgroups' n sums in d_part (arrays stride apart, the first k of
+// them) to the counters slot[0 .. k) in pinned memory, and the codec's error
+// flag with them.  frontier: the first two are also the next frontier's
+// vertices and edges.  Waits for the stream.
+int fold_counters(g5_bfs *b, int64_t stride, int n, const int *slot, int k, bool frontier)
+{
+    g5::FoldOut o{};
+    for (int j = 0; j < k; ++j) o.host[j] = b->h_cnt + slot[j];
+    if (frontier) {
+        o.dev[0] = b->d_cnt + kQLen;
+        o.dev[1] = b->d_cnt + kEdges;
+    }
+    o.from = b->d_cnt + kCodecErr;
+    o.to = b->h_cnt + kCodecErr;
+    o.ncopy = 1;
+    G5_HIP(g5::fold_parts(b->d_part, stride, n, o, b->s));
+    G5_HIP(hipStreamSynchronize(b->s));
     return G5_OK;
 }
 
@@ -470,12 +637,11 @@ int expand_level(g5_bfs *b)
 // algorithmic bytes, 16 B row-offset pair per frontier vertex, 4 B column id
 // + 8 B visited word per frontier edge, 8 B out word + 4 B parent per newly
 // reached vertex.
-int account_level(g5_bfs *b, int64_t qlen, int64_t n_new)
+int account_level(g5_bfs *b, int64_t qlen, int64_t E, int64_t n_new)
 {
     if (!b->prof || qlen == 0) return G5_OK;
     float ms = 0;
     G5_HIP(hipEventElapsedTime(&ms, b->ek0, b->ek1));
-    const int64_t E = b->h_cnt[kEdges];
     b->exp_ms += ms;
     b->exp_launches += 1;
     b->exp_edges += E;
@@ -486,8 +652,9 @@ int account_level(g5_bfs *b, int64_t qlen, int64_t n_new)
 // After a bottom-up level: k_bottom_up time and its algorithmic bytes, 16 B
 // row-offset pair per unvisited vertex scanned, 4 B column + 8 B frontier
 // word per neighbour checked, 4 B parent per newly reached vertex, 16 B
-// (visited read + next write) per 64-vertex word.
-int account_bottom_up(g5_bfs *b, int64_t n_new)
+// (visited read + next write) per 64-vertex word; with the commit in the same
+// pass 4 B level per new vertex and 8 B visited per word more.
+int account_bottom_up(g5_bfs *b, int64_t n_new, bool commit)
 {
     if (!b->prof) return G5_OK;
     float ms = 0;
@@ -496,14 +663,7 @@ int account_bottom_up(g5_bfs *b, int64_t n_new)
     b->bu_ms += ms;
     b->bu_launches += 1;
     b->bu_edges += E;
-    b->bu_bytes += 16.0 * V + 12.0 * E + 4.0 * n_new + 16.0 * b->wc;
-    return G5_OK;
-}
-
-int sync_counters(g5_bfs *b)
-{
-    G5_HIP(hipMemcpyAsync(b->h_cnt, b->d_cnt, kNCnt * 8, hipMemcpyDeviceToHost, b->s));
-    G5_HIP(hipStreamSynchronize(b->s));
+    b->bu_bytes += 16.0 * V + 12.0 * E + (commit ? 8.0 : 4.0) * n_new + (commit ? 24.0 : 16.0) * b->wc;
     return G5_OK;
 }
 
@@ -539,21 +699,15 @@ int reset_search(g5_bfs *b, int64_t root, bool isolated = false)
     const int64_t rr = root - g->row_start, rc = root - g->col_start;
     const int64_t root_row = (root >= 0 && rr >= 0 && rr < g->n_rows) ? rr : -1;
     const int64_t root_col = (root >= 0 && rc >= 0 && rc < g->n_cols) ? rc : -1;
-    if (isolated) {
-        G5_HIP(hipMemcpyAsync(b->d_visited, b->d_isolated, (size_t)b->wc * 8, hipMemcpyDeviceToDevice, s));
-    } else {
-        G5_HIP(g5::fill_u64(b->d_visited, b->wc, 0, s));
-    }
-    G5_HIP(g5::fill_u64(b->d_out, b->wc, 0, s));
-    G5_HIP(g5::fill_u32(b->d_parent, g->n_cols, kNoParent, s));
-    G5_HIP(g5::fill_i32(b->d_level, g->n_cols, -1, s));
-    G5_HIP(g5::fill_i64(b->d_cnt, kNCnt, 0, s));
-    hipLaunchKernelGGL(k_start, 1, 1, 0, s, root_row, root_col, b->d_queue, b->d_visited, b->d_out, b->d_level,
-                       b->d_parent, b->d_cnt);
+    hipLaunchKernelGGL(k_start, g5::grid_for(g->n_cols / 4, 256, 4096), 256, 0, s, root_row, root_col, b->wc,
+                       g->n_cols, isolated ? (const uint64_t *)b->d_isolated : (const uint64_t *)nullptr,
+                       (const int64_t *)g->d_rowptr, b->d_visited, b->d_out, b->d_next, b->d_parent, b->d_level,
+                       b->d_queue, b->d_qoff, b->d_cnt);
     G5_HIP(hipGetLastError());
     b->root = root;
     b->depth = 0;
     b->qlen = root_row >= 0 ? 1 : 0;
+    b->queue_ok = b->qoff_ok = true;
     b->inbits_valid = false;
     return G5_OK;
 }
@@ -585,7 +739,6 @@ int reset_search(g5_bfs *b, int64_t root, bool isolated = false)
 constexpr int kLvBlock = 256;
 constexpr int kLvGrid = 4096;   // two rounds of 8 workgroups per CU, which differ in what they take
 constexpr int kLvTile = 1024;   // edges of a top-down tile
-constexpr int kLvSrc = 512;     // sources of a tile that are staged in LDS
 constexpr int kLvBuf = 1024;    // new vertices a workgroup keeps
 constexpr int kLvMem = 4096;    // words of LDS: the buffer and staged sources, or the scans' rows
 constexpr int kEdgeBits = 34;   // of a packed total; the vertices take the rest
@@ -651,13 +804,10 @@ __global__ __launch_bounds__(kLvBlock) void k_reset(LevelArgs a, const uint64_t 
     // n is a multiple of 64
     uint4 *p4 = (uint4 *)a.parent, *l4 = (uint4 *)a.level;
     for (int64_t i = t; i < a.n / 4; i += stride) {
-        uint4 p = {kNoParent, kNoParent, kNoParent, kNoParent}, l = {~0u, ~0u, ~0u, ~0u};
-        if (i == root >> 2) {
-            (&p.x)[root & 3] = kRootMark;
-            (&l.x)[root & 3] = 0;
-        }
-        p4[i] = p;
-        l4[i] = l;
+        const int at = i == root >> 2 ? (int)(root & 3) : 4;
+        p4[i] = make_uint4(at == 0 ? kRootMark : kNoParent, at == 1 ? kRootMark : kNoParent,
+                           at == 2 ? kRootMark : kNoParent, at == 3 ? kRootMark : kNoParent);
+        l4[i] = make_uint4(at == 0 ? 0u : ~0u, at == 1 ? 0u : ~0u, at == 2 ? 0u : ~0u, at == 3 ? 0u : ~0u);
     }
     if (blockIdx.x == 0) {
         for (int i = threadIdx.x; i < (int)(sizeof(LevelCtl) / 8); i += kLvBlock) ((uint64_t *)a.ctl)[i] = 0;
@@ -728,11 +878,11 @@ __device__ __forceinline__ void level_top_down(const LevelArgs &a, int d, const 
     __shared__ int64_t s_range[2];
     __shared__ int s_n;
     __shared__ unsigned int s_lost;
-    int32_t *s_off = (int32_t *)s_mem;                        // kLvSrc
-    uint32_t *s_u = s_mem + kLvSrc;                           // kLvSrc
-    int64_t *s_rb = (int64_t *)(s_mem + 2 * kLvSrc);          // kLvSrc
-    uint32_t *s_v = s_mem + 4 * kLvSrc, *s_d = s_v + kLvBuf;  // kLvBuf each
-    static_assert(4 * kLvSrc + 2 * kLvBuf <= kLvMem && kLvBuf >= kLvTile, "LDS");
+    int32_t *s_off = (int32_t *)s_mem;                        // kTileSrc
+    uint32_t *s_u = s_mem + kTileSrc;                           // kTileSrc
+    int64_t *s_rb = (int64_t *)(s_mem + 2 * kTileSrc);          // kTileSrc
+    uint32_t *s_v = s_mem + 4 * kTileSrc, *s_d = s_v + kLvBuf;  // kLvBuf each
+    static_assert(4 * kTileSrc + 2 * kLvBuf <= kLvMem && kLvBuf >= kLvTile, "LDS");
     const uint64_t *__restrict__ front = a.front;
     if (threadIdx.x == 0) {
         s_n = 0;
@@ -751,25 +901,9 @@ __device__ __forceinline__ void level_top_down(const LevelArgs &a, int d, const 
         const int64_t *__restrict__ qoff = a.qoff + g * a.gcap;
         const int64_t t0 = (t - gr.tile0[g]) * kLvTile, t1 = min(gr.edges[g], t0 + (int64_t)kLvTile);
         const int64_t qn = gr.n[g];
-        if (threadIdx.x < 128) {
-            const int64_t r = g5_wave_src_of(qoff, 0, qn - 1, threadIdx.x < 64 ? t0 : t1 - 1);
-            if ((threadIdx.x & 63) == 0) s_range[threadIdx.x >> 6] = r;
-        } else if (threadIdx.x == 128) {
-            s_lost = lost_yet(a, d);
-        }
-        __syncthreads();
-        const int64_t lo = s_range[0], hi = s_range[1];
+        if (threadIdx.x == 128) s_lost = lost_yet(a, d);
+        const TileSrc src = stage_sources(q, qoff, qn, a.rowptr, t0, t1, s_range, s_off, s_u, s_rb);
         const bool collect = s_lost == 0;
-        const bool staged = hi - lo < kLvSrc;  // sources of two edges and more on average
-        if (staged)
-            for (int j = threadIdx.x; j <= (int)(hi - lo); j += kLvBlock) {
-                const uint32_t u = q[lo + j];
-                const int64_t o = qoff[lo + j];
-                s_u[j] = u;
-                s_rb[j] = a.rowptr[u] - o;
-                s_off[j] = (int32_t)max(o - t0, (int64_t)-1);
-            }
-        __syncthreads();
         // a thread's edges together, so that their loads are in flight at once
         constexpr int U = kLvTile / kLvBlock;
         uint32_t u[U], v[U];
@@ -780,21 +914,7 @@ __device__ __forceinline__ void level_top_down(const LevelArgs &a, int d, const 
             u[k] = v[k] = kNoParent;
             if (e >= t1) continue;
             int64_t at;
-            if (staged) {
-                const int32_t rel = (int32_t)(e - t0);
-                int x = 0, y = (int)(hi - lo);  // last source that starts at or before rel
-                while (x < y) {
-                    const int mid = (x + y + 1) >> 1;
-                    if (s_off[mid] <= rel) x = mid;
-                    else y = mid - 1;
-                }
-                u[k] = s_u[x];
-                at = s_rb[x] + e;
-            } else {
-                const int64_t x = src_of(qoff, lo, hi, e);
-                u[k] = q[x];
-                at = a.rowptr[u[k]] + (e - qoff[x]);
-            }
+            u[k] = edge_source(src, q, qoff, a.rowptr, t0, e, s_off, s_u, s_rb, at);
             v[k] = a.cols[at];
         }
 #pragma unroll
@@ -1012,6 +1132,8 @@ int run_levels(g5_bfs *b, int64_t root)
     b->d_next = bm[(nlevels + 1) % 3];
     b->d_third = bm[(nlevels + 2) % 3];
     b->qlen = 0;
+    b->queue_ok = true;
+    b->qoff_ok = false;
     b->root = root;
     b->inbits_valid = false;
     return G5_OK;
@@ -1032,7 +1154,7 @@ extern "C" int g5_bfs_create(g5_graph *g, g5_bfs **out)
     };
     hipError_t e = hipStreamCreate(&b->s);
     const int64_t nmax = std::max(g->n_rows, g->n_cols);
-    const size_t scr = g5::scan_scratch_words(nmax + 1) + g5::scan_scratch_words(b->wc + 1) + 64;
+    const size_t scr = g5::scan_scratch_words(nmax + 1) + 64;
     if (e == hipSuccess) e = hipMalloc(&b->d_visited, (size_t)std::max<int64_t>(b->wc, 1) * 8);
     if (e == hipSuccess) e = hipMalloc(&b->d_out, (size_t)std::max<int64_t>(b->wc, 1) * 8);
     if (e == hipSuccess) e = hipMalloc(&b->d_next, (size_t)std::max<int64_t>(b->wc, 1) * 8);
@@ -1043,6 +1165,8 @@ extern "C" int g5_bfs_create(g5_graph *g, g5_bfs **out)
     if (e == hipSuccess) e = hipMalloc(&b->d_qoff, (size_t)(g->n_rows + 2) * 8);
     if (e == hipSuccess) e = hipMalloc(&b->d_scratch, scr * 8);
     if (e == hipSuccess) e = hipMalloc(&b->d_cnt, kNCnt * 8);
+    if (e == hipSuccess) e = hipMalloc(&b->d_part, 4 * kParts * 8);
+    static_assert(kParts >= 2 * g5::kTiles && kParts >= kSumGrid, "a sum per workgroup and tile");
     if (e == hipSuccess) e = hipHostMalloc(&b->h_cnt, (kNCnt + 1) * 8, hipHostMallocDefault);  // k_level's end last
     if (g->n_rows == g->n_cols && g->row_start == g->col_start) {  // g5_bfs_run
         // twice n / 8 vertices spread evenly: a level that finds more runs on
@@ -1069,7 +1193,7 @@ extern "C" int g5_bfs_free(g5_bfs *b)
     if (!b) return G5_OK;
     if (b->s) (void)hipStreamSynchronize(b->s);
     void *dev[] = {b->d_visited, b->d_out,     b->d_next, b->d_parent, b->d_level, b->d_queue,
-                   b->d_outq,    b->d_qoff,    b->d_scratch, b->d_cnt, b->d_words, b->d_isolated, b->d_inbits,
+                   b->d_outq,    b->d_qoff,    b->d_scratch, b->d_cnt, b->d_part, b->d_words, b->d_isolated, b->d_inbits,
                    b->d_third,   b->d_gq[0],   b->d_gq[1], b->d_goff[0], b->d_goff[1], b->d_ctl};
     for (void *p : dev)
         if (p) (void)hipFree(p);
@@ -1097,16 +1221,13 @@ extern "C" int g5_bfs_expand(g5_bfs *b, int *any_new)
 {
     G5_REQUIRE(b && any_new, G5_E_ARG, "g5_bfs_expand: null argument");
     G5_REQUIRE(b->depth >= 0, G5_E_STATE, "g5_bfs_expand: g5_bfs_start not called");
-    int rc = expand_level(b);
-    if (rc) return rc;
-    hipLaunchKernelGGL(k_set_cnt, 1, 1, 0, b->s, b->d_cnt, (int)kOutLen, (int64_t)0);
-    hipLaunchKernelGGL(k_count_bits, g5::grid_for(b->wc, 256, 2048), 256, 0, b->s,
-                       (const uint64_t *)b->d_out, b->wc, b->d_cnt + kOutLen);
-    G5_HIP(hipGetLastError());
-    rc = sync_counters(b);
-    if (rc) return rc;
+    int rc = prepare_queue(b, b->d_out);
+    if (!rc) rc = expand_level(b, b->d_out, true, -1);
     // the out bits are this block's newly reached columns
-    rc = account_level(b, b->qlen, b->h_cnt[kOutLen]);
+    const int slot[] = {kOutLen};
+    if (!rc && b->prof) G5_HIP(hipMemcpyAsync(b->h_cnt, b->d_cnt, 2 * 8, hipMemcpyDeviceToHost, b->s));
+    if (!rc) rc = fold_counters(b, kParts, kExpandGrid, slot, 1, false);
+    if (!rc) rc = account_level(b, b->h_cnt[kQLen], b->h_cnt[kEdges], b->h_cnt[kOutLen]);
     if (rc) return rc;
     *any_new = b->h_cnt[kOutLen] > 0;
     return G5_OK;
@@ -1116,9 +1237,11 @@ extern "C" int g5_bfs_outqueue(g5_bfs *b, uint32_t *q, int64_t *n)
 {
     G5_REQUIRE(b && n, G5_E_ARG, "g5_bfs_outqueue: null argument");
     G5_REQUIRE(b->depth >= 0, G5_E_STATE, "g5_bfs_outqueue: g5_bfs_start not called");
-    G5_HIP(g5::bitmap_to_queue(b->d_out, b->wc, b->d_outq, b->d_cnt + kOutLen, b->d_scratch, b->s));
-    int rc = sync_counters(b);
-    if (rc) return rc;
+    g5::QueueOut o{};
+    o.q = b->d_outq;
+    o.h_n = b->h_cnt + kOutLen;
+    G5_HIP(g5::bitmap_to_queue(b->d_out, b->wc, nullptr, o, b->d_part, false, b->s));
+    G5_HIP(hipStreamSynchronize(b->s));
     const int64_t len = b->h_cnt[kOutLen];
     G5_REQUIRE(len <= *n, G5_E_OVERFLOW, "g5_bfs_outqueue: queue of %lld entries exceeds capacity %lld",
                (long long)len, (long long)*n);
@@ -1128,6 +1251,15 @@ extern "C" int g5_bfs_outqueue(g5_bfs *b, uint32_t *q, int64_t *n)
         G5_HIP(hipMemcpy(q, b->d_outq, (size_t)len * 4, hipMemcpyDeviceToHost));
     }
     return G5_OK;
+}
+
+// the level's newly reached columns: bits, which may be d_out
+static hipError_t commit_out(g5_bfs *b, const uint64_t *bits)
+{
+    if (b->wc == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_commit, g5::tile_count(b->wc), 256, 0, b->s, bits, b->d_out, b->d_visited, b->d_level, b->wc,
+                       g5::tile_words(b->wc), (int32_t)(b->depth + 1), (const int64_t *)nullptr, (int64_t *)nullptr);
+    return hipGetLastError();
 }
 
 extern "C" int g5_bfs_set_outqueue(g5_bfs *b, const uint32_t *q, int64_t n)
@@ -1143,14 +1275,10 @@ extern "C" int g5_bfs_set_outqueue(g5_bfs *b, const uint32_t *q, int64_t n)
         G5_HIP(g5::fill_u64(b->d_out, b->wc, 0, b->s));
         if (n) {
             G5_HIP(hipMemcpyAsync(b->d_outq, q, (size_t)n * 4, hipMemcpyHostToDevice, b->s));
-            G5_HIP(g5::queue_to_bitmap(b->d_outq, n, b->d_out, b->s));
+            G5_HIP(g5::queue_to_bitmap(b->d_outq, n, b->d_out, b->wc, nullptr, b->s));
         }
     }
-    hipLaunchKernelGGL(k_set_cnt, 1, 1, 0, b->s, b->d_cnt, (int)kNew, (int64_t)0);
-    hipLaunchKernelGGL(k_commit, g5::grid_for(b->wc, 256, 2048), 256, 0, b->s, b->d_out, b->d_visited,
-                       b->d_level, b->wc, (int32_t)(b->depth + 1), b->d_cnt,
-                       (const int64_t *)nullptr);
-    G5_HIP(hipGetLastError());
+    G5_HIP(commit_out(b, b->d_out));
     G5_HIP(hipStreamSynchronize(b->s));
     return G5_OK;
 }
@@ -1166,18 +1294,23 @@ extern "C" int g5_bfs_set_inqueue(g5_bfs *b, const uint32_t *q, int64_t n)
             G5_REQUIRE(q[i] < (uint64_t)g->n_rows && (i == 0 || q[i] > q[i - 1]), G5_E_ARG,
                        "g5_bfs_set_inqueue: queue not sorted/unique/in range at %lld", (long long)i);
         if (n) G5_HIP(hipMemcpyAsync(b->d_queue, q, (size_t)n * 4, hipMemcpyHostToDevice, b->s));
-        hipLaunchKernelGGL(k_set_cnt, 1, 1, 0, b->s, b->d_cnt, (int)kQLen, n);
         b->qlen = n;
+        b->qoff_ok = false;
     } else {
         G5_REQUIRE(g->n_rows == g->n_cols && g->row_start == g->col_start, G5_E_STATE,
                    "g5_bfs_set_inqueue: own out-queue as in-queue needs a diagonal block");
-        G5_HIP(g5::bitmap_to_queue(b->d_out, b->wc, b->d_queue, b->d_cnt + kQLen, b->d_scratch, b->s));
-        int rc = sync_counters(b);
-        if (rc) return rc;
-        b->qlen = b->h_cnt[kQLen];
+        g5::QueueOut o{};
+        o.q = b->d_queue;
+        o.qoff = b->d_qoff;
+        o.d_n = b->d_cnt + kQLen;
+        o.d_e = b->d_cnt + kEdges;
+        o.h_n = b->h_cnt + kQLen;
+        G5_HIP(g5::bitmap_to_queue(b->d_out, b->wc, (const int64_t *)g->d_rowptr, o, b->d_part, false, b->s));
+        b->qoff_ok = true;
     }
-    G5_HIP(hipGetLastError());
     G5_HIP(hipStreamSynchronize(b->s));
+    if (!q) b->qlen = b->h_cnt[kQLen];
+    b->queue_ok = true;
     b->inbits_valid = false;
     b->depth++;
     return G5_OK;
@@ -1215,13 +1348,7 @@ extern "C" int g5_bfs_set_out_bitmap(g5_bfs *b, const uint64_t *d_bits)
 {
     G5_REQUIRE(b, G5_E_ARG, "g5_bfs_set_out_bitmap: null handle");
     G5_REQUIRE(b->depth >= 0, G5_E_STATE, "g5_bfs_set_out_bitmap: g5_bfs_start not called");
-    if (d_bits && d_bits != b->d_out && b->wc)
-        G5_HIP(hipMemcpyAsync(b->d_out, d_bits, (size_t)b->wc * 8, hipMemcpyDeviceToDevice, b->s));
-    hipLaunchKernelGGL(k_set_cnt, 1, 1, 0, b->s, b->d_cnt, (int)kNew, (int64_t)0);
-    hipLaunchKernelGGL(k_commit, g5::grid_for(b->wc, 256, 2048), 256, 0, b->s, b->d_out, b->d_visited,
-                       b->d_level, b->wc, (int32_t)(b->depth + 1), b->d_cnt,
-                       (const int64_t *)nullptr);
-    G5_HIP(hipGetLastError());
+    G5_HIP(commit_out(b, d_bits && b->wc ? d_bits : b->d_out));
     G5_HIP(hipStreamSynchronize(b->s));
     return G5_OK;
 }
@@ -1230,12 +1357,12 @@ extern "C" int g5_bfs_set_in_bitmap(g5_bfs *b, const uint64_t *d_bits)
 {
     G5_REQUIRE(b && d_bits, G5_E_ARG, "g5_bfs_set_in_bitmap: null argument");
     G5_REQUIRE(b->depth >= 0, G5_E_STATE, "g5_bfs_set_in_bitmap: g5_bfs_start not called");
-    G5_HIP(g5::bitmap_to_queue(d_bits, b->wr, b->d_queue, b->d_cnt + kQLen, b->d_scratch, b->s));
     if (!b->d_inbits) G5_HIP(hipMalloc(&b->d_inbits, (size_t)(b->wr ? b->wr : 1) * 8));
-    if (b->wr) G5_HIP(hipMemcpyAsync(b->d_inbits, d_bits, (size_t)b->wr * 8, hipMemcpyDeviceToDevice, b->s));
-    int rc = sync_counters(b);
-    if (rc) return rc;
-    b->qlen = b->h_cnt[kQLen];
+    // the queue is made by an expansion that runs top-down, which needs it
+    hipLaunchKernelGGL(k_copy_words, g5::grid_for(b->wr, 256, 4096), 256, 0, b->s, d_bits, b->d_inbits, b->wr);
+    G5_HIP(hipGetLastError());
+    G5_HIP(hipStreamSynchronize(b->s));
+    b->queue_ok = b->qoff_ok = false;
     b->inbits_valid = true;
     b->depth++;
     return G5_OK;
@@ -1251,23 +1378,18 @@ extern "C" int g5_bfs_expand_bottom_up(g5_bfs *b, const g5_graph *gt, int *any_n
                    gt->col_start == g->row_start,
                G5_E_ARG, "g5_bfs_expand_bottom_up: gt is not the transposed block");
     hipStream_t s = b->s;
-    G5_HIP(g5::fill_i64(b->d_cnt + kNew, kBuVerts - kNew + 1, 0, s));
     if (b->prof) G5_HIP(hipEventRecord(b->ek0, s));
     // rows of gt = this block's columns, its columns = this block's rows: the
     // kernel's frontier bits are the row frontier, its parents local row ids
-    hipLaunchKernelGGL(k_bottom_up, g5::grid_for(b->wc, 4, 4096), 256, 0,
-                       s, (const int64_t *)gt->d_rowptr, (const uint32_t *)gt->d_cols,
-                       (const uint64_t *)b->d_visited, (const uint64_t *)b->d_inbits, b->d_out, b->d_parent, b->wc,
-                       b->d_cnt);
+    const int grid = g5::grid_for(b->wc, 4, kParts);
+    hipLaunchKernelGGL(k_bottom_up<false>, grid, 256, 0, s, (const int64_t *)gt->d_rowptr,
+                       (const uint32_t *)gt->d_cols, b->d_visited, (const uint64_t *)b->d_inbits, b->d_out,
+                       b->d_parent, (int32_t *)nullptr, 0, b->wc, b->d_part);
     G5_HIP(hipGetLastError());
     if (b->prof) G5_HIP(hipEventRecord(b->ek1, s));
-    hipLaunchKernelGGL(k_set_cnt, 1, 1, 0, s, b->d_cnt, (int)kOutLen, (int64_t)0);
-    hipLaunchKernelGGL(k_count_bits, g5::grid_for(b->wc, 256, 2048), 256, 0, s, (const uint64_t *)b->d_out, b->wc,
-                       b->d_cnt + kOutLen);
-    G5_HIP(hipGetLastError());
-    int rc = sync_counters(b);
-    if (rc) return rc;
-    rc = account_bottom_up(b, b->h_cnt[kOutLen]);
+    const int slot[] = {kOutLen, kNewEdges, kBuEdges, kBuVerts};
+    int rc = fold_counters(b, kParts, grid, slot, 4, false);
+    if (!rc) rc = account_bottom_up(b, b->h_cnt[kOutLen], false);
     if (rc) return rc;
     *any_new = b->h_cnt[kOutLen] > 0;
     return G5_OK;
@@ -1298,12 +1420,12 @@ extern "C" int g5_bfs_nedge(g5_bfs *b, int64_t *nedge)
 {
     G5_REQUIRE(b && nedge, G5_E_ARG, "g5_bfs_nedge: null argument");
     G5_REQUIRE(b->g->n_rows == b->g->n_cols, G5_E_STATE, "g5_bfs_nedge: needs a 1x1 block");
-    hipLaunchKernelGGL(k_set_cnt, 1, 1, 0, b->s, b->d_cnt, (int)kOutLen, (int64_t)0);
-    hipLaunchKernelGGL(k_nedge, g5::grid_for(b->g->n_rows / 4, 256, kSumGrid), 256, 0, b->s,
-                       (const uint32_t *)b->g->d_gdeg, (const int32_t *)b->d_level, b->g->n_rows,
-                       b->d_cnt + kOutLen);
+    const int grid = g5::grid_for(b->g->n_rows / 4, 256, kSumGrid);
+    hipLaunchKernelGGL(k_nedge, grid, 256, 0, b->s, (const uint32_t *)b->g->d_gdeg, (const int32_t *)b->d_level,
+                       b->g->n_rows, b->d_part);
     G5_HIP(hipGetLastError());
-    int rc = sync_counters(b);
+    const int slot[] = {kOutLen};
+    int rc = fold_counters(b, kParts, grid, slot, 1, false);
     if (rc) return rc;
     *nedge = b->h_cnt[kOutLen] / 2;
     return G5_OK;
@@ -1314,15 +1436,12 @@ extern "C" int g5_bfs_summary(g5_bfs *b, int64_t *nedge, uint64_t *checksum)
     G5_REQUIRE(b && nedge && checksum, G5_E_ARG, "g5_bfs_summary: null argument");
     G5_REQUIRE(b->g->n_rows == b->g->n_cols && b->g->row_start == b->g->col_start, G5_E_STATE,
                "g5_bfs_summary: needs a diagonal (1x1) block");
-    // kOutLen and kNewEdges as the two sums (free between levels)
-    static_assert(kNewEdges == kOutLen + 1, "the summary's two slots must be adjacent");
-    hipLaunchKernelGGL(k_set_cnt, 1, 1, 0, b->s, b->d_cnt, (int)kOutLen, (int64_t)0);
-    hipLaunchKernelGGL(k_set_cnt, 1, 1, 0, b->s, b->d_cnt, (int)kNewEdges, (int64_t)0);
-    hipLaunchKernelGGL(k_summary, g5::grid_for(b->g->n_rows, 256, kSumGrid), 256, 0, b->s,
-                       (const uint32_t *)b->g->d_gdeg, (const int32_t *)b->d_level, (const uint32_t *)b->d_parent,
-                       b->g->n_rows, b->d_cnt + kOutLen);
+    const int grid = g5::grid_for(b->g->n_rows, 256, kSumGrid);
+    hipLaunchKernelGGL(k_summary, grid, 256, 0, b->s, (const uint32_t *)b->g->d_gdeg, (const int32_t *)b->d_level,
+                       (const uint32_t *)b->d_parent, b->g->n_rows, b->d_part);
     G5_HIP(hipGetLastError());
-    int rc = sync_counters(b);
+    const int slot[] = {kOutLen, kNewEdges};
+    int rc = fold_counters(b, kParts, grid, slot, 2, false);
     if (rc) return rc;
     *nedge = b->h_cnt[kOutLen] / 2;
     *checksum = (uint64_t)b->h_cnt[kNewEdges];
@@ -1364,34 +1483,38 @@ extern "C" int g5_bfs_run(g5_bfs *b, int64_t root, int flags, int32_t *nlevels, 
     const int64_t n = g->n_rows;
     int64_t m_u = g->nnz;  // edges not yet checked top-down
     bool bu = false;       // the first level is always top-down
+    int64_t E = 0;         // the frontier's edges
+    if (b->prof) G5_HIP(hipMemcpyAsync(&b->h_cnt[kEdges], b->d_cnt + kEdges, 8, hipMemcpyDeviceToHost, s));
+    const int64_t tile = g5::tile_words(b->wc);
+    const int tiles = g5::tile_count(b->wc), bu_grid = g5::grid_for(b->wc, 4, kParts);
+    // d_out is the frontier, d_next the next one (clear before a top-down level)
     for (;;) {
-        G5_HIP(g5::fill_i64(b->d_cnt + kNew, kBuVerts - kNew + 1, 0, s));
-        uint64_t *fresh = b->d_out;
         if (bu) {
             if (b->prof) G5_HIP(hipEventRecord(b->ek0, s));
-            hipLaunchKernelGGL(k_bottom_up, g5::grid_for(b->wc, 4, 4096),
-                               256, 0, s, (const int64_t *)g->d_rowptr,
-                               (const uint32_t *)g->d_cols, (const uint64_t *)b->d_visited,
-                               (const uint64_t *)b->d_out, b->d_next, b->d_parent, b->wc, b->d_cnt);
+            hipLaunchKernelGGL(k_bottom_up<true>, bu_grid, 256, 0, s, (const int64_t *)g->d_rowptr,
+                               (const uint32_t *)g->d_cols, b->d_visited, (const uint64_t *)b->d_out, b->d_next,
+                               b->d_parent, b->d_level, (int32_t)(b->depth + 1), b->wc, b->d_part);
             G5_HIP(hipGetLastError());
             if (b->prof) G5_HIP(hipEventRecord(b->ek1, s));
-            fresh = b->d_next;
+            const int slot[] = {kNew, kNewEdges, kBuEdges, kBuVerts};
+            rc = fold_counters(b, kParts, bu_grid, slot, 4, true);
         } else {
-            rc = expand_level(b);
+            rc = expand_level(b, b->d_next, false, b->depth == 0 ? -1 : E);
             if (rc) return rc;
+            hipLaunchKernelGGL(k_commit, tiles, 256, 0, s, (const uint64_t *)b->d_next, b->d_next, b->d_visited,
+                               b->d_level, b->wc, tile, (int32_t)(b->depth + 1), (const int64_t *)g->d_rowptr,
+                               b->d_part);
+            G5_HIP(hipGetLastError());
+            const int slot[] = {kNew, kNewEdges};
+            rc = fold_counters(b, g5::kTiles, tiles, slot, 2, true);
         }
-        // a bottom-up level already summed its new vertices' degrees
-        hipLaunchKernelGGL(k_commit, g5::grid_for(b->wc, 256, 2048), 256, 0, s, fresh, b->d_visited, b->d_level,
-                           b->wc, (int32_t)(b->depth + 1), b->d_cnt,
-                           bu ? (const int64_t *)nullptr : (const int64_t *)g->d_rowptr);
-        G5_HIP(hipGetLastError());
-        if (bu) std::swap(b->d_out, b->d_next);
-        rc = sync_counters(b);
         if (rc) return rc;
+        std::swap(b->d_out, b->d_next);
         // the previous level's codec round trip has completed by now
         G5_REQUIRE(b->h_cnt[kCodecErr] == 0, G5_E_STREAM, "g5_bfs_run: codec round trip lost values");
         const int64_t n_new = b->h_cnt[kNew];
-        rc = bu ? account_bottom_up(b, n_new) : account_level(b, b->qlen, n_new);
+        if (b->depth == 0) E = b->h_cnt[kEdges];
+        rc = bu ? account_bottom_up(b, n_new, true) : account_level(b, b->qlen, E, n_new);
         if (rc) return rc;
         if (n_new == 0) break;
         // the next level's direction
@@ -1405,8 +1528,17 @@ extern "C" int g5_bfs_run(g5_bfs *b, int64_t root, int flags, int32_t *nlevels, 
         // the out-bitmap holds exactly the new vertices; a queue of them is
         // needed by a top-down level and by the codec
         b->qlen = n_new;
-        if (!bu_next || codec)
-            G5_HIP(g5::bitmap_to_queue(b->d_out, b->wc, b->d_queue, b->d_cnt + kQLen, b->d_scratch, s));
+        E = m_f;
+        if (!bu_next || codec) {
+            g5::QueueOut o{};
+            o.q = b->d_queue;
+            o.qoff = b->d_qoff;
+            o.clear = b->d_next;
+            o.n_clear = bu_next ? 0 : b->wc;
+            // a top-down level's commit has left its tiles' sums
+            G5_HIP(g5::bitmap_to_queue(b->d_out, b->wc, bu_next ? nullptr : (const int64_t *)g->d_rowptr, o,
+                                       b->d_part, !bu, s));
+        }
         if (codec) {
             // encode -> decode in place with no host synchronisation; checked
             // at the next level's counter read
@@ -1420,6 +1552,10 @@ extern "C" int g5_bfs_run(g5_bfs *b, int64_t root, int flags, int32_t *nlevels, 
     G5_HIP(hipEventSynchronize(b->ev1));
     if (ms) G5_HIP(hipEventElapsedTime(ms, b->ev0, b->ev1));
     if (nlevels) *nlevels = b->depth + 1;
+    // no frontier is left
+    b->qlen = 0;
+    b->queue_ok = true;
+    b->qoff_ok = false;
     return G5_OK;
 }
 

@@ -63,12 +63,45 @@ constexpr int kWave = 64;
 size_t scan_scratch_words(int64_t n);
 hipError_t exclusive_scan_i64(int64_t *d_data, int64_t n, int64_t *d_total, int64_t *scratch,
                               hipStream_t s);
-// Bitmap -> sorted queue of set-bit indices (+ base).  Writes the count to
-// *d_count.  scratch as for exclusive_scan_i64 over n_words.
-hipError_t bitmap_to_queue(const uint64_t *d_bits, int64_t n_words, uint32_t *d_queue,
-                           int64_t *d_count, int64_t *scratch, hipStream_t s);
-// Queue -> bitmap (bitmap must be cleared first).
-hipError_t queue_to_bitmap(const uint32_t *d_queue, int64_t n, uint64_t *d_bits, hipStream_t s);
+// Bitmap tiles: the n_words words of a bitmap in at most kTiles shares of
+// tile_words(n_words) words (a multiple of 64); a pass over the bitmap gives
+// workgroup t tile t and leaves what it summed in part[t].
+constexpr int kTiles = 1024;
+inline int64_t tile_words(int64_t n_words)
+{
+    const int64_t w = (n_words + kTiles - 1) / kTiles;
+    return w < 64 ? 64 : (w + 63) / 64 * 64;
+}
+inline int tile_count(int64_t n_words) { return (int)((n_words + tile_words(n_words) - 1) / tile_words(n_words)); }
+// Bitmap -> sorted queue of its set bits, in two launches.  With rowptr also
+// the queue's degree prefix (qoff).  The count goes to *d_n (device) and *h_n
+// (pinned), the degree total to *d_e; null pointers are left out.  part: 2 *
+// kTiles entries; have_parts: they hold every tile's bits (and, kTiles
+// further, degrees) already.  clear: n_clear words are set to 0 on the way.
+struct QueueOut {
+    uint32_t *q;
+    int64_t *qoff;
+    int64_t *d_n, *d_e, *h_n;
+    uint64_t *clear;
+    int64_t n_clear;
+};
+hipError_t bitmap_to_queue(const uint64_t *d_bits, int64_t n_words, const int64_t *rowptr, const QueueOut &out,
+                           int64_t *part, bool have_parts, hipStream_t s);
+// Up to 4 sums of n entries each, part[j * stride ...], to pinned memory
+// (host[0 .. k)) and to the device (null: left out); then ncopy entries from the device to pinned
+// memory.  One launch: a level's counters reach the host without a copy.
+struct FoldOut {
+    int64_t *host[4], *dev[4];
+    const int64_t *from;
+    int64_t *to;
+    int ncopy;
+};
+hipError_t fold_parts(const int64_t *part, int64_t stride, int n, const FoldOut &out, hipStream_t s);
+// Queue -> bitmap of n_words words (which must be cleared first): ids beyond
+// them are left out, and one of them sets *h_bad (pinned; null if the caller
+// knows that there are none).
+hipError_t queue_to_bitmap(const uint32_t *d_queue, int64_t n, uint64_t *d_bits, int64_t n_words, int64_t *h_bad,
+                           hipStream_t s);
 hipError_t fill_u64(uint64_t *d, int64_t n, uint64_t v, hipStream_t s);
 hipError_t fill_u32(uint32_t *d, int64_t n, uint32_t v, hipStream_t s);
 hipError_t fill_i32(int32_t *d, int64_t n, int32_t v, hipStream_t s);
@@ -182,6 +215,13 @@ __device__ __forceinline__ int64_t g5_block_sum256(int64_t v)
     const int64_t t = s_part[0] + s_part[1] + s_part[2] + s_part[3];
     __syncthreads();  // s_part is free again for the next call
     return t;
+}
+
+// lane l's value, to every lane (l the same in all of them)
+__device__ __forceinline__ uint64_t g5_bcast64(uint64_t x, int l)
+{
+    return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(x >> 32), l) << 32) |
+           (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, l);
 }
 
 // last s in [lo, hi] with off[s] <= e (off ascends, off[lo] <= e), by a whole

@@ -155,73 +155,216 @@ hipError_t exclusive_scan_i64(int64_t *d, int64_t n, int64_t *d_total, int64_t *
     return hipGetLastError();
 }
 
-// ---------------------------------------------------------------- bitmap <-> queue
+// ---------------------------------------------------------------- sums
 
-// One thread per word.  Word popcounts are scanned per 256-word block; the
-// block offsets come from a scan of the block totals.
-__global__ void k_bm_counts(const uint64_t *bits, int64_t n_words, int64_t *blk)
+// K arrays; all loads of a round are in flight at once
+template <int K>
+__global__ __launch_bounds__(1024) void k_fold(const int64_t *__restrict__ part, int64_t stride, int n, FoldOut out)
 {
-    __shared__ int64_t lw[4];
-    const int64_t w = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    const int64_t c = (w < n_words) ? __popcll(bits[w]) : 0;
-    int64_t tot;
-    block_excl_scan(c, lw, &tot);
-    if (threadIdx.x == 0) blk[blockIdx.x] = tot;
-}
-
-__global__ void k_bm_write(const uint64_t *bits, int64_t n_words, const int64_t *blk_off,
-                           uint32_t *queue, int64_t *d_count)
-{
-    __shared__ int64_t lw[4];
-    const int64_t w = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    uint64_t word = (w < n_words) ? bits[w] : 0;
-    int64_t tot;
-    int64_t pos = block_excl_scan(__popcll(word), lw, &tot) + blk_off[blockIdx.x];
-    while (word) {
-        const int b = __ffsll((long long)word) - 1;
-        queue[pos++] = (uint32_t)(w * 64 + b);
-        word &= word - 1;
+    __shared__ int64_t s_wave[K][16];
+    int64_t c[K] = {};
+    for (int i0 = 0; i0 < n; i0 += 4096) {
+        int64_t x[K][4];
+#pragma unroll
+        for (int j = 0; j < K; ++j)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int i = i0 + k * 1024 + threadIdx.x;
+                x[j][k] = i < n ? part[j * stride + i] : 0;
+            }
+#pragma unroll
+        for (int j = 0; j < K; ++j) c[j] += (x[j][0] + x[j][1]) + (x[j][2] + x[j][3]);
     }
-    if (d_count && blockIdx.x == gridDim.x - 1 && threadIdx.x == blockDim.x - 1) *d_count = pos;
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+        c[j] = g5_wave_sum(c[j]);
+        if (__lane_id() == 0) s_wave[j][threadIdx.x >> 6] = c[j];
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < out.ncopy) out.to[threadIdx.x] = out.from[threadIdx.x];
+    if (threadIdx.x >= 64) return;
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+        const int64_t t = g5_wave_sum(threadIdx.x < 16 ? s_wave[j][threadIdx.x] : 0);
+        if (threadIdx.x == 0) {
+            if (out.host[j]) *out.host[j] = t;
+            if (out.dev[j]) *out.dev[j] = t;
+        }
+    }
 }
 
-hipError_t bitmap_to_queue(const uint64_t *bits, int64_t n_words, uint32_t *queue,
-                           int64_t *d_count, int64_t *scratch, hipStream_t s)
+hipError_t fold_parts(const int64_t *part, int64_t stride, int n, const FoldOut &out, hipStream_t s)
 {
-    if (n_words <= 0) return fill_i64(d_count, 1, 0, s);
-    const int64_t blocks = (n_words + 255) / 256;
-    int64_t *blk = scratch;
-    hipLaunchKernelGGL(k_bm_counts, (unsigned)blocks, 256, 0, s, bits, n_words, blk);
-    hipError_t e = exclusive_scan_i64(blk, blocks, nullptr, scratch + blocks + 1, s);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_bm_write, (unsigned)blocks, 256, 0, s, bits, n_words,
-                       (const int64_t *)blk, queue, d_count);
+    const int k = out.host[3] ? 4 : out.host[2] ? 3 : out.host[1] ? 2 : 1;
+    hipLaunchKernelGGL(k == 4 ? k_fold<4> : k == 3 ? k_fold<3> : k == 2 ? k_fold<2> : k_fold<1>, 1, 1024, 0, s, part,
+                       stride, n, out);
     return hipGetLastError();
 }
 
-// Sorted queue: the first entry of each run of equal words ORs the run's bits
-// with one atomic (runs that cross a wave boundary simply take two atomics).
-__global__ void k_q2bm(const uint32_t *q, int64_t n, uint64_t *bits)
+// ---------------------------------------------------------------- bitmap <-> queue
+//
+// A tile's workgroup takes 64 words at a time, 16 to a wave (lane j holds
+// word j); a word's vertices are then the wave's lanes, so that row offsets
+// are read and the queue is written in order.  A workgroup finds its tile's
+// place by adding up the tiles before it (at most kTiles) instead of waiting
+// for a scan of them: two launches where counts, scan of one to three
+// launches and write took three to five, and a thread wrote each word's
+// entries one by one.  2^22 vertices: 10 us -> MEASURE.
+constexpr int kWordsWave = 16;
+
+// the degrees of this wave's vertices whose bits (lane j: word w0 + j) are
+// set, in d[j] of each word's lanes; returns the lane's sum
+__device__ __forceinline__ int64_t wave_degrees(uint64_t bits, int64_t w0, const int64_t *__restrict__ rowptr,
+                                                int lane, uint32_t (&d)[kWordsWave])
 {
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t v = q[i];
-    const uint32_t w = v >> 6;
-    const bool lead = (i == 0) || ((q[i - 1] >> 6) != w) || ((threadIdx.x & 63) == 0);
-    if (!lead) return;
-    uint64_t acc = 0;
-    int64_t j = i;
-    do {
-        acc |= 1ull << (q[j] & 63);
-        ++j;
-    } while (j < n && (q[j] >> 6) == w && (((threadIdx.x + (j - i)) & 63) != 0));
-    atomicOr((unsigned long long *)&bits[w], (unsigned long long)acc);
+    int64_t sum = 0;
+    int64_t lo[kWordsWave], hi[kWordsWave];
+#pragma unroll
+    for (int j = 0; j < kWordsWave; ++j) {
+        const uint64_t b = g5_bcast64(bits, j);
+        const int64_t v = (w0 + j) * 64 + lane;
+        const bool set = b >> lane & 1;
+        lo[j] = set ? rowptr[v] : 0;
+        hi[j] = set ? rowptr[v + 1] : 0;
+    }
+#pragma unroll
+    for (int j = 0; j < kWordsWave; ++j) {
+        d[j] = (uint32_t)(hi[j] - lo[j]);
+        sum += d[j];
+    }
+    return sum;
 }
 
-hipError_t queue_to_bitmap(const uint32_t *q, int64_t n, uint64_t *bits, hipStream_t s)
+__global__ __launch_bounds__(256) void k_bm_sums(const uint64_t *__restrict__ bits, int64_t n_words, int64_t tile,
+                                                 const int64_t *__restrict__ rowptr, int64_t *__restrict__ part)
+{
+    const int lane = __lane_id();
+    const int64_t end = min(n_words, (blockIdx.x + 1) * tile);
+    int64_t c = 0, e = 0;
+    for (int64_t w0 = blockIdx.x * tile + (threadIdx.x >> 6) * kWordsWave; w0 < end; w0 += 64) {
+        const uint64_t b = lane < kWordsWave && w0 + lane < end ? bits[w0 + lane] : 0ull;
+        c += __popcll(b);
+        if (rowptr && __ballot(b != 0)) {
+            uint32_t d[kWordsWave];
+            e += wave_degrees(b, w0, rowptr, lane, d);
+        }
+    }
+    c = g5_block_sum256(c);
+    if (threadIdx.x == 0) part[blockIdx.x] = c;
+    if (!rowptr) return;
+    e = g5_block_sum256(e);
+    if (threadIdx.x == 0) part[kTiles + blockIdx.x] = e;
+}
+
+template <bool kOffsets>
+__global__ __launch_bounds__(256) void k_bm_write(const uint64_t *__restrict__ bits, int64_t n_words, int64_t tile,
+                                                  const int64_t *__restrict__ rowptr,
+                                                  const int64_t *__restrict__ part, QueueOut out)
+{
+    __shared__ int64_t s_n[4], s_e[4];
+    const int lane = __lane_id(), wave = threadIdx.x >> 6;
+    for (int64_t w = blockIdx.x * 256ll + threadIdx.x; w < out.n_clear; w += gridDim.x * 256ll) out.clear[w] = 0;
+    // tiles before this one
+    int64_t pos = 0, eoff = 0;
+    for (int t = threadIdx.x; t < (int)blockIdx.x; t += 256) {
+        pos += part[t];
+        if (kOffsets) eoff += part[kTiles + t];
+    }
+    pos = g5_block_sum256(pos);
+    if (kOffsets) eoff = g5_block_sum256(eoff);
+    const int64_t end = min(n_words, (blockIdx.x + 1) * tile);
+    for (int64_t g = blockIdx.x * tile; g < end; g += 64) {
+        const int64_t w0 = g + wave * kWordsWave;
+        const uint64_t b = lane < kWordsWave && w0 + lane < end ? bits[w0 + lane] : 0ull;
+        uint32_t d[kWordsWave] = {};
+        int64_t n = __popcll(b), e = 0;
+        const bool any = __ballot(b != 0) != 0;
+        if (kOffsets && any) e = wave_degrees(b, w0, rowptr, lane, d);
+        n = g5_wave_sum(n);
+        if (kOffsets) e = g5_wave_sum(e);
+        if (lane == 0) {
+            s_n[wave] = n;
+            if (kOffsets) s_e[wave] = e;
+        }
+        __syncthreads();
+        int64_t at = pos, eat = eoff;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            at += k < wave ? s_n[k] : 0;
+            pos += s_n[k];
+            if (kOffsets) {
+                eat += k < wave ? s_e[k] : 0;
+                eoff += s_e[k];
+            }
+        }
+        __syncthreads();
+        if (!any) continue;
+#pragma unroll
+        for (int j = 0; j < kWordsWave; ++j) {
+            const uint64_t word = g5_bcast64(b, j);
+            if (!word) continue;
+            const bool set = word >> lane & 1;
+            const int64_t i = at + __popcll(word & ((1ull << lane) - 1));
+            if (set) out.q[i] = (uint32_t)((w0 + j) * 64 + lane);
+            at += __popcll(word);
+            if (kOffsets) {
+                const int64_t inc = g5_wave_incl_scan((int64_t)d[j]);
+                if (set) out.qoff[i] = eat + inc - d[j];
+                eat += (int64_t)g5_bcast64((uint64_t)inc, 63);
+            }
+        }
+    }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+        if (out.d_n) *out.d_n = pos;
+        if (out.h_n) *out.h_n = pos;
+        if (kOffsets && out.d_e) *out.d_e = eoff;
+    }
+}
+
+hipError_t bitmap_to_queue(const uint64_t *bits, int64_t n_words, const int64_t *rowptr, const QueueOut &out,
+                           int64_t *part, bool have_parts, hipStream_t s)
+{
+    const int64_t tile = tile_words(n_words);
+    const int tiles = n_words > 0 ? tile_count(n_words) : 1;  // an empty bitmap: the counts
+    if (!have_parts && n_words > 0)
+        hipLaunchKernelGGL(k_bm_sums, tiles, 256, 0, s, bits, n_words, tile, rowptr, part);
+    if (rowptr) hipLaunchKernelGGL(k_bm_write<true>, tiles, 256, 0, s, bits, n_words, tile, rowptr, part, out);
+    else hipLaunchKernelGGL(k_bm_write<false>, tiles, 256, 0, s, bits, n_words, tile, rowptr, part, out);
+    return hipGetLastError();
+}
+
+// A wave takes 64 consecutive ids.  Neighbours with the same word combine
+// their bits (a lane takes in the lanes 1, 2, 4, ... further that hold its
+// word; a bit more than once does no harm), and the first of each run of equal
+// words writes them with one atomic: a queue in ascending order takes about
+// one per word and wave, and any other order stays right.
+__global__ __launch_bounds__(256) void k_q2bm(const uint32_t *__restrict__ q, int64_t n,
+                                              uint64_t *__restrict__ bits, int64_t n_words, int64_t *h_bad)
+{
+    const int lane = __lane_id();
+    const int64_t last = (n + 63) / 64 * 64;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < last; i += (int64_t)gridDim.x * blockDim.x) {
+        const uint32_t v = i < n ? q[i] : 0u;
+        const bool ok = i < n && (int64_t)(v >> 6) < n_words;
+        if (i < n && !ok && h_bad) *h_bad = 1;
+        const uint32_t w = ok ? v >> 6 : ~0u;
+        uint64_t acc = ok ? 1ull << (v & 63) : 0ull;
+        const uint32_t before = __shfl_up(w, 1, 64);
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t ow = __shfl_down(w, d, 64);
+            const uint64_t o = __shfl_down(acc, d, 64);
+            if (lane + d < 64 && ow == w) acc |= o;
+        }
+        if (ok && (lane == 0 || before != w)) atomicOr((unsigned long long *)&bits[w], (unsigned long long)acc);
+    }
+}
+
+hipError_t queue_to_bitmap(const uint32_t *q, int64_t n, uint64_t *bits, int64_t n_words, int64_t *h_bad,
+                           hipStream_t s)
 {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_q2bm, (unsigned)((n + 255) / 256), 256, 0, s, q, n, bits);
+    hipLaunchKernelGGL(k_q2bm, grid_for(n, 256, 16384), 256, 0, s, q, n, bits, n_words, h_bad);
     return hipGetLastError();
 }
 
@@ -365,16 +508,95 @@ extern "C" int g5_fill_u64(uint64_t *d, int64_t n, uint64_t value)
 }
 
 namespace {
-// *ndiff += the positions where a and b differ
+
+// What the calls below need on a device: the tiles' sums and a few pinned
+// words, 16 KiB.  A thread keeps one per device it has called them on (the
+// first kDevices; on others a call allocates its own), so that a call
+// neither allocates nor waits for a free; they go with the thread.
+struct Work {
+    int device = -1;
+    int64_t *part = nullptr;  // 2 * kTiles, on the device
+    int64_t *host = nullptr;  // 8, pinned
+    Work() = default;
+    Work(const Work &) = delete;
+    Work &operator=(const Work &) = delete;
+    ~Work()
+    {
+        if (part) (void)hipFree(part);
+        if (host) (void)hipHostFree(host);
+    }
+    hipError_t get()
+    {
+        hipError_t e = hipSuccess;
+        if (!part) e = hipMalloc(&part, 2 * g5::kTiles * 8);
+        if (e == hipSuccess && !host) e = hipHostMalloc(&host, 8 * 8, hipHostMallocDefault);
+        return e;
+    }
+};
+constexpr int kDevices = 8;
+
+// the calling thread's, for its current device; own: the caller's, for a
+// device beyond those that are kept
+hipError_t work_for(Work *&w, Work &own)
+{
+    static thread_local Work kept[kDevices];
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    w = &own;
+    for (Work &k : kept)
+        if (k.device == dev || k.device < 0) {
+            w = &k;
+            break;
+        }
+    w->device = dev;
+    return w->get();
+}
+
+// part[workgroup] = its positions where a and b differ
 __global__ __launch_bounds__(256) void k_diff_u32(const uint32_t *__restrict__ a, const uint32_t *__restrict__ b,
-                                                  int64_t n, unsigned long long *__restrict__ ndiff)
+                                                  int64_t n, int64_t *__restrict__ part)
 {
     int64_t c = 0;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
         c += a[i] != b[i];
     c = g5_block_sum256(c);
-    if (threadIdx.x == 0 && c) atomicAdd(ndiff, (unsigned long long)c);
+    if (threadIdx.x == 0) part[blockIdx.x] = c;
 }
+
+// part[workgroup] = its ids at or beyond n_words * 64
+__global__ __launch_bounds__(256) void k_beyond(const uint32_t *__restrict__ q, int64_t n, int64_t n_words,
+                                                int64_t *__restrict__ part)
+{
+    int64_t c = 0;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        c += (int64_t)(q[i] >> 6) >= n_words;
+    c = g5_block_sum256(c);
+    if (threadIdx.x == 0) part[blockIdx.x] = c;
+}
+
+__global__ __launch_bounds__(256) void k_popcount(const uint64_t *__restrict__ bits, int64_t n_words,
+                                                  int64_t *__restrict__ part)
+{
+    int64_t c = 0;
+    for (int64_t w = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; w < n_words; w += (int64_t)gridDim.x * blockDim.x)
+        c += __popcll(bits[w]);
+    c = g5_block_sum256(c);
+    if (threadIdx.x == 0) part[blockIdx.x] = c;
+}
+
+// waits for the sum of w.part[0 .. n)
+hipError_t sum_of(Work &w, int n, int64_t *sum)
+{
+    g5::FoldOut o{};
+    o.host[0] = w.host;
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = g5::fold_parts(w.part, 0, n, o, nullptr);
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+    if (e == hipSuccess) *sum = w.host[0];
+    return e;
+}
+
 }  // namespace
 
 extern "C" int g5_diff_u32(const uint32_t *d_a, const uint32_t *d_b, int64_t n, int64_t *ndiff)
@@ -382,17 +604,11 @@ extern "C" int g5_diff_u32(const uint32_t *d_a, const uint32_t *d_b, int64_t n, 
     G5_REQUIRE(n >= 0 && ndiff && (n == 0 || (d_a && d_b)), G5_E_ARG, "g5_diff_u32: bad arguments");
     *ndiff = 0;
     if (n == 0) return G5_OK;
-    unsigned long long *d = nullptr, h = 0;
-    G5_HIP(hipMalloc(&d, 8));
-    hipError_t e = g5::fill_u64((uint64_t *)d, 1, 0, nullptr);
-    if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_diff_u32, g5::grid_for(n, 256, 8192), 256, 0, nullptr, d_a, d_b, n, d);
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess) e = hipMemcpy(&h, d, 8, hipMemcpyDeviceToHost);
-    (void)hipFree(d);
-    G5_HIP(e);
-    *ndiff = (int64_t)h;
+    Work own, *w = nullptr;
+    G5_HIP(work_for(w, own));
+    const int grid = g5::grid_for(n, 256, 2 * g5::kTiles);
+    hipLaunchKernelGGL(k_diff_u32, grid, 256, 0, nullptr, d_a, d_b, n, w->part);
+    G5_HIP(sum_of(*w, grid, ndiff));
     return G5_OK;
 }
 
@@ -400,83 +616,46 @@ extern "C" int g5_bitmap_to_queue(const uint64_t *d_bits, int64_t n_words, uint3
 {
     G5_REQUIRE(n_words >= 0 && n && (n_words == 0 || (d_bits && d_queue)), G5_E_ARG,
                "g5_bitmap_to_queue: bad arguments");
-    int64_t *d_tmp = nullptr;
-    const size_t words = g5::scan_scratch_words((n_words + 255) / 256 + 1) + (n_words + 255) / 256 + 8;
-    G5_HIP(hipMalloc(&d_tmp, words * 8));
-    hipError_t e = g5::bitmap_to_queue(d_bits, n_words, d_queue, d_tmp, d_tmp + 1, nullptr);
-    if (e == hipSuccess) e = hipMemcpy(n, d_tmp, 8, hipMemcpyDeviceToHost);
-    (void)hipFree(d_tmp);
-    G5_HIP(e);
+    Work own, *w = nullptr;
+    G5_HIP(work_for(w, own));
+    g5::QueueOut o{};
+    o.q = d_queue;
+    o.h_n = w->host;
+    G5_HIP(g5::bitmap_to_queue(d_bits, n_words, nullptr, o, w->part, false, nullptr));
+    G5_HIP(hipStreamSynchronize(nullptr));
+    *n = w->host[0];
     return G5_OK;
 }
-
-namespace {
-__global__ void k_popcount(const uint64_t *__restrict__ bits, int64_t n_words, unsigned long long *__restrict__ out)
-{
-    int64_t c = 0;
-    for (int64_t w = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; w < n_words; w += (int64_t)gridDim.x * blockDim.x)
-        c += __popcll(bits[w]);
-    c = g5_block_sum256(c);
-    if (threadIdx.x == 0 && c) atomicAdd(out, (unsigned long long)c);
-}
-}  // namespace
 
 extern "C" int g5_bitmap_count(const uint64_t *d_bits, int64_t n_words, int64_t *count)
 {
     G5_REQUIRE(n_words >= 0 && count && (n_words == 0 || d_bits), G5_E_ARG, "g5_bitmap_count: bad arguments");
     *count = 0;
     if (n_words == 0) return G5_OK;
-    unsigned long long *d_c = nullptr;
-    G5_HIP(hipMalloc(&d_c, 8));
-    hipError_t e = g5::fill_u64((uint64_t *)d_c, 1, 0, nullptr);
-    if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_popcount, g5::grid_for(n_words, 256, 2048), 256, 0, nullptr, d_bits, n_words, d_c);
-        e = hipGetLastError();
-    }
-    unsigned long long h = 0;
-    if (e == hipSuccess) e = hipMemcpy(&h, d_c, 8, hipMemcpyDeviceToHost);
-    (void)hipFree(d_c);
-    G5_HIP(e);
-    *count = (int64_t)h;
+    Work own, *w = nullptr;
+    G5_HIP(work_for(w, own));
+    const int grid = g5::grid_for(n_words, 256, 2 * g5::kTiles);
+    hipLaunchKernelGGL(k_popcount, grid, 256, 0, nullptr, d_bits, n_words, w->part);
+    G5_HIP(sum_of(*w, grid, count));
     return G5_OK;
 }
-
-namespace {
-// ids at or beyond n_words * 64 are counted in *bad and skipped
-__global__ void k_q2bm_checked(const uint32_t *__restrict__ q, int64_t n, uint64_t *__restrict__ bits,
-                               int64_t n_words, unsigned long long *__restrict__ bad)
-{
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const uint32_t v = q[i];
-        if ((int64_t)(v >> 6) >= n_words) {
-            atomicAdd(bad, 1ull);
-            continue;
-        }
-        atomicOr((unsigned long long *)&bits[v >> 6], 1ull << (v & 63));
-    }
-}
-}  // namespace
 
 extern "C" int g5_queue_to_bitmap(const uint32_t *d_queue, int64_t n, uint64_t *d_bits, int64_t n_words)
 {
     G5_REQUIRE(n >= 0 && n_words >= 0 && (n == 0 || d_queue) && (n_words == 0 || d_bits), G5_E_ARG,
                "g5_queue_to_bitmap: bad arguments");
+    Work own, *w = nullptr;
+    G5_HIP(work_for(w, own));
+    w->host[0] = 0;
     G5_HIP(g5::fill_u64(d_bits, n_words, 0, nullptr));
-    if (n == 0) {
-        G5_HIP(hipStreamSynchronize(nullptr));
-        return G5_OK;
-    }
-    unsigned long long *d_bad = nullptr, h_bad = 0;
-    G5_HIP(hipMalloc(&d_bad, 8));
-    hipError_t e = hipMemset(d_bad, 0, 8);
-    if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_q2bm_checked, g5::grid_for(n, 256, 16384), 256, 0, nullptr, d_queue, n, d_bits, n_words,
-                           d_bad);
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess) e = hipMemcpy(&h_bad, d_bad, 8, hipMemcpyDeviceToHost);
-    (void)hipFree(d_bad);
-    G5_HIP(e);
-    G5_REQUIRE(h_bad == 0, G5_E_ARG, "g5_queue_to_bitmap: %llu ids beyond %lld words", h_bad, (long long)n_words);
+    G5_HIP(g5::queue_to_bitmap(d_queue, n, d_bits, n_words, w->host, nullptr));
+    G5_HIP(hipStreamSynchronize(nullptr));
+    if (w->host[0] == 0) return G5_OK;
+    int64_t bad = 0;
+    const int grid = g5::grid_for(n, 256, 2 * g5::kTiles);
+    hipLaunchKernelGGL(k_beyond, grid, 256, 0, nullptr, d_queue, n, n_words, w->part);
+    G5_HIP(sum_of(*w, grid, &bad));
+    G5_REQUIRE(bad == 0, G5_E_ARG, "g5_queue_to_bitmap: %lld ids beyond %lld words", (long long)bad,
+               (long long)n_words);
     return G5_OK;
 }
