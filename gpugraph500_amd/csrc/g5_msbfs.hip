@@ -249,6 +249,8 @@ struct g5_msbfs {
     // join: roots [0, 64), lanes [64, 128), added frontier [128, 130), root
     // degrees [130, 194); batch run: the roots' reach [0, 64)
     int64_t *d_join = nullptr;
+    uint64_t *d_dup = nullptr;  // push levels: the edges that the minimum pass looks at
+    int64_t dup_tiles = 0;
     unsigned long long *d_sums = nullptr;  // leave: checksums [0, 64), generated-degree sums [64, 128)
     // the last batch run: device time of the search and of its finalising
     // pass (ev_fin between them), and whether its level bytes are final
@@ -830,8 +832,13 @@ __global__ __launch_bounds__(kBlock) void k_pull_block(
 // The frontier's vertices u (active bitmap -> sorted queue) push their lane
 // bits along their edges: next[v] |= frontier[u] & ~visited[v].  The edge
 // whose atomicOr sets a (v, root) bit first stores its source in the pair's
-// parent slot; a second pass over the same edges lowers every newly reached
-// pair's slot to the minimum frontier neighbour with atomicMin.  Work is balanced by edges: each block tile takes
+// parent slot; a second pass over the edges that found one of their pairs set
+// (a bit per edge, written by the first pass a wave at a time) lowers their
+// pairs' slots to the minimum frontier neighbour with atomicMin.  At scale 24
+// it takes 213 us of the largest push level (350 over all edges), at scale 26
+// 825 (1300).  The first pass is bound by atomics on memory, of which the card
+// completes 20 to 28 billion a second whatever they touch.  Work is balanced
+// by edges: each block tile takes
 // kPushTile consecutive edges of the frontier and finds each edge's source by
 // binary search in the frontier's degree prefix.  The push kernels work on
 // the lanes in lm (all lanes on push levels, the pushed lanes of a split
@@ -921,8 +928,10 @@ __device__ __forceinline__ int64_t fq_src(const int64_t *__restrict__ qoff, int6
 // in mark, the next frontier's active bitmap.  The first pass writes the
 // level bytes of the pairs it sets (every candidate parent of a pair is of
 // the same level).
+// The first pass returns whether another edge had set one of its pairs before:
+// only such an edge can hold a smaller parent than the one stored.
 template <bool kMin>
-__device__ __forceinline__ void push_edge(uint32_t u, uint32_t uo, uint32_t v, uint32_t vo,
+__device__ __forceinline__ bool push_edge(uint32_t u, uint32_t uo, uint32_t v, uint32_t vo,
                                           const uint64_t *__restrict__ visited,
                                           const uint64_t *__restrict__ frontier, uint64_t *__restrict__ next,
                                           int32_t *__restrict__ parent, uint8_t *__restrict__ level, uint8_t lv,
@@ -934,14 +943,16 @@ __device__ __forceinline__ void push_edge(uint32_t u, uint32_t uo, uint32_t v, u
     if (!kMin) {
         // (a plain load of next[v] first, to skip atomics whose bits are set,
         // cost more than it saved: level 2 at scale 26 1.95 -> 1.7 ms without)
-        if (!f) return;
+        if (!f) return false;
         const uint64_t old = (uint64_t)atomicOr((unsigned long long *)&next[v], (unsigned long long)f);
         const uint64_t fresh = f & ~old;
         // the edge that sets a (v, root) bit first stores its source as the
         // pair's first parent candidate; the kMin pass lowers it
         if (fresh) write_slots(parent, level, vo, fresh, uo, lv);
         if (mark && old == 0) atomicOr((unsigned long long *)&mark[v >> 6], 1ull << (v & 63));
-    } else if (f) {
+        return fresh != f;
+    }
+    if (f) {
         uint64_t bits = f;
         int32_t *rec = &parent[(int64_t)vo * 64];
         while (bits) {
@@ -951,6 +962,7 @@ __device__ __forceinline__ void push_edge(uint32_t u, uint32_t uo, uint32_t v, u
             bits &= bits - 1;
         }
     }
+    return false;
 }
 
 // The candidate pass of a split level (its targets, the block and wave
@@ -1026,8 +1038,13 @@ struct PushArgs {
     uint64_t *next;
     int32_t *parent;
     uint8_t *level;
+    // a bit per edge of the first `dup_tiles` tiles: set by the first pass
+    // where the edge found a pair set before
+    uint64_t *dup;
+    int64_t dup_tiles;
 };
 
+// kMin (the minimum pass): only the edges that the first pass marked
 template <bool kMin, bool kCand>
 __device__ __forceinline__ void push_tiles(const PushArgs &a, const PushQueue &q, const Parts &s, PushTile &t,
                                            uint8_t lv, uint64_t lm, uint64_t *__restrict__ mark, int64_t vend,
@@ -1039,6 +1056,11 @@ __device__ __forceinline__ void push_tiles(const PushArgs &a, const PushQueue &q
         const uint32_t *__restrict__ fq = q.v + s.base[g];
         const int64_t *__restrict__ qoff = q.off + s.base[g];
         const int64_t t0 = (tile - s.tile0[g]) * kPushTile, t1 = min(s.edges[g], t0 + (int64_t)kPushTile);
+        uint64_t *dup = !kCand && tile < a.dup_tiles ? a.dup + tile * (kPushTile / 64) : nullptr;
+        if (kMin && dup) {
+            const bool any = threadIdx.x < (t1 - t0 + 63) / 64 && dup[threadIdx.x] != 0;
+            if (!__syncthreads_or(any)) continue;
+        }
         if (threadIdx.x < 128) {
             const int64_t r = g5_wave_src_of(qoff, 0, s.n[g] - 1, threadIdx.x < 64 ? t0 : t1 - 1);
             if (lane == 0) t.lo_hi[threadIdx.x >> 6] = r;
@@ -1046,7 +1068,8 @@ __device__ __forceinline__ void push_tiles(const PushArgs &a, const PushQueue &q
         __syncthreads();
         const int64_t lo = t.lo_hi[0], hi = t.lo_hi[1];
         const int ns = (int)min(hi - lo + 1, (int64_t)kPushTile + 1);
-        if (ns <= kPushTile) {
+        const bool staged = ns <= kPushTile;
+        if (staged) {
             for (int j = threadIdx.x; j < ns; j += kBlock) {
                 const uint32_t u = fq[lo + j];
                 const int64_t o = qoff[lo + j];
@@ -1056,35 +1079,43 @@ __device__ __forceinline__ void push_tiles(const PushArgs &a, const PushQueue &q
                 t.off[j] = (int32_t)max(o - t0, (int64_t)0);
             }
             __syncthreads();
-            int j = 0;  // the sources of a thread's edges ascend
-            for (int64_t e = t0 + threadIdx.x; e < t1; e += kBlock) {
-                const int32_t rel = (int32_t)(e - t0);
-                int x = j, y = ns - 1;  // last j with off[j] <= rel
-                while (x < y) {
-                    const int mid = (x + y + 1) >> 1;
-                    if (t.off[mid] <= rel) x = mid;
-                    else y = mid - 1;
+        }
+        int j = 0;  // the sources of a thread's edges ascend
+        for (int64_t e0 = t0 + (threadIdx.x & ~63); e0 < t1; e0 += kBlock) {
+            const int64_t e = e0 + lane;
+            bool again = false;
+            if (e < t1 && (!kMin || !dup || (dup[(e0 - t0) >> 6] >> lane & 1))) {
+                uint32_t u, uo;
+                int64_t pos;
+                if (staged) {
+                    const int32_t rel = (int32_t)(e - t0);
+                    int x = j, y = ns - 1;  // last j with off[j] <= rel
+                    while (x < y) {
+                        const int mid = (x + y + 1) >> 1;
+                        if (t.off[mid] <= rel) x = mid;
+                        else y = mid - 1;
+                    }
+                    j = x;
+                    u = t.u[j];
+                    uo = t.uo[j];
+                    pos = t.rb[j] + e;
+                } else {
+                    const int64_t si = fq_src(qoff, lo, hi, e);
+                    u = fq[si];
+                    uo = a.new2old[u];
+                    pos = a.rowptr[u] + (e - qoff[si]);
                 }
-                j = x;
-                const int64_t pos = t.rb[j] + e;
                 const uint32_t v = a.cols[pos];
-                if (v >= vend) continue;
-                if (kCand) push_cand(t.u[j], t.uo[j], v, a.visited, a.frontier, cand, npm, lm);
-                else
-                    push_edge<kMin>(t.u[j], t.uo[j], v, a.cols_orig[pos], a.visited, a.frontier, a.next, a.parent,
-                                    a.level, lv, lm, mark);
+                if (v < vend) {
+                    if (kCand) push_cand(u, uo, v, a.visited, a.frontier, cand, npm, lm);
+                    else
+                        again = push_edge<kMin>(u, uo, v, a.cols_orig[pos], a.visited, a.frontier, a.next, a.parent,
+                                                a.level, lv, lm, mark);
+                }
             }
-        } else {
-            for (int64_t e = t0 + threadIdx.x; e < t1; e += kBlock) {
-                const int64_t si = fq_src(qoff, lo, hi, e);
-                const uint32_t u = fq[si];
-                const int64_t pos = a.rowptr[u] + (e - qoff[si]);
-                const uint32_t v = a.cols[pos];
-                if (v >= vend) continue;
-                if (kCand) push_cand(u, a.new2old[u], v, a.visited, a.frontier, cand, npm, lm);
-                else
-                    push_edge<kMin>(u, a.new2old[u], v, a.cols_orig[pos], a.visited, a.frontier, a.next, a.parent,
-                                    a.level, lv, lm, mark);
+            if (!kMin && !kCand && dup) {
+                const uint64_t w = __ballot(again);
+                if (lane == 0) dup[(e0 - t0) >> 6] = w;
             }
         }
         __syncthreads();
@@ -1142,8 +1173,8 @@ __global__ void k_push_begin(uint64_t *__restrict__ act_next, int64_t nw, uint64
 // fewer edges than the frontier (levels past the peak: few new vertices of low
 // degree) it runs by rows: each new vertex scans its row in ascending
 // original-id order, and the first frontier neighbour of each new lane is its
-// parent.  Otherwise over the frontier's edges again, lowering the parents of
-// the pairs found at this level.  Both give the same minimum.
+// parent.  Otherwise over the frontier's marked edges again, lowering the
+// parents of the pairs found at this level.  Both give the same minimum.
 // A push level (whole) also counts each lane's frontier edges of the next
 // level here, from the new vertices' queue (k_queue sees them word by word,
 // mostly a few lanes at a time).
@@ -1996,8 +2027,12 @@ PushArgs push_args(const g5_msbfs *m, int p)
 {
     const Relabeled &R = m->rl;
     return PushArgs{R.rowptr, R.cols, R.cols_orig, R.new2old, m->d_visited, p == 0 ? m->d_fa : m->d_fb,
-                    p == 0 ? m->d_fb : m->d_fa, m->d_parent, m->d_level};
+                    p == 0 ? m->d_fb : m->d_fa, m->d_parent, m->d_level, m->d_dup, m->dup_tiles};
 }
+
+// tiles of edges whose marks are kept: 8 MiB of them at most (a push level of
+// more edges gives the minimum pass all the edges beyond)
+int64_t dup_tiles_of(int64_t nnz) { return std::min<int64_t>(nnz / kPushTile + 2 * kGroups, (1 << 26) / kPushTile); }
 
 unsigned queue_grid(int64_t nwords) { return (unsigned)g5::grid_for(queue_units(nwords), 1, kPushVertGrid); }
 
@@ -2411,6 +2446,8 @@ extern "C" int g5_msbfs_create(g5_graph *g, g5_msbfs **out)
     if (e == hipSuccess) e = hipHostMalloc(&m->h_cnt, kHostSlots * 8, hipHostMallocDefault);
     if (e == hipSuccess) e = hipMalloc(&m->d_lane, kLaneStripes * 64 * 8);
     if (e == hipSuccess) e = hipMalloc(&m->d_scratch, (g5::scan_scratch_words(n + 1) + 16) * 8);
+    m->dup_tiles = dup_tiles_of(g->nnz);
+    if (e == hipSuccess) e = hipMalloc(&m->d_dup, (size_t)m->dup_tiles * (kPushTile / 8));
     if (e == hipSuccess) e = hipMalloc(&m->d_roots, 64 * 8 + 64 * 4);  // roots, then lane_of
     if (e == hipSuccess) e = hipMalloc(&m->d_join, 194 * 8);
     if (e == hipSuccess) e = hipMalloc(&m->d_sums, 128 * 8);
@@ -2446,7 +2483,7 @@ extern "C" int g5_msbfs_footprint(const g5_graph *g, int64_t *graph_bytes, int64
                         + 3 * (n / 64) * 8             // active bitmaps, level flags
                         + 2 * 12 * queue_units(n / 64) * (kUnitWords * 64) + 2 * kGroups * (int64_t)sizeof(QueueTotal)  // push queues
                         + 64 * 5 * n                   // parent and level records
-                        + kDirtyCap * 8 + kStripes * kCntStride * 8 + kLaneStripes * 64 * 8 +
+                        + dup_tiles_of(g->nnz) * (kPushTile / 8) + kDirtyCap * 8 + kStripes * kCntStride * 8 + kLaneStripes * 64 * 8 +
                         ((int64_t)g5::scan_scratch_words(n + 1) + 16) * 8 + 64 * 12 + 194 * 8 + 128 * 8 +
                         3 * 4 * n + 8 * (n + 1) + 2 * 4 * nnz  // relabelled copy: ids, degrees, rows
                         + 2 * 8 * n;                       // head, head_orig
@@ -2465,7 +2502,7 @@ extern "C" int g5_msbfs_free(g5_msbfs *m)
             if (ge) (void)hipGraphExecDestroy(ge);
     void *dev[] = {m->d_qv[0],   m->d_qv[1],   m->d_qo[0],    m->d_qo[1],   m->d_qt,    m->d_act,   m->d_visited, m->d_fa,
                    m->d_fb,      m->d_parent,  m->d_cnt,      m->d_scratch, m->d_roots, m->d_join,
-                   m->d_sums,    m->rl.new2old, m->rl.old2new, m->rl.rowptr, m->rl.cols, m->rl.gdeg,
+                   m->d_sums,    m->d_dup, m->rl.new2old, m->rl.old2new, m->rl.rowptr, m->rl.cols, m->rl.gdeg,
                    m->d_lane,    m->rl.head,    m->d_level,   m->d_dirty,  m->rl.head_orig,
                    m->rl.cols_orig, m->d_lvflag};
     for (void *p : dev)

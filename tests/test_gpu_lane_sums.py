@@ -115,3 +115,28 @@ def test_thread_bound_follows_a_smaller_wave_bound_until_it_is_set(scale, edgefa
     check()
     with pytest.raises(g5.G5Error):
         m.tune(wave_max=7)
+
+
+@pytest.mark.parametrize("sources, targets", [(3, 64), (40, 1000), (700, 3000), (2000, 40)])
+def test_push_levels_keep_the_smallest_parent(sources, targets):
+    """Every target has several parents at one level: the edges that find a pair
+    set are looked at again, in tiles of few and of many sources."""
+    rng = np.random.default_rng(sources)
+    n = 1 + sources + targets
+    e = [np.stack([np.zeros(sources, np.int64), 1 + np.arange(sources)], 1)]
+    for _ in range(5):
+        t = 1 + sources + np.arange(targets)
+        e.append(np.stack([1 + rng.integers(0, sources, targets), t], 1))
+    s = 1 + np.arange(sources)
+    e.append(np.stack([s, 1 + sources + rng.integers(0, targets, sources)], 1))
+    ref = O.build_csr(rng.permutation(n)[np.concatenate(e)])
+    g = g5.Graph.upload(ref.rowptr, ref.cols, ref.n_rows, gdeg=ref.gdeg)
+    m = g5.MSBFS(g)
+    m.set_mode(2)
+    roots = [int(r) for r in rng.choice(n, min(n, 64), replace=False)]
+    for _ in range(2):
+        m.run(roots)
+        for lane in range(0, len(roots), 5):
+            pred, lev = m.result(lane)
+            opred, olev, _ = O.bfs_bin(ref, roots[lane])
+            assert np.array_equal(pred, opred) and np.array_equal(lev, olev)
