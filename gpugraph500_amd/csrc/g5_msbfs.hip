@@ -104,6 +104,14 @@ constexpr int kLevelRec = 12;  // per level: ms[4], edges[4], new pairs, pushed,
 // around the line (scales 15 to 19, edgefactors 64 to 4) the two are within
 // 3 % either way.  lane_ratio 128 is 0.99-1.01 (scale 20 and below), 1.04
 // (22) and 1.07 (24) times as fast as 64; push_ratio 4 to 64 are within 7 %.
+// Below kFuseNnz stored neighbours a pull level's three bins share one launch:
+// none of them fills the card, and a level takes as long as the longest chain
+// of the longest bin instead of the sum of theirs (a search at scale 14 0.434
+// -> 0.381 ms, 16 0.507 -> 0.457, 18 0.640 -> 0.626, edgefactor 4 at scale 21
+// 1.04 -> 1.02).  Beyond it the block and wave bins lose more by the thread
+// bin's registers, which halve their wavefronts (scale 20 0.99 -> 1.07, 24
+// 6.4 -> 6.9).
+constexpr int64_t kFuseNnz = (int64_t)1 << 24;
 constexpr int64_t kLargeNnz = (int64_t)1 << 22;
 constexpr int64_t kLeastWaveMax = 32;  // of a search whose thread_max was not set
 struct Tune {
@@ -517,7 +525,8 @@ __device__ __forceinline__ void write_out(const KeptHits &k, int lane, int32_t *
 // ids, the head-step parents' from head_orig and the cols_orig loads issued
 // at the hits) complete under that scan instead of stalling the wave.
 template <bool kActive>
-__global__ __launch_bounds__(kBlock) void k_pull_thread(
+__device__ __forceinline__ void pull_thread(
+    int64_t group, int64_t ngroups,
     int64_t first_v, int64_t nlist, const int64_t *__restrict__ rowptr, const uint32_t *__restrict__ cols,
     const uint64_t *__restrict__ head, const uint64_t *__restrict__ head_orig,
     const uint32_t *__restrict__ cols_orig, uint64_t *__restrict__ visited,
@@ -538,8 +547,8 @@ __global__ __launch_bounds__(kBlock) void k_pull_thread(
     // wave-uniform loop: the wave takes 64 consecutive vertices per step, one
     // word of the next frontier's active bitmap (the bin starts at a multiple
     // of 64)
-    for (int64_t base = blockIdx.x * (int64_t)kBlock + (threadIdx.x & ~63); base < nlist;
-         base += (int64_t)gridDim.x * kBlock) {
+    for (int64_t base = group * (int64_t)kBlock + (threadIdx.x & ~63); base < nlist;
+         base += ngroups * kBlock) {
         const int64_t i = base + lane;
         const uint32_t v = (uint32_t)(first_v + i);
         const int64_t fword = (first_v + base) >> 6;
@@ -627,7 +636,8 @@ constexpr int kWaveFirst = 16;  // 8: same time
 static_assert(kWaveFirst <= 64, "a step spans at most one neighbour per lane");
 
 template <bool kActive>
-__global__ __launch_bounds__(kBlock) void k_pull_wave(
+__device__ __forceinline__ void pull_wave(
+    int64_t group, int64_t ngroups,
     int64_t first_v, int64_t nlist, const int64_t *__restrict__ rowptr, const uint32_t *__restrict__ cols,
     const uint64_t *__restrict__ head, const uint64_t *__restrict__ head_orig,
     const uint32_t *__restrict__ cols_orig, uint64_t *__restrict__ visited,
@@ -642,9 +652,9 @@ __global__ __launch_bounds__(kBlock) void k_pull_wave(
     const int lane = __lane_id();
     const uint64_t lanes = (uint64_t)cnt_all[kPullLanes];
     const int64_t first_step = cnt_all[kWaveStep];
-    const int64_t stride = (int64_t)gridDim.x * (kBlock / 64);
+    const int64_t stride = ngroups * (kBlock / 64);
     int64_t nbits = 0, nedges = 0, nverts = 0, ngath = 0, nnext = 0, enext = 0;
-    for (int64_t i = blockIdx.x * (int64_t)(kBlock / 64) + (threadIdx.x >> 6); i < nlist; i += stride) {
+    for (int64_t i = group * (int64_t)(kBlock / 64) + (threadIdx.x >> 6); i < nlist; i += stride) {
         const uint32_t v = (uint32_t)(first_v + i);
         const uint64_t vis = visited[v];
         const uint64_t unv = ~vis & lanes;
@@ -725,7 +735,8 @@ __global__ __launch_bounds__(kBlock) void k_pull_wave(
 constexpr int kBlockUnroll = 1;
 
 template <bool kActive>
-__global__ __launch_bounds__(kBlock) void k_pull_block(
+__device__ __forceinline__ void pull_block(
+    int64_t group, int64_t ngroups,
     int64_t first_v, int64_t nlist, const int64_t *__restrict__ rowptr, const uint32_t *__restrict__ cols,
     const uint64_t *__restrict__ head, const uint64_t *__restrict__ head_orig,
     const uint32_t *__restrict__ cols_orig, uint64_t *__restrict__ visited,
@@ -742,7 +753,7 @@ __global__ __launch_bounds__(kBlock) void k_pull_block(
     const int lane = __lane_id(), wv = threadIdx.x >> 6;
     const uint64_t lanes = (uint64_t)cnt_all[kPullLanes];
     int64_t nbits = 0, nedges = 0, nverts = 0, nnext = 0, enext = 0;
-    for (int64_t i = blockIdx.x; i < nlist; i += gridDim.x) {
+    for (int64_t i = group; i < nlist; i += ngroups) {
         const uint32_t v = (uint32_t)(first_v + i);
         if (threadIdx.x == 0) s_vis = visited[v];
         __syncthreads();
@@ -827,6 +838,55 @@ __global__ __launch_bounds__(kBlock) void k_pull_block(
     }
     block_add(cnt_all + kUnitSlots * bin, {nbits, nedges, nverts, ngath, nnext, enext});
 }
+
+struct PullArgs {
+    const int64_t *rowptr;
+    const uint32_t *cols;
+    const uint64_t *head, *head_orig;
+    const uint32_t *cols_orig;
+    uint64_t *visited;
+    const uint64_t *frontier, *active;
+    uint64_t *next;
+    int32_t *parent;
+    uint8_t *level;
+    const uint32_t *new2old;
+    int64_t *cnt;
+    uint64_t *act_next, *lvflag;
+};
+#define G5_PULL(fn, group, ngroups, first, n, bin)                                                                 \
+    fn<kActive>(group, ngroups, first, n, a.rowptr, a.cols, a.head, a.head_orig, a.cols_orig, a.visited, a.frontier, \
+                a.active, a.next, a.parent, a.level, a.new2old, a.cnt, bin, a.act_next, a.lvflag)
+
+template <bool kActive>
+__global__ __launch_bounds__(kBlock) void k_pull_block(PullArgs a, int64_t first, int64_t n)
+{
+    G5_PULL(pull_block, blockIdx.x, gridDim.x, first, n, 0);
+}
+template <bool kActive>
+__global__ __launch_bounds__(kBlock) void k_pull_wave(PullArgs a, int64_t first, int64_t n)
+{
+    G5_PULL(pull_wave, blockIdx.x, gridDim.x, first, n, 1);
+}
+template <bool kActive>
+__global__ __launch_bounds__(kBlock) void k_pull_thread(PullArgs a, int64_t first, int64_t n)
+{
+    G5_PULL(pull_thread, blockIdx.x, gridDim.x, first, n, 2);
+}
+
+// The three bins in one launch (kFuseNnz), those with the longest chains first.
+struct PullBins {
+    int64_t first[kBins], n[kBins];
+    unsigned groups[kBins];
+};
+template <bool kActive>
+__global__ __launch_bounds__(kBlock) void k_pull_all(PullArgs a, PullBins b)
+{
+    const unsigned g0 = b.groups[0], g1 = g0 + b.groups[1];
+    if (blockIdx.x < g0) G5_PULL(pull_block, blockIdx.x, g0, b.first[0], b.n[0], 0);
+    else if (blockIdx.x < g1) G5_PULL(pull_wave, blockIdx.x - g0, b.groups[1], b.first[1], b.n[1], 1);
+    else G5_PULL(pull_thread, blockIdx.x - g1, b.groups[2], b.first[2], b.n[2], 2);
+}
+#undef G5_PULL
 
 // ---- push (top-down) levels for sparse frontiers ----
 // The frontier's vertices u (active bitmap -> sorted queue) push their lane
@@ -1975,27 +2035,31 @@ __global__ __launch_bounds__(kBlock) void k_leave(uint64_t *__restrict__ visited
 void pull_bins(g5_msbfs *m, hipStream_t s, int p, bool act_check, bool prof, const int64_t *bf)
 {
     const Relabeled &R = m->rl;
-    const uint64_t *front = p == 0 ? m->d_fa : m->d_fb;
-    uint64_t *next = p == 0 ? m->d_fb : m->d_fa;
     const int64_t nw = m->n / 64;
-    const uint64_t *act = m->d_act + (p == 0 ? 0 : nw);
-    uint64_t *act_next = m->d_act + (p == 0 ? nw : 0);
+    PullArgs a{R.rowptr, R.cols, R.head, R.head_orig, R.cols_orig, m->d_visited, p == 0 ? m->d_fa : m->d_fb,
+               m->d_act + (p == 0 ? 0 : nw), p == 0 ? m->d_fb : m->d_fa, m->d_parent, m->d_level, R.new2old, m->d_cnt,
+               m->d_act + (p == 0 ? nw : 0), m->d_lvflag};
+    PullBins b{};
+    for (int k = 0; k < kBins; ++k) {
+        b.first[k] = bf[k];
+        b.n[k] = bf[k + 1] - bf[k];
+        b.groups[k] = !b.n[k]  ? 0u
+                      : k == 0 ? (unsigned)std::min<int64_t>(b.n[k], 4096)
+                      : k == 1 ? (unsigned)g5::grid_for(b.n[k], kBlock / 64, 16384)
+                               : (unsigned)g5::grid_for(b.n[k], kBlock, 16384);
+    }
+    if (!prof && m->g->nnz < kFuseNnz) {
+        hipLaunchKernelGGL(act_check ? k_pull_all<true> : k_pull_all<false>, b.groups[0] + b.groups[1] + b.groups[2],
+                           kBlock, 0, s, a, b);
+        return;
+    }
     for (int k = 0; k < kBins; ++k) {
         if (prof) (void)hipEventRecord(m->ek[k], s);
-        const int64_t first = bf[k], cnt = bf[k + 1] - first;
-        if (!cnt) continue;
-#define G5_PULL_ARGS first, cnt, (const int64_t *)R.rowptr, (const uint32_t *)R.cols, (const uint64_t *)R.head, \
-                     (const uint64_t *)R.head_orig, (const uint32_t *)R.cols_orig, \
-                     m->d_visited, front, act, next, m->d_parent, m->d_level, (const uint32_t *)R.new2old, m->d_cnt, \
-                     k, act_next, m->d_lvflag
-        const unsigned grid = k == 0 ? (unsigned)std::min<int64_t>(cnt, 4096)
-                              : k == 1 ? g5::grid_for(cnt, kBlock / 64, 16384)
-                                       : g5::grid_for(cnt, kBlock, 16384);
-        auto kern = k == 0 ? (act_check ? k_pull_block<true> : k_pull_block<false>)
+        if (!b.n[k]) continue;
+        auto kern = k == 0   ? (act_check ? k_pull_block<true> : k_pull_block<false>)
                     : k == 1 ? (act_check ? k_pull_wave<true> : k_pull_wave<false>)
                              : (act_check ? k_pull_thread<true> : k_pull_thread<false>);
-        hipLaunchKernelGGL(kern, grid, kBlock, 0, s, G5_PULL_ARGS);
-#undef G5_PULL_ARGS
+        hipLaunchKernelGGL(kern, b.groups[k], kBlock, 0, s, a, b.first[k], b.n[k]);
     }
     if (prof) (void)hipEventRecord(m->ek[kBins], s);
 }

@@ -140,3 +140,23 @@ def test_push_levels_keep_the_smallest_parent(sources, targets):
             pred, lev = m.result(lane)
             opred, olev, _ = O.bfs_bin(ref, roots[lane])
             assert np.array_equal(pred, opred) and np.array_equal(lev, olev)
+
+
+@pytest.mark.parametrize("shape", [dict(thread_max=0, wave_max=0), dict(thread_max=0, wave_max=1 << 20),
+                                   dict(thread_max=1 << 20, wave_max=1 << 20), dict(thread_max=9, wave_max=40),
+                                   dict(thread_max=9, wave_max=1 << 20), dict(thread_max=40, wave_max=40)])
+def test_bins_in_one_launch_and_in_three(shape):
+    """Pull levels with any of the bins empty; accounting runs them one by one."""
+    ref = O.build_csr(O.kronecker_edges(12))
+    g = g5.Graph.upload(ref.rowptr, ref.cols, ref.n_rows, gdeg=ref.gdeg)
+    m = g5.MSBFS(g)
+    m.tune(**shape)
+    m.set_mode(1)
+    roots = [int(r) for r in O.select_roots(ref, 1 << 12)][:40]
+    want = [O.bfs_bin(ref, r)[:2] for r in roots]
+    for prof in (False, True, False):
+        m.profile(prof)
+        m.run(roots)
+        for lane in range(0, len(roots), 3):
+            pred, lev = m.result(lane)
+            assert np.array_equal(pred, want[lane][0]) and np.array_equal(lev, want[lane][1])
