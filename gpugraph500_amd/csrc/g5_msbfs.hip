@@ -55,9 +55,10 @@
 // the same results): one thread per vertex up to thread_max neighbours, one wavefront
 // (64 neighbours per step, first hits from an exclusive prefix-OR across
 // lanes) up to wave_max, one 256-thread workgroup beyond (Tune; 256 and 2048
-// by default, 32 and 2048 on graphs of fewer than 2^22 stored neighbours).  Each pull level's launch
-// sequence is captured once into a hipGraph per frontier parity and
-// replayed; the level number lives in device memory.
+// by default, 32 and 2048 on graphs of fewer than 2^22 stored neighbours).  A pull level is
+// three to five launches (as a captured hipGraph, after a launch that set what
+// arguments hold now, it took 8 us more: a search of 64 roots at scale 16 with
+// four pull levels 0.457 ms, now 0.424).
 //
 // Output in HBM, final when g5_msbfs_run returns: the 64 predecessor maps
 // as one vertex-major array parent int32[n][64] and the 64 level maps as
@@ -133,18 +134,13 @@ struct Tune {
 // root) pairs, edges read, vertices worked on, frontier words gathered, and
 // the next frontier's vertices and edges; then the OR of the next frontier's
 // words (the lanes still searching).  Then set-once slots: the level number,
-// the frontier queue's length and its edge total (push; the host's copy only),
-// the lanes the block and wave kernels work on, the lanes
-// in use, the first word of level flags the level before wrote, the lanes
-// the thread kernel works on and the wave kernel's first step (the last five
-// written before each pull level, k_set_pull_lanes).
+// the frontier queue's length and its edge total (push; the host's copy only).
 enum MsCnt {
     kNewBits = 0, kEdgesRead = 1, kVisitedVerts = 2, kGathers = 3, kNextVerts = 4, kNextEdges = 5,
     kUnitSlots = 6,
     kLive = kUnits * kUnitSlots,
     kAccum = kLive + 1,
-    kDepth = kAccum, kFqLen = kAccum + 2, kFqEdges = kAccum + 3, kPullLanes = kAccum + 4,
-    kUsed = kAccum + 5, kFlagWord = kAccum + 6, kThreadLanes = kAccum + 7, kWaveStep = kAccum + 8,
+    kDepth = kAccum, kFqLen = kAccum + 2, kFqEdges = kAccum + 3,
     kCntStride = 40
 };
 // Many workgroups adding into one address serialise in one L2 channel, so
@@ -152,7 +148,7 @@ enum MsCnt {
 // kStripes (stripes 320 B apart) and k_level_end folds the stripes for the
 // host; stripe 0 also holds the set-once slots.
 constexpr int kStripes = 32;
-static_assert(kWaveStep < kCntStride, "counter stripe too small");
+static_assert(kFqEdges < kCntStride, "counter stripe too small");
 // Per-lane frontier edges (counted by push levels, from their new-vertex
 // queue): kLaneStripes stripes of 64 slots, summed on the host.
 constexpr int kLaneStripes = 8;
@@ -210,7 +206,6 @@ struct g5_msbfs {
     int64_t *d_scratch = nullptr;
     int64_t *d_roots = nullptr;
     Relabeled rl;
-    hipGraphExec_t graph[2][2] = {};  // [frontier parity][active-bitmap check]
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     int nroots = 0;
     int64_t roots[64];
@@ -366,13 +361,24 @@ __device__ __forceinline__ uint64_t lanes_excl_or(uint64_t f)
 // kActive (all pull kernels): skip neighbours whose bit in the active bitmap
 // is clear before gathering their frontier word (pays only when few sources
 // are active).  The block and wave kernels work on the lanes in
-// cnt[kPullLanes] only, the thread kernel on those in cnt[kThreadLanes] (the
+// PullLanes::pull only, the thread kernel on those in PullLanes::thread (the
 // same, except on a split level: there it takes every lane, the pushed ones
 // too, since its rows are scanned to the end anyway): a vertex is done when
 // every unvisited lane among them is found.
 constexpr int kHits = 6;  // 4: +0.5 ms at level 3 (spilled hits' scattered stores), 8: 3 waves per SIMD, slower
 constexpr int kThreadUnroll = 8;  // 4: +0.6 ms at level 3, 16: +0.7 ms at level 4; 12 after the short first step: the same
 constexpr int kThreadFirst = 2;  // 1: same time, more neighbours read
+
+// What a pull level works on: the lanes of the block and wave bins and those
+// of the thread bin, the lanes in use, the first word of level flags that the
+// level just before wrote (its thread bin's; INT64_MAX after a push level): the
+// thread bin trusts the flags from there on; and the wave bin's first step
+// (kWaveFirst neighbours, or 64 on split levels, whose rows are scanned to the
+// end).
+struct PullLanes {
+    uint64_t pull, thread, used;
+    int64_t flag_word, wave_step;
+};
 
 // the record outputs of a pull level: parent and level records by original
 // id, the level byte of the pairs it reaches, new2old and the columns'
@@ -533,13 +539,12 @@ __device__ __forceinline__ void pull_thread(
     const uint64_t *__restrict__ frontier,
     const uint64_t *__restrict__ active, uint64_t *__restrict__ next, int32_t *__restrict__ parent,
     uint8_t *__restrict__ level, const uint32_t *__restrict__ new2old, int64_t *__restrict__ cnt_all, int bin,
-    uint64_t *__restrict__ act_next, uint64_t *__restrict__ lvflag)
+    uint64_t *__restrict__ act_next, uint64_t *__restrict__ lvflag, const PullLanes &pl)
 {
     __shared__ uint64_t s_live[kBlock / 64];
     const int lane = __lane_id();
-    const uint64_t lanes = (uint64_t)cnt_all[kThreadLanes];
-    const uint64_t used = (uint64_t)cnt_all[kUsed];
-    const int64_t flags_from = cnt_all[kFlagWord];
+    const uint64_t lanes = pl.thread, used = pl.used;
+    const int64_t flags_from = pl.flag_word;
     const PullOut out{parent, level, new2old, cols_orig, level_byte(cnt_all)};
     int64_t ngath = 0, nbits = 0, nedges = 0, nverts = 0, nnext = 0, enext = 0;
     uint64_t live = 0;
@@ -630,7 +635,7 @@ __device__ __forceinline__ void pull_thread(
 // only kWaveFirst neighbours (the other lanes idle): on dense levels most
 // vertices are done after a few, and every gather past the early exit is a
 // wasted line fill.  On split levels every row is scanned to its end, so
-// there the first step is a whole one (cnt[kWaveStep]).
+// there the first step is a whole one (PullLanes::wave_step).
 constexpr int kWaveUnroll = 1;
 constexpr int kWaveFirst = 16;  // 8: same time
 static_assert(kWaveFirst <= 64, "a step spans at most one neighbour per lane");
@@ -644,14 +649,14 @@ __device__ __forceinline__ void pull_wave(
     const uint64_t *__restrict__ frontier,
     const uint64_t *__restrict__ active, uint64_t *__restrict__ next, int32_t *__restrict__ parent,
     uint8_t *__restrict__ level, const uint32_t *__restrict__ new2old, int64_t *__restrict__ cnt_all, int bin,
-    uint64_t *__restrict__ act_next, uint64_t *__restrict__ lvflag)
+    uint64_t *__restrict__ act_next, uint64_t *__restrict__ lvflag, const PullLanes &pl)
 {
     __shared__ uint32_t s_par[kBlock / 64][64];
     uint32_t *__restrict__ sp = s_par[threadIdx.x >> 6];
     const uint8_t lv = level_byte(cnt_all);
     const int lane = __lane_id();
-    const uint64_t lanes = (uint64_t)cnt_all[kPullLanes];
-    const int64_t first_step = cnt_all[kWaveStep];
+    const uint64_t lanes = pl.pull;
+    const int64_t first_step = pl.wave_step;
     const int64_t stride = ngroups * (kBlock / 64);
     int64_t nbits = 0, nedges = 0, nverts = 0, ngath = 0, nnext = 0, enext = 0;
     for (int64_t i = group * (int64_t)(kBlock / 64) + (threadIdx.x >> 6); i < nlist; i += stride) {
@@ -743,7 +748,7 @@ __device__ __forceinline__ void pull_block(
     const uint64_t *__restrict__ frontier,
     const uint64_t *__restrict__ active, uint64_t *__restrict__ next, int32_t *__restrict__ parent,
     uint8_t *__restrict__ level, const uint32_t *__restrict__ new2old, int64_t *__restrict__ cnt_all, int bin,
-    uint64_t *__restrict__ act_next, uint64_t *__restrict__ lvflag)
+    uint64_t *__restrict__ act_next, uint64_t *__restrict__ lvflag, const PullLanes &pl)
 {
     __shared__ uint64_t s_wave[kBlockUnroll][kBlock / 64];
     __shared__ uint64_t s_vis;
@@ -751,7 +756,7 @@ __device__ __forceinline__ void pull_block(
     const uint8_t lv = level_byte(cnt_all);
     int64_t ngath = 0;
     const int lane = __lane_id(), wv = threadIdx.x >> 6;
-    const uint64_t lanes = (uint64_t)cnt_all[kPullLanes];
+    const uint64_t lanes = pl.pull;
     int64_t nbits = 0, nedges = 0, nverts = 0, nnext = 0, enext = 0;
     for (int64_t i = group; i < nlist; i += ngroups) {
         const uint32_t v = (uint32_t)(first_v + i);
@@ -852,10 +857,11 @@ struct PullArgs {
     const uint32_t *new2old;
     int64_t *cnt;
     uint64_t *act_next, *lvflag;
+    PullLanes lanes;
 };
 #define G5_PULL(fn, group, ngroups, first, n, bin)                                                                 \
     fn<kActive>(group, ngroups, first, n, a.rowptr, a.cols, a.head, a.head_orig, a.cols_orig, a.visited, a.frontier, \
-                a.active, a.next, a.parent, a.level, a.new2old, a.cnt, bin, a.act_next, a.lvflag)
+                a.active, a.next, a.parent, a.level, a.new2old, a.cnt, bin, a.act_next, a.lvflag, a.lanes)
 
 template <bool kActive>
 __global__ __launch_bounds__(kBlock) void k_pull_block(PullArgs a, int64_t first, int64_t n)
@@ -1465,22 +1471,6 @@ __global__ __launch_bounds__(kBlock) void k_build_active(const uint64_t *__restr
     }
 }
 
-// One thread: the lanes the next block and wave kernels work on, those the
-// next thread kernel works on, the lanes in use, the first word of level
-// flags that the level just before wrote (its thread kernel's bin; INT64_MAX
-// after a push level): the thread kernel trusts the flags from there on, and
-// the wave kernel's first step (kWaveFirst neighbours, or 64 on split
-// levels, whose rows are scanned to the end).
-__global__ void k_set_pull_lanes(int64_t *cnt, uint64_t lanes, uint64_t thread_lanes, uint64_t used,
-                                 int64_t flag_word, int64_t wave_step)
-{
-    cnt[kWaveStep] = wave_step;
-    cnt[kPullLanes] = (int64_t)lanes;
-    cnt[kThreadLanes] = (int64_t)thread_lanes;
-    cnt[kUsed] = (int64_t)used;
-    cnt[kFlagWord] = flag_word;
-}
-
 // one workgroup: the stripes' and the per-lane edges' sums, the pushed queue's
 // totals (when there was one) and the set-once slots go to the host's counters,
 // in pinned memory; the stripes are clear again, the level advances
@@ -2028,17 +2018,15 @@ __global__ __launch_bounds__(kBlock) void k_leave(uint64_t *__restrict__ visited
 }
 
 // The three pull kernels of parity p (act: they consult the active bitmap;
-// prof: events between them).  They work on the lanes in cnt[kPullLanes]
-// (the thread kernel: cnt[kThreadLanes]).
-// They share one argument list; only the thread kernel reads `head` and
+// prof: events between them).  They share one argument list; only the thread kernel reads `head` and
 // `head_orig`.
-void pull_bins(g5_msbfs *m, hipStream_t s, int p, bool act_check, bool prof, const int64_t *bf)
+void pull_bins(g5_msbfs *m, hipStream_t s, int p, const PullLanes &lanes, bool act_check, bool prof, const int64_t *bf)
 {
     const Relabeled &R = m->rl;
     const int64_t nw = m->n / 64;
     PullArgs a{R.rowptr, R.cols, R.head, R.head_orig, R.cols_orig, m->d_visited, p == 0 ? m->d_fa : m->d_fb,
                m->d_act + (p == 0 ? 0 : nw), p == 0 ? m->d_fb : m->d_fa, m->d_parent, m->d_level, R.new2old, m->d_cnt,
-               m->d_act + (p == 0 ? nw : 0), m->d_lvflag};
+               m->d_act + (p == 0 ? nw : 0), m->d_lvflag, lanes};
     PullBins b{};
     for (int k = 0; k < kBins; ++k) {
         b.first[k] = bf[k];
@@ -2049,8 +2037,9 @@ void pull_bins(g5_msbfs *m, hipStream_t s, int p, bool act_check, bool prof, con
                                : (unsigned)g5::grid_for(b.n[k], kBlock, 16384);
     }
     if (!prof && m->g->nnz < kFuseNnz) {
-        hipLaunchKernelGGL(act_check ? k_pull_all<true> : k_pull_all<false>, b.groups[0] + b.groups[1] + b.groups[2],
-                           kBlock, 0, s, a, b);
+        const unsigned groups = b.groups[0] + b.groups[1] + b.groups[2];  // 0: no edges
+        if (groups)
+            hipLaunchKernelGGL(act_check ? k_pull_all<true> : k_pull_all<false>, groups, kBlock, 0, s, a, b);
         return;
     }
     for (int k = 0; k < kBins; ++k) {
@@ -2064,13 +2053,13 @@ void pull_bins(g5_msbfs *m, hipStream_t s, int p, bool act_check, bool prof, con
     if (prof) (void)hipEventRecord(m->ek[kBins], s);
 }
 
-// One pull level of parity p (the launches a hipGraph captures).
-int level_launches(g5_msbfs *m, hipStream_t s, int p, bool act_check, bool prof = false)
+// One pull level of parity p.
+int pull_level(g5_msbfs *m, hipStream_t s, int p, const PullLanes &lanes, bool act_check, bool prof)
 {
     uint64_t *next = p == 0 ? m->d_fb : m->d_fa;
     const int64_t nw = m->n / 64;
     uint64_t *act_next = m->d_act + (p == 0 ? nw : 0);
-    pull_bins(m, s, p, act_check, prof, m->rl.bin_first);
+    pull_bins(m, s, p, lanes, act_check, prof, m->rl.bin_first);
     // the thread kernel wrote its words of the active bitmap; the block and
     // wave bins' words (and the live lanes among them) come from next
     const int64_t nw01 = (m->rl.bin_first[2] + 63) / 64;
@@ -2078,7 +2067,8 @@ int level_launches(g5_msbfs *m, hipStream_t s, int p, bool act_check, bool prof 
         hipLaunchKernelGGL((k_build_active<false, true>), g5::grid_for(nw01, 16, 4096), kBlock, 0, s,
                            (const uint64_t *)next, nw01, (const int64_t *)m->rl.rowptr, act_next, m->d_cnt, ~0ull);
     hipLaunchKernelGGL(k_level_end, 1, kBlock, 0, s, m->d_cnt, m->d_lane, (const QueueTotal *)nullptr, m->h_cnt);
-    return hipGetLastError() == hipSuccess ? G5_OK : G5_E_HIP;
+    G5_HIP(hipGetLastError());
+    return G5_OK;
 }
 
 // queue i of the engine
@@ -2141,15 +2131,15 @@ int push_level(g5_msbfs *m, hipStream_t s, int p, bool listed_in, bool queue_in,
 }
 
 // One split level on parity p: the block and wave kernels on the lanes in
-// cnt[kPullLanes] and the thread kernel on every frontier lane, then the push
-// kernels on the lanes pm (disjoint from cnt[kPullLanes]) into the block and
+// lanes.pull and the thread kernel on every frontier lane, then the push
+// kernels on the lanes pm (disjoint from lanes.pull) into the block and
 // wave bins only (the thread kernel pulls every lane of its vertices), which
 // the pull kernels have written for the other lanes.  When those bins'
 // vertices times the pushed lanes fit in n words, one pass lowers per-pair
 // candidates (push_cand) and k_cand_commit writes the pairs out; otherwise the
 // passes of a push level run.  Ends with the bins' part of next's active
 // bitmap, counts and live lanes.
-int split_level(g5_msbfs *m, hipStream_t s, int p, uint64_t pm, bool act_check, bool prof)
+int split_level(g5_msbfs *m, hipStream_t s, int p, uint64_t pm, const PullLanes &lanes, bool act_check, bool prof)
 {
     const Relabeled &R = m->rl;
     const int64_t nw = m->n / 64;
@@ -2158,7 +2148,7 @@ int split_level(g5_msbfs *m, hipStream_t s, int p, uint64_t pm, bool act_check, 
     const PushArgs a = push_args(m, p);
     const PushQueue q = push_queue(m, 1 - m->listed);
     uint32_t *cand = m->d_qv[m->listed];  // the other queue, of one entry per vertex, holds the candidates
-    pull_bins(m, s, p, act_check, prof, R.split_first);
+    pull_bins(m, s, p, lanes, act_check, prof, R.split_first);
     if (prof) G5_HIP(hipEventRecord(m->ek_push[0], s));
     // the frontier vertices with a pushed lane, in the frontier's own active
     // bitmap (the pull kernels are done with it; the thread kernel has
@@ -2198,23 +2188,6 @@ int split_level(g5_msbfs *m, hipStream_t s, int p, uint64_t pm, bool act_check, 
     if (prof) G5_HIP(hipEventRecord(m->ek_push[1], s));
     hipLaunchKernelGGL(k_level_end, 1, kBlock, 0, s, m->d_cnt, m->d_lane, (const QueueTotal *)q.tot, m->h_cnt);
     G5_HIP(hipGetLastError());
-    return G5_OK;
-}
-
-int capture_graphs(g5_msbfs *m)
-{
-    for (int p = 0; p < 2; ++p)
-        for (int a = 0; a < 2; ++a) {
-            hipGraph_t gr = nullptr;
-            G5_HIP(hipStreamBeginCapture(m->s, hipStreamCaptureModeThreadLocal));
-            int rc = level_launches(m, m->s, p, a != 0);
-            hipError_t e = hipStreamEndCapture(m->s, &gr);
-            if (rc) return rc;
-            G5_HIP(e);
-            e = hipGraphInstantiate(&m->graph[p][a], gr, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(gr);
-            G5_HIP(e);
-        }
     return G5_OK;
 }
 
@@ -2307,16 +2280,6 @@ int compute_bins(g5_msbfs *m)
     return rc;
 }
 
-void destroy_graphs(g5_msbfs *m)
-{
-    for (auto &gp : m->graph)
-        for (hipGraphExec_t &ge : gp)
-            if (ge) {
-                (void)hipGraphExecDestroy(ge);
-                ge = nullptr;
-            }
-}
-
 // the lanes in use: a batch run's roots' lanes, continuous mode's busy lanes
 uint64_t used_lanes(const g5_msbfs *m)
 {
@@ -2376,17 +2339,11 @@ int run_level(g5_msbfs *m, int64_t *new_bits_out, uint64_t *live_out)
         int rc = push_level(m, s, p, listed_in, queue_in, m->prof);
         if (rc) return rc;
     } else {
-        hipLaunchKernelGGL(k_set_pull_lanes, 1, 1, 0, s, m->d_cnt, m->front_lanes & ~pm, m->front_lanes, used_lanes(m),
-                           m->flag_word, pm ? (int64_t)64 : (int64_t)kWaveFirst);
-        if (pm) {
-            int rc = split_level(m, s, p, pm, act_check, m->prof);
-            if (rc) return rc;
-        } else if (m->prof) {
-            int rc = level_launches(m, s, p, act_check, true);
-            if (rc) return rc;
-        } else {
-            G5_HIP(hipGraphLaunch(m->graph[p][act_check ? 1 : 0], s));
-        }
+        const PullLanes lanes{m->front_lanes & ~pm, m->front_lanes, used_lanes(m), m->flag_word,
+                              pm ? (int64_t)64 : (int64_t)kWaveFirst};
+        int rc = pm ? split_level(m, s, p, pm, lanes, act_check, m->prof)
+                    : pull_level(m, s, p, lanes, act_check, m->prof);
+        if (rc) return rc;
     }
     G5_HIP(hipStreamSynchronize(s));  // k_level_end has written h_cnt
     int64_t new_bits = 0;
@@ -2529,8 +2486,6 @@ extern "C" int g5_msbfs_create(g5_graph *g, g5_msbfs **out)
     if (rc) return fail(rc);
     rc = compute_bins(m);
     if (rc) return fail(rc);
-    rc = capture_graphs(m);
-    if (rc) return fail(rc);
     *out = m;
     return G5_OK;
 }
@@ -2561,9 +2516,6 @@ extern "C" int g5_msbfs_free(g5_msbfs *m)
 {
     if (!m) return G5_OK;
     if (m->s) (void)hipStreamSynchronize(m->s);
-    for (auto &gp : m->graph)
-        for (hipGraphExec_t ge : gp)
-            if (ge) (void)hipGraphExecDestroy(ge);
     void *dev[] = {m->d_qv[0],   m->d_qv[1],   m->d_qo[0],    m->d_qo[1],   m->d_qt,    m->d_act,   m->d_visited, m->d_fa,
                    m->d_fb,      m->d_parent,  m->d_cnt,      m->d_scratch, m->d_roots, m->d_join,
                    m->d_sums,    m->d_dup, m->rl.new2old, m->rl.old2new, m->rl.rowptr, m->rl.cols, m->rl.gdeg,
@@ -3034,7 +2986,7 @@ int64_t *tune_slot(g5_msbfs *m, int key)
     }
 }
 
-// Installs t: new degree bins and re-captured level graphs when the bounds move.
+// Installs t: new degree bins when the bounds move.
 int apply_tune(g5_msbfs *m, const Tune &t)
 {
     const bool rebin = t.thread_max != m->tune.thread_max || t.wave_max != m->tune.wave_max ||
@@ -3042,10 +2994,7 @@ int apply_tune(g5_msbfs *m, const Tune &t)
     m->tune = t;
     if (!rebin) return G5_OK;
     G5_HIP(hipStreamSynchronize(m->s));
-    int rc = compute_bins(m);
-    if (rc) return rc;
-    destroy_graphs(m);
-    return capture_graphs(m);
+    return compute_bins(m);
 }
 
 }  // namespace
@@ -3190,12 +3139,6 @@ extern "C" int g5_msbfs_place(g5_msbfs *m, const int64_t *roots, int nroots, int
         *out = best;
         return G5_OK;
     };
-    // the captured pull levels hold the records' address
-    auto swap_records = [&](int32_t *to) -> int {
-        m->d_parent = to;
-        destroy_graphs(m);
-        return capture_graphs(m);
-    };
     float cur = 0;
     int kept = 0;
     int rc = time_runs(&cur);
@@ -3214,18 +3157,17 @@ extern "C" int g5_msbfs_place(g5_msbfs *m, const int64_t *roots, int nroots, int
             rc = g5::fail_hip(e, "g5_msbfs_place: copy", __FILE__, __LINE__);
             break;
         }
-        rc = swap_records((int32_t *)q);
+        m->d_parent = (int32_t *)q;
         float ms = 0;
-        if (!rc) rc = time_runs(&ms);
+        rc = time_runs(&ms);
         if (!rc && ms < cur * 0.98f) {
             // the copy ran the same roots as the original: both hold their maps
             (void)hipFree(old);
             cur = ms;
             ++kept;
         } else {
-            const int rc2 = swap_records(old);
+            m->d_parent = old;
             (void)hipFree(q);
-            if (!rc) rc = rc2;
         }
     }
     m->prof = prof;

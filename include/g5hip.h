@@ -264,8 +264,8 @@ int g5_msbfs_set_mode(g5_msbfs *m, int mode);
 /* Per-kernel accounting.  Units 0..2 are the pull kernels of the degree bins
  * (0: workgroup per vertex, degree > 2048; 1: wavefront per vertex,
  * 257..2048; 2: thread per vertex, 1..256), unit 3 the push levels and the
- * pushed lanes of split levels.  Enabling runs pull levels as direct launches timed with
- * events (otherwise each pull level replays a captured hipGraph); bytes are
+ * pushed lanes of split levels.  Enabling runs the bins of pull levels one by one, timed with
+ * events (otherwise small graphs' share a launch); bytes are
  * the algorithmic bytes of the unit's launches. */
 int g5_msbfs_profile(g5_msbfs *m, int enable);
 int g5_msbfs_stats(g5_msbfs *m, int unit, double *ms, int64_t *launches, double *bytes);

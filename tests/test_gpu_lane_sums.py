@@ -160,3 +160,17 @@ def test_bins_in_one_launch_and_in_three(shape):
         for lane in range(0, len(roots), 3):
             pred, lev = m.result(lane)
             assert np.array_equal(pred, want[lane][0]) and np.array_equal(lev, want[lane][1])
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_graph_without_edges(mode):
+    n = 128
+    g = g5.Graph.upload(np.zeros(n + 1, np.int64), np.zeros(0, np.uint32), n, gdeg=np.zeros(n, np.int64))
+    m = g5.MSBFS(g)
+    m.set_mode(mode)
+    for prof in (False, True):
+        m.profile(prof)
+        m.run([0, 5, 127])
+        for lane, r in enumerate((0, 5, 127)):
+            pred, lev = m.result(lane)
+            assert pred[r] == r and lev[r] == 0 and (np.delete(pred, r) == -1).all()
