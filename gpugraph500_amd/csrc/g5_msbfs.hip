@@ -204,7 +204,6 @@ struct g5_msbfs {
     int64_t *d_cnt = nullptr, *h_cnt = nullptr;
     int64_t *d_lane = nullptr;  // [kLaneStripes][64] per-lane frontier edges
     int64_t *d_scratch = nullptr;
-    int64_t *d_roots = nullptr;
     Relabeled rl;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     int nroots = 0;
@@ -249,12 +248,14 @@ struct g5_msbfs {
     // continuous mode (g5_msbfs_open): lanes in use
     bool cont = false;
     uint64_t busy = 0;
-    // join: roots [0, 64), lanes [64, 128), added frontier [128, 130), root
-    // degrees [130, 194); batch run: the roots' reach [0, 64)
-    int64_t *d_join = nullptr;
+    int64_t *d_reach = nullptr;  // batch run: the roots' reach
+    // pinned, written by kernels: a join's added frontier and root degrees
+    // [0, 66), a batch run's lanes [66, 98), sums or reaches [98, 226)
+    int64_t *h_io = nullptr;
     uint64_t *d_dup = nullptr;  // push levels: the edges that the minimum pass looks at
     int64_t dup_tiles = 0;
     unsigned long long *d_sums = nullptr;  // leave: checksums [0, 64), generated-degree sums [64, 128)
+    bool sums_clear = false;               // d_sums is 0 (k_sums_out leaves it so)
     // the last batch run: device time of the search and of its finalising
     // pass (ev_fin between them), and whether its level bytes are final
     // (depth below 255)
@@ -1414,15 +1415,6 @@ __global__ __launch_bounds__(kBlock) void k_queue(const uint64_t *__restrict__ b
     }
 }
 
-// one workgroup of kBlock threads: clear every stripe's accumulated slots (the
-// first level's; every level's end leaves them clear for the next)
-__global__ void k_level_begin(int64_t *cnt, int64_t *lane_edges)
-{
-    for (int i = threadIdx.x; i < kStripes * kCntStride; i += blockDim.x)
-        if (i % kCntStride < kAccum) cnt[i] = 0;
-    for (int i = threadIdx.x; i < kLaneStripes * 64; i += blockDim.x) lane_edges[i] = 0;
-}
-
 // active[w] bit i = ((next[64w + i] & lm) != 0).  A wave takes four
 // 64-vertex words per step (four independent loads in flight per lane).
 // kCount: also add the active vertices and their edges to the push unit's
@@ -1521,13 +1513,63 @@ __global__ __launch_bounds__(kBlock) void k_level_end(int64_t *cnt, int64_t *lan
     if (threadIdx.x == 0) cnt[kDepth] += 1;
 }
 
-// visited := unused lanes, both active bitmaps := 0 and, unless the caller
-// clears them entry by entry (fronts false), both frontier buffers := 0
-__global__ void k_ms_init(uint64_t *__restrict__ visited, uint64_t *__restrict__ fa, uint64_t *__restrict__ fb,
-                          uint64_t *__restrict__ act, int64_t n, uint64_t unused_lanes, bool fronts)
+// Up to 64 roots by value: a search's start needs no copy.
+struct Roots {
+    int64_t v[64];
+};
+
+// A search's start, in one launch (it was four, two copies to the device and a
+// wait, and its end another copy and wait: with the same taken from a join, a
+// leave, a step and nedge, 64 roots and their edge counts at scale 16 take 494
+// us instead of 532, and the scale-20 queue's service 3.21 ms instead of 3.48):
+// visited := unused lanes, both active bitmaps
+// := 0 and, unless the caller clears them entry by entry (fronts false), both
+// frontier buffers := 0; every stripe's accumulated slots clear (the first
+// level's; every level's end leaves them clear for the next).  Its first
+// `front` workgroups do what a batch run needs besides: reach[r] = the edges of
+// root r's neighbours (its second level's frontier edges), a workgroup per
+// root; and records of edgeless vertices that held a root `old` before (with
+// edges, a relabelled id below bin_end: left alone) read unreached again, a
+// wave each.
+__global__ __launch_bounds__(kBlock) void k_ms_init(uint64_t *__restrict__ visited, uint64_t *__restrict__ fa,
+                                                    uint64_t *__restrict__ fb, uint64_t *__restrict__ act, int64_t n,
+                                                    uint64_t unused_lanes, bool fronts, int64_t *__restrict__ cnt,
+                                                    int64_t *__restrict__ lane_edges, int front, Roots roots,
+                                                    int nroots, Roots old, int nold,
+                                                    const uint32_t *__restrict__ old2new,
+                                                    const int64_t *__restrict__ rowptr,
+                                                    const uint32_t *__restrict__ cols, int64_t bin_end,
+                                                    int64_t *__restrict__ reach, int32_t *__restrict__ parent,
+                                                    uint8_t *__restrict__ level)
 {
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
+    if ((int)blockIdx.x < front) {
+        const int r = blockIdx.x;
+        if (r < nold && threadIdx.x < 64) {
+            const int64_t o = old.v[r];
+            if ((int64_t)old2new[o] >= bin_end) {
+                parent[o * 64 + threadIdx.x] = -1;
+                level[o * 64 + threadIdx.x] = 0xFF;
+            }
+        }
+        if (r < nroots) {
+            const int64_t v = old2new[roots.v[r]];
+            int64_t t = 0;
+            for (int64_t j = rowptr[v] + threadIdx.x; j < rowptr[v + 1]; j += kBlock) {
+                const uint32_t u = cols[j];
+                t += rowptr[u + 1] - rowptr[u];
+            }
+            t = g5_block_sum256(t);
+            if (threadIdx.x == 0) reach[r] = t;
+        }
+        return;
+    }
+    const int64_t b = blockIdx.x - front, stride = (int64_t)(gridDim.x - front) * kBlock;
+    if (b == 0) {
+        for (int i = threadIdx.x; i < kStripes * kCntStride; i += kBlock)
+            if (i % kCntStride < kAccum) cnt[i] = 0;
+        for (int i = threadIdx.x; i < kLaneStripes * 64; i += kBlock) lane_edges[i] = 0;
+    }
+    for (int64_t i = b * kBlock + threadIdx.x; i < n; i += stride) {
         visited[i] = unused_lanes;
         if (fronts) {
             fa[i] = 0;
@@ -1537,13 +1579,12 @@ __global__ void k_ms_init(uint64_t *__restrict__ visited, uint64_t *__restrict__
     }
 }
 
-// reach[r] = the edges of root r's neighbours (its second level's frontier
-// edges); one workgroup per root
-__global__ __launch_bounds__(256) void k_root_reach(const int64_t *__restrict__ roots, const uint32_t *__restrict__ old2new,
+// The roots' reaches alone (g5_msbfs_reach)
+__global__ __launch_bounds__(256) void k_root_reach(Roots roots, const uint32_t *__restrict__ old2new,
                                                     const int64_t *__restrict__ rowptr,
                                                     const uint32_t *__restrict__ cols, int64_t *__restrict__ reach)
 {
-    const int64_t v = old2new[roots[blockIdx.x]];
+    const int64_t v = old2new[roots.v[blockIdx.x]];
     int64_t t = 0;
     for (int64_t j = rowptr[v] + threadIdx.x; j < rowptr[v + 1]; j += blockDim.x) {
         const uint32_t u = cols[j];
@@ -1551,6 +1592,13 @@ __global__ __launch_bounds__(256) void k_root_reach(const int64_t *__restrict__ 
     }
     t = g5_block_sum256(t);
     if (threadIdx.x == 0) reach[blockIdx.x] = t;
+}
+
+// d_sums[0 .. n) to pinned memory; they are 0 again for the next sums
+__global__ void k_sums_out(unsigned long long *sums, int64_t *host)
+{
+    host[threadIdx.x] = (int64_t)sums[threadIdx.x];
+    sums[threadIdx.x] = 0;
 }
 
 // One thread per root (roots may share a vertex, hence the atomics).  Root r
@@ -1562,7 +1610,7 @@ __global__ __launch_bounds__(256) void k_root_reach(const int64_t *__restrict__ 
 // reached and done: it never enters the frontier, so no frontier word of a
 // vertex outside the degree bins (which the pull kernels never rewrite) is
 // ever non-zero.
-__global__ void k_ms_roots(const int64_t *__restrict__ roots, int nroots, const uint32_t *__restrict__ old2new,
+__global__ void k_ms_roots(Roots roots, int nroots, const uint32_t *__restrict__ old2new,
                            const int64_t *__restrict__ rowptr, uint64_t *__restrict__ visited,
                            uint64_t *__restrict__ frontier, uint64_t *__restrict__ active,
                            int32_t *__restrict__ parent, uint8_t *__restrict__ level, int64_t *__restrict__ cnt,
@@ -1572,7 +1620,7 @@ __global__ void k_ms_roots(const int64_t *__restrict__ roots, int nroots, const 
     const int r = threadIdx.x;
     int64_t v = 0, d = -1, key = -1;
     if (r < nroots) {
-        v = old2new[roots[r]];
+        v = old2new[roots.v[r]];
         d = rowptr[v + 1] - rowptr[v];
         key = reach[r];
     }
@@ -1583,8 +1631,8 @@ __global__ void k_ms_roots(const int64_t *__restrict__ roots, int nroots, const 
         for (int j = 0; j < nroots; ++j) lane += (s_key[j] > key || (s_key[j] == key && j < r)) ? 1 : 0;
         lane_of[r] = lane;
         atomicOr((unsigned long long *)&visited[v], 1ull << lane);
-        parent[roots[r] * 64 + lane] = (int32_t)roots[r];
-        level[roots[r] * 64 + lane] = 0;
+        parent[roots.v[r] * 64 + lane] = (int32_t)roots.v[r];
+        level[roots.v[r] * 64 + lane] = 0;
         if (d != 0) {
             atomicOr((unsigned long long *)&frontier[v], 1ull << lane);
             atomicOr((unsigned long long *)&active[v >> 6], 1ull << (v & 63));
@@ -1878,14 +1926,17 @@ __global__ void k_lane_masks(uint64_t *__restrict__ visited, int64_t n, uint64_t
         visited[i] = (visited[i] | set) & ~clear;
 }
 
-// One wave, a thread per root: root jr[i] (original id) starts lane jr[64 + i]
+// One wave, a thread per root: root jr.v[i] (original id) starts lane lanes.l[i]
 // in the frontier the next level reads (roots may share a vertex, hence the
 // atomics; the one that finds its frontier word empty counts the vertex).  A
 // root without neighbours is only marked visited: its search is complete (and
 // vertices outside the degree bins are never rewritten by the pull kernels, so
 // no frontier bit may be left there).  added[0..1] = new frontier vertices and
 // their edges, added[2 + i] = root i's degree.
-__global__ __launch_bounds__(64) void k_join(const int64_t *__restrict__ jr, int n,
+struct JoinLanes {
+    uint8_t l[64];
+};
+__global__ __launch_bounds__(64) void k_join(Roots jr, JoinLanes lanes, int n,
                                              const uint32_t *__restrict__ old2new,
                                              const int64_t *__restrict__ rowptr, uint64_t *__restrict__ visited,
                                              uint64_t *__restrict__ front, uint64_t *__restrict__ act,
@@ -1897,8 +1948,8 @@ __global__ __launch_bounds__(64) void k_join(const int64_t *__restrict__ jr, int
     const int i = threadIdx.x;
     int64_t nv = 0, ne = 0;
     if (i < n) {
-        const int64_t root = jr[i];
-        const int lane = (int)jr[64 + i];
+        const int64_t root = jr.v[i];
+        const int lane = lanes.l[i];
         const int64_t v = old2new[root];
         const unsigned long long bit = 1ull << lane;
         const int64_t deg = rowptr[v + 1] - rowptr[v];
@@ -2254,6 +2305,7 @@ int bins_for(g5_msbfs *m, int64_t thread_max, int64_t *bf)
     hipStream_t s = m->s;
     const Relabeled &R = m->rl;
     unsigned long long *d = (unsigned long long *)m->d_sums;  // transient scratch, free between calls
+    m->sums_clear = false;
     unsigned long long hb[kBins] = {0, 0, 0};
     G5_HIP(g5::fill_u64((uint64_t *)d, kBins, 0, s));
     hipLaunchKernelGGL(k_bin_counts, g5::grid_for(m->n, 256, 16384), 256, 0, s, (const int64_t *)R.rowptr, m->n,
@@ -2318,11 +2370,29 @@ uint64_t split_lanes(const g5_msbfs *m)
     return pm == m->front_lanes ? 0 : pm;
 }
 
+// Sums of up to 128 values over a kernel's workgroups: d_sums clear, then
+// (after the kernel's launch) to pinned memory, waited for.
+hipError_t begin_sums(g5_msbfs *m)
+{
+    hipError_t e = m->sums_clear ? hipSuccess : g5::fill_u64((uint64_t *)m->d_sums, 128, 0, m->s);
+    m->sums_clear = false;
+    return e;
+}
+hipError_t end_sums(g5_msbfs *m, int n)
+{
+    hipLaunchKernelGGL(k_sums_out, 1, n, 0, m->s, m->d_sums, m->h_io + 98);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipStreamSynchronize(m->s);
+    m->sums_clear = e == hipSuccess;
+    return e;
+}
+
 // One level at parity m->p: push or pull by the frontier's edges (a pull
 // level may push some lanes, split_lanes), then the level's counters on the
 // host; sets *new_bits (new (vertex, root) pairs) and *live (OR of the next
-// frontier), and moves the frontier state on.
-int run_level(g5_msbfs *m, int64_t *new_bits_out, uint64_t *live_out)
+// frontier), and moves the frontier state on.  end: recorded once its work is
+// queued.
+int run_level(g5_msbfs *m, int64_t *new_bits_out, uint64_t *live_out, hipEvent_t end = nullptr)
 {
     hipStream_t s = m->s;
     const int p = m->p;
@@ -2345,6 +2415,7 @@ int run_level(g5_msbfs *m, int64_t *new_bits_out, uint64_t *live_out)
                     : pull_level(m, s, p, lanes, act_check, m->prof);
         if (rc) return rc;
     }
+    if (end) G5_HIP(hipEventRecord(end, s));
     G5_HIP(hipStreamSynchronize(s));  // k_level_end has written h_cnt
     int64_t new_bits = 0;
     const int64_t *h = m->h_cnt;
@@ -2372,9 +2443,10 @@ int run_level(g5_msbfs *m, int64_t *new_bits_out, uint64_t *live_out)
         rec[10] = (double)act_verts;
         rec[11] = (double)act_edges;
         if (push || pm) {
-            // 16 B row offsets per frontier vertex; per frontier edge and
-            // pass (two passes) 4 B column + 8 B frontier word + 8 B visited
-            // word + 8 B next word; 16 B visited read-modify-write per newly
+            // 16 B row offsets per frontier vertex; per frontier edge 4 B
+            // column + 8 B frontier word + 8 B visited word + 8 B next word and
+            // its mark, written and read (the marked edges' second look is left
+            // out); 16 B visited read-modify-write per newly
             // reached vertex; 4 B first parent candidate + 4 B parent + 1 B
             // level per new (vertex, root) pair
             float kms = 0;
@@ -2383,7 +2455,7 @@ int run_level(g5_msbfs *m, int64_t *new_bits_out, uint64_t *live_out)
             const double E = (double)h[kFqEdges];
             m->k_ms[kPushUnit] += kms;
             m->k_launches[kPushUnit] += 1;
-            m->k_bytes[kPushUnit] += 16.0 * h[kFqLen] + 56.0 * E + 16.0 * h[kUnitSlots * kPushUnit + kVisitedVerts] +
+            m->k_bytes[kPushUnit] += 16.0 * h[kFqLen] + 28.25 * E + 16.0 * h[kUnitSlots * kPushUnit + kVisitedVerts] +
                                      9.0 * h[kUnitSlots * kPushUnit + kNewBits];
             rec[kPushUnit] = kms;
             rec[4 + kPushUnit] = E;
@@ -2469,8 +2541,8 @@ extern "C" int g5_msbfs_create(g5_graph *g, g5_msbfs **out)
     if (e == hipSuccess) e = hipMalloc(&m->d_scratch, (g5::scan_scratch_words(n + 1) + 16) * 8);
     m->dup_tiles = dup_tiles_of(g->nnz);
     if (e == hipSuccess) e = hipMalloc(&m->d_dup, (size_t)m->dup_tiles * (kPushTile / 8));
-    if (e == hipSuccess) e = hipMalloc(&m->d_roots, 64 * 8 + 64 * 4);  // roots, then lane_of
-    if (e == hipSuccess) e = hipMalloc(&m->d_join, 194 * 8);
+    if (e == hipSuccess) e = hipMalloc(&m->d_reach, 64 * 8);
+    if (e == hipSuccess) e = hipHostMalloc(&m->h_io, 226 * 8, hipHostMallocDefault);
     if (e == hipSuccess) e = hipMalloc(&m->d_sums, 128 * 8);
     if (e == hipSuccess) e = hipEventCreate(&m->ev0);
     if (e == hipSuccess) e = hipEventCreate(&m->ev1);
@@ -2503,7 +2575,7 @@ extern "C" int g5_msbfs_footprint(const g5_graph *g, int64_t *graph_bytes, int64
                         + 2 * 12 * queue_units(n / 64) * (kUnitWords * 64) + 2 * kGroups * (int64_t)sizeof(QueueTotal)  // push queues
                         + 64 * 5 * n                   // parent and level records
                         + dup_tiles_of(g->nnz) * (kPushTile / 8) + kDirtyCap * 8 + kStripes * kCntStride * 8 + kLaneStripes * 64 * 8 +
-                        ((int64_t)g5::scan_scratch_words(n + 1) + 16) * 8 + 64 * 12 + 194 * 8 + 128 * 8 +
+                        ((int64_t)g5::scan_scratch_words(n + 1) + 16) * 8 + 64 * 8 + 128 * 8 +
                         3 * 4 * n + 8 * (n + 1) + 2 * 4 * nnz  // relabelled copy: ids, degrees, rows
                         + 2 * 8 * n;                       // head, head_orig
     if (graph_bytes) *graph_bytes = 8 * (g->n_rows + 1) + 4 * g->nnz + 4 * g->n_rows;
@@ -2517,13 +2589,14 @@ extern "C" int g5_msbfs_free(g5_msbfs *m)
     if (!m) return G5_OK;
     if (m->s) (void)hipStreamSynchronize(m->s);
     void *dev[] = {m->d_qv[0],   m->d_qv[1],   m->d_qo[0],    m->d_qo[1],   m->d_qt,    m->d_act,   m->d_visited, m->d_fa,
-                   m->d_fb,      m->d_parent,  m->d_cnt,      m->d_scratch, m->d_roots, m->d_join,
+                   m->d_fb,      m->d_parent,  m->d_cnt,      m->d_scratch, m->d_reach,
                    m->d_sums,    m->d_dup, m->rl.new2old, m->rl.old2new, m->rl.rowptr, m->rl.cols, m->rl.gdeg,
                    m->d_lane,    m->rl.head,    m->d_level,   m->d_dirty,  m->rl.head_orig,
                    m->rl.cols_orig, m->d_lvflag};
     for (void *p : dev)
         if (p) (void)hipFree(p);
     if (m->h_cnt) (void)hipHostFree(m->h_cnt);
+    if (m->h_io) (void)hipHostFree(m->h_io);
     hipEvent_t evs[] = {m->ev0, m->ev1, m->ev_fin};
     for (hipEvent_t ev : evs)
         if (ev) (void)hipEventDestroy(ev);
@@ -2547,24 +2620,26 @@ extern "C" int g5_msbfs_run(g5_msbfs *m, const int64_t *roots, int nroots, int32
     m->busy = 0;
     m->nroots = nroots;
     std::copy(roots, roots + nroots, m->roots);
-    int64_t *d_roots = m->d_roots;
-    G5_HIP(hipMemcpyAsync(d_roots, roots, (size_t)nroots * 8, hipMemcpyHostToDevice, s));
-    const bool dirty_listed = (int64_t)m->dirty.size() <= kDirtyCap;
-    if (dirty_listed && !m->dirty.empty())
-        G5_HIP(hipMemcpyAsync(m->d_dirty, m->dirty.data(), m->dirty.size() * 8, hipMemcpyHostToDevice, s));
-    G5_HIP(hipStreamSynchronize(s));
-    G5_HIP(hipEventRecord(m->ev0, s));
+    Roots r{}, old{};
+    std::copy(roots, roots + nroots, r.v);
     // records of edgeless vertices that held an earlier root read unreached
     // again (every edgeless vertex's, when too many roots came since)
     const int64_t bin_end = m->rl.bin_first[kBins];
-    if (!dirty_listed) {
+    const int64_t dirty = (int64_t)m->dirty.size();
+    const int nold = dirty <= 64 ? (int)dirty : 0;
+    std::copy(m->dirty.begin(), m->dirty.begin() + nold, old.v);
+    if (dirty > 64 && dirty <= kDirtyCap) {
+        G5_HIP(hipMemcpyAsync(m->d_dirty, m->dirty.data(), (size_t)dirty * 8, hipMemcpyHostToDevice, s));
+        G5_HIP(hipStreamSynchronize(s));
+    }
+    G5_HIP(hipEventRecord(m->ev0, s));
+    if (dirty > kDirtyCap) {
         if (m->n > bin_end)
             hipLaunchKernelGGL(k_ms_clear_range, g5::grid_for(m->n - bin_end, 4, 16384), 256, 0, s,
                                (const uint32_t *)m->rl.new2old, bin_end, m->n, m->d_parent, m->d_level);
-    } else if (!m->dirty.empty()) {
-        hipLaunchKernelGGL(k_ms_clear_roots, g5::grid_for((int64_t)m->dirty.size(), 4, 4096), 256, 0, s,
-                           (const int64_t *)m->d_dirty, (int64_t)m->dirty.size(), (const uint32_t *)m->rl.old2new,
-                           bin_end, m->d_parent, m->d_level);
+    } else if (dirty > 64) {
+        hipLaunchKernelGGL(k_ms_clear_roots, g5::grid_for(dirty, 4, 4096), 256, 0, s, (const int64_t *)m->d_dirty,
+                           dirty, (const uint32_t *)m->rl.old2new, bin_end, m->d_parent, m->d_level);
     }
     m->dirty.assign(roots, roots + nroots);
     const uint64_t unused = nroots == 64 ? 0ull : ~((1ull << nroots) - 1);
@@ -2572,19 +2647,19 @@ extern "C" int g5_msbfs_run(g5_msbfs *m, const int64_t *roots, int nroots, int32
     // buffer is clear and its frontier buffer is non-zero only at the entries
     // of its frontier queue: clear those instead of both buffers
     const bool listed = m->listed_ok && m->last_empty && m->listed_len * kListedFrac < m->n;
-    hipLaunchKernelGGL(k_ms_init, g5::grid_for(m->n, 256, 16384), 256, 0, s, m->d_visited, m->d_fa, m->d_fb,
-                       m->d_act, m->n, unused, !listed);
-    hipLaunchKernelGGL(k_level_begin, 1, kBlock, 0, s, m->d_cnt, m->d_lane);
+    const int front = std::max(nroots, nold);
+    hipLaunchKernelGGL(k_ms_init, front + g5::grid_for(m->n, kBlock, 16384), kBlock, 0, s, m->d_visited, m->d_fa,
+                       m->d_fb, m->d_act, m->n, unused, !listed, m->d_cnt, m->d_lane, front, r, nroots, old, nold,
+                       (const uint32_t *)m->rl.old2new, (const int64_t *)m->rl.rowptr, (const uint32_t *)m->rl.cols,
+                       bin_end, m->d_reach, m->d_parent, m->d_level);
     if (listed && m->listed_len) {
         uint64_t *last_front = m->p == 0 ? m->d_fb : m->d_fa;  // parity p ^ 1 read it
         hipLaunchKernelGGL(k_push_begin, g5::grid_for(m->listed_len, 256, 4096), 256, 0, s, (uint64_t *)nullptr,
                            (int64_t)0, last_front, m->n, false, push_queue(m, m->listed), (QueueTotal *)nullptr);
     }
-    hipLaunchKernelGGL(k_root_reach, nroots, 256, 0, s, (const int64_t *)d_roots, (const uint32_t *)m->rl.old2new,
-                       (const int64_t *)m->rl.rowptr, (const uint32_t *)m->rl.cols, m->d_join);
-    hipLaunchKernelGGL(k_ms_roots, 1, 64, 0, s, (const int64_t *)d_roots, nroots, (const uint32_t *)m->rl.old2new,
+    hipLaunchKernelGGL(k_ms_roots, 1, 64, 0, s, r, nroots, (const uint32_t *)m->rl.old2new,
                        (const int64_t *)m->rl.rowptr, m->d_visited, m->d_fa, m->d_act, m->d_parent, m->d_level,
-                       m->d_cnt, (int32_t *)(m->d_roots + 64), (const int64_t *)m->d_join);
+                       m->d_cnt, (int32_t *)(m->h_io + 66), (const int64_t *)m->d_reach);
     G5_HIP(hipGetLastError());
     int levels = 1;
     m->lvl.clear();
@@ -2621,9 +2696,8 @@ extern "C" int g5_msbfs_run(g5_msbfs *m, const int64_t *roots, int nroots, int32
                            m->d_parent, m->d_level);
     G5_HIP(hipGetLastError());
     G5_HIP(hipEventRecord(m->ev1, s));
-    G5_HIP(hipMemcpyAsync(m->lane_of, m->d_roots + 64, 64 * 4, hipMemcpyDeviceToHost, s));
     G5_HIP(hipEventSynchronize(m->ev1));
-    G5_HIP(hipStreamSynchronize(s));
+    std::copy((const int32_t *)(m->h_io + 66), (const int32_t *)(m->h_io + 66) + 64, m->lane_of);
     G5_HIP(hipEventElapsedTime(&m->search_ms, m->ev0, m->ev_fin));
     G5_HIP(hipEventElapsedTime(&m->finalize_ms, m->ev_fin, m->ev1));
     // level L is stored as the byte L: final up to level 254 (255: unreached)
@@ -2640,9 +2714,10 @@ extern "C" int g5_msbfs_open(g5_msbfs *m)
     hipStream_t s = m->s;
     // every lane free: free lanes count as visited everywhere, so they never
     // keep a vertex from the fully-visited early exit
-    hipLaunchKernelGGL(k_ms_init, g5::grid_for(m->n, 256, 16384), 256, 0, s, m->d_visited, m->d_fa, m->d_fb,
-                       m->d_act, m->n, ~0ull, true);
-    hipLaunchKernelGGL(k_level_begin, 1, kBlock, 0, s, m->d_cnt, m->d_lane);
+    hipLaunchKernelGGL(k_ms_init, g5::grid_for(m->n, kBlock, 16384), kBlock, 0, s, m->d_visited, m->d_fa, m->d_fb,
+                       m->d_act, m->n, ~0ull, true, m->d_cnt, m->d_lane, 0, Roots{}, 0, Roots{}, 0,
+                       (const uint32_t *)nullptr, (const int64_t *)nullptr, (const uint32_t *)nullptr, (int64_t)0,
+                       (int64_t *)nullptr, (int32_t *)nullptr, (uint8_t *)nullptr);
     G5_HIP(hipGetLastError());
     G5_HIP(hipStreamSynchronize(s));
     m->cont = true;
@@ -2669,28 +2744,27 @@ extern "C" int g5_msbfs_join(g5_msbfs *m, const int64_t *roots, const int *lanes
     G5_REQUIRE(m->cont, G5_E_STATE, "g5_msbfs_join: g5_msbfs_open not called");
     if (n == 0) return G5_OK;
     uint64_t mask = 0;
-    int64_t h[128];
+    Roots jr{};
+    JoinLanes jl{};
     for (int i = 0; i < n; ++i) {
         G5_REQUIRE(lanes[i] >= 0 && lanes[i] < 64, G5_E_ARG, "g5_msbfs_join: lane %d out of range", lanes[i]);
         G5_REQUIRE(!((m->busy | mask) >> lanes[i] & 1), G5_E_STATE, "g5_msbfs_join: lane %d is not free", lanes[i]);
         G5_REQUIRE(roots[i] >= 0 && roots[i] < m->n, G5_E_ARG, "g5_msbfs_join: root %lld out of range",
                    (long long)roots[i]);
         mask |= 1ull << lanes[i];
-        h[i] = roots[i];
-        h[64 + i] = lanes[i];
+        jr.v[i] = roots[i];
+        jl.l[i] = (uint8_t)lanes[i];
     }
     hipStream_t s = m->s;
     uint64_t *front = m->p == 0 ? m->d_fa : m->d_fb;
     uint64_t *act = m->d_act + (m->p == 0 ? 0 : m->n / 64);
-    G5_HIP(hipMemcpyAsync(m->d_join, h, sizeof(h), hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL(k_lane_masks, g5::grid_for(m->n, 256, 16384), 256, 0, s, m->d_visited, m->n, 0ull, mask);
-    hipLaunchKernelGGL(k_join, 1, 64, 0, s, (const int64_t *)m->d_join, n, (const uint32_t *)m->rl.old2new,
+    hipLaunchKernelGGL(k_join, 1, 64, 0, s, jr, jl, n, (const uint32_t *)m->rl.old2new,
                        (const int64_t *)m->rl.rowptr, m->d_visited, front, act, m->d_parent, m->d_level,
-                       (const int64_t *)m->d_cnt, m->d_join + 128);
+                       (const int64_t *)m->d_cnt, m->h_io);
     G5_HIP(hipGetLastError());
-    int64_t added[66] = {};
-    G5_HIP(hipMemcpyAsync(added, m->d_join + 128, (size_t)(2 + n) * 8, hipMemcpyDeviceToHost, s));
     G5_HIP(hipStreamSynchronize(s));
+    const int64_t *added = m->h_io;
     m->busy |= mask;
     for (int i = 0; i < n; ++i) {
         m->lane_root[lanes[i]] = roots[i];
@@ -2723,12 +2797,10 @@ extern "C" int g5_msbfs_step(g5_msbfs *m, uint64_t *live, float *ms)
     G5_HIP(hipEventRecord(m->ev0, m->s));
     int64_t new_bits = 0;
     uint64_t l = 0;
-    int rc = run_level(m, &new_bits, &l);
+    int rc = run_level(m, &new_bits, &l, m->ev1);
     if (rc) return rc;
     for (int r = 0; r < 64; ++r)
         if (m->busy >> r & 1) ++m->lane_steps[r];
-    G5_HIP(hipEventRecord(m->ev1, m->s));
-    G5_HIP(hipEventSynchronize(m->ev1));
     if (ms) G5_HIP(hipEventElapsedTime(ms, m->ev0, m->ev1));
     *live = l & m->busy;
     return G5_OK;
@@ -2741,7 +2813,7 @@ extern "C" int g5_msbfs_leave(g5_msbfs *m, uint64_t lanes, int64_t *nedge, uint6
     G5_REQUIRE((lanes & ~m->busy) == 0, G5_E_STATE, "g5_msbfs_leave: lane not in use");
     if (!lanes) return G5_OK;
     hipStream_t s = m->s;
-    G5_HIP(g5::fill_u64((uint64_t *)m->d_sums, 128, 0, s));
+    G5_HIP(begin_sums(m));
     int lg = 0;  // 2^lg >= the leaving lanes
     while ((1 << lg) < __builtin_popcountll(lanes)) ++lg;
     auto leave = lg == 0   ? k_leave<0>
@@ -2754,10 +2826,8 @@ extern "C" int g5_msbfs_leave(g5_msbfs *m, uint64_t lanes, int64_t *nedge, uint6
     hipLaunchKernelGGL(leave, g5::grid_for(m->n, kBlock, kLeaveGrid), kBlock, 0, s, m->d_visited,
                        (const int32_t *)m->d_parent, (const uint32_t *)m->rl.new2old, (const uint32_t *)m->rl.gdeg,
                        m->n, lanes, m->d_sums);
-    G5_HIP(hipGetLastError());
-    unsigned long long h[128];
-    G5_HIP(hipMemcpyAsync(h, m->d_sums, sizeof(h), hipMemcpyDeviceToHost, s));
-    G5_HIP(hipStreamSynchronize(s));
+    G5_HIP(end_sums(m, 128));
+    const unsigned long long *h = (const unsigned long long *)(m->h_io + 98);
     for (int r = 0; r < 64; ++r)
         if (lanes >> r & 1) {
             if (checksum) checksum[r] = h[r];
@@ -2913,15 +2983,11 @@ extern "C" int g5_msbfs_times(g5_msbfs *m, float *search_ms, float *finalize_ms)
 extern "C" int g5_msbfs_nedge(g5_msbfs *m, int64_t *nedge)
 {
     G5_REQUIRE(m && nedge, G5_E_ARG, "g5_msbfs_nedge: null argument");
-    G5_HIP(g5::fill_u64((uint64_t *)m->d_sums, 64, 0, m->s));  // free between calls
+    G5_HIP(begin_sums(m));
     hipLaunchKernelGGL(k_ms_nedge, g5::grid_for(m->n, kBlock * kNedgeGroups, kNedgeGrid), kBlock, 0, m->s,
                        (const uint64_t *)m->d_visited, (const uint32_t *)m->rl.gdeg, m->n, m->d_sums);
-    G5_HIP(hipGetLastError());
-    // h_cnt is read by a level right after its own copy, so it is free too
-    static_assert(kHostSlots >= 64, "the lanes' sums do not fit the pinned slots");
-    G5_HIP(hipMemcpyAsync(m->h_cnt, m->d_sums, 64 * 8, hipMemcpyDeviceToHost, m->s));
-    G5_HIP(hipStreamSynchronize(m->s));
-    const int64_t *h = m->h_cnt;
+    G5_HIP(end_sums(m, 64));
+    const int64_t *h = m->h_io + 98;
     for (int r = 0; r < m->nroots; ++r) nedge[r] = (int64_t)((unsigned long long)h[internal_lane(m, r)] / 2);
     return G5_OK;
 }
@@ -3185,12 +3251,12 @@ extern "C" int g5_msbfs_reach(g5_msbfs *m, const int64_t *roots, int n, int64_t 
         G5_REQUIRE(roots[i] >= 0 && roots[i] < m->n, G5_E_ARG, "g5_msbfs_reach: root %lld out of range",
                    (long long)roots[i]);
     hipStream_t s = m->s;
-    G5_HIP(hipStreamSynchronize(s));  // d_roots and d_sums are free between calls
-    G5_HIP(hipMemcpyAsync(m->d_roots, roots, (size_t)n * 8, hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_root_reach, n, 256, 0, s, (const int64_t *)m->d_roots, (const uint32_t *)m->rl.old2new,
-                       (const int64_t *)m->rl.rowptr, (const uint32_t *)m->rl.cols, (int64_t *)m->d_sums);
+    Roots r{};
+    std::copy(roots, roots + n, r.v);
+    hipLaunchKernelGGL(k_root_reach, n, 256, 0, s, r, (const uint32_t *)m->rl.old2new, (const int64_t *)m->rl.rowptr,
+                       (const uint32_t *)m->rl.cols, m->h_io + 98);
     G5_HIP(hipGetLastError());
-    G5_HIP(hipMemcpyAsync(reach, m->d_sums, (size_t)n * 8, hipMemcpyDeviceToHost, s));
     G5_HIP(hipStreamSynchronize(s));
+    std::copy(m->h_io + 98, m->h_io + 98 + n, reach);
     return G5_OK;
 }
