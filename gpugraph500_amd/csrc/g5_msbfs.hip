@@ -55,7 +55,8 @@
 // the same results): one thread per vertex up to thread_max neighbours, one wavefront
 // (64 neighbours per step, first hits from an exclusive prefix-OR across
 // lanes) up to wave_max, one 256-thread workgroup beyond (Tune; 256 and 2048
-// by default, 32 and 2048 on graphs of fewer than 2^22 stored neighbours).  A pull level is
+// by default, 64 or 32 and 2048 on graphs of fewer than 2^22 or 2^20 stored
+// neighbours).  A pull level is
 // three to five launches (as a captured hipGraph, after a launch that set what
 // arguments hold now, it took 8 us more: a search of 64 roots at scale 16 with
 // four pull levels 0.457 ms, now 0.424).
@@ -80,6 +81,7 @@
 // parent tree by pointer jumping, as the reference validator derives
 // depths from the predecessor map (validate/validate.h:107-232).
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "g5_internal.hpp"
@@ -97,14 +99,16 @@ constexpr int kLevelRec = 12;  // per level: ms[4], edges[4], new pairs, pushed,
 // Shape parameters (g5_msbfs_tune / g5_msbfs_autotune).  Any values give the
 // same results; they only move work between kernels.  The bounds a search
 // starts with were measured on Kronecker graphs, 64 (and 17) roots each.
-// From 2^22 stored neighbours on, thread_max 256 with split_max 32 is 1.02
-// (scale 17, edgefactor 16), 1.09 (18), 1.14 (20), 1.06 (22), 1.17 (24) times
-// as fast as 32 with 16 (64: 1.01-1.05, 128: 1.04-1.07).  Below it a thread's
+// From 2^22 stored neighbours on, thread_max 256 with split_max 32 is 1.07
+// (scale 17, edgefactor 24), 1.19 (18), 1.14 (20), 1.06 (22), 1.17 (24) times
+// as fast as 32 with 16 (64: 1.01-1.10, 128: 1.04-1.07).  Below it a thread's
 // longer list is a launch's longest chain and too few wavefronts run to hide
-// it: 256 takes 1.08 (scale 16), 1.06 (14) and 1.04 (12) times as long as 32;
-// around the line (scales 15 to 19, edgefactors 64 to 4) the two are within
-// 3 % either way.  lane_ratio 128 is 0.99-1.01 (scale 20 and below), 1.04
+// it: 64 with 32 is the fastest down to 2^20 (1.03 times as fast as 32 at scale
+// 15, 1.00 at 16, 1.04 at 16 with edgefactor 32, 1.07 at 18 with 4; 256: 1.01,
+// 0.97, 1.04, 1.04), 32 with 16 below (64: 0.97 at scales 10, 12 and 14).
+// lane_ratio 128 is 0.99-1.01 (scale 20 and below), 1.04
 // (22) and 1.07 (24) times as fast as 64; push_ratio 4 to 64 are within 7 %.
+constexpr int64_t kLargeNnz = (int64_t)1 << 22, kMiddleNnz = (int64_t)1 << 20;
 // Below kFuseNnz stored neighbours a pull level's three bins share one launch:
 // none of them fills the card, and a level takes as long as the longest chain
 // of the longest bin instead of the sum of theirs (a search at scale 14 0.434
@@ -113,7 +117,13 @@ constexpr int kLevelRec = 12;  // per level: ms[4], edges[4], new pairs, pushed,
 // bin's registers, which halve their wavefronts (scale 20 0.99 -> 1.07, 24
 // 6.4 -> 6.9).
 constexpr int64_t kFuseNnz = (int64_t)1 << 24;
-constexpr int64_t kLargeNnz = (int64_t)1 << 22;
+// With fewer than kPartMax vertices in the thread bin its waves take 16 of them
+// a step instead of 64: four times the waves, of which there is one per SIMD or
+// less otherwise, each with a quarter of the records to write one after the
+// other (scale 12 0.294 -> 0.254 ms, 16 0.417 -> 0.377, 18 0.593 -> 0.554; 19,
+// 340 thousand of them, 0.752 -> 0.757, 20 with edgefactor 8 0.87 -> 0.91; 8 a
+// step: 0.97-1.00 times that up to scale 16, 1.03-1.1 at 17 and 18).
+constexpr int64_t kPartMax = (int64_t)1 << 18;
 constexpr int64_t kLeastWaveMax = 32;  // of a search whose thread_max was not set
 struct Tune {
     int64_t thread_max = 32;   // degree bound of the thread-per-vertex bin
@@ -531,7 +541,7 @@ __device__ __forceinline__ void write_out(const KeptHits &k, int lane, int32_t *
 // end of the next step's scan, so the loads it needs (the vertices' original
 // ids, the head-step parents' from head_orig and the cols_orig loads issued
 // at the hits) complete under that scan instead of stalling the wave.
-template <bool kActive>
+template <bool kActive, int kPer>
 __device__ __forceinline__ void pull_thread(
     int64_t group, int64_t ngroups,
     int64_t first_v, int64_t nlist, const int64_t *__restrict__ rowptr, const uint32_t *__restrict__ cols,
@@ -550,15 +560,17 @@ __device__ __forceinline__ void pull_thread(
     int64_t ngath = 0, nbits = 0, nedges = 0, nverts = 0, nnext = 0, enext = 0;
     uint64_t live = 0;
     KeptHits pend;  // the previous step's hits, translated, not yet written
-    // wave-uniform loop: the wave takes 64 consecutive vertices per step, one
-    // word of the next frontier's active bitmap (the bin starts at a multiple
-    // of 64)
-    for (int64_t base = group * (int64_t)kBlock + (threadIdx.x & ~63); base < nlist;
-         base += ngroups * kBlock) {
-        const int64_t i = base + lane;
+    // wave-uniform loop: the wave takes kPer (64 or 16) consecutive vertices per
+    // step, a word or a quarter of one of the next frontier's active bitmap (the
+    // bin starts at a multiple of 64)
+    typedef typename std::conditional<kPer == 64, uint64_t, uint16_t>::type Flags;
+    Flags *__restrict__ lvf = (Flags *)lvflag, *__restrict__ actn = (Flags *)act_next;
+    for (int64_t base = (group * (kBlock / 64) + (threadIdx.x >> 6)) * kPer; base < nlist;
+         base += ngroups * (kBlock / 64) * kPer) {
+        const int64_t i = kPer == 64 || lane < kPer ? base + lane : nlist;
         const uint32_t v = (uint32_t)(first_v + i);
-        const int64_t fword = (first_v + base) >> 6;
-        const uint64_t fw = fword >= flags_from ? lvflag[fword] : 0ull;
+        const int64_t fword = (first_v + base) / kPer;
+        const uint64_t fw = (first_v + base) >> 6 >= flags_from ? lvf[fword] : (Flags)0;
         KeptHits cur;
         cur.lvmode = (fw >> lane & 1) ? kLvFlagged : 0u;
         uint32_t from_head = 0;
@@ -603,10 +615,10 @@ __device__ __forceinline__ void pull_thread(
         live |= cur.found;
         {
             const uint64_t nf = __ballot(cur.lvmode == kLvWhole);
-            if (lane == 0) lvflag[fword] = nf;
+            if (lane == 0) lvf[fword] = (Flags)nf;
         }
         const uint64_t word = __ballot(cur.found != 0);
-        if (lane == 0) act_next[(first_v + base) >> 6] = word;
+        if (lane == 0) actn[fword] = (Flags)word;
         translate(cur, v, from_head, new2old, head_orig);
         write_out(pend, lane, parent, level, out.lv);
         pend = cur;
@@ -861,23 +873,23 @@ struct PullArgs {
     PullLanes lanes;
 };
 #define G5_PULL(fn, group, ngroups, first, n, bin)                                                                 \
-    fn<kActive>(group, ngroups, first, n, a.rowptr, a.cols, a.head, a.head_orig, a.cols_orig, a.visited, a.frontier, \
+    fn(group, ngroups, first, n, a.rowptr, a.cols, a.head, a.head_orig, a.cols_orig, a.visited, a.frontier, \
                 a.active, a.next, a.parent, a.level, a.new2old, a.cnt, bin, a.act_next, a.lvflag, a.lanes)
 
 template <bool kActive>
 __global__ __launch_bounds__(kBlock) void k_pull_block(PullArgs a, int64_t first, int64_t n)
 {
-    G5_PULL(pull_block, blockIdx.x, gridDim.x, first, n, 0);
+    G5_PULL((pull_block<kActive>), blockIdx.x, gridDim.x, first, n, 0);
 }
 template <bool kActive>
 __global__ __launch_bounds__(kBlock) void k_pull_wave(PullArgs a, int64_t first, int64_t n)
 {
-    G5_PULL(pull_wave, blockIdx.x, gridDim.x, first, n, 1);
+    G5_PULL((pull_wave<kActive>), blockIdx.x, gridDim.x, first, n, 1);
 }
 template <bool kActive>
 __global__ __launch_bounds__(kBlock) void k_pull_thread(PullArgs a, int64_t first, int64_t n)
 {
-    G5_PULL(pull_thread, blockIdx.x, gridDim.x, first, n, 2);
+    G5_PULL((pull_thread<kActive, 64>), blockIdx.x, gridDim.x, first, n, 2);
 }
 
 // The three bins in one launch (kFuseNnz), those with the longest chains first.
@@ -885,13 +897,13 @@ struct PullBins {
     int64_t first[kBins], n[kBins];
     unsigned groups[kBins];
 };
-template <bool kActive>
+template <bool kActive, int kPer>
 __global__ __launch_bounds__(kBlock) void k_pull_all(PullArgs a, PullBins b)
 {
     const unsigned g0 = b.groups[0], g1 = g0 + b.groups[1];
-    if (blockIdx.x < g0) G5_PULL(pull_block, blockIdx.x, g0, b.first[0], b.n[0], 0);
-    else if (blockIdx.x < g1) G5_PULL(pull_wave, blockIdx.x - g0, b.groups[1], b.first[1], b.n[1], 1);
-    else G5_PULL(pull_thread, blockIdx.x - g1, b.groups[2], b.first[2], b.n[2], 2);
+    if (blockIdx.x < g0) G5_PULL((pull_block<kActive>), blockIdx.x, g0, b.first[0], b.n[0], 0);
+    else if (blockIdx.x < g1) G5_PULL((pull_wave<kActive>), blockIdx.x - g0, b.groups[1], b.first[1], b.n[1], 1);
+    else G5_PULL((pull_thread<kActive, kPer>), blockIdx.x - g1, b.groups[2], b.first[2], b.n[2], 2);
 }
 #undef G5_PULL
 
@@ -2088,9 +2100,12 @@ void pull_bins(g5_msbfs *m, hipStream_t s, int p, const PullLanes &lanes, bool a
                                : (unsigned)g5::grid_for(b.n[k], kBlock, 16384);
     }
     if (!prof && m->g->nnz < kFuseNnz) {
+        const bool part = b.n[2] < kPartMax;
+        if (part && b.n[2]) b.groups[2] = (unsigned)g5::grid_for(b.n[2], kBlock / 4, 16384);
         const unsigned groups = b.groups[0] + b.groups[1] + b.groups[2];  // 0: no edges
-        if (groups)
-            hipLaunchKernelGGL(act_check ? k_pull_all<true> : k_pull_all<false>, groups, kBlock, 0, s, a, b);
+        auto kern = part ? (act_check ? k_pull_all<true, 16> : k_pull_all<false, 16>)
+                         : (act_check ? k_pull_all<true, 64> : k_pull_all<false, 64>);
+        if (groups) hipLaunchKernelGGL(kern, groups, kBlock, 0, s, a, b);
         return;
     }
     for (int k = 0; k < kBins; ++k) {
@@ -2511,8 +2526,8 @@ extern "C" int g5_msbfs_create(g5_graph *g, g5_msbfs **out)
     g5_msbfs *m = new g5_msbfs();
     m->g = g;
     m->n = g->n_rows;
-    if (g->nnz >= kLargeNnz) {
-        m->tune.thread_max = m->tune.thread_auto = 256;
+    if (g->nnz >= kMiddleNnz) {
+        m->tune.thread_max = m->tune.thread_auto = g->nnz >= kLargeNnz ? 256 : 64;
         m->tune.split_max = 32;
     }
     const int64_t n = std::max<int64_t>(m->n, 64);

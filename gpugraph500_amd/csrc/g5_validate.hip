@@ -328,9 +328,12 @@ constexpr int kEdgeGrid = 4096;
 // step's row starts make a 64-bit mask, from which every lane takes its row by
 // a population count.  An edge (v, u) with u < v gathers u's depth; its other
 // copy (u, v) is left to that check.  u == parent(v) counts one found parent.
-// Bound by the gathers' addresses, about one per clock and CU whatever they
-// hit (nnz / 2 nibbles: 2.1 ms at scale 24, of which 0.6 ms are the columns and
-// 1.7 ms remain with a footprint that fits the L2 whole).  A thread per light
+// Bound by the gathers' line requests (nnz / 2 nibbles: 2.1 ms at scale 24, 275
+// million requests to the L2s, which serve random lines at 230 to 270 billion a
+// second, and 97 million misses beyond: 6 TB/s; 1.7 ms remain with a footprint
+// that fits the L2 whole, and the VALU is busy for a sixth).  Looking only at
+// the neighbours below v, which end where a binary search says, halves the
+// steps but took 2.3 ms: the requests stay, and the search adds its own.  A thread per light
 // row and a wave per 2048 neighbours of a heavy one, gathering a byte for every
 // entry, took 8.6 ms; 2 or 8 steps in flight 2.3 and 2.1 ms.
 template <typename T>

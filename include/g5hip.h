@@ -295,7 +295,7 @@ int g5_msbfs_info(g5_msbfs *m, int64_t *bins, int cap);
 /* Shape parameters of the batched search (results never depend on them):
  * G5_TUNE_THREAD_MAX / G5_TUNE_WAVE_MAX bound the degree bins of the
  * thread-per-vertex and wavefront-per-vertex pull kernels (default 256, 2048,
- * or 32, 2048 on graphs of fewer than 2^22 stored neighbours; higher degrees
+ * or 64 or 32, 2048 on graphs of fewer than 2^22 or 2^20 stored neighbours; higher degrees
  * take a workgroup per vertex; while THREAD_MAX has not been
  * set it follows a smaller WAVE_MAX, down to 32); G5_TUNE_PUSH_RATIO pushes a
  * level whose frontier edges are below nnz / ratio (16); G5_TUNE_ACTIVE_RATIO
@@ -304,7 +304,7 @@ int g5_msbfs_info(g5_msbfs *m, int64_t *bins, int cap);
  * lanes whose frontier edges are below nnz / ratio (128; 0 = never), which
  * stops one lagging root from making every vertex scan its whole list;
  * G5_TUNE_SPLIT_MAX: such split levels bound the thread-per-vertex bin at
- * min(split_max, thread_max) (32, or 16 on graphs of fewer than 2^22
+ * min(split_max, thread_max) (32, or 16 on graphs of fewer than 2^20
  * stored neighbours), as every row is scanned to its end there.
  * g5_msbfs_autotune searches these by coordinate descent over candidate
  * values (passes rounds, two timed batch searches of roots per candidate),

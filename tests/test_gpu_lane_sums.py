@@ -87,7 +87,8 @@ def test_leaving_lanes_match_the_oracle():
             assert int(ne[x]) == O.nedge(ref, lev) and int(ck[x]) == checksum(pred)
 
 
-@pytest.mark.parametrize("scale, edgefactor, thread, split", [(11, 16, 32, 16), (18, 16, 256, 32)])
+@pytest.mark.parametrize("scale, edgefactor, thread, split", [(11, 16, 32, 16), (16, 16, 64, 32),
+                                                             (18, 16, 256, 32)])
 def test_thread_bound_follows_a_smaller_wave_bound_until_it_is_set(scale, edgefactor, thread, split):
     g = g5.Graph.kronecker(scale, edgefactor)
     m = g5.MSBFS(g)
@@ -174,3 +175,30 @@ def test_graph_without_edges(mode):
         for lane, r in enumerate((0, 5, 127)):
             pred, lev = m.result(lane)
             assert pred[r] == r and lev[r] == 0 and (np.delete(pred, r) == -1).all()
+
+
+@pytest.mark.parametrize("n", [64, 128, 1 << 12, (1 << 18) - 64, 1 << 18])
+def test_thread_bin_in_quarters_of_words(n):
+    """Rings and pairs over all ids: every vertex in the thread bin, up to the
+    size where a wave takes whole words, partly filled words at its end."""
+    rng = np.random.default_rng(n)
+    v = rng.permutation(n)[:n - 21]
+    e = np.stack([v, np.roll(v, 1)], 1)
+    far = rng.integers(0, len(v), (n // 3, 2))
+    e = np.concatenate([e, v[far[far[:, 0] != far[:, 1]]]])
+    e = e[np.lexsort((e[:, 1], e[:, 0]))]
+    both = np.unique(np.concatenate([e, e[:, ::-1]]), axis=0)
+    both = both[both[:, 0] != both[:, 1]]
+    rowptr = np.concatenate([[0], np.cumsum(np.bincount(both[:, 0], minlength=n))])
+    g = g5.Graph.upload(rowptr, both[:, 1].astype(np.uint32), n, gdeg=np.diff(rowptr))
+    roots = [int(v[i]) for i in rng.integers(0, len(v), 40)]
+    a, b = g5.MSBFS(g), g5.MSBFS(g)
+    a.set_mode(1)
+    b.set_mode(2)  # push only: no pull kernels
+    for _ in range(2):
+        a.run(roots)
+        b.run(roots)
+        for lane in range(0, 40, 6):
+            for x, y in zip(a.result(lane), b.result(lane)):
+                assert np.array_equal(x, y)
+    assert a.nedge().tolist() == b.nedge().tolist()
