@@ -189,7 +189,10 @@ struct Relabeled {
     int64_t split_first[kBins + 1] = {0};  // the same on split levels (min(split_max, thread_max))
 };
 
-// the total of a part of a push queue, in a line of its own
+// the total of a part of a push queue, in a line of its own.  Unless the level
+// before left its frontier's queue, the totals of the queue for it are clear
+// before a push level: k_ms_init, the end of a pull or split level and a join
+// see to that
 struct QueueTotal {
     unsigned long long x;  // entries << kQueueEdgeBits | edges
     unsigned long long pad[15];
@@ -1228,10 +1231,11 @@ __global__ __launch_bounds__(kBlock) void k_push_edges(PushArgs a, PushQueue q, 
 // next itself, whole or at the entries of the queue whose words it holds (the
 // frontier queue of the push level before); clear: the totals of a queue that
 // is built next.
-__global__ void k_push_begin(uint64_t *__restrict__ act_next, int64_t nw, uint64_t *__restrict__ next, int64_t n,
-                             bool whole, PushQueue listed, QueueTotal *__restrict__ clear)
+__device__ __forceinline__ void push_begin(int64_t group, int64_t ngroups, uint64_t *__restrict__ act_next,
+                                           int64_t nw, uint64_t *__restrict__ next, int64_t n, bool whole,
+                                           const PushQueue &listed, QueueTotal *__restrict__ clear)
 {
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+    const int64_t t = group * kBlock + threadIdx.x, stride = ngroups * kBlock;
     if (clear && t < kGroups) clear[t].x = 0;
     for (int64_t i = t; i < nw; i += stride) act_next[i] = 0;
     if (whole) {
@@ -1246,6 +1250,13 @@ __global__ void k_push_begin(uint64_t *__restrict__ act_next, int64_t nw, uint64
         const int g = part_of(s, i);
         next[listed.v[s.base[g] + i - s.n0[g]]] = 0;
     }
+}
+
+__global__ __launch_bounds__(kBlock) void k_push_begin(uint64_t *__restrict__ act_next, int64_t nw,
+                                                       uint64_t *__restrict__ next, int64_t n, bool whole,
+                                                       PushQueue listed, QueueTotal *__restrict__ clear)
+{
+    push_begin(blockIdx.x, gridDim.x, act_next, nw, next, n, whole, listed, clear);
 }
 
 // The minimum pass of a push level.  When the newly reached vertices have
@@ -1329,7 +1340,7 @@ __global__ __launch_bounds__(kBlock) void k_push_min(PushArgs a, PushQueue q, Pu
 // A lane's vertices (one per word) lie next to each other in the queue, so one
 // scan over the lanes gives every entry its place and edge offset.
 template <int kKind>
-__global__ __launch_bounds__(kBlock) void k_queue(const uint64_t *__restrict__ bits, int64_t nwords,
+__device__ __forceinline__ void queue_units_of(int64_t group, int64_t ngroups, const uint64_t *__restrict__ bits, int64_t nwords,
                                                   const int64_t *__restrict__ rowptr, PushQueue q,
                                                   const uint64_t *__restrict__ next, uint64_t *__restrict__ visited,
                                                   uint64_t lm, int64_t *__restrict__ cnt)
@@ -1341,7 +1352,7 @@ __global__ __launch_bounds__(kBlock) void k_queue(const uint64_t *__restrict__ b
     int64_t nbits = 0, nv = 0, ne = 0;
     uint64_t live = 0;
     const int64_t units = queue_units(nwords);
-    for (int64_t unit = blockIdx.x; unit < units; unit += gridDim.x) {
+    for (int64_t unit = group; unit < units; unit += ngroups) {
         const int64_t w0 = unit * kUnitWords + wv * W;
         uint64_t word = 0;  // lane k < W: word w0 + k
         if (lane < W && w0 + lane < nwords) word = bits[w0 + lane];
@@ -1427,6 +1438,29 @@ __global__ __launch_bounds__(kBlock) void k_queue(const uint64_t *__restrict__ b
     }
 }
 
+template <int kKind>
+__global__ __launch_bounds__(kBlock) void k_queue(const uint64_t *__restrict__ bits, int64_t nwords,
+                                                  const int64_t *__restrict__ rowptr, PushQueue q,
+                                                  const uint64_t *__restrict__ next, uint64_t *__restrict__ visited,
+                                                  uint64_t lm, int64_t *__restrict__ cnt)
+{
+    queue_units_of<kKind>(blockIdx.x, gridDim.x, bits, nwords, rowptr, q, next, visited, lm, cnt);
+}
+
+// A push level's beginning and, in the workgroups behind the first nb, its
+// frontier's queue q from the active bitmap act (neither touches what the other
+// does; q's totals are clear, see QueueTotal)
+__global__ __launch_bounds__(kBlock) void k_push_start(uint64_t *__restrict__ act_next, int64_t nw,
+                                                       uint64_t *__restrict__ next, int64_t n, bool whole,
+                                                       PushQueue listed, unsigned nb,
+                                                       const uint64_t *__restrict__ act,
+                                                       const int64_t *__restrict__ rowptr, PushQueue q)
+{
+    if (blockIdx.x < nb) push_begin(blockIdx.x, nb, act_next, nw, next, n, whole, listed, nullptr);
+    else
+        queue_units_of<0>(blockIdx.x - nb, gridDim.x - nb, act, nw, rowptr, q, nullptr, nullptr, ~0ull, nullptr);
+}
+
 // active[w] bit i = ((next[64w + i] & lm) != 0).  A wave takes four
 // 64-vertex words per step (four independent loads in flight per lane).
 // kCount: also add the active vertices and their edges to the push unit's
@@ -1479,7 +1513,8 @@ __global__ __launch_bounds__(kBlock) void k_build_active(const uint64_t *__restr
 // totals (when there was one) and the set-once slots go to the host's counters,
 // in pinned memory; the stripes are clear again, the level advances
 __global__ __launch_bounds__(kBlock) void k_level_end(int64_t *cnt, int64_t *lane_edges,
-                                                      const QueueTotal *__restrict__ pushed, int64_t *__restrict__ host)
+                                                      const QueueTotal *pushed, QueueTotal *clear,
+                                                      int64_t *__restrict__ host)
 {
     static_assert(kAccum <= kBlock / 2 && kStripes % 8 == 0 && kLaneStripes == 8, "fold");
     // a thread per slot and 8 stripes, all loads in flight at once
@@ -1513,6 +1548,7 @@ __global__ __launch_bounds__(kBlock) void k_level_end(int64_t *cnt, int64_t *lan
     if (threadIdx.x >= 64 && threadIdx.x < 128) {  // the second wave
         const int g = threadIdx.x - 64;
         const unsigned long long x = pushed && g < kGroups ? pushed[g].x : 0ull;
+        if (clear && g < kGroups) clear[g].x = 0;
         const int64_t n = g5_wave_sum((int64_t)(x >> kQueueEdgeBits));
         const int64_t m = g5_wave_sum((int64_t)(x & ((1ull << kQueueEdgeBits) - 1)));
         if (g == 0) {
@@ -1546,7 +1582,8 @@ struct Roots {
 __global__ __launch_bounds__(kBlock) void k_ms_init(uint64_t *__restrict__ visited, uint64_t *__restrict__ fa,
                                                     uint64_t *__restrict__ fb, uint64_t *__restrict__ act, int64_t n,
                                                     uint64_t unused_lanes, bool fronts, int64_t *__restrict__ cnt,
-                                                    int64_t *__restrict__ lane_edges, int front, Roots roots,
+                                                    int64_t *__restrict__ lane_edges,
+                                                    QueueTotal *__restrict__ clear, int front, Roots roots,
                                                     int nroots, Roots old, int nold,
                                                     const uint32_t *__restrict__ old2new,
                                                     const int64_t *__restrict__ rowptr,
@@ -1580,6 +1617,7 @@ __global__ __launch_bounds__(kBlock) void k_ms_init(uint64_t *__restrict__ visit
         for (int i = threadIdx.x; i < kStripes * kCntStride; i += kBlock)
             if (i % kCntStride < kAccum) cnt[i] = 0;
         for (int i = threadIdx.x; i < kLaneStripes * 64; i += kBlock) lane_edges[i] = 0;
+        if (threadIdx.x < kGroups) clear[threadIdx.x].x = 0;
     }
     for (int64_t i = b * kBlock + threadIdx.x; i < n; i += stride) {
         visited[i] = unused_lanes;
@@ -1953,8 +1991,10 @@ __global__ __launch_bounds__(64) void k_join(Roots jr, JoinLanes lanes, int n,
                                              const int64_t *__restrict__ rowptr, uint64_t *__restrict__ visited,
                                              uint64_t *__restrict__ front, uint64_t *__restrict__ act,
                                              int32_t *__restrict__ parent, uint8_t *__restrict__ level,
-                                             const int64_t *__restrict__ cnt, int64_t *__restrict__ added)
+                                             const int64_t *__restrict__ cnt, QueueTotal *__restrict__ clear,
+                                             int64_t *__restrict__ added)
 {
+    if (threadIdx.x < kGroups) clear[threadIdx.x].x = 0;  // that queue lacks the roots
     // the next level finds the root's neighbours with byte cnt[kDepth]
     const uint8_t root_byte = (uint8_t)(cnt[kDepth] - 1);
     const int i = threadIdx.x;
@@ -2119,6 +2159,12 @@ void pull_bins(g5_msbfs *m, hipStream_t s, int p, const PullLanes &lanes, bool a
     if (prof) (void)hipEventRecord(m->ek[kBins], s);
 }
 
+// queue i of the engine
+PushQueue push_queue(const g5_msbfs *m, int i)
+{
+    return PushQueue{m->d_qv[i], m->d_qo[i], m->d_qt + i * kGroups, queue_units(m->n / 64)};
+}
+
 // One pull level of parity p.
 int pull_level(g5_msbfs *m, hipStream_t s, int p, const PullLanes &lanes, bool act_check, bool prof)
 {
@@ -2132,15 +2178,10 @@ int pull_level(g5_msbfs *m, hipStream_t s, int p, const PullLanes &lanes, bool a
     if (nw01)
         hipLaunchKernelGGL((k_build_active<false, true>), g5::grid_for(nw01, 16, 4096), kBlock, 0, s,
                            (const uint64_t *)next, nw01, (const int64_t *)m->rl.rowptr, act_next, m->d_cnt, ~0ull);
-    hipLaunchKernelGGL(k_level_end, 1, kBlock, 0, s, m->d_cnt, m->d_lane, (const QueueTotal *)nullptr, m->h_cnt);
+    hipLaunchKernelGGL(k_level_end, 1, kBlock, 0, s, m->d_cnt, m->d_lane, (const QueueTotal *)nullptr,
+                       push_queue(m, 1 - m->listed).tot, m->h_cnt);
     G5_HIP(hipGetLastError());
     return G5_OK;
-}
-
-// queue i of the engine
-PushQueue push_queue(const g5_msbfs *m, int i)
-{
-    return PushQueue{m->d_qv[i], m->d_qo[i], m->d_qt + i * kGroups, queue_units(m->n / 64)};
 }
 
 PushArgs push_args(const g5_msbfs *m, int p)
@@ -2153,6 +2194,14 @@ PushArgs push_args(const g5_msbfs *m, int p)
 // tiles of edges whose marks are kept: 8 MiB of them at most (a push level of
 // more edges gives the minimum pass all the edges beyond)
 int64_t dup_tiles_of(int64_t nnz) { return std::min<int64_t>(nnz / kPushTile + 2 * kGroups, (1 << 26) / kPushTile); }
+
+// A push level's workgroups: an edge a thread up to the whole grid (starting
+// 4096 workgroups that find no tile takes 7 us, 64 of them 3).  The first
+// level's edges are not known.
+unsigned push_grid(int64_t edges)
+{
+    return edges < 0 ? 1024u : (unsigned)std::max(64, g5::grid_for(edges, kBlock, kPushGrid));
+}
 
 unsigned queue_grid(int64_t nwords) { return (unsigned)g5::grid_for(queue_units(nwords), 1, kPushVertGrid); }
 
@@ -2176,21 +2225,23 @@ int push_level(g5_msbfs *m, hipStream_t s, int p, bool listed_in, bool queue_in,
     const PushArgs a = push_args(m, p);
     const PushQueue q = push_queue(m, 1 - m->listed), nq = push_queue(m, m->listed);
     const bool whole = !(listed_in && m->listed_len * kListedFrac < m->n);
-    hipLaunchKernelGGL(k_push_begin, g5::grid_for(whole ? m->n : std::max(nw, m->listed_len), 256, 4096), 256, 0, s,
-                       act_next, nw, a.next, m->n, whole, m->listed_len ? nq : PushQueue{},
-                       queue_in ? (QueueTotal *)nullptr : q.tot);
+    const unsigned nb = (unsigned)g5::grid_for(whole ? m->n : std::max(nw, m->listed_len), kBlock, 4096);
     if (prof) G5_HIP(hipEventRecord(m->ek[0], s));
-    if (!queue_in)
-        hipLaunchKernelGGL(k_queue<0>, queue_grid(nw), kBlock, 0, s, act, nw, (const int64_t *)R.rowptr, q,
-                           (const uint64_t *)nullptr, (uint64_t *)nullptr, ~0ull, m->d_cnt);
-    hipLaunchKernelGGL(k_push_edges<false>, kPushGrid, kBlock, 0, s, a, q, m->d_cnt, ~0ull, act_next, m->n,
+    if (queue_in)
+        hipLaunchKernelGGL(k_push_begin, nb, kBlock, 0, s, act_next, nw, a.next, m->n, whole,
+                           m->listed_len ? nq : PushQueue{}, (QueueTotal *)nullptr);
+    else
+        hipLaunchKernelGGL(k_push_start, nb + queue_grid(nw), kBlock, 0, s, act_next, nw, a.next, m->n, whole,
+                           m->listed_len ? nq : PushQueue{}, nb, act, (const int64_t *)R.rowptr, q);
+    hipLaunchKernelGGL(k_push_edges<false>, push_grid(m->act_edges), kBlock, 0, s, a, q, m->d_cnt, ~0ull, act_next, m->n,
                        (uint32_t *)nullptr, 0, nq.tot);
     hipLaunchKernelGGL(k_queue<1>, queue_grid(nw), kBlock, 0, s, (const uint64_t *)act_next, nw,
                        (const int64_t *)R.rowptr, nq, (const uint64_t *)a.next, m->d_visited, ~0ull, m->d_cnt);
-    hipLaunchKernelGGL(k_push_min, kPushGrid, kBlock, 0, s, a, q, nq, (const int64_t *)m->d_cnt, ~0ull, m->n, true,
+    hipLaunchKernelGGL(k_push_min, push_grid(m->act_edges), kBlock, 0, s, a, q, nq, (const int64_t *)m->d_cnt, ~0ull, m->n, true,
                        m->d_lane);
     if (prof) G5_HIP(hipEventRecord(m->ek[1], s));
-    hipLaunchKernelGGL(k_level_end, 1, kBlock, 0, s, m->d_cnt, m->d_lane, (const QueueTotal *)q.tot, m->h_cnt);
+    hipLaunchKernelGGL(k_level_end, 1, kBlock, 0, s, m->d_cnt, m->d_lane, (const QueueTotal *)q.tot,
+                       (QueueTotal *)nullptr, m->h_cnt);
     G5_HIP(hipGetLastError());
     m->listed = 1 - m->listed;  // q lists the buffer that the next push level writes
     return G5_OK;
@@ -2205,7 +2256,7 @@ int push_level(g5_msbfs *m, hipStream_t s, int p, bool listed_in, bool queue_in,
 // candidates (push_cand) and k_cand_commit writes the pairs out; otherwise the
 // passes of a push level run.  Ends with the bins' part of next's active
 // bitmap, counts and live lanes.
-int split_level(g5_msbfs *m, hipStream_t s, int p, uint64_t pm, const PullLanes &lanes, bool act_check, bool prof)
+int split_level(g5_msbfs *m, hipStream_t s, int p, uint64_t pm, int64_t pe, const PullLanes &lanes, bool act_check, bool prof)
 {
     const Relabeled &R = m->rl;
     const int64_t nw = m->n / 64;
@@ -2230,14 +2281,14 @@ int split_level(g5_msbfs *m, hipStream_t s, int p, uint64_t pm, const PullLanes 
     if (vend * npm <= m->n) {
         if (vend) {
             G5_HIP(g5::fill_u32(cand, vend * npm, ~0u, s));
-            hipLaunchKernelGGL(k_push_edges<true>, kPushGrid, kBlock, 0, s, a, q, m->d_cnt, pm, (uint64_t *)nullptr,
+            hipLaunchKernelGGL(k_push_edges<true>, push_grid(pe), kBlock, 0, s, a, q, m->d_cnt, pm, (uint64_t *)nullptr,
                                vend, cand, npm, (QueueTotal *)nullptr);
             hipLaunchKernelGGL(k_cand_commit, g5::grid_for(vend, kBlock, 4096), kBlock, 0, s, (const uint32_t *)cand,
                                npm, pm, vend, (const uint32_t *)R.new2old, a.next, m->d_visited, m->d_parent,
                                m->d_level, m->d_cnt);
         }
     } else {
-        hipLaunchKernelGGL(k_push_edges<false>, kPushGrid, kBlock, 0, s, a, q, m->d_cnt, pm, (uint64_t *)nullptr, vend,
+        hipLaunchKernelGGL(k_push_edges<false>, push_grid(pe), kBlock, 0, s, a, q, m->d_cnt, pm, (uint64_t *)nullptr, vend,
                            (uint32_t *)nullptr, 0, (QueueTotal *)nullptr);
         // the newly reached vertices of the lanes pm
         hipLaunchKernelGGL((k_build_active<false, false>), g5::grid_for(nw_push, 16, 4096), kBlock, 0, s,
@@ -2245,14 +2296,15 @@ int split_level(g5_msbfs *m, hipStream_t s, int p, uint64_t pm, const PullLanes 
         hipLaunchKernelGGL(k_queue<2>, queue_grid(nw_push), kBlock, 0, s, (const uint64_t *)act_next, nw_push,
                            (const int64_t *)R.rowptr, PushQueue{}, (const uint64_t *)a.next, m->d_visited, pm,
                            m->d_cnt);
-        hipLaunchKernelGGL(k_push_min, kPushGrid, kBlock, 0, s, a, q, PushQueue{}, (const int64_t *)m->d_cnt, pm, vend,
+        hipLaunchKernelGGL(k_push_min, push_grid(pe), kBlock, 0, s, a, q, PushQueue{}, (const int64_t *)m->d_cnt, pm, vend,
                            false, m->d_lane);
     }
     if (nw_push)
         hipLaunchKernelGGL((k_build_active<true, true>), g5::grid_for(nw_push, 16, 4096), kBlock, 0, s,
                            (const uint64_t *)a.next, nw_push, (const int64_t *)R.rowptr, act_next, m->d_cnt, ~0ull);
     if (prof) G5_HIP(hipEventRecord(m->ek_push[1], s));
-    hipLaunchKernelGGL(k_level_end, 1, kBlock, 0, s, m->d_cnt, m->d_lane, (const QueueTotal *)q.tot, m->h_cnt);
+    hipLaunchKernelGGL(k_level_end, 1, kBlock, 0, s, m->d_cnt, m->d_lane, (const QueueTotal *)q.tot, q.tot,
+                       m->h_cnt);
     G5_HIP(hipGetLastError());
     return G5_OK;
 }
@@ -2362,7 +2414,7 @@ uint64_t used_lanes(const g5_msbfs *m)
 // 30 ms split, at scale 27.)  Only right after a push level or a join:
 // after a pull level every lane has had a dense level, and the unvisited
 // vertices left are few (a split there has measured slower).  0: no split.
-uint64_t split_lanes(const g5_msbfs *m)
+uint64_t split_lanes(const g5_msbfs *m, int64_t &pe)
 {
     const int64_t nnz = m->g->nnz;
     if (m->mode != 0 || m->tune.lane_ratio <= 0 || !m->split_ok) return 0;
@@ -2375,7 +2427,7 @@ uint64_t split_lanes(const g5_msbfs *m)
         return m->lane_edges[a] != m->lane_edges[b] ? m->lane_edges[a] < m->lane_edges[b] : a < b;
     });
     uint64_t pm = 0;
-    int64_t pe = 0;
+    pe = 0;
     for (int i = 0; i < nc; ++i) {
         const int64_t e = m->lane_edges[order[i]];
         if ((pe + e) * m->tune.push_ratio >= nnz) break;
@@ -2419,14 +2471,15 @@ int run_level(g5_msbfs *m, int64_t *new_bits_out, uint64_t *live_out, hipEvent_t
     const int64_t nnz = m->g->nnz;
     const bool push = m->mode == 2 || (m->mode == 0 && (act_edges < 0 || act_edges * m->tune.push_ratio < nnz));
     const bool act_check = act_edges < 0 || act_edges * m->tune.active_ratio < nnz;
-    const uint64_t pm = push ? 0 : split_lanes(m);
+    int64_t pe = 0;  // of the pushed lanes
+    const uint64_t pm = push ? 0 : split_lanes(m, pe);
     if (push) {
         int rc = push_level(m, s, p, listed_in, queue_in, m->prof);
         if (rc) return rc;
     } else {
         const PullLanes lanes{m->front_lanes & ~pm, m->front_lanes, used_lanes(m), m->flag_word,
                               pm ? (int64_t)64 : (int64_t)kWaveFirst};
-        int rc = pm ? split_level(m, s, p, pm, lanes, act_check, m->prof)
+        int rc = pm ? split_level(m, s, p, pm, pe, lanes, act_check, m->prof)
                     : pull_level(m, s, p, lanes, act_check, m->prof);
         if (rc) return rc;
     }
@@ -2664,7 +2717,8 @@ extern "C" int g5_msbfs_run(g5_msbfs *m, const int64_t *roots, int nroots, int32
     const bool listed = m->listed_ok && m->last_empty && m->listed_len * kListedFrac < m->n;
     const int front = std::max(nroots, nold);
     hipLaunchKernelGGL(k_ms_init, front + g5::grid_for(m->n, kBlock, 16384), kBlock, 0, s, m->d_visited, m->d_fa,
-                       m->d_fb, m->d_act, m->n, unused, !listed, m->d_cnt, m->d_lane, front, r, nroots, old, nold,
+                       m->d_fb, m->d_act, m->n, unused, !listed, m->d_cnt, m->d_lane, push_queue(m, 1 - m->listed).tot,
+                       front, r, nroots, old, nold,
                        (const uint32_t *)m->rl.old2new, (const int64_t *)m->rl.rowptr, (const uint32_t *)m->rl.cols,
                        bin_end, m->d_reach, m->d_parent, m->d_level);
     if (listed && m->listed_len) {
@@ -2730,7 +2784,7 @@ extern "C" int g5_msbfs_open(g5_msbfs *m)
     // every lane free: free lanes count as visited everywhere, so they never
     // keep a vertex from the fully-visited early exit
     hipLaunchKernelGGL(k_ms_init, g5::grid_for(m->n, kBlock, 16384), kBlock, 0, s, m->d_visited, m->d_fa, m->d_fb,
-                       m->d_act, m->n, ~0ull, true, m->d_cnt, m->d_lane, 0, Roots{}, 0, Roots{}, 0,
+                       m->d_act, m->n, ~0ull, true, m->d_cnt, m->d_lane, push_queue(m, 1 - m->listed).tot, 0, Roots{}, 0, Roots{}, 0,
                        (const uint32_t *)nullptr, (const int64_t *)nullptr, (const uint32_t *)nullptr, (int64_t)0,
                        (int64_t *)nullptr, (int32_t *)nullptr, (uint8_t *)nullptr);
     G5_HIP(hipGetLastError());
@@ -2776,7 +2830,7 @@ extern "C" int g5_msbfs_join(g5_msbfs *m, const int64_t *roots, const int *lanes
     hipLaunchKernelGGL(k_lane_masks, g5::grid_for(m->n, 256, 16384), 256, 0, s, m->d_visited, m->n, 0ull, mask);
     hipLaunchKernelGGL(k_join, 1, 64, 0, s, jr, jl, n, (const uint32_t *)m->rl.old2new,
                        (const int64_t *)m->rl.rowptr, m->d_visited, front, act, m->d_parent, m->d_level,
-                       (const int64_t *)m->d_cnt, m->h_io);
+                       (const int64_t *)m->d_cnt, push_queue(m, 1 - m->listed).tot, m->h_io);
     G5_HIP(hipGetLastError());
     G5_HIP(hipStreamSynchronize(s));
     const int64_t *added = m->h_io;
