@@ -117,6 +117,13 @@ constexpr int64_t kLargeNnz = (int64_t)1 << 22, kMiddleNnz = (int64_t)1 << 20;
 // bin's registers, which halve their wavefronts (scale 20 0.99 -> 1.07, 24
 // 6.4 -> 6.9).
 constexpr int64_t kFuseNnz = (int64_t)1 << 24;
+// There the wave bin's workgroups take several vertices a wave, three of them
+// per CU: one vertex a wave, they fill the card several times over before the
+// thread bin's start, and end in a counter update each (scale 16 0.362 -> 0.337
+// ms, 17 0.407 -> 0.381, 18 0.468 -> 0.446; 256 of them 0.366 / 0.412 / 0.484,
+// 512 0.346 / 0.373 / 0.445, the same up to scale 14; on larger graphs, where
+// the bins are launched apart, 768 take 1.02 to 1.15 times as long as all).
+constexpr unsigned kFuseWaveGroups = 768;
 // With fewer than kPartMax vertices in the thread bin its waves take 16 of them
 // a step instead of 64: four times the waves, of which there is one per SIMD or
 // less otherwise, each with a quarter of the records to write one after the
@@ -2142,6 +2149,7 @@ void pull_bins(g5_msbfs *m, hipStream_t s, int p, const PullLanes &lanes, bool a
     if (!prof && m->g->nnz < kFuseNnz) {
         const bool part = b.n[2] < kPartMax;
         if (part && b.n[2]) b.groups[2] = (unsigned)g5::grid_for(b.n[2], kBlock / 4, 16384);
+        b.groups[1] = std::min(b.groups[1], kFuseWaveGroups);
         const unsigned groups = b.groups[0] + b.groups[1] + b.groups[2];  // 0: no edges
         auto kern = part ? (act_check ? k_pull_all<true, 16> : k_pull_all<false, 16>)
                          : (act_check ? k_pull_all<true, 64> : k_pull_all<false, 64>);
@@ -2213,9 +2221,9 @@ unsigned queue_grid(int64_t nwords) { return (unsigned)g5::grid_for(queue_units(
 // left if it pushed.  The edge that makes next[v] non-zero sets v's active
 // bit; k_queue then commits and counts the vertices of that bitmap and leaves
 // their queue, the next level's frontier's, so a push level makes no pass over
-// all n words.  Six launches or five (19 with separate queue, degree, prefix,
-// count and commit passes: a batch's four push levels at scale 16 took 260 us,
-// now 160).
+// all n words.  Five launches (19 with separate queue, degree, prefix, count
+// and commit passes: with those, a batch of 64 roots at scale 16 and its
+// per-root edge sums were 114 launches and 739 us, without 61 and 614 us).
 int push_level(g5_msbfs *m, hipStream_t s, int p, bool listed_in, bool queue_in, bool prof)
 {
     const Relabeled &R = m->rl;
