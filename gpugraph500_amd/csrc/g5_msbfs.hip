@@ -115,7 +115,8 @@ constexpr int64_t kLargeNnz = (int64_t)1 << 22, kMiddleNnz = (int64_t)1 << 20;
 // -> 0.381 ms, 16 0.507 -> 0.457, 18 0.640 -> 0.626, edgefactor 4 at scale 21
 // 1.04 -> 1.02).  Beyond it the block and wave bins lose more by the thread
 // bin's registers, which halve their wavefronts (scale 20 0.99 -> 1.07, 24
-// 6.4 -> 6.9).
+// 6.4 -> 6.9; on a second stream beside the thread bin 0.99 -> 1.03 and the
+// same).
 constexpr int64_t kFuseNnz = (int64_t)1 << 24;
 // There the wave bin's workgroups take several vertices a wave, three of them
 // per CU: one vertex a wave, they fill the card several times over before the
