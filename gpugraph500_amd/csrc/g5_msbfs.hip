@@ -936,6 +936,12 @@ __global__ __launch_bounds__(kBlock) void k_pull_all(PullArgs a, PullBins b)
 // the block and wave bins, whose kernels leave the pushed lanes out).
 // a push level clears next entry by entry when the list is below n / kListedFrac
 constexpr int64_t kListedFrac = 32;
+// A push level of n / kScanFrac edges or more leaves next's bitmap to k_queue,
+// which reads all of next for it, instead of setting a bit with an atomic per
+// vertex reached: level 2 of 64 roots at scale 24 670 -> 630 us of edges and
+// queue, at scale 26 2078 -> 1940.  Only after another push level: past the
+// peak, after pull levels, few vertices are new (scale 26 430 -> 469).
+constexpr int64_t kScanFrac = 8;
 constexpr int kPushTile = 1024;  // 20 KB of LDS per block (2048: 40 KB, 4 waves per SIMD)
 constexpr int kPushGrid = 4096;
 constexpr int kPushVertGrid = 2048;
@@ -1343,15 +1349,17 @@ __global__ __launch_bounds__(kBlock) void k_push_min(PushArgs a, PushQueue q, Pu
 //   kKind 1   the same for a push level's newly reached vertices (next's
 //             bitmap), with the level's commit (visited |= next) and counts:
 //             pairs, the next frontier's vertices and edges, the live lanes
+//   kKind 3   the same as 1, with the bitmap made on the way: every word of next
+//             is read
 //   kKind 2   a split level's vertices reached by the pushed lanes lm: commit
 //             and counts of pairs and vertices, no queue
 // A lane's vertices (one per word) lie next to each other in the queue, so one
 // scan over the lanes gives every entry its place and edge offset.
 template <int kKind>
-__device__ __forceinline__ void queue_units_of(int64_t group, int64_t ngroups, const uint64_t *__restrict__ bits, int64_t nwords,
-                                                  const int64_t *__restrict__ rowptr, PushQueue q,
-                                                  const uint64_t *__restrict__ next, uint64_t *__restrict__ visited,
-                                                  uint64_t lm, int64_t *__restrict__ cnt)
+__device__ __forceinline__ void queue_units_of(int64_t group, int64_t ngroups, uint64_t *__restrict__ bits,
+                                               int64_t nwords, const int64_t *__restrict__ rowptr, PushQueue q,
+                                               const uint64_t *__restrict__ next, uint64_t *__restrict__ visited,
+                                               uint64_t lm, int64_t *__restrict__ cnt)
 {
     constexpr int W = kUnitWords / (kBlock / 64);
     __shared__ unsigned long long s_wave[kBlock / 64], s_at;
@@ -1363,13 +1371,24 @@ __device__ __forceinline__ void queue_units_of(int64_t group, int64_t ngroups, c
     for (int64_t unit = group; unit < units; unit += ngroups) {
         const int64_t w0 = unit * kUnitWords + wv * W;
         uint64_t word = 0;  // lane k < W: word w0 + k
-        if (lane < W && w0 + lane < nwords) word = bits[w0 + lane];
+        uint64_t x[W];
+        if (kKind == 3) {
+#pragma unroll
+            for (int k = 0; k < W; ++k) x[k] = w0 + k < nwords ? next[(w0 + k) * 64 + lane] : 0ull;
+#pragma unroll
+            for (int k = 0; k < W; ++k) {
+                const uint64_t found = __ballot(x[k] != 0);
+                if (lane == k) word = found;
+            }
+            if (lane < W && w0 + lane < nwords) bits[w0 + lane] = word;
+        } else if (lane < W && w0 + lane < nwords) {
+            word = bits[w0 + lane];
+        }
         const bool any = __ballot(word != 0) != 0;
         uint32_t deg[W];
         unsigned long long sum = 0;
         if (any) {
             int64_t lo[W], hi[W];
-            uint64_t x[W];
 #pragma unroll
             for (int k = 0; k < W; ++k) {
                 const int64_t v = (w0 + k) * 64 + lane;
@@ -1378,7 +1397,7 @@ __device__ __forceinline__ void queue_units_of(int64_t group, int64_t ngroups, c
                     lo[k] = mine ? rowptr[v] : 0;
                     hi[k] = mine ? rowptr[v + 1] : 0;
                 }
-                if (kKind != 0) x[k] = mine ? next[v] & lm : 0ull;
+                if (kKind == 1 || kKind == 2) x[k] = mine ? next[v] & lm : 0ull;
             }
 #pragma unroll
             for (int k = 0; k < W; ++k) {
@@ -1392,7 +1411,7 @@ __device__ __forceinline__ void queue_units_of(int64_t group, int64_t ngroups, c
                     visited[v] |= x[k];
                     nbits += __popcll(x[k]);
                     ++nv;
-                    if (kKind == 1) {
+                    if (kKind != 2) {
                         ne += deg[k];
                         live |= x[k];
                     }
@@ -1430,7 +1449,7 @@ __device__ __forceinline__ void queue_units_of(int64_t group, int64_t ngroups, c
         __syncthreads();  // s_wave is rewritten by the next unit
     }
     if (kKind == 2) block_add(cnt + kUnitSlots * kPushUnit, {nbits, (int64_t)0, nv});
-    if (kKind == 1) {
+    if (kKind == 1 || kKind == 3) {
         live = g5_wave_or(live);
         if (lane == 0) s_live[wv] = live;
         // its barrier orders s_live
@@ -1447,7 +1466,7 @@ __device__ __forceinline__ void queue_units_of(int64_t group, int64_t ngroups, c
 }
 
 template <int kKind>
-__global__ __launch_bounds__(kBlock) void k_queue(const uint64_t *__restrict__ bits, int64_t nwords,
+__global__ __launch_bounds__(kBlock) void k_queue(uint64_t *__restrict__ bits, int64_t nwords,
                                                   const int64_t *__restrict__ rowptr, PushQueue q,
                                                   const uint64_t *__restrict__ next, uint64_t *__restrict__ visited,
                                                   uint64_t lm, int64_t *__restrict__ cnt)
@@ -1461,7 +1480,7 @@ __global__ __launch_bounds__(kBlock) void k_queue(const uint64_t *__restrict__ b
 __global__ __launch_bounds__(kBlock) void k_push_start(uint64_t *__restrict__ act_next, int64_t nw,
                                                        uint64_t *__restrict__ next, int64_t n, bool whole,
                                                        PushQueue listed, unsigned nb,
-                                                       const uint64_t *__restrict__ act,
+                                                       uint64_t *__restrict__ act,
                                                        const int64_t *__restrict__ rowptr, PushQueue q)
 {
     if (blockIdx.x < nb) push_begin(blockIdx.x, nb, act_next, nw, next, n, whole, listed, nullptr);
@@ -2220,7 +2239,8 @@ unsigned queue_grid(int64_t nwords) { return (unsigned)g5::grid_for(queue_units(
 // only non-zero words of this level's next: listed_in) and the list is short,
 // otherwise whole -- and with the frontier's queue, which the level before
 // left if it pushed.  The edge that makes next[v] non-zero sets v's active
-// bit; k_queue then commits and counts the vertices of that bitmap and leaves
+// bit (a level of many edges after another leaves that to k_queue); k_queue
+// then commits and counts the vertices of that bitmap and leaves
 // their queue, the next level's frontier's, so a push level makes no pass over
 // all n words.  Five launches (19 with separate queue, degree, prefix, count
 // and commit passes: with those, a batch of 64 roots at scale 16 and its
@@ -2229,7 +2249,7 @@ int push_level(g5_msbfs *m, hipStream_t s, int p, bool listed_in, bool queue_in,
 {
     const Relabeled &R = m->rl;
     const int64_t nw = m->n / 64;
-    const uint64_t *act = m->d_act + (p == 0 ? 0 : nw);
+    uint64_t *act = m->d_act + (p == 0 ? 0 : nw);
     uint64_t *act_next = m->d_act + (p == 0 ? nw : 0);
     const PushArgs a = push_args(m, p);
     const PushQueue q = push_queue(m, 1 - m->listed), nq = push_queue(m, m->listed);
@@ -2242,9 +2262,10 @@ int push_level(g5_msbfs *m, hipStream_t s, int p, bool listed_in, bool queue_in,
     else
         hipLaunchKernelGGL(k_push_start, nb + queue_grid(nw), kBlock, 0, s, act_next, nw, a.next, m->n, whole,
                            m->listed_len ? nq : PushQueue{}, nb, act, (const int64_t *)R.rowptr, q);
-    hipLaunchKernelGGL(k_push_edges<false>, push_grid(m->act_edges), kBlock, 0, s, a, q, m->d_cnt, ~0ull, act_next, m->n,
-                       (uint32_t *)nullptr, 0, nq.tot);
-    hipLaunchKernelGGL(k_queue<1>, queue_grid(nw), kBlock, 0, s, (const uint64_t *)act_next, nw,
+    const bool scan = queue_in && m->act_edges >= m->n / kScanFrac;
+    hipLaunchKernelGGL(k_push_edges<false>, push_grid(m->act_edges), kBlock, 0, s, a, q, m->d_cnt, ~0ull,
+                       scan ? (uint64_t *)nullptr : act_next, m->n, (uint32_t *)nullptr, 0, nq.tot);
+    hipLaunchKernelGGL(scan ? k_queue<3> : k_queue<1>, queue_grid(nw), kBlock, 0, s, act_next, nw,
                        (const int64_t *)R.rowptr, nq, (const uint64_t *)a.next, m->d_visited, ~0ull, m->d_cnt);
     hipLaunchKernelGGL(k_push_min, push_grid(m->act_edges), kBlock, 0, s, a, q, nq, (const int64_t *)m->d_cnt, ~0ull, m->n, true,
                        m->d_lane);
@@ -2283,7 +2304,7 @@ int split_level(g5_msbfs *m, hipStream_t s, int p, uint64_t pm, int64_t pe, cons
                        (const int64_t *)R.rowptr, act_cur, m->d_cnt, pm);
     hipLaunchKernelGGL(k_push_begin, 1, 256, 0, s, (uint64_t *)nullptr, (int64_t)0, (uint64_t *)nullptr, (int64_t)0,
                        true, PushQueue{}, q.tot);
-    hipLaunchKernelGGL(k_queue<0>, queue_grid(nw), kBlock, 0, s, (const uint64_t *)act_cur, nw,
+    hipLaunchKernelGGL(k_queue<0>, queue_grid(nw), kBlock, 0, s, act_cur, nw,
                        (const int64_t *)R.rowptr, q, (const uint64_t *)nullptr, (uint64_t *)nullptr, ~0ull, m->d_cnt);
     const int64_t vend = R.split_first[2], nw_push = (vend + 63) / 64;
     const int npm = __builtin_popcountll(pm);
@@ -2302,7 +2323,7 @@ int split_level(g5_msbfs *m, hipStream_t s, int p, uint64_t pm, int64_t pe, cons
         // the newly reached vertices of the lanes pm
         hipLaunchKernelGGL((k_build_active<false, false>), g5::grid_for(nw_push, 16, 4096), kBlock, 0, s,
                            (const uint64_t *)a.next, nw_push, (const int64_t *)R.rowptr, act_next, m->d_cnt, pm);
-        hipLaunchKernelGGL(k_queue<2>, queue_grid(nw_push), kBlock, 0, s, (const uint64_t *)act_next, nw_push,
+        hipLaunchKernelGGL(k_queue<2>, queue_grid(nw_push), kBlock, 0, s, act_next, nw_push,
                            (const int64_t *)R.rowptr, PushQueue{}, (const uint64_t *)a.next, m->d_visited, pm,
                            m->d_cnt);
         hipLaunchKernelGGL(k_push_min, push_grid(pe), kBlock, 0, s, a, q, PushQueue{}, (const int64_t *)m->d_cnt, pm, vend,

@@ -202,3 +202,25 @@ def test_thread_bin_in_quarters_of_words(n):
             for x, y in zip(a.result(lane), b.result(lane)):
                 assert np.array_equal(x, y)
     assert a.nedge().tolist() == b.nedge().tolist()
+
+
+@pytest.mark.parametrize("n", [640, 4096, 40000])
+def test_push_levels_with_and_without_a_bitmap_of_marks(n):
+    """Push only: a few sources, then nearly all vertices at once (more edges
+    than n / 8 after a push level), then their neighbours."""
+    rng = np.random.default_rng(n)
+    k = n // 2
+    e = np.concatenate([np.stack([rng.integers(0, 4, k), 4 + np.arange(k)], 1),
+                        np.stack([4 + rng.integers(0, k, n - 4 - k), np.arange(4 + k, n)], 1),
+                        np.stack([np.arange(3), np.arange(1, 4)], 1)])
+    ref = O.build_csr(rng.permutation(n)[e])
+    g = g5.Graph.upload(ref.rowptr, ref.cols, ref.n_rows, gdeg=ref.gdeg)
+    m = g5.MSBFS(g)
+    m.set_mode(2)
+    roots = [int(r) for r in rng.choice(n, 64, replace=False)]
+    for _ in range(2):
+        m.run(roots)
+        for lane in range(0, 64, 7):
+            pred, lev = m.result(lane)
+            opred, olev, _ = O.bfs_bin(ref, roots[lane])
+            assert np.array_equal(pred, opred) and np.array_equal(lev, olev)
