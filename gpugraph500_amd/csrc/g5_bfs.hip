@@ -1356,6 +1356,11 @@ extern "C" int g5_bfs_set_out_bitmap(g5_bfs *b, const uint64_t *d_bits)
 {
     G5_REQUIRE(b, G5_E_ARG, "g5_bfs_set_out_bitmap: null handle");
     G5_REQUIRE(b->depth >= 0, G5_E_STATE, "g5_bfs_set_out_bitmap: g5_bfs_start not called");
+    // bits in this GPU's memory are read where they lie
+    if (d_bits && b->wc && d_bits != b->d_out && !g5::in_memory_of(b->g->device, d_bits, b->wc)) {
+        G5_HIP(hipMemcpyAsync(b->d_out, d_bits, (size_t)b->wc * 8, hipMemcpyDefault, b->s));
+        d_bits = b->d_out;
+    }
     G5_HIP(commit_out(b, d_bits && b->wc ? d_bits : b->d_out));
     G5_HIP(hipStreamSynchronize(b->s));
     return G5_OK;
@@ -1367,8 +1372,12 @@ extern "C" int g5_bfs_set_in_bitmap(g5_bfs *b, const uint64_t *d_bits)
     G5_REQUIRE(b->depth >= 0, G5_E_STATE, "g5_bfs_set_in_bitmap: g5_bfs_start not called");
     if (!b->d_inbits) G5_HIP(hipMalloc(&b->d_inbits, (size_t)(b->wr ? b->wr : 1) * 8));
     // the queue is made by an expansion that runs top-down, which needs it
-    hipLaunchKernelGGL(k_copy_words, g5::grid_for(b->wr, 256, 4096), 256, 0, b->s, d_bits, b->d_inbits, b->wr);
-    G5_HIP(hipGetLastError());
+    if (g5::in_memory_of(b->g->device, d_bits, b->wr)) {
+        hipLaunchKernelGGL(k_copy_words, g5::grid_for(b->wr, 256, 4096), 256, 0, b->s, d_bits, b->d_inbits, b->wr);
+        G5_HIP(hipGetLastError());
+    } else if (b->wr) {
+        G5_HIP(hipMemcpyAsync(b->d_inbits, d_bits, (size_t)b->wr * 8, hipMemcpyDefault, b->s));
+    }
     G5_HIP(hipStreamSynchronize(b->s));
     b->queue_ok = b->qoff_ok = false;
     b->inbits_valid = true;

@@ -107,6 +107,11 @@ hipError_t fill_u32(uint32_t *d, int64_t n, uint32_t v, hipStream_t s);
 hipError_t fill_i32(int32_t *d, int64_t n, int32_t v, hipStream_t s);
 hipError_t fill_i64(int64_t *d, int64_t n, int64_t v, hipStream_t s);
 int grid_for(int64_t n, int block, int max_grid = 1 << 20);
+// whether p is the start of n aligned words in one allocation of the GPU
+// `device`, which its kernels may read in place.  Anything else is for a copy:
+// it reaches another GPU's and the host's memory, and refuses a range that
+// passes an allocation's end.
+bool in_memory_of(int device, const uint64_t *p, int64_t n);
 // Once per device, with that device current: the device's address of the
 // static scratch of g5_s4_roundtrip_noalloc (g5_noalloc.hip).
 int noalloc_setup(int device);

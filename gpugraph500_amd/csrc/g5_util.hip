@@ -21,6 +21,7 @@ void set_error(const char *fmt, ...)
 int fail_hip(hipError_t e, const char *what, const char *file, int line)
 {
     set_error("%s failed: %s (%s:%d)", what, hipGetErrorString(e), file, line);
+    (void)hipGetLastError();  // reported here, not by the next call's look after a launch
     return e == hipErrorOutOfMemory ? G5_E_NOMEM : G5_E_HIP;
 }
 
@@ -191,6 +192,20 @@ __global__ __launch_bounds__(1024) void k_fold(const int64_t *__restrict__ part,
             if (out.dev[j]) *out.dev[j] = t;
         }
     }
+}
+
+bool in_memory_of(int device, const uint64_t *p, int64_t n)
+{
+    hipPointerAttribute_t a{};
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess || a.type != hipMemoryTypeDevice || a.device != device ||
+        hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)p) != hipSuccess) {
+        (void)hipGetLastError();  // memory that the runtime does not know is no error here
+        return false;
+    }
+    const size_t at = (size_t)((const char *)p - (const char *)base);
+    return ((uintptr_t)p & 7) == 0 && at <= size && (size_t)n * 8 <= size - at;
 }
 
 hipError_t fold_parts(const int64_t *part, int64_t stride, int n, const FoldOut &out, hipStream_t s)

@@ -46,7 +46,7 @@ struct g5_validator {
     const g5_graph *g = nullptr;
     hipStream_t s = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    int64_t *d_pred = nullptr;       // a host map's copy
+    int64_t *d_pred = nullptr;       // the copy of a map that lies elsewhere
     const int64_t *pred = nullptr;   // the map being validated
     uint64_t *d_j[2] = {nullptr, nullptr};
     uint16_t *d_d16 = nullptr;
@@ -501,9 +501,12 @@ int validate(g5_validator *v, int64_t root, int64_t nglob, const int64_t *pred, 
         if (ms) *ms = 0.f;
         return G5_OK;
     }
-    // a device map is read where it lies
-    if (!pred_on_device) G5_HIP(hipMemcpyAsync(v->d_pred, pred, (size_t)n * 8, hipMemcpyHostToDevice, s));
-    v->pred = pred_on_device ? pred : v->d_pred;
+    // a map in this GPU's memory is read where it lies
+    const bool here = pred_on_device && g5::in_memory_of(g->device, (const uint64_t *)pred, n);
+    if (!here)
+        G5_HIP(hipMemcpyAsync(v->d_pred, pred, (size_t)n * 8,
+                              pred_on_device ? hipMemcpyDefault : hipMemcpyHostToDevice, s));
+    v->pred = here ? pred : v->d_pred;
     G5_HIP(g5::fill_u64((uint64_t *)v->d_acc, kNAcc, 0, s));
     const int grid = g5::grid_for(n, 256, kVertGrid);
     hipLaunchKernelGGL(k_val_walk, grid, 256, 0, s, v->pred, n, root, nglob, (const uint32_t *)g->d_gdeg, v->d_d4,
