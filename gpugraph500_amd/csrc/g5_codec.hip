@@ -642,8 +642,9 @@ __device__ int64_t dec_tail_wave(const uint8_t *bi, int64_t nb, int64_t cap, uin
 }
 
 // The end of a decode, one wave: the tail's values and the record, to
-// device memory and, when given, the host's.  flag (round trip; may be null)
-// is set to 1 unless the stream held exactly n_expect values.
+// device memory and, when given, the host's.  n_expect (round trip; else < 0):
+// the record's flag slot, or flag when given (never a slot of the record), is
+// set to 1 unless the stream held exactly that many values.
 __device__ void dec_finish(const uint8_t *stream, int64_t nwords, int64_t err, int64_t L,
                            int64_t tailpos, int64_t cap, uint32_t *__restrict__ out, int64_t n_expect,
                            int64_t *__restrict__ flag, int64_t *__restrict__ meta, int64_t *__restrict__ host, int l)
@@ -657,8 +658,9 @@ __device__ void dec_finish(const uint8_t *stream, int64_t nwords, int64_t err, i
         }
     }
     if (l == 0) {
-        const int64_t lost = flag && (err || L + n != n_expect);
-        if (lost) *flag = 1;
+        const int64_t lost = n_expect >= 0 && (err || L + n != n_expect);
+        if (lost && flag) *flag = 1;
+        meta[kMetaFlag] = lost;
         meta[kMetaErr] = err;
         meta[kMetaTail] = n;
         meta[kMetaNw] = nwords;
@@ -935,7 +937,7 @@ __global__ __launch_bounds__(kTileThreads) void k_dec_small(const uint32_t *__re
                                                             int64_t *__restrict__ meta, int64_t *__restrict__ host)
 {
     __shared__ DecSmall s;
-    dec_small(in, nwords, cap, out, 0, nullptr, meta, host, s);
+    dec_small(in, nwords, cap, out, -1, nullptr, meta, host, s);
 }
 
 // encode, then decode from the words the encode wrote to memory, as a
@@ -947,7 +949,6 @@ __global__ __launch_bounds__(kTileThreads) void k_rt_small(const uint32_t *in, i
 {
     __shared__ EncSmall se;
     __shared__ DecSmall sd;
-    if (threadIdx.x < kMetaSlots) meta[threadIdx.x] = 0;
     const int64_t nw = enc_small(in, n, words, se);
     if (threadIdx.x == 0) *nw_out = nw;
     __threadfence();  // the words are read back below, by other waves
@@ -1138,7 +1139,7 @@ int S4Codec::decode(const uint32_t *d_in, size_t nwords, uint32_t *d_out, size_t
         }
     }
     if (!small) {
-        rc = decode_launch(d_in, nullptr, (int64_t)nwords, (int64_t)nwords, (int64_t)cap_values, d_out, 0, nullptr,
+        rc = decode_launch(d_in, nullptr, (int64_t)nwords, (int64_t)nwords, (int64_t)cap_values, d_out, -1, nullptr,
                            h_meta, s);
         if (rc) return rc;
         if (acct) G5_HIP(acct->stop());
@@ -1160,18 +1161,18 @@ int S4Codec::roundtrip(const uint32_t *d_in, int64_t n, uint32_t *d_words_out, s
                "s4 round trip: word capacity %zu below the bound for %lld values", cap_words, (long long)n);
     int rc = reserve(n);
     if (rc) return rc;
-    int64_t *flag = d_flag ? d_flag : d_meta + kMetaFlag;
     // the record goes home when it is asked for (a borrowed layout has no pinned memory)
     int64_t *host = owned && !d_flag ? h_meta : nullptr;
     if (n <= kSmallValues) {
-        hipLaunchKernelGGL(k_rt_small, 1, kTileThreads, 0, s, d_in, n, d_words_out, d_nw, d_out, d_meta, flag, host);
+        hipLaunchKernelGGL(k_rt_small, 1, kTileThreads, 0, s, d_in, n, d_words_out, d_nw, d_out, d_meta, d_flag,
+                           host);
         G5_HIP(hipGetLastError());
         return G5_OK;
     }
     rc = encode_launch(d_in, n, d_words_out, nullptr, s);
     if (rc) return rc;
     // the stream's length stays on the device; sizes the host needs follow from n
-    return decode_launch(d_words_out, d_nw, 0, (int64_t)g5_s4_max_words((size_t)n), n, d_out, n, flag, host, s);
+    return decode_launch(d_words_out, d_nw, 0, (int64_t)g5_s4_max_words((size_t)n), n, d_out, n, d_flag, host, s);
 }
 
 int S4Codec::roundtrip_result(size_t *nwords, const char *who)
@@ -1229,7 +1230,7 @@ extern "C" int g5_s4_roundtrip(const uint32_t *d_in, size_t n, uint32_t *d_words
     g5::S4Codec &c = abi_codec();
     int rc = c.reserve((int64_t)n);
     if (rc) return rc;
-    // the flag lives in the decoder's record, which the header search clears
+    // the flag lives in the decoder's record, which the decode writes
     rc = c.roundtrip(d_in, (int64_t)n, d_words, cap_words, d_out, nullptr, nullptr);
     if (rc) return rc;
     return c.roundtrip_result(nwords, "g5_s4_roundtrip");

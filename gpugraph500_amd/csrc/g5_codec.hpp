@@ -44,7 +44,7 @@ struct S4Codec {
     // d_in), with no host synchronisation: *d_flag (device) is set to 1 if
     // the round trip did not give back exactly n values, and left alone
     // otherwise (d_flag null: the flag slot of the decoder's record, which
-    // the round trip clears first).
+    // every round trip writes, holds the answer alone).
     int roundtrip(const uint32_t *d_in, int64_t n, uint32_t *d_words_out, size_t cap_words, uint32_t *d_out,
                   int64_t *d_flag, hipStream_t s);
     // After a roundtrip with d_flag null, on the null stream: waits for it,

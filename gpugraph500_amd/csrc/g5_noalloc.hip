@@ -11,9 +11,9 @@
 // with that device current (g5_init, or the entry point's first call on a
 // device), and only that address is used.  Every call on one GPU shares the
 // array: calls that overlap on one GPU race.  Nothing in the array must
-// start at zero: the header search clears the decoder's record (and its
-// error and lost-values flag) before anything reads it, as in the allocating
-// round trip, whose scratch is also reused from call to call.
+// start at zero: a decode writes its record (with its error and lost-values
+// flag) before anything reads it, as in the allocating round trip, whose
+// scratch is also reused from call to call.
 #include <mutex>
 
 #include "g5_codec.hpp"
