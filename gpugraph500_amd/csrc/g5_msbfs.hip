@@ -132,6 +132,24 @@ constexpr unsigned kFuseWaveGroups = 768;
 // 340 thousand of them, 0.752 -> 0.757, 20 with edgefactor 8 0.87 -> 0.91; 8 a
 // step: 0.97-1.00 times that up to scale 16, 1.03-1.1 at 17 and 18).
 constexpr int64_t kPartMax = (int64_t)1 << 18;
+// A thread keeps kHits hits and stores the rest one by one, scattered; rows that
+// meet many words of few lanes each have more.  So the thread bin is bounded as
+// on split levels where it takes more than kHits of the frontier's words to hold
+// all its lanes (the mean word times Relabeled::skew, as rows meet the words of
+// vertices with many neighbours more often) and the level, if the search grows
+// on as it did, finds more than kHits pairs per vertex.  That comes up on graphs
+// without hubs: a level where every row of 100 neighbours meets words of 1.3
+// lanes takes 1.26 ms instead of 2.77 (a million vertices), one of 40 and 3.7
+// lanes 0.77 instead of 1.82; with 64 and 13.7 lanes the thread bin is the faster
+// one (0.75, 0.81).  Searches of 64 roots with all rows of d neighbours, at 32 / at
+// 256 / by this rule: 2^20 vertices, d = 40 2.28 / 2.89 / 1.87 ms, 100 2.15 / 3.22
+// / 1.73; 2^19, 200 0.93 / 1.55 / 0.88; degrees 32 to 400 at 2^20 2.38 / 3.56 / 2.08.
+// Without the second condition a ring of near neighbours (half a pair per
+// vertex and level) takes 69 ms instead of 55.  Below kSparseVerts vertices the
+// records stay in the caches (2^17, 40: 0.31, by the rule 0.37).  Kronecker
+// graphs of that size have a skew of 20 and more and never get here.
+constexpr int64_t kSparseVerts = (int64_t)1 << 18;
+constexpr int64_t kSparseThreadMax = 32;
 constexpr int64_t kLeastWaveMax = 32;  // of a search whose thread_max was not set
 struct Tune {
     int64_t thread_max = 32;   // degree bound of the thread-per-vertex bin
@@ -143,8 +161,8 @@ struct Tune {
                                // frontier's edges < nnz / active_ratio
     int64_t lane_ratio = 128;  // a pull level pushes the lanes whose frontier
                                // edges < nnz / lane_ratio (0: never)
-    int64_t split_max = 16;    // split levels bound the thread bin at
-                               // min(split_max, thread_max)
+    int64_t split_max = 16;    // split levels, and those of kSparseVerts, bound the
+                               // thread bin at min(split_max, thread_max)
 };
 
 // Level counters.  Per accounting unit u (the kBins pull bins, then
@@ -194,7 +212,8 @@ struct Relabeled {
     uint64_t *head_orig = nullptr;
     uint32_t *gdeg = nullptr;
     int64_t bin_first[kBins + 1] = {0};  // bin b holds new ids [bin_first[b], bin_first[b+1])
-    int64_t split_first[kBins + 1] = {0};  // the same on split levels (min(split_max, thread_max))
+    int64_t split_first[kBins + 1] = {0};  // the same on split levels and of sparse words
+    double skew = 1;  // mean degree of a row's neighbours over the rows' own (1: all rows alike)
 };
 
 // the total of a part of a push queue, in a line of its own.  Unless the level
@@ -243,6 +262,7 @@ struct g5_msbfs {
     // frontier's active vertices / edges (edges < 0: unknown, take push)
     int p = 0;
     int64_t act_verts = 0, act_edges = -1;
+    int64_t act_pairs = 0, last_pairs = 0;  // its (vertex, root) pairs, and those of the frontier before
     // the lanes with a non-empty frontier, and the lanes whose frontier edges
     // for the frontier the next level reads lane_edges holds (every lane
     // after a push level, which counts them from its new-vertex queue; the
@@ -1733,18 +1753,21 @@ __global__ void k_degree_keys(const int64_t *__restrict__ rowptr, int64_t n, uin
     }
 }
 
-// vertices with degree > wave_max, in (thread_max, wave_max], in (0, thread_max]
+// vertices with degree > wave_max, in (thread_max, wave_max], in (0, thread_max],
+// and the sum of the degrees' squares (a degree counts 2^20 at most)
 __global__ void k_bin_counts(const int64_t *__restrict__ rowptr, int64_t n, int64_t thread_max, int64_t wave_max,
                              unsigned long long *__restrict__ bins)
 {
-    unsigned long long c[kBins] = {0, 0, 0};
+    unsigned long long c[kBins + 1] = {0, 0, 0, 0};
     for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < n; v += (int64_t)gridDim.x * blockDim.x) {
         const int64_t d = rowptr[v + 1] - rowptr[v];
         if (d > wave_max) ++c[0];
         else if (d > thread_max) ++c[1];
         else if (d > 0) ++c[2];
+        const unsigned long long x = (unsigned long long)min(d, (int64_t)1 << 20);
+        c[kBins] += x * x;
     }
-    for (int k = 0; k < kBins; ++k) {
+    for (int k = 0; k <= kBins; ++k) {
         const unsigned long long t = (unsigned long long)g5_block_sum256((int64_t)c[k]);
         if (threadIdx.x == 0 && t) atomicAdd(&bins[k], t);
     }
@@ -2193,16 +2216,16 @@ PushQueue push_queue(const g5_msbfs *m, int i)
     return PushQueue{m->d_qv[i], m->d_qo[i], m->d_qt + i * kGroups, queue_units(m->n / 64)};
 }
 
-// One pull level of parity p.
-int pull_level(g5_msbfs *m, hipStream_t s, int p, const PullLanes &lanes, bool act_check, bool prof)
+// One pull level of parity p on the bins bf.
+int pull_level(g5_msbfs *m, hipStream_t s, int p, const PullLanes &lanes, bool act_check, bool prof, const int64_t *bf)
 {
     uint64_t *next = p == 0 ? m->d_fb : m->d_fa;
     const int64_t nw = m->n / 64;
     uint64_t *act_next = m->d_act + (p == 0 ? nw : 0);
-    pull_bins(m, s, p, lanes, act_check, prof, m->rl.bin_first);
+    pull_bins(m, s, p, lanes, act_check, prof, bf);
     // the thread kernel wrote its words of the active bitmap; the block and
     // wave bins' words (and the live lanes among them) come from next
-    const int64_t nw01 = (m->rl.bin_first[2] + 63) / 64;
+    const int64_t nw01 = (bf[2] + 63) / 64;
     if (nw01)
         hipLaunchKernelGGL((k_build_active<false, true>), g5::grid_for(nw01, 16, 4096), kBlock, 0, s,
                            (const uint64_t *)next, nw01, (const int64_t *)m->rl.rowptr, act_next, m->d_cnt, ~0ull);
@@ -2403,12 +2426,12 @@ int bins_for(g5_msbfs *m, int64_t thread_max, int64_t *bf)
     const Relabeled &R = m->rl;
     unsigned long long *d = (unsigned long long *)m->d_sums;  // transient scratch, free between calls
     m->sums_clear = false;
-    unsigned long long hb[kBins] = {0, 0, 0};
-    G5_HIP(g5::fill_u64((uint64_t *)d, kBins, 0, s));
+    unsigned long long hb[kBins + 1] = {0, 0, 0, 0};
+    G5_HIP(g5::fill_u64((uint64_t *)d, kBins + 1, 0, s));
     hipLaunchKernelGGL(k_bin_counts, g5::grid_for(m->n, 256, 16384), 256, 0, s, (const int64_t *)R.rowptr, m->n,
                        thread_max, m->tune.wave_max, d);
     G5_HIP(hipGetLastError());
-    G5_HIP(hipMemcpyAsync(hb, d, kBins * 8, hipMemcpyDeviceToHost, s));
+    G5_HIP(hipMemcpyAsync(hb, d, (kBins + 1) * 8, hipMemcpyDeviceToHost, s));
     G5_HIP(hipStreamSynchronize(s));
     bf[0] = 0;
     for (int k = 0; k < kBins; ++k) bf[k + 1] = bf[k] + (int64_t)hb[k];
@@ -2417,6 +2440,8 @@ int bins_for(g5_msbfs *m, int64_t thread_max, int64_t *bf)
     // round up, moving at most 63 vertices each into the bin before (any bin
     // gives the same results)
     const int64_t end = bf[kBins];
+    const double nnz = (double)m->g->nnz;
+    m->rl.skew = nnz > 0 ? std::max(1.0, (double)hb[kBins] * (double)end / (nnz * nnz)) : 1.0;
     for (int k = 1; k < kBins; ++k) bf[k] = std::min(end, std::max(bf[k - 1], (bf[k] + 63) / 64 * 64));
     return G5_OK;
 }
@@ -2467,6 +2492,15 @@ uint64_t split_lanes(const g5_msbfs *m, int64_t &pe)
     return pm == m->front_lanes ? 0 : pm;
 }
 
+// whether the rows of a pull level meet many words of few lanes (kSparseVerts)
+bool sparse_words(const g5_msbfs *m)
+{
+    const double pairs = (double)m->act_pairs;
+    return m->tune.thread_max > kSparseThreadMax && m->n >= kSparseVerts &&
+           (double)__builtin_popcountll(m->front_lanes) * (double)m->act_verts > kHits * pairs * m->rl.skew &&
+           pairs * pairs > (double)kHits * (double)m->rl.bin_first[kBins] * (double)m->last_pairs;
+}
+
 // Sums of up to 128 values over a kernel's workgroups: d_sums clear, then
 // (after the kernel's launch) to pinned memory, waited for.
 hipError_t begin_sums(g5_msbfs *m)
@@ -2503,6 +2537,7 @@ int run_level(g5_msbfs *m, int64_t *new_bits_out, uint64_t *live_out, hipEvent_t
     const bool act_check = act_edges < 0 || act_edges * m->tune.active_ratio < nnz;
     int64_t pe = 0;  // of the pushed lanes
     const uint64_t pm = push ? 0 : split_lanes(m, pe);
+    const int64_t *bf = pm || sparse_words(m) ? m->rl.split_first : m->rl.bin_first;  // a pull level's bins
     if (push) {
         int rc = push_level(m, s, p, listed_in, queue_in, m->prof);
         if (rc) return rc;
@@ -2510,7 +2545,7 @@ int run_level(g5_msbfs *m, int64_t *new_bits_out, uint64_t *live_out, hipEvent_t
         const PullLanes lanes{m->front_lanes & ~pm, m->front_lanes, used_lanes(m), m->flag_word,
                               pm ? (int64_t)64 : (int64_t)kWaveFirst};
         int rc = pm ? split_level(m, s, p, pm, pe, lanes, act_check, m->prof)
-                    : pull_level(m, s, p, lanes, act_check, m->prof);
+                    : pull_level(m, s, p, lanes, act_check, m->prof, bf);
         if (rc) return rc;
     }
     if (end) G5_HIP(hipEventRecord(end, s));
@@ -2566,7 +2601,6 @@ int run_level(g5_msbfs *m, int64_t *new_bits_out, uint64_t *live_out, hipEvent_t
             // pair; per newly reached vertex its original id and at least
             // one parent's (4 + 4 B)
             for (int k = 0; k < kBins; ++k) {
-                const int64_t *bf = pm ? m->rl.split_first : m->rl.bin_first;
                 if (bf[k + 1] == bf[k]) continue;
                 float kms = 0;
                 G5_HIP(hipEventElapsedTime(&kms, m->ek[k], m->ek[k + 1]));
@@ -2587,11 +2621,12 @@ int run_level(g5_msbfs *m, int64_t *new_bits_out, uint64_t *live_out, hipEvent_t
     m->front_lanes = (uint64_t)h[kLive];
     m->act_verts = next_verts;
     m->act_edges = next_edges;
+    m->last_pairs = m->act_pairs;
+    m->act_pairs = new_bits;
     m->p ^= 1;
     // the level flags this level's thread kernel wrote (none: a push level,
     // or an empty thread bin)
-    const int64_t *tf = pm ? m->rl.split_first : m->rl.bin_first;
-    m->flag_word = push || tf[2] == tf[3] ? INT64_MAX : tf[2] / 64;
+    m->flag_word = push || bf[2] == bf[3] ? INT64_MAX : bf[2] / 64;
     return G5_OK;
 }
 
@@ -2767,6 +2802,7 @@ extern "C" int g5_msbfs_run(g5_msbfs *m, const int64_t *roots, int nroots, int32
     m->p = 0;
     m->flag_word = INT64_MAX;
     m->act_edges = -1;
+    m->act_pairs = m->last_pairs = nroots;
     m->front_lanes = nroots == 64 ? ~0ull : (1ull << nroots) - 1;
     m->lane_known = 0;
     m->split_levels = 0;
@@ -2826,6 +2862,7 @@ extern "C" int g5_msbfs_open(g5_msbfs *m)
     m->flag_word = INT64_MAX;
     m->act_verts = 0;
     m->act_edges = 0;
+    m->act_pairs = m->last_pairs = 0;
     m->front_lanes = 0;
     m->listed_ok = true;  // k_ms_init cleared both frontier buffers
     m->listed_len = 0;
@@ -2878,7 +2915,10 @@ extern "C" int g5_msbfs_join(g5_msbfs *m, const int64_t *roots, const int *lanes
         m->lane_edges[lanes[i]] = added[2 + i];
         m->lane_known |= 1ull << lanes[i];
         m->last_empty = false;  // the roots sit in the buffer the next level reads
-        if (added[2 + i]) m->front_lanes |= 1ull << lanes[i];
+        if (added[2 + i]) {
+            m->front_lanes |= 1ull << lanes[i];
+            ++m->act_pairs;
+        }
     }
     m->split_ok = true;
     m->queue_ok = false;  // the roots are not in it

@@ -305,7 +305,8 @@ int g5_msbfs_info(g5_msbfs *m, int64_t *bins, int cap);
  * stops one lagging root from making every vertex scan its whole list;
  * G5_TUNE_SPLIT_MAX: such split levels bound the thread-per-vertex bin at
  * min(split_max, thread_max) (32, or 16 on graphs of fewer than 2^20
- * stored neighbours), as every row is scanned to its end there.
+ * stored neighbours), as every row is scanned to its end there; so do levels of
+ * graphs without hubs whose rows meet many frontier words of few lanes each.
  * g5_msbfs_autotune searches these by coordinate descent over candidate
  * values (passes rounds, two timed batch searches of roots per candidate),
  * keeps the fastest and reports its time and the number of candidates run. */
