@@ -121,10 +121,18 @@ constexpr int64_t kFuseNnz = (int64_t)1 << 24;
 // There the wave bin's workgroups take several vertices a wave, three of them
 // per CU: one vertex a wave, they fill the card several times over before the
 // thread bin's start, and end in a counter update each (scale 16 0.362 -> 0.337
-// ms, 17 0.407 -> 0.381, 18 0.468 -> 0.446; 256 of them 0.366 / 0.412 / 0.484,
+// ms, 17 0.407 -> 0.381, 18 0.468 -> 0.446, 19 0.70 -> 0.61, edgefactor 8 at 20 0.91 ->
+// 0.83, 4 at 21 1.06 -> 0.97; 256 of them 0.366 / 0.412 / 0.484,
 // 512 0.346 / 0.373 / 0.445, the same up to scale 14; on larger graphs, where
 // the bins are launched apart, 768 take 1.02 to 1.15 times as long as all).
 constexpr unsigned kFuseWaveGroups = 768;
+// The bins share a launch for the thread bin's sake.  From kFuseWaveNnz stored
+// neighbours on, a wave bin of more vertices than the thread bin is the level,
+// and loses by it: with a thread_max of 32 a ring of near neighbours (2^17 rows
+// of 100) takes 1.91 ms in one launch and 1.45 in three, all rows of 40 at 2^18
+// 0.84 and 0.66, of 100 at 2^17 0.42 and 0.40.  Below: 2^16 rows of 100 0.38 and
+// 0.42, near ones of 40 1.16 and 1.70.
+constexpr int64_t kFuseWaveNnz = (int64_t)1 << 23;
 // With fewer than kPartMax vertices in the thread bin its waves take 16 of them
 // a step instead of 64: four times the waves, of which there is one per SIMD or
 // less otherwise, each with a quarter of the records to write one after the
@@ -2189,7 +2197,7 @@ void pull_bins(g5_msbfs *m, hipStream_t s, int p, const PullLanes &lanes, bool a
                       : k == 1 ? (unsigned)g5::grid_for(b.n[k], kBlock / 64, 16384)
                                : (unsigned)g5::grid_for(b.n[k], kBlock, 16384);
     }
-    if (!prof && m->g->nnz < kFuseNnz) {
+    if (!prof && m->g->nnz < (b.n[1] > b.n[2] ? kFuseWaveNnz : kFuseNnz)) {
         const bool part = b.n[2] < kPartMax;
         if (part && b.n[2]) b.groups[2] = (unsigned)g5::grid_for(b.n[2], kBlock / 4, 16384);
         b.groups[1] = std::min(b.groups[1], kFuseWaveGroups);

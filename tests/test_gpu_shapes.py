@@ -74,3 +74,21 @@ def test_words_of_few_lanes(make, n, d, lanes, some):
     while m.step()[0]:
         pass
     same_maps(m, push, range(0, lanes, 9))
+
+
+@pytest.mark.parametrize("n,d", [(1 << 17, 56), (1 << 17, 72), (1 << 16, 130), ((1 << 17) + 128, 64)])
+def test_wave_bins_of_most_vertices(n, d):
+    """Below and beyond 2^23 stored neighbours: in a launch with the other bins,
+    and in one of their own."""
+    g, deg = regular(n, d, n + d)
+    m, push = g5.MSBFS(g), g5.MSBFS(g)
+    m.tune(thread_max=32, split_max=16)
+    assert m.bins()[1] > m.bins()[2] and g.nnz < 1 << 24
+    push.set_mode(2)
+    roots = np.random.default_rng(n).choice(n, 50, replace=False)
+    push.run(roots)
+    for mode in (1, 0, 0):
+        m.set_mode(mode)
+        m.run(roots)
+        same_maps(m, push, range(0, 50, 7))
+        assert m.nedge().tolist() == push.nedge().tolist()
