@@ -92,3 +92,28 @@ def test_wave_bins_of_most_vertices(n, d):
         m.run(roots)
         same_maps(m, push, range(0, 50, 7))
         assert m.nedge().tolist() == push.nedge().tolist()
+
+
+@pytest.mark.parametrize("n,left,whole", [(1 << 18, 1, False), (1 << 18, 0, True), ((1 << 18) + 64, 21, True),
+                                          ((1 << 18) + 1024, 21, True), (1 << 19, 5, True)])
+def test_thread_bin_in_whole_words(n, left, whole):
+    """Thread bins of 2^18 vertices and more in a launch with the other bins, the
+    last word full or not; `left` ids have no edge."""
+    rng = np.random.default_rng(n + left)
+    v = rng.permutation(n)[left:]
+    far = rng.integers(0, len(v), (2, n // 3))
+    # some rows for the other bins, which end at a multiple of 64
+    hubs = v[rng.integers(0, 40, 20000 if n > (1 << 18) + 64 else 0)]
+    g, deg = upload(np.concatenate([v, v[far[0]], hubs]),
+                    np.concatenate([np.roll(v, 1), v[far[1]], v[rng.integers(0, len(v), len(hubs))]]), n)
+    m, push = g5.MSBFS(g), g5.MSBFS(g)
+    m.tune(wave_max=400)
+    assert (m.bins()[2] >= 1 << 18) == whole
+    push.set_mode(2)
+    roots = [int(v[i]) for i in rng.integers(0, len(v), 40)]
+    push.run(roots)
+    for mode in (1, 0, 1):
+        m.set_mode(mode)
+        m.run(roots)
+        same_maps(m, push, range(0, 40, 6))
+        assert m.nedge().tolist() == push.nedge().tolist()
