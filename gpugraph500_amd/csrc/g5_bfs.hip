@@ -1487,8 +1487,11 @@ extern "C" int g5_bfs_run(g5_bfs *b, int64_t root, int flags, int32_t *nlevels, 
     G5_HIP(hipEventRecord(b->ev0, s));
     // k_level decides the levels on the device; the codec's launches, the
     // accounting and a forced direction need the host's view of each level,
-    // and a packed total holds 2^30 vertices and 2^34 edges
-    if (!codec && !topdown_only && !b->prof && g->n_rows <= (int64_t)1 << 30 && g->nnz < (int64_t)1 << kEdgeBits) {
+    // a packed total holds 2^30 vertices and 2^34 edges, and a root outside the
+    // block (one that does not start at vertex 0) has no row to start from
+    const bool here = root >= g->row_start && root - g->row_start < g->n_rows;
+    if (!codec && !topdown_only && !b->prof && here && g->n_rows <= (int64_t)1 << 30 &&
+        g->nnz < (int64_t)1 << kEdgeBits) {
         rc = run_levels(b, root);
         if (rc) return rc;
         if (ms) G5_HIP(hipEventElapsedTime(ms, b->ev0, b->ev1));
