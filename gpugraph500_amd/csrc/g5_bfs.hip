@@ -107,8 +107,10 @@ struct g5_bfs {
     uint64_t *d_inbits = nullptr;
     bool inbits_valid = false;
     // g5_bfs_run's levels on the device (k_level): a third frontier bitmap,
-    // the two levels' queues and their
-    // prefixes (kGroups times gcap entries each) and the control record
+    // the two levels' queues and their prefixes (kGroups times gcap entries
+    // each) and the control record.  6 bytes a vertex: allocated with the handle
+    // of a whole graph, at the first g5_bfs_run of a grid's block, whose hooks
+    // do without (level_buffers)
     uint64_t *d_third = nullptr;
     uint32_t *d_gq[2] = {nullptr, nullptr};
     int64_t *d_goff[2] = {nullptr, nullptr};
@@ -1085,6 +1087,34 @@ __global__ __launch_bounds__(kLvBlock) void k_level(LevelArgs a, int d, const in
         level_bottom_up(a, d, rowptr, cols, front, visited, next, third, parent, level, s_late, s_mem);
 }
 
+// The buffers of k_level's levels; false if the memory is not there (the host
+// drives the levels then).
+bool level_buffers(g5_bfs *b)
+{
+    if (b->d_ctl) return true;
+    // twice n / 8 vertices spread evenly: a level that finds more runs on
+    // bottom-up
+    b->gcap = std::max<int64_t>(kMinQueue, b->g->n_rows / 4 / kGroups);
+    hipError_t e = hipMalloc(&b->d_third, (size_t)std::max<int64_t>(b->wc, 1) * 8);
+    for (int k = 0; k < 2; ++k) {
+        if (e == hipSuccess) e = hipMalloc(&b->d_gq[k], (size_t)(kGroups * b->gcap) * 4);
+        if (e == hipSuccess) e = hipMalloc(&b->d_goff[k], (size_t)(kGroups * b->gcap) * 8);
+    }
+    if (e == hipSuccess) e = hipMalloc(&b->d_ctl, sizeof(LevelCtl));
+    if (e == hipSuccess) return true;
+    (void)hipGetLastError();
+    auto drop = [](auto *&p) {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+    };
+    drop(b->d_third);
+    for (int k = 0; k < 2; ++k) {
+        drop(b->d_gq[k]);
+        drop(b->d_goff[k]);
+    }
+    return false;
+}
+
 // The whole search with k_level; levels are launched in batches.
 int run_levels(g5_bfs *b, int64_t root)
 {
@@ -1176,22 +1206,12 @@ extern "C" int g5_bfs_create(g5_graph *g, g5_bfs **out)
     if (e == hipSuccess) e = hipMalloc(&b->d_part, 4 * kParts * 8);
     static_assert(kParts >= 2 * g5::kTiles && kParts >= kSumGrid, "a sum per workgroup and tile");
     if (e == hipSuccess) e = hipHostMalloc(&b->h_cnt, (kNCnt + 1) * 8, hipHostMallocDefault);  // k_level's end last
-    if (g->n_rows == g->n_cols && g->row_start == g->col_start) {  // g5_bfs_run
-        // twice n / 8 vertices spread evenly: a level that finds more runs on
-        // bottom-up
-        b->gcap = std::max<int64_t>(kMinQueue, nmax / 4 / kGroups);
-        if (e == hipSuccess) e = hipMalloc(&b->d_third, (size_t)std::max<int64_t>(b->wc, 1) * 8);
-        for (int k = 0; k < 2; ++k) {
-            if (e == hipSuccess) e = hipMalloc(&b->d_gq[k], (size_t)(kGroups * b->gcap) * 4);
-            if (e == hipSuccess) e = hipMalloc(&b->d_goff[k], (size_t)(kGroups * b->gcap) * 8);
-        }
-        if (e == hipSuccess) e = hipMalloc(&b->d_ctl, sizeof(LevelCtl));
-    }
     if (e == hipSuccess) e = hipEventCreate(&b->ev0);
     if (e == hipSuccess) e = hipEventCreate(&b->ev1);
     if (e == hipSuccess) e = hipEventCreate(&b->ek0);
     if (e == hipSuccess) e = hipEventCreate(&b->ek1);
     if (e != hipSuccess) return fail(g5::fail_hip(e, "g5_bfs_create allocation", __FILE__, __LINE__));
+    if (g->n_rows == g->n_cols && g->row_start == g->col_start && g->n_rows >= g->nglobal) (void)level_buffers(b);
     *out = b;
     return G5_OK;
 }
@@ -1480,18 +1500,19 @@ extern "C" int g5_bfs_run(g5_bfs *b, int64_t root, int flags, int32_t *nlevels, 
         int rc = b->codec.reserve((int64_t)g->n_cols);
         if (rc) return rc;
     }
-    hipStream_t s = b->s;
-    G5_HIP(hipStreamSynchronize(s));
-    int rc = find_isolated(b);
-    if (rc) return rc;
-    G5_HIP(hipEventRecord(b->ev0, s));
     // k_level decides the levels on the device; the codec's launches, the
     // accounting and a forced direction need the host's view of each level,
     // a packed total holds 2^30 vertices and 2^34 edges, and a root outside the
     // block (one that does not start at vertex 0) has no row to start from
     const bool here = root >= g->row_start && root - g->row_start < g->n_rows;
-    if (!codec && !topdown_only && !b->prof && here && g->n_rows <= (int64_t)1 << 30 &&
-        g->nnz < (int64_t)1 << kEdgeBits) {
+    const bool on_device = !codec && !topdown_only && !b->prof && here && g->n_rows <= (int64_t)1 << 30 &&
+                           g->nnz < (int64_t)1 << kEdgeBits && level_buffers(b);
+    hipStream_t s = b->s;
+    G5_HIP(hipStreamSynchronize(s));
+    int rc = find_isolated(b);
+    if (rc) return rc;
+    G5_HIP(hipEventRecord(b->ev0, s));
+    if (on_device) {
         rc = run_levels(b, root);
         if (rc) return rc;
         if (ms) G5_HIP(hipEventElapsedTime(ms, b->ev0, b->ev1));

@@ -1,5 +1,7 @@
-"""g5_bfs_run on the diagonal blocks of a grid, whose rows need not start at
-vertex 0."""
+"""The single-root engine on a grid's blocks: g5_bfs_run on the diagonal ones,
+whose rows need not start at vertex 0, and the memory that the hooks take."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -38,7 +40,28 @@ def test_root_of_the_first_block(blocks):
     b = blocks[0]
     rowptr = b.download()[0]
     a, h = g5.BFS(b), g5.BFS(b)
+    a.start(0)  # a handle that the hooks have used
+    a.expand()
     for root in np.flatnonzero(np.diff(rowptr))[[0, 5, -1]].tolist():
         assert a.run(root)[0] == h.run(root, topdown=True)[0] > 1
         for x, y in zip(a.result(), h.result()):
             assert np.array_equal(x, y)
+
+
+def free_bytes():
+    free, total = ctypes.c_int64(), ctypes.c_int64()
+    g5.check(g5.lib().g5_mem_info(ctypes.byref(free), ctypes.byref(total)))
+    return free.value
+
+
+def test_diagonal_blocks_take_what_the_others_take():
+    """The buffers of a whole search (6 bytes a vertex, 25 MB an engine here) come
+    with the first one."""
+    took = []
+    for b in g5.Graph.kronecker_2d(23, PARTS, PARTS):
+        before = free_bytes()
+        engines = [g5.BFS(b) for _ in range(4)]
+        took.append(before - free_bytes())
+        for e in engines:
+            e.free()
+    assert max(took[0], took[3]) <= max(took[1], took[2]) + (16 << 20), took
