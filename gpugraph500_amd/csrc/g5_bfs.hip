@@ -1509,9 +1509,9 @@ extern "C" int g5_bfs_run(g5_bfs *b, int64_t root, int flags, int32_t *nlevels, 
                            g->nnz < (int64_t)1 << kEdgeBits && level_buffers(b);
     hipStream_t s = b->s;
     G5_HIP(hipStreamSynchronize(s));
+    G5_HIP(hipEventRecord(b->ev0, s));  // a first search's time holds the look for edgeless vertices
     int rc = find_isolated(b);
     if (rc) return rc;
-    G5_HIP(hipEventRecord(b->ev0, s));
     if (on_device) {
         rc = run_levels(b, root);
         if (rc) return rc;
