@@ -186,6 +186,18 @@ def root_sets(g, scale, n):
     return timed, tune
 
 
+def account_single(b, roots, **how):
+    """Per-kernel totals of one search of every root.  Accounting has the host
+    drive the levels (k_expand, k_bottom_up), which a plain search decides on
+    the device, so no search that is timed runs under it."""
+    b.profile(True)
+    for r in roots.tolist():
+        b.run(r, **how)
+    totals = b.kernel_stats()
+    b.profile(False)
+    return totals
+
+
 def tune_probe(args):
     """Child process (no profiler): the batched search's shapes for this
     graph -- the persisted ones for its scale and degree histogram, or an
@@ -241,7 +253,8 @@ def pmc_probe(args):
 
 def probe(args):
     """Workloads for profiler runs (rocprofv3 before this script):
-    single    the 64 single-root searches (profiled) and the copy calibration kernel
+    single    the 64 single-root searches, once more with accounting, and the copy
+              calibration kernel
     exchange  the c3 and c2 sub-records by themselves
     batched   one profiled and six timed batched searches with the given shapes
               (after the parent records' placement, --place trials)
@@ -254,9 +267,8 @@ def probe(args):
         b = g5.BFS(g)
         for r in roots[:2].tolist():
             b.run(r)
-        b.profile(True)
         ms = [b.run(r)[1] for r in roots.tolist()]
-        out = {"mean_ms": float(np.mean(ms)), "kernels": b.kernel_stats()}
+        out = {"mean_ms": float(np.mean(ms)), "kernels": account_single(b, roots)}
         b.free()
         g.free()
         src = g5.DeviceArray(COPY_WORDS, np.uint64)
@@ -376,7 +388,6 @@ def bench_c4(args, g5, traffic, traffic_info, probe_tuned):
     b = g5.BFS(g)
     for r in roots[:max(args.warmup, 1)].tolist():
         b.run(r)
-    b.profile(True)
     single_ms, nedge = [], []
     val = g5.Validator(g) if args.validate == "on" else None
     d_pred = g5.DeviceArray(g.n_rows, np.int64) if val else None
@@ -390,7 +401,7 @@ def bench_c4(args, g5, traffic, traffic_info, probe_tuned):
             bad, vne, _, vms = val.validate_device(r, d_pred)
             val_fail += int(bad != 0 or vne != nedge[-1])
             val_ms.append(vms)
-    kst1 = b.kernel_stats()
+    kst1 = account_single(b, roots)
     nedge = np.array(nedge, np.float64)
     single_teps = nedge / (np.array(single_ms) / 1e3)
     single_h = hmean(single_teps) / 1e9
@@ -552,6 +563,8 @@ def bench_c4(args, g5, traffic, traffic_info, probe_tuned):
                            "levels_final": bool(levels_final)},
         "single_root_mean_ms": float(np.mean(single_ms)),
         "single_root_kernel": single_kernel,
+        "single_root_kernel_of": "one more search per root with accounting, its levels driven by the host; "
+                                 "single_root_mean_ms is without, the levels decided on the device",
         "roofline": roofline,
         "autotune": tuned,
         "placement": placement,
@@ -702,7 +715,6 @@ def bench_c2(args, g5):
         plain.append(b.nedge())
     for r in roots[:max(args.warmup, 1)].tolist():
         b.run(r, codec=True)
-    b.profile(True)
     step_ms, per_root_ms, nedge = [], None, None
     for i in range(args.warmup + args.steps):
         g5.lib().g5_device_sync()
@@ -721,7 +733,7 @@ def bench_c2(args, g5):
     per_root_ms = np.array(per_root_ms) / args.steps
     teps = nedge / (per_root_ms / 1e3)
     value = hmean(teps) / 1e9
-    kst1 = b.kernel_stats()
+    kst1 = account_single(b, roots, codec=True)
     kname = max(kst1, key=lambda k: kst1[k]["ms"])
     st = kst1[kname]
     gbs = st["bytes"] / (st["ms"] / 1e3) / 1e9 if st["ms"] > 0 else 0.0
@@ -752,7 +764,6 @@ def bench_c1(args, g5):
     b = g5.BFS(g)
     for r in roots[:max(args.warmup, 1)].tolist():
         b.run(r)
-    b.profile(True)
     step_ms, per_root_ms, nedge = [], None, None
     for i in range(args.warmup + args.steps):
         g5.lib().g5_device_sync()
@@ -769,7 +780,7 @@ def bench_c1(args, g5):
         nedge = np.array(ne_r, np.float64)
     per_root_ms = np.array(per_root_ms) / args.steps
     value = hmean(nedge / (per_root_ms / 1e3)) / 1e9
-    kst1 = b.kernel_stats()
+    kst1 = account_single(b, roots)
     kname = max(kst1, key=lambda k: kst1[k]["ms"])
     st = kst1[kname]
     gbs = st["bytes"] / (st["ms"] / 1e3) / 1e9 if st["ms"] > 0 else 0.0

@@ -171,7 +171,8 @@ int g5_bfs_level_device(g5_bfs *b, int32_t *d_level);
  * parents are again the minimum-id frontier vertex of its row range. */
 int g5_bfs_expand_bottom_up(g5_bfs *b, const g5_graph *gt, int *any_new);
 /* The whole 1x1 runBFS (globalbfs.hh:548-1263) resident in HBM: no host
- * round trip per level.  Dense levels run bottom-up (every unvisited vertex
+ * round trip per level (one per level with the codec, a forced direction or
+ * accounting).  Dense levels run bottom-up (every unvisited vertex
  * stops at its first -- minimum-id -- frontier neighbour), chosen by the
  * direction switch of Beamer et al. (SC'12: bottom-up once the frontier's
  * edges exceed the unexplored edges / 20, top-down again below n / 24
@@ -190,12 +191,17 @@ int g5_bfs_tune(g5_bfs *b, int64_t alpha, int64_t beta);
  * g5_bfs_expand calls:
  * enable (resets the totals), then read total device ms, launches,
  * algorithmic bytes (16 B per frontier vertex, 12 B per frontier edge, 12 B
- * per newly reached vertex) and frontier edges. */
+ * per newly reached vertex) and frontier edges.  While it is enabled the host
+ * drives g5_bfs_run's levels, as it does with the codec or a forced direction,
+ * through these kernels; otherwise the levels are decided on the device by a
+ * kernel that is not accounted.  Results are the same; time a search with
+ * accounting disabled. */
 int g5_bfs_profile(g5_bfs *b, int enable);
 int g5_bfs_stats(g5_bfs *b, double *ms, int64_t *launches, double *bytes, int64_t *edges);
 /* The same per kernel: 0 = k_expand (as g5_bfs_stats), 1 = k_bottom_up (16 B
  * per unvisited vertex scanned, 12 B per neighbour checked, 4 B per newly
- * reached vertex, 16 B per 64-vertex word; edges = neighbours checked). */
+ * reached vertex, 16 B per 64-vertex word, and 4 and 8 B more where the level's
+ * commit is in the same pass, as in g5_bfs_run; edges = neighbours checked). */
 int g5_bfs_kernel_stats(g5_bfs *b, int kernel, double *ms, int64_t *launches, double *bytes, int64_t *edges);
 /* TEPS numerator of the last search: generated undirected edges with a
  * reached endpoint (validate/validate.h:439-485). */
