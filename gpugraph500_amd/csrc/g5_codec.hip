@@ -14,8 +14,9 @@
 //   varint tail of n - L values, deltas restarting at 0, 7-bit groups LSB
 //   first, stop bit on the last byte, zero padded to a word (variablebyte.h).
 //
-// Encode and decode are the same few launches whatever the length, so that a
-// level's queue costs launches in proportion to what depends on what:
+// Encode is two launches and decode four to nine, a hop table more for every
+// factor of 8 in the groups, so that a level's queue costs launches in proportion
+// to what depends on what (short queues, below, one):
 //   k_enc_sizes   widths and, per workgroup's miniblocks, their word total
 //   k_enc_write   each workgroup adds up the totals before its own, packs its
 //                 miniblocks (each lane assembles whole output words from the

@@ -16,8 +16,9 @@
 // leaves its source in the pair's parent slot), then the new (vertex, root)
 // parent slots are lowered with atomicMin over the same edges -- the same
 // minimum-id parent -- or, when the new vertices have fewer edges than the
-// frontier, by a scan of the new vertices' rows (k_min_rows).  A 1-bit-per-vertex active bitmap lets gathers skip vertices with
-// an empty frontier word.
+// frontier, by a scan of the new vertices' rows (both in k_push_min).  A
+// 1-bit-per-vertex active bitmap lets gathers skip vertices with an empty
+// frontier word.
 //
 // Split levels: a pull scan stops only when all of the vertex's unvisited
 // lanes are found, so one lane whose frontier is still small (a root of low
@@ -341,8 +342,8 @@ __device__ __forceinline__ void write_slots(int32_t *__restrict__ parent, uint8_
     }
 }
 
-// the level byte of the pairs the running level reaches (the level number
-// lives in device memory, so captured level graphs replay unchanged)
+// the level byte of the pairs the running level reaches (the level number lives
+// in device memory: k_level_end advances it, a join's k_join reads it)
 __device__ __forceinline__ uint8_t level_byte(const int64_t *__restrict__ cnt) { return (uint8_t)cnt[kDepth]; }
 
 // lane-to-wave broadcast; l must be wave-uniform
@@ -2270,10 +2271,10 @@ unsigned queue_grid(int64_t nwords) { return (unsigned)g5::grid_for(queue_units(
 // only non-zero words of this level's next: listed_in) and the list is short,
 // otherwise whole -- and with the frontier's queue, which the level before
 // left if it pushed.  The edge that makes next[v] non-zero sets v's active
-// bit (a level of many edges after another leaves that to k_queue); k_queue
-// then commits and counts the vertices of that bitmap and leaves
+// bit; k_queue then commits and counts the vertices of that bitmap and leaves
 // their queue, the next level's frontier's, so a push level makes no pass over
-// all n words.  Five launches (19 with separate queue, degree, prefix, count
+// all n words -- but for one of many edges after another push level, whose bitmap
+// k_queue makes from the words (kScanFrac).  Five launches (19 with separate queue, degree, prefix, count
 // and commit passes: with those, a batch of 64 roots at scale 16 and its
 // per-root edge sums were 114 launches and 739 us, without 61 and 614 us).
 int push_level(g5_msbfs *m, hipStream_t s, int p, bool listed_in, bool queue_in, bool prof)

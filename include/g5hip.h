@@ -268,11 +268,12 @@ int g5_msbfs_nedge(g5_msbfs *m, int64_t *nedge);
  * identical in every mode. */
 int g5_msbfs_set_mode(g5_msbfs *m, int mode);
 /* Per-kernel accounting.  Units 0..2 are the pull kernels of the degree bins
- * (0: workgroup per vertex, degree > 2048; 1: wavefront per vertex,
- * 257..2048; 2: thread per vertex, 1..256), unit 3 the push levels and the
- * pushed lanes of split levels.  Enabling runs the bins of pull levels one by one, timed with
- * events (otherwise small graphs' share a launch); bytes are
- * the algorithmic bytes of the unit's launches. */
+ * (0: workgroup per vertex, degrees above G5_TUNE_WAVE_MAX; 1: wavefront per
+ * vertex, degrees from G5_TUNE_THREAD_MAX + 1; 2: thread per vertex; the levels
+ * that G5_TUNE_SPLIT_MAX speaks of bound unit 2 lower), unit 3 the push levels
+ * and the pushed lanes of split levels.  Enabling runs the bins of pull levels
+ * one by one, timed with events (otherwise small graphs' share a launch); bytes
+ * are the algorithmic bytes of the unit's launches. */
 int g5_msbfs_profile(g5_msbfs *m, int enable);
 int g5_msbfs_stats(g5_msbfs *m, int unit, double *ms, int64_t *launches, double *bytes);
 /* Per level of the last profiled run, 12 doubles each: ms of units 0..3 (as
