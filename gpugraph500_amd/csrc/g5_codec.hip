@@ -204,6 +204,7 @@ __device__ int64_t enc_tail_wave(const uint32_t *__restrict__ in, int64_t n, int
     }
     const int64_t tailpos = 4 + 4 * ((nblk + 15) / 16) + pn;
     const int64_t nt = n - L;
+    if (nt == 0) return tailpos;
     for (int k = l; k < kTailBytes; k += 64) bytes[k] = 0;
     wave_sync();
     uint32_t run = 0;
@@ -795,7 +796,7 @@ struct EncSmall {
     uint8_t w[kTile];
     int64_t pos[kTile];
     uint32_t d[kTileWaves][128];
-    int64_t nw;
+    int64_t packed, nw;  // the miniblocks' words, the stream's
 };
 
 // n <= kSmallValues; returns the stream's length to every thread
@@ -804,6 +805,14 @@ __device__ __forceinline__ int64_t enc_small(const uint32_t *in, int64_t n, uint
 {
     const int wv = threadIdx.x >> 6, l = threadIdx.x & 63;
     const int cnt = (int)(n / 128);
+    if (cnt == 0) {  // a tail alone
+        if (wv == 0) {
+            const int64_t nw = enc_tail_wave(in, n, 0, 0, 0, out, s.bytes, l);
+            if (l == 0) s.nw = nw;
+        }
+        __syncthreads();
+        return s.nw;
+    }
     Mini m[kPerWave] = {};
 #pragma unroll
     for (int k = 0; k < kPerWave; ++k)
@@ -818,10 +827,8 @@ __device__ __forceinline__ int64_t enc_small(const uint32_t *in, int64_t n, uint
         const uint32_t words = enc_positions(s.w, 0, s.pos, l);
         wave_sync();
         enc_headers(0, cnt, s.w, s.pos, out, l);
-        if (l == 0) s.nw = words;
+        if (l == 0) s.packed = words;
     }
-    __syncthreads();
-    const int64_t pn = s.nw;
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < kPerWave; ++k) {
@@ -829,7 +836,7 @@ __device__ __forceinline__ int64_t enc_small(const uint32_t *in, int64_t n, uint
         if (q < cnt) enc_pack(m[k], s.w[q], out + 8 + 4 * (q >> 4) + s.pos[q], s.d[wv], l);
     }
     if (wv == kTileWaves - 1) {  // the wave with the fewest miniblocks
-        const int64_t nw = enc_tail_wave(in, n, (int64_t)cnt * 128, cnt, pn, out, s.bytes, l);
+        const int64_t nw = enc_tail_wave(in, n, (int64_t)cnt * 128, cnt, s.packed, out, s.bytes, l);
         if (l == 0) s.nw = nw;
     }
     __syncthreads();
@@ -892,7 +899,7 @@ __device__ __forceinline__ void dec_small(const uint32_t *in, int64_t nwords, in
     }
     __syncthreads();
     err = s.err;
-    if (!err) {
+    if (!err && cnt) {
         if (wv == 0) dec_places(s.words, s.grp, cnt, s.w, s.off, l);
         __syncthreads();
         uint32_t d0[kPerWave], d1[kPerWave];
@@ -952,8 +959,7 @@ __global__ __launch_bounds__(kTileThreads) void k_rt_small(const uint32_t *in, i
     __shared__ DecSmall sd;
     const int64_t nw = enc_small(in, n, words, se);
     if (threadIdx.x == 0) *nw_out = nw;
-    __threadfence();  // the words are read back below, by other waves
-    __syncthreads();
+    // enc_small's last barrier lets the workgroup's other waves read the words
     dec_small(words, nw, n, out, n, flag, meta, host, sd);
 }
 
